@@ -4,10 +4,9 @@
 // FP32 master weights are rounded to bfloat16 (nearest even) for every matrix
 // product and activations are rounded to bfloat16 on input to a product;
 // accumulation is FP32.  Inference runs on the matrix cores (bf16 MFMA, 16 samples
-// per tile).  Training: per 64-sample block the backward pass keeps pre-activations and
-// deltas in LDS and forms the weight gradients as sample reductions; per-block
-// partial gradients are summed in a fixed order by the Adam kernel, so training
-// is bitwise reproducible.
+// per tile), and so does training (bf16 MFMA forward, FP32 MFMA deltas and weight
+// gradients); per-block partial gradients are summed in a fixed order by the Adam
+// kernel, so training is bitwise reproducible.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -42,40 +41,6 @@ __device__ inline float gelu(float z) {
     const float t = tanhf(C_GELU * (z + 0.044715f * z * z * z));
     return 0.5f * z * (1.f + t);
 }
-__device__ inline float gelu_d(float z) {
-    const float u = C_GELU * (z + 0.044715f * z * z * z);
-    const float t = tanhf(u);
-    const float du = C_GELU * (1.f + 3.f * 0.044715f * z * z);
-    return 0.5f * (1.f + t) + 0.5f * z * (1.f - t * t) * du;
-}
-
-// one hidden layer: z[o] = b[o] + sum_i bf16(h[i]) * wq[i][o]
-template <int NIN>
-__device__ inline void layer(const float* __restrict__ wq, const float* __restrict__ h, float* z) {
-    float hb[NIN];
-#pragma unroll
-    for (int i = 0; i < NIN; ++i) hb[i] = bf16r(h[i]);
-#pragma unroll
-    for (int o = 0; o < MH; ++o) {
-        float s = wq[NIN * MH + o];  // bias follows the weight block
-#pragma unroll
-        for (int i = 0; i < NIN; ++i) s = fmaf(hb[i], wq[i * MH + o], s);
-        z[o] = s;
-    }
-}
-
-__device__ inline void head(const float* __restrict__ wq, const float* h, float* y) {
-    float hb[MH];
-#pragma unroll
-    for (int i = 0; i < MH; ++i) hb[i] = bf16r(h[i]);
-#pragma unroll
-    for (int o = 0; o < MO; ++o) {
-        float s = wq[O_B4 + o];
-#pragma unroll
-        for (int i = 0; i < MH; ++i) s = fmaf(hb[i], wq[O_W4 + i * MO + o], s);
-        y[o] = s;
-    }
-}
 
 // ---- inference on the matrix cores -------------------------------------------------
 // v_mfma_f32_16x16x16_bf16 with the hidden units as rows and 16 samples as columns.
@@ -85,8 +50,7 @@ __device__ inline void head(const float* __restrict__ wq, const float* h, float*
 // therefore the B operand of K-step kt = mt of the next layer, lane for lane: the
 // activations never leave registers.  Each wave holds every weight as A fragments
 // (80 VGPRs) and sweeps 16-sample tiles; products of bfloat16 operands are exact in
-// FP32 and accumulate in FP32, so only the summation order differs from the
-// sample-per-lane forward pass of the training kernel below.
+// FP32 and accumulate in FP32.
 typedef short bf16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -199,128 +163,344 @@ __global__ void k_mfma_probe_bf16(const float* A, const float* B, float* out) {
     for (int i = 0; i < 4; ++i) out[l * 4 + i] = d[i];
 }
 
-// backward of one 64-sample block: partial gradient (NPARAM) and partial loss sum
-__global__ __launch_bounds__(64) void k_mlp_backward(int n, int nscale, const float* __restrict__ X,
-                                                     const float* __restrict__ T, const float* __restrict__ wq,
-                                                     float* __restrict__ partial, float* __restrict__ lossp) {
-    // [layer][unit][sample], rows padded to 65 words so that lanes reading one
-    // sample column of different units hit different banks
-    __shared__ float sZ[3][MH][65];   // pre-activations; after the deltas, bf16(gelu(z))
-    __shared__ float sD[3][MH][65];   // deltas of the hidden layers
-    __shared__ float sX[MI][65];
-    __shared__ float sY[MO][65];      // output deltas
-    const int s = threadIdx.x;
-    const int gs = blockIdx.x * 64 + s;
-    const bool ok = gs < n;
-    float x[MI], a[MH], b[MH];
-#pragma unroll
-    for (int i = 0; i < MI; ++i) x[i] = ok ? X[(size_t)gs * MI + i] : 0.f;
-#pragma unroll
-    for (int i = 0; i < MI; ++i) sX[i][s] = x[i];
-    layer<MI>(wq + O_W1, x, a);
-#pragma unroll
-    for (int j = 0; j < MH; ++j) { sZ[0][j][s] = a[j]; a[j] = gelu(a[j]); }
-    layer<MH>(wq + O_W2, a, b);
-#pragma unroll
-    for (int j = 0; j < MH; ++j) { sZ[1][j][s] = b[j]; b[j] = gelu(b[j]); }
-    layer<MH>(wq + O_W3, b, a);
-#pragma unroll
-    for (int j = 0; j < MH; ++j) { sZ[2][j][s] = a[j]; a[j] = gelu(a[j]); }
-    float y[MO];
-    head(wq, a, y);
-    float dy[MO], l = 0.f;
-#pragma unroll
-    for (int o = 0; o < MO; ++o) {
-        const float d = ok ? y[o] - T[(size_t)gs * MO + o] : 0.f;
-        l += d * d;
-        dy[o] = 2.f * d / (float)nscale;
-        sY[o][s] = dy[o];
-    }
-    // hidden deltas: dz3 = W4 dy * g'(z3); dz2 = W3 dz3 * g'(z2); dz1 = W2 dz2 * g'(z1)
-#pragma unroll
-    for (int j = 0; j < MH; ++j) {
-        float t = 0.f;
-#pragma unroll
-        for (int o = 0; o < MO; ++o) t = fmaf(wq[O_W4 + j * MO + o], dy[o], t);
-        a[j] = t * gelu_d(sZ[2][j][s]);
-        sD[2][j][s] = a[j];
-    }
-#pragma unroll
-    for (int i = 0; i < MH; ++i) {
-        float t = 0.f;
-#pragma unroll
-        for (int j = 0; j < MH; ++j) t = fmaf(wq[O_W3 + i * MH + j], a[j], t);
-        b[i] = t * gelu_d(sZ[1][i][s]);
-        sD[1][i][s] = b[i];
-    }
-#pragma unroll
-    for (int i = 0; i < MH; ++i) {
-        float t = 0.f;
-#pragma unroll
-        for (int j = 0; j < MH; ++j) t = fmaf(wq[O_W2 + i * MH + j], b[j], t);
-        sD[0][i][s] = t * gelu_d(sZ[0][i][s]);
-    }
-    // the weight gradients need the (rounded) activations, not the pre-activations;
-    // each lane converts its own sample column
-#pragma unroll
-    for (int L = 0; L < 3; ++L)
-#pragma unroll
-        for (int j = 0; j < MH; ++j) sZ[L][j][s] = bf16r(gelu(sZ[L][j][s]));
-    // block loss
-    for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off, 64);
-    if (s == 0) lossp[blockIdx.x] = l;
-    __syncthreads();
-    // weight gradients: sample reductions, one parameter per lane per pass
-    float* P = partial + (size_t)blockIdx.x * NPARAM;
-    for (int p = s; p < NPARAM; p += 64) {
-        float g = 0.f;
-        if (p < O_B1) {                       // W1[i][j]
-            const int i = p / MH, j = p % MH;
-            for (int k = 0; k < 64; ++k) g = fmaf(bf16r(sX[i][k]), sD[0][j][k], g);
-        } else if (p < O_W2) {                // b1
-            const int j = p - O_B1;
-            for (int k = 0; k < 64; ++k) g += sD[0][j][k];
-        } else if (p < O_B2) {                // W2[i][j]: h1 = bf16(gelu(z1))
-            const int q = p - O_W2, i = q / MH, j = q % MH;
-            for (int k = 0; k < 64; ++k) g = fmaf(sZ[0][i][k], sD[1][j][k], g);
-        } else if (p < O_W3) {
-            const int j = p - O_B2;
-            for (int k = 0; k < 64; ++k) g += sD[1][j][k];
-        } else if (p < O_B3) {                // W3[i][j]: h2 = bf16(gelu(z2))
-            const int q = p - O_W3, i = q / MH, j = q % MH;
-            for (int k = 0; k < 64; ++k) g = fmaf(sZ[1][i][k], sD[2][j][k], g);
-        } else if (p < O_W4) {
-            const int j = p - O_B3;
-            for (int k = 0; k < 64; ++k) g += sD[2][j][k];
-        } else if (p < O_B4) {                // W4[i][o]: h3 = bf16(gelu(z3))
-            const int q = p - O_W4, i = q / MO, o = q % MO;
-            for (int k = 0; k < 64; ++k) g = fmaf(sZ[2][i][k], sY[o][k], g);
-        } else {
-            const int o = p - O_B4;
-            for (int k = 0; k < 64; ++k) g += sY[o][k];
-        }
-        P[p] = g;
-    }
+// ---- training step on the matrix cores ----------------------------------------------
+// Forward, backward and weight gradients of 16-sample tiles, one tile per wave at a time;
+// a wave keeps its sums of all 9 673 gradient entries in registers over its tiles, the
+// block adds its four waves in a fixed order and writes one partial, so a minibatch of
+// 65 536 samples writes 256 partials (the card's CUs) instead of one per 64 samples.
+//   forward: the tiles of k_mlp_forward_mfma (bf16 products, FP32 accumulation);
+//   deltas:  dz_l = (W_{l+1} dz_{l+1}) * gelu'(z_l) on v_mfma_f32_16x16x4f32.  The deltas
+//            stay FP32 (the bf16 weights are exact in FP32); register i of output tile mt
+//            holds unit 16 mt + 4 q + i, which is K-step (mt, i) of the next product;
+//   weight gradients h_l^T dz_{l+1} contract over the samples, which sit in the lane
+//            columns, so h and dz go through a transposed copy in LDS (row = unit, 16
+//            samples, padded to 20 words: a lane's four samples are one 16-byte read, no
+//            bank conflicts); v_mfma_f32_16x16x4f32 again.
+// Bound: the FP32 matrix cores (304 instructions of 32 cycles per tile) and, near it, the
+// 48 tanh per lane.  65 536 samples: 1 903 us for the sample-per-lane form with a
+// reduction per parameter before it, 98 us now.
+typedef float f4_t __attribute__((ext_vector_type(4)));
+
+__device__ inline f4_t mfma_f32(float a, float b, f4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ inline float bf16_value(short b) {
+    const unsigned u = (unsigned)(unsigned short)b << 16;
+    return __uint_as_float(u);
 }
 
-// gradient = ordered sum of the block partials; optional Adam step on the masters
-__global__ void k_mlp_reduce_adam(int nblocks, const float* __restrict__ partial, float* __restrict__ grad,
-                                  float* master, float* wq, float* m1, float* m2, float lr, float bc1, float bc2,
-                                  int do_step) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= NPARAM) return;
-    float g = 0.f;
-    for (int b = 0; b < nblocks; ++b) g += partial[(size_t)b * NPARAM + p];
+constexpr int TRAIN_BLOCKS = 256;         // partials of a minibatch at most: one block per CU
+constexpr int TW = 68, TS = 20;           // LDS row strides (words): weights, transposed tiles
+constexpr int LW2 = 0, LW3 = LW2 + MH * TW, LW4 = LW3 + MH * TW;         // FP32 weights by row
+constexpr int LFW = LW4 + MH * TS;                                      // bf16 A fragments, 2 words a lane
+constexpr int NFRAG = 40;                                               // 4 + 16 + 16 + 4
+constexpr int LWAVE = LFW + NFRAG * 64 * 2;                             // per-wave tiles from here
+constexpr int WTILE = 2 * MH * TS + 2 * 16 * TS;                        // h, dz, x, dy
+constexpr int TRAIN_LDS = LWAVE + 4 * WTILE;
+static_assert(NPARAM <= LWAVE, "the block's gradient sums reuse the weights' LDS");
+static_assert(TRAIN_LDS * 4 <= 160 * 1024, "LDS of one CU");
+
+// gelu(z) as bfloat16 bits (the B operands of the next layer) and gelu'(z) in place of z
+__device__ inline void gelu_and_slope(f32x4_t z[4], bf16x4_t h[4]) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float v = z[t][j];
+            const float th = tanhf(C_GELU * (v + 0.044715f * v * v * v));
+            const float du = C_GELU * (1.f + 3.f * 0.044715f * v * v);
+            h[t][j] = bf16_bits(0.5f * v * (1.f + th));
+            z[t][j] = 0.5f * (1.f + th) + 0.5f * v * (1.f - th * th) * du;
+        }
+}
+
+// orders this wave's LDS writes before its reads of other lanes' values
+__device__ inline void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__global__ __launch_bounds__(256) void k_mlp_train_mfma(int n, int nscale, const float* __restrict__ X,
+                                                        const float* __restrict__ T, const float* __restrict__ wq,
+                                                        float* __restrict__ partial, float* __restrict__ lossp) {
+    __shared__ __align__(16) float sm[TRAIN_LDS];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, q = lane >> 4, c = lane & 15;
+    for (int k = threadIdx.x; k < MH * MH; k += 256) {
+        const int i = k / MH, j = k % MH;
+        sm[LW2 + i * TW + j] = wq[O_W2 + k];
+        sm[LW3 + i * TW + j] = wq[O_W3 + k];
+    }
+    for (int k = threadIdx.x; k < MH * 16; k += 256) {
+        const int i = k >> 4, o = k & 15;
+        sm[LW4 + i * TS + o] = o < MO ? wq[O_W4 + i * MO + o] : 0.f;
+    }
+    bf16x4_t* const frag = reinterpret_cast<bf16x4_t*>(sm + LFW);
+    for (int k = threadIdx.x; k < NFRAG * 64; k += 256) {
+        const int f = k >> 6, l = k & 63, lq = l >> 4, lc = l & 15;
+        bf16x4_t v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float x;
+            if (f < 4) {
+                const int i = 4 * lq + j;
+                x = i < MI ? wq[O_W1 + i * MH + 16 * f + lc] : 0.f;
+            } else if (f < 36) {
+                const int g = (f - 4) & 15, i = 16 * (g & 3) + 4 * lq + j;
+                x = wq[(f < 20 ? O_W2 : O_W3) + i * MH + 16 * (g >> 2) + lc];
+            } else {
+                const int i = 16 * (f - 36) + 4 * lq + j;
+                x = lc < MO ? wq[O_W4 + i * MO + lc] : 0.f;
+            }
+            v[j] = bf16_bits(x);
+        }
+        frag[k] = v;
+    }
+    __syncthreads();
+
+    float* const sh = sm + LWAVE + w * WTILE;   // h of a layer, then
+    float* const sd = sh + MH * TS;             // deltas of the layer above it
+    float* const sx = sd + MH * TS;             // bf16(x), rows 11.. zero
+    float* const sy = sx + 16 * TS;             // output deltas, rows 9.. zero
+    const f4_t z0 = {0.f, 0.f, 0.f, 0.f};
+    f4_t g2[4][4], g3[4][4], g1[4], g4[4];
+    float gb1[4], gb2[4], gb3[4], gb4 = 0.f, loss = 0.f;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        g1[a] = z0; g4[a] = z0; gb1[a] = gb2[a] = gb3[a] = 0.f;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) { g2[a][b] = z0; g3[a][b] = z0; }
+    }
+    // rows of unit 16 t + c, samples 4 q .. 4 q + 3 of a transposed tile
+    auto row = [&](const float* s, int t) { return *reinterpret_cast<const f4_t*>(s + (16 * t + c) * TS + 4 * q); };
+    auto put_h = [&](const bf16x4_t* h) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sh[(16 * t + 4 * q + i) * TS + c] = bf16_value(h[t][i]);
+    };
+    auto put_d = [&](const f4_t* d) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sd[(16 * t + 4 * q + i) * TS + c] = d[t][i];
+    };
+    // sum over the tile's samples of h (64 rows) x d (64 columns); bias sums of d
+    auto outer = [&](f4_t g[4][4], float* gb) {
+        f4_t d[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            d[b] = row(sd, b);
+            gb[b] += (d[b][0] + d[b][1]) + (d[b][2] + d[b][3]);
+        }
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const f4_t h = row(sh, a);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) g[a][b] = mfma_f32(h[k], d[b][k], g[a][b]);
+        }
+    };
+    // (W d) * slope, W rows in LDS at lw: the deltas of the layer below
+    auto back = [&](int lw, const f4_t* d, const f32x4_t* slope, f4_t* out) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[r] = z0;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            f4_t a[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                a[r] = *reinterpret_cast<const f4_t*>(sm + lw + (16 * r + c) * TW + 16 * t + 4 * q);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) out[r] = mfma_f32(a[r][i], d[t][i], out[r]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) out[r][i] *= slope[r][i];
+    };
+
+    const int ntile = (n + 15) / 16;
+    for (int tile = blockIdx.x * 4 + w; tile < ntile; tile += gridDim.x * 4) {
+        const int s = tile * 16 + c;
+        const bool ok = s < n;
+        bf16x4_t hx, h1[4], h2[4], h3[4];
+        f32x4_t s1[4], s2[4], s3[4];   // pre-activations, then gelu'
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int k = 4 * q + j;
+            hx[j] = (ok && k < MI) ? bf16_bits(X[(size_t)s * MI + k]) : (short)0;
+            sx[k * TS + c] = bf16_value(hx[j]);
+        }
+        auto bias = [&](int o, int t) {
+            f32x4_t b;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) b[i] = wq[o + 16 * t + 4 * q + i];
+            return b;
+        };
+#pragma unroll
+        for (int t = 0; t < 4; ++t) s1[t] = mfma_bf16(frag[t * 64 + lane], hx, bias(O_B1, t));
+        gelu_and_slope(s1, h1);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            s2[t] = bias(O_B2, t);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s2[t] = mfma_bf16(frag[(4 + 4 * t + k) * 64 + lane], h1[k], s2[t]);
+        }
+        gelu_and_slope(s2, h2);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            s3[t] = bias(O_B3, t);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s3[t] = mfma_bf16(frag[(20 + 4 * t + k) * 64 + lane], h2[k], s3[t]);
+        }
+        gelu_and_slope(s3, h3);
+        f32x4_t y;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[i] = 4 * q + i < MO ? wq[O_B4 + 4 * q + i] : 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) y = mfma_bf16(frag[(36 + k) * 64 + lane], h3[k], y);
+        f4_t dy;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int o = 4 * q + i;
+            const float d = (ok && o < MO) ? y[i] - T[(size_t)s * MO + o] : 0.f;
+            loss += d * d;
+            dy[i] = 2.f * d / (float)nscale;
+            sy[o * TS + c] = dy[i];
+        }
+        // dz3 and the gradients of the output layer
+        f4_t da[4], db[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const f4_t a = *reinterpret_cast<const f4_t*>(sm + LW4 + (16 * r + c) * TS + 4 * q);
+            f4_t t = z0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) t = mfma_f32(a[i], dy[i], t);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) da[r][i] = t[i] * s3[r][i];
+        }
+        put_h(h3);
+        wave_lds_sync();
+        {
+            const f4_t d = row(sy, 0);
+            gb4 += (d[0] + d[1]) + (d[2] + d[3]);
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const f4_t h = row(sh, a);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) g4[a] = mfma_f32(h[k], d[k], g4[a]);
+            }
+        }
+        wave_lds_sync();
+        put_h(h2);
+        put_d(da);
+        wave_lds_sync();
+        outer(g3, gb3);
+        back(LW3, da, s2, db);
+        wave_lds_sync();
+        put_h(h1);
+        put_d(db);
+        wave_lds_sync();
+        outer(g2, gb2);
+        back(LW2, db, s1, da);
+        wave_lds_sync();
+        put_d(da);
+        wave_lds_sync();
+        {
+            const f4_t x = row(sx, 0);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const f4_t d = row(sd, b);
+                gb1[b] += (d[0] + d[1]) + (d[2] + d[3]);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) g1[b] = mfma_f32(x[k], d[k], g1[b]);
+            }
+        }
+        wave_lds_sync();
+    }
+    // block sums: waves 0..3 in order, in the weights' LDS; accumulator register i of lane
+    // (q, c) is row 4 q + i, column c of its tile
+    auto quarter = [&](float v) {   // over the four lane groups (the samples of a tile)
+        v += __shfl_xor(v, 16, 64);
+        return v + __shfl_xor(v, 32, 64);
+    };
+#pragma unroll
+    for (int a = 0; a < 4; ++a) { gb1[a] = quarter(gb1[a]); gb2[a] = quarter(gb2[a]); gb3[a] = quarter(gb3[a]); }
+    gb4 = quarter(gb4);
+    for (int off = 32; off > 0; off >>= 1) loss += __shfl_down(loss, off, 64);
+    for (int turn = 0; turn < 4; ++turn) {
+        __syncthreads();
+        if (turn != w) continue;
+        auto add = [&](int p, float v) { sm[p] = w == 0 ? v : sm[p] + v; };
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = 16 * a + 4 * q + i;
+                if (4 * q + i < MI) add(O_W1 + (4 * q + i) * MH + 16 * a + c, g1[a][i]);
+                if (c < MO) add(O_W4 + r * MO + c, g4[a][i]);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    add(O_W2 + r * MH + 16 * b + c, g2[a][b][i]);
+                    add(O_W3 + r * MH + 16 * b + c, g3[a][b][i]);
+                }
+            }
+            if (q == 0) {
+                add(O_B1 + 16 * a + c, gb1[a]);
+                add(O_B2 + 16 * a + c, gb2[a]);
+                add(O_B3 + 16 * a + c, gb3[a]);
+            }
+        }
+        if (q == 0 && c < MO) add(O_B4 + c, gb4);
+        if (lane == 0) sm[LWAVE] = w == 0 ? loss : sm[LWAVE] + loss;
+    }
+    __syncthreads();
+    float* const P = partial + (size_t)blockIdx.x * NPARAM;
+    for (int p = threadIdx.x; p < NPARAM; p += 256) P[p] = sm[p];
+    if (threadIdx.x == 0) lossp[blockIdx.x] = sm[LWAVE];
+}
+
+// gradient = sum of the block partials in a fixed order (four lanes a quarter of the
+// partials each, then the quarters in order); optional Adam step on the masters.  64
+// parameters per block: 151 blocks keep the 38 KB partials streaming (242 us for 1 024
+// partials with one lane per parameter before, 8 us for 256 now).  lsum (may
+// be null) accumulates the minibatch's loss sum.
+__global__ __launch_bounds__(256) void k_mlp_reduce_adam(int nblocks, const float* __restrict__ partial,
+                                                         float* __restrict__ grad, float* master, float* wq,
+                                                         float* m1, float* m2, float lr, float bc1, float bc2,
+                                                         int do_step, const float* __restrict__ lossp, double* lsum) {
+    __shared__ float part[4][64];
+    const int j = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + j;
+    const int per = (nblocks + 3) / 4, b0 = w * per, b1 = min(nblocks, b0 + per);
+    float s = 0.f;
+    if (p < NPARAM) {
+#pragma unroll 8
+        for (int b = b0; b < b1; ++b) s += partial[(size_t)b * NPARAM + p];
+    }
+    part[w][j] = s;
+    __syncthreads();
+    if (lsum && blockIdx.x == 0 && threadIdx.x == 64) {
+        double l = lsum[0];
+        for (int b = 0; b < nblocks; ++b) l += lossp[b];
+        lsum[0] = l;
+    }
+    if (w != 0 || p >= NPARAM) return;
+    const float g = ((part[0][j] + part[1][j]) + part[2][j]) + part[3][j];
     grad[p] = g;
     if (!do_step) return;
     const float a = 0.9f * m1[p] + 0.1f * g;
     const float v = 0.999f * m2[p] + 0.001f * g * g;
     m1[p] = a;
     m2[p] = v;
-    const float w = master[p] - lr * (a / bc1) / (sqrtf(v / bc2) + 1e-8f);
-    master[p] = w;
+    const float x = master[p] - lr * (a / bc1) / (sqrtf(v / bc2) + 1e-8f);
+    master[p] = x;
     const bool is_bias = (p >= O_B1 && p < O_W2) || (p >= O_B2 && p < O_W3) || (p >= O_B3 && p < O_W4) || p >= O_B4;
-    wq[p] = is_bias ? w : bf16r(w);
+    wq[p] = is_bias ? x : bf16r(x);
 }
 
 // mean-square loss from the block losses: the same double sum, in block order, and
@@ -333,7 +513,8 @@ __global__ void k_mlp_loss_sum(int nblocks, const float* __restrict__ lossp, int
 }
 
 // Scratch of the allocation-free loss/gradient entry point: the per-block partial
-// gradients (NPARAM floats per 64-sample block) followed by the block losses.  One
+// gradients (NPARAM floats per block of k_mlp_train_mfma, room for one block per 64
+// samples) followed by the block losses.  One
 // copy per GPU, held until the process ends; host code uses the address that
 // hipGetSymbolAddress returns for the current device, never the symbol itself.
 // Every call overwrites what it reads (each block writes all of its partials and
@@ -351,12 +532,14 @@ struct hpg_mlp {
     hipStream_t stream = nullptr;
     float *master = nullptr, *wq = nullptr, *m1 = nullptr, *m2 = nullptr, *grad = nullptr;
     float *partial = nullptr, *lossp = nullptr, *X = nullptr, *T = nullptr, *Y = nullptr;
+    double* lsum = nullptr;  // loss sum of a training run's last epoch
     int cap_blocks = 0, cap_n = 0, step = 0;
     int dev = 0;  // device the MLP was created on
     std::string err;
     ~hpg_mlp() {
         for (float* p : {master, wq, m1, m2, grad, partial, lossp, X, T, Y})
             if (p) hipFree(p);
+        if (lsum) hipFree(lsum);
         if (stream) hipStreamDestroy(stream);
     }
 };
@@ -400,14 +583,18 @@ void resolve_scratch(int dev) {
     g_scratch[dev] = static_cast<float*>(p);
 }
 
+// blocks (= partials) of a minibatch: at least one 16-sample tile per wave, one block per
+// CU at most, so larger minibatches give each wave more tiles instead of more partials
+int train_blocks(int n) { return std::max(1, std::min((n + 63) / 64, TRAIN_BLOCKS)); }
+
 // enqueue the backward pass of n samples (block partials and block losses into
 // partial / lossp) and the ordered gradient sum into grad, no weight update
 void enqueue_loss_grad(hpg_mlp* m, const float* X, const float* T, int n, float* partial, float* lossp,
                        float* grad) {
-    const int nb = (n + 63) / 64;
-    hipLaunchKernelGGL(k_mlp_backward, dim3(nb), dim3(64), 0, m->stream, n, n * MO, X, T, m->wq, partial, lossp);
-    hipLaunchKernelGGL(k_mlp_reduce_adam, dim3((NPARAM + 255) / 256), dim3(256), 0, m->stream, nb, partial, grad,
-                       m->master, m->wq, m->m1, m->m2, 0.f, 1.f, 1.f, 0);
+    const int nb = train_blocks(n);
+    hipLaunchKernelGGL(k_mlp_train_mfma, dim3(nb), dim3(256), 0, m->stream, n, n * MO, X, T, m->wq, partial, lossp);
+    hipLaunchKernelGGL(k_mlp_reduce_adam, dim3((NPARAM + 63) / 64), dim3(256), 0, m->stream, nb, partial, grad,
+                       m->master, m->wq, m->m1, m->m2, 0.f, 1.f, 1.f, 0, (const float*)nullptr, (double*)nullptr);
 }
 
 void ensure_blocks(hpg_mlp* m, int nb) {
@@ -440,6 +627,7 @@ int hpg_mlp_create(unsigned seed, hpg_mlp** out) {
         resolve_scratch(m->dev);
         ck(hipStreamCreate(&m->stream), "hipStreamCreate");
         for (float** p : {&m->master, &m->wq, &m->m1, &m->m2, &m->grad}) ck(hipMalloc(p, NPARAM * 4), "hipMalloc");
+        ck(hipMalloc(&m->lsum, sizeof(double)), "hipMalloc");
         ck(hipMemsetAsync(m->m1, 0, NPARAM * 4, m->stream), "memset");
         ck(hipMemsetAsync(m->m2, 0, NPARAM * 4, m->stream), "memset");
         // He-style uniform init from a fixed LCG, biases zero
@@ -523,7 +711,7 @@ int hpg_mlp_loss_grad(hpg_mlp* m, const float* X, const float* T, int n, float* 
     if (!m || !X || !T || n <= 0) return -2;
     try {
         ensure_n(m, n);
-        const int nb = (n + 63) / 64;
+        const int nb = train_blocks(n);
         ensure_blocks(m, nb);
         ck(hipMemcpyAsync(m->X, X, (size_t)n * MI * 4, hipMemcpyHostToDevice, m->stream), "H2D");
         ck(hipMemcpyAsync(m->T, T, (size_t)n * MO * 4, hipMemcpyHostToDevice, m->stream), "H2D");
@@ -545,8 +733,7 @@ int hpg_mlp_loss_grad(hpg_mlp* m, const float* X, const float* T, int n, float* 
 // summation order as hpg_mlp_loss_grad, so loss and gradient are bitwise equal.
 int hpg_mlp_loss_grad_noalloc(hpg_mlp* m, const float* X, const float* T, int n, float* loss, float* grad) {
     if (!m || !X || !T || !loss || !grad || n <= 0) return -2;
-    const int nb = (n + 63) / 64;
-    if (nb > NOALLOC_MAX_BLOCKS) {
+    if ((n + 63) / 64 > NOALLOC_MAX_BLOCKS) {
         m->err = "hpg_mlp_loss_grad_noalloc: n exceeds the scratch capacity of " +
                  std::to_string(HPG_MLP_NOALLOC_MAX_SAMPLES) + " samples";
         return -2;
@@ -554,6 +741,7 @@ int hpg_mlp_loss_grad_noalloc(hpg_mlp* m, const float* X, const float* T, int n,
     try {
         float* sp = (m->dev >= 0 && m->dev < MAX_DEVICES) ? g_scratch[m->dev] : nullptr;
         if (!sp) throw std::runtime_error("scratch address not resolved for this device");
+        const int nb = train_blocks(n);
         float* lossp = sp + (size_t)nb * NPARAM;
         enqueue_loss_grad(m, X, T, n, sp, lossp, grad);
         hipLaunchKernelGGL(k_mlp_loss_sum, dim3(1), dim3(64), 0, m->stream, nb, lossp, n * MO, loss);
@@ -570,29 +758,26 @@ int hpg_mlp_train(hpg_mlp* m, const float* X, const float* T, int n, int epochs,
     try {
         ensure_n(m, n);
         batch = ((batch + 63) / 64) * 64;
-        ensure_blocks(m, batch / 64);
+        ensure_blocks(m, train_blocks(std::min(batch, n)));
         ck(hipMemcpyAsync(m->X, X, (size_t)n * MI * 4, hipMemcpyHostToDevice, m->stream), "H2D");
         ck(hipMemcpyAsync(m->T, T, (size_t)n * MO * 4, hipMemcpyHostToDevice, m->stream), "H2D");
         double lsum = 0.0;
-        std::vector<float> lp(batch / 64);
+        ck(hipMemcpyAsync(m->lsum, &lsum, sizeof(double), hipMemcpyHostToDevice, m->stream), "H2D");
         for (int ep = 0; ep < epochs; ++ep) {
-            lsum = 0.0;
             for (int b0 = 0; b0 < n; b0 += batch) {
-                const int nb_s = std::min(batch, n - b0), nb = (nb_s + 63) / 64;
+                const int nb_s = std::min(batch, n - b0), nb = train_blocks(nb_s);
                 ++m->step;
                 const float bc1 = 1.f - std::pow(0.9f, (float)m->step), bc2 = 1.f - std::pow(0.999f, (float)m->step);
-                hipLaunchKernelGGL(k_mlp_backward, dim3(nb), dim3(64), 0, m->stream, nb_s, nb_s * MO,
+                hipLaunchKernelGGL(k_mlp_train_mfma, dim3(nb), dim3(256), 0, m->stream, nb_s, nb_s * MO,
                                    m->X + (size_t)b0 * MI, m->T + (size_t)b0 * MO, m->wq, m->partial, m->lossp);
-                hipLaunchKernelGGL(k_mlp_reduce_adam, dim3((NPARAM + 255) / 256), dim3(256), 0, m->stream, nb,
-                                   m->partial, m->grad, m->master, m->wq, m->m1, m->m2, lr, bc1, bc2, 1);
-                if (ep == epochs - 1) {
-                    ck(hipMemcpyAsync(lp.data(), m->lossp, nb * 4, hipMemcpyDeviceToHost, m->stream), "D2H");
-                    ck(hipStreamSynchronize(m->stream), "sync");
-                    for (int k = 0; k < nb; ++k) lsum += lp[k];
-                }
+                // the last epoch's loss accumulates on the device: nothing waits between steps
+                hipLaunchKernelGGL(k_mlp_reduce_adam, dim3((NPARAM + 63) / 64), dim3(256), 0, m->stream, nb,
+                                   m->partial, m->grad, m->master, m->wq, m->m1, m->m2, lr, bc1, bc2, 1, m->lossp,
+                                   ep == epochs - 1 ? m->lsum : nullptr);
             }
             ck(hipGetLastError(), "train launch");
         }
+        ck(hipMemcpyAsync(&lsum, m->lsum, sizeof(double), hipMemcpyDeviceToHost, m->stream), "D2H");
         ck(hipStreamSynchronize(m->stream), "sync");
         if (last) *last = (float)(lsum / ((double)n * MO));
     } catch (const std::exception& e) { m->err = e.what(); return -1; }
