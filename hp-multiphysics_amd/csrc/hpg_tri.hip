@@ -1233,8 +1233,9 @@ struct CallBuffers {
     }
 };
 
-template <int P, int NVn>
-void jacobian_colour(hpg_ctx* c, const JacArgs& ja, int N) {
+// cns: one column of a colour's batch elements at a time, through the global state
+template <int P>
+void jacobian_colour_cns(hpg_ctx* c, const JacArgs& ja, int N) {
     const int nel = ja.end - ja.begin;
     const dim3 b1(nblk(nel, 64)), t1(64), bN(nblk((long)nel * N)), tN(256);
     const Level& L = c->lv[c->log2p];
@@ -1244,38 +1245,54 @@ void jacobian_colour(hpg_ctx* c, const JacArgs& ja, int N) {
     // keyed to colour 0 here, not to the elements' own colour; that does not matter:
     // every scratch entry starts at zero, so both lftog paths store lf_re + lf_im
     const std::vector<int> offs = {ja.begin, ja.end};
-    hipLaunchKernelGGL(k_jac_dw<NVn>, b1, t1, 0, c->stream, ja);
+    hipLaunchKernelGGL(k_jac_dw<NVC>, b1, t1, 0, c->stream, ja);
     for (int col = -1; col < N; ++col) {
         JacArgs a = ja;
-        a.mode = col < 0 ? -1 : col / NVn;
-        a.var = col < 0 ? 0 : col % NVn;
-        if (col >= 0) hipLaunchKernelGGL((k_jac_perturb<P, NVn>), b1, t1, 0, c->stream, a);
-        if (c->physics == HPG_PHYSICS_CNS) {
-            CnsElemArgs e;
-            e.pnts = c->pnts; e.tri_pnt = c->tri_pnt; e.tri_seg = c->tri_seg; e.tri_sgn = c->tri_sgn;
-            e.order = ja.jel; e.begin = 0; e.end = 0;
-            e.ugv = c->ugv; e.ugs = c->ugs; e.ugi = c->ugi;
-            e.resv = ja.jrv; e.ress = ja.jrs; e.resi = ja.jri;
-            e.rrv = ja.jqv; e.rrs = ja.jqs; e.rri = ja.jqi;
-            e.ops = L.cpack; e.sm0 = c->sm0; e.im0 = c->im0;
-            e.ph = c->cph; e.beta = beta; e.keep = 0.0;
-            e.fcv = c->fcv; e.fcs = c->fcs; e.colour = 0;
-            launch_elem_cns<P>(c, e, full, &offs);
-        } else {
-            ElemArgs e{};
-            e.pnts = c->pnts; e.tri_pnt = c->tri_pnt; e.tri_seg = c->tri_seg; e.tri_sgn = c->tri_sgn;
-            e.order = ja.jel; e.begin = 0; e.end = 0;
-            e.ugv = c->ugv; e.ugs = c->ugs; e.ugi = c->ugi;
-            e.resv = ja.jrv; e.ress = ja.jrs; e.resi = ja.jri;
-            e.rrv = ja.jqv; e.rrs = ja.jqs; e.rri = ja.jqi;
-            e.ops = L.pack; e.sm0 = c->sm0; e.im0 = c->im0;
-            e.rho = c->prm.rho; e.mu = c->prm.mu; e.adis = c->prm.adis; e.beta = beta;
-            e.fcv = c->fcv; e.fcs = c->fcs; e.colour = 0; e.keep = 0.0;
-            e.lin = nullptr; e.gbase = 0;
-            launch_elem<P>(c, e, full, &offs);
-        }
-        hipLaunchKernelGGL((k_jac_collect<P, NVn>), bN, tN, 0, c->stream, a);
+        a.mode = col < 0 ? -1 : col / NVC;
+        a.var = col < 0 ? 0 : col % NVC;
+        if (col >= 0) hipLaunchKernelGGL((k_jac_perturb<P, NVC>), b1, t1, 0, c->stream, a);
+        CnsElemArgs e;
+        e.pnts = c->pnts; e.tri_pnt = c->tri_pnt; e.tri_seg = c->tri_seg; e.tri_sgn = c->tri_sgn;
+        e.order = ja.jel; e.begin = 0; e.end = 0;
+        e.ugv = c->ugv; e.ugs = c->ugs; e.ugi = c->ugi;
+        e.resv = ja.jrv; e.ress = ja.jrs; e.resi = ja.jri;
+        e.rrv = ja.jqv; e.rrs = ja.jqs; e.rri = ja.jqi;
+        e.ops = L.cpack; e.sm0 = c->sm0; e.im0 = c->im0;
+        e.ph = c->cph; e.beta = beta; e.keep = 0.0;
+        e.fcv = c->fcv; e.fcs = c->fcs; e.colour = 0;
+        launch_elem_cns<P>(c, e, full, &offs);
+        hipLaunchKernelGGL((k_jac_collect<P, NVC>), bN, tN, 0, c->stream, a);
     }
+    check(hipGetLastError(), "jacobian launch");
+}
+
+// ins: the unperturbed residuals of the batch elements, then all their columns in one
+// launch (entries are independent: no colours, no scatter, the state is only read)
+template <int P>
+void jacobian_ins(hpg_ctx* c, const int* d_tind, int nel, int N, double eps_r, double eps_a, double* base, double* K) {
+    const Level& L = c->lv[c->log2p];
+    ElemArgs e{};
+    e.pnts = c->pnts; e.tri_pnt = c->tri_pnt; e.tri_seg = c->tri_seg; e.tri_sgn = c->tri_sgn;
+    e.order = d_tind;
+    e.ugv = c->ugv; e.ugs = c->ugs; e.ugi = c->ugi;
+    e.ops = L.pack; e.sm0 = c->sm0; e.im0 = c->im0;
+    e.rho = c->prm.rho; e.mu = c->prm.mu; e.adis = c->prm.adis; e.beta = c->prm.beta[0];
+    e.fcv = c->fcv; e.fcs = c->fcs;
+    e.jeps_r = eps_r; e.jeps_a = eps_a; e.jbase = base;
+    const bool full = e.beta > 0.0;
+    auto launch = [&](int cols, double* k) {
+        e.jcols = cols; e.jK = k; e.begin = 0; e.end = nel * cols;
+        const int nlogical = (e.end + 63) / 64;
+        if (full) {
+            static const int cap = resident_blocks((const void*)k_elem_ins_jac<P, true>);
+            hipLaunchKernelGGL((k_elem_ins_jac<P, true>), dim3(persistent_grid(nlogical, cap)), dim3(256), 0, c->stream, e);
+        } else {
+            static const int cap = resident_blocks((const void*)k_elem_ins_jac<P, false>);
+            hipLaunchKernelGGL((k_elem_ins_jac<P, false>), dim3(persistent_grid(nlogical, cap)), dim3(256), 0, c->stream, e);
+        }
+    };
+    launch(1, nullptr);
+    launch(N, K);
     check(hipGetLastError(), "jacobian launch");
 }
 
@@ -1899,7 +1916,29 @@ int hpg_element_jacobian(hpg_ctx* c, const int* tind, int nel, double eps_r, dou
             if (seen[tind[j]]) throw std::runtime_error("element listed twice");
             seen[tind[j]] = 1;
         }
-        // group the batch by colour (stable in the caller's order)
+        CallBuffers B(c->stream);
+        if (c->physics == HPG_PHYSICS_INS) {
+            int* d_tind = B.get<int>(nel);
+            check(hipMemcpyAsync(d_tind, tind, (size_t)nel * 4, hipMemcpyHostToDevice, c->stream), "H2D");
+            // a slice of the batch at a time: the entry index of a launch is a 32-bit int
+            // and the scratch for K stays within 256 MiB however large the batch is
+            const int slice = (int)std::min<size_t>(nel, std::max<size_t>(1, (size_t)(1 << 25) / ((size_t)N * N)));
+            double* base = B.get<double>((size_t)slice * N);
+            double* dK = B.get<double>((size_t)slice * N * N);
+            for (int j0 = 0; j0 < nel; j0 += slice) {
+                const int nj = std::min(slice, nel - j0);
+                switch (L.p) {
+                    case 1: jacobian_ins<1>(c, d_tind + j0, nj, N, eps_r, eps_a, base, dK); break;
+                    case 2: jacobian_ins<2>(c, d_tind + j0, nj, N, eps_r, eps_a, base, dK); break;
+                    case 4: jacobian_ins<4>(c, d_tind + j0, nj, N, eps_r, eps_a, base, dK); break;
+                    default: throw std::runtime_error("unsupported p");
+                }
+                check(hipMemcpyAsync(K + (size_t)j0 * N * N, dK, (size_t)nj * N * N * 8, hipMemcpyDeviceToHost, c->stream), "D2H");
+                check(hipStreamSynchronize(c->stream), "sync");
+            }
+            return 0;
+        }
+        // cns: group the batch by colour (stable in the caller's order)
         const int ncol = (int)c->coff.size() - 1;
         std::vector<int> cnt(ncol + 1, 0), jel(nel), jpos(nel);
         for (int j = 0; j < nel; ++j) ++cnt[c->tcol[tind[j]] + 1];
@@ -1910,7 +1949,6 @@ int hpg_element_jacobian(hpg_ctx* c, const int* tind, int nel, double eps_r, dou
             jel[q] = tind[j];
             jpos[q] = j;
         }
-        CallBuffers B(c->stream);
         JacArgs ja{};
         ja.jel = B.get<int>(nel);
         ja.jpos = B.get<int>(nel);
@@ -1932,11 +1970,10 @@ int hpg_element_jacobian(hpg_ctx* c, const int* tind, int nel, double eps_r, dou
             JacArgs a = ja;
             a.begin = joff[col];
             a.end = joff[col + 1];
-            const bool cns = c->physics == HPG_PHYSICS_CNS;
             switch (L.p) {
-                case 1: cns ? jacobian_colour<1, 4>(c, a, N) : jacobian_colour<1, 3>(c, a, N); break;
-                case 2: cns ? jacobian_colour<2, 4>(c, a, N) : jacobian_colour<2, 3>(c, a, N); break;
-                case 4: cns ? jacobian_colour<4, 4>(c, a, N) : jacobian_colour<4, 3>(c, a, N); break;
+                case 1: jacobian_colour_cns<1>(c, a, N); break;
+                case 2: jacobian_colour_cns<2>(c, a, N); break;
+                case 4: jacobian_colour_cns<4>(c, a, N); break;
                 default: throw std::runtime_error("unsupported p");
             }
         }

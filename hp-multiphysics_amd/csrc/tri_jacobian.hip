@@ -1,5 +1,6 @@
 // Forward-difference element Jacobian of tri_hp::element_jacobian
-// (tri_hp/nstage.cpp:131-165, fixed-mesh branch) for a batch of elements.
+// (tri_hp/nstage.cpp:131-165, fixed-mesh branch) for a batch of cns elements, through the
+// global state (the ins batches run as independent entries of one launch, k_elem_ins_jac).
 //
 // The batch is split by element colour.  Elements of one colour share no vertex or
 // side, so one column (mode, var) of every element of the colour is formed at once:

@@ -62,6 +62,12 @@ struct ElemArgsT {
     const double* srcs;
     const double* srci;
     const double* sfac;
+    // element Jacobians (the Jacobian launch only): entry idx is column idx % jcols of batch
+    // element order[idx / jcols]; jK null: the unperturbed residuals into jbase
+    int jcols;
+    double jeps_r, jeps_a;
+    T* jbase;  // batch x N, N = TM * NV
+    T* jK;     // batch x N x N
     // curved elements (the curved launch only): per entry of order[begin:end), the
     // side-mode coefficients of the element's coordinates, (3 sides, sm0 modes, x/y)
     // with the side sign applied, zero on straight sides
