@@ -216,6 +216,8 @@ struct hpg_ctx {
     double *eres = nullptr, *eout = nullptr;
     float* eres32 = nullptr;  // the FP32 inner solve's element-major residual
     int *vb_ptr = nullptr, *vb_ent = nullptr;
+    int *sedge = nullptr, *enext = nullptr;  // each side's first edge in eseg, each edge's next one
+    float* eout32 = nullptr;
     int *vs_ptr, *vs_side, *vs_end, *vt_ptr, *vt_tri, *vt_loc, *st_tri, *st_loc;
     unsigned char *vess, *sess;
     unsigned char *fcv, *fcs;  // first colour touching each vertex / side
@@ -388,78 +390,87 @@ void launch_elem(hpg_ctx* c, const ElemArgs& a0, bool full, const std::vector<in
     }
 }
 
-// element-major residual over a0.order[begin:end) (null order: mesh order) in one
-// persistent launch (timing records 1 / 0 like the colour launches)
-template <int P>
-void launch_elem_em(hpg_ctx* c, const ElemArgs& a, bool full) {
+// element-major residual over a.order[begin:end) (null order: mesh order) and the
+// boundary-edge fluxes e in one persistent launch (timing records 1 / 0 like the colour
+// launches, 3 / 2 in FP32)
+template <int P, typename T>
+void launch_elem_em(hpg_ctx* c, const ElemArgsT<T>& a, const EdgeArgsT<T>& e, bool full) {
     const int nlogical = (a.end - a.begin + 63) / 64;
-    if (nlogical == 0) return;
+    const int eblk = e.end > 0 ? (int)nblk8(e.end) : 0;
+    if (nlogical == 0 && eblk == 0) return;
+    constexpr bool F64 = sizeof(T) == 8;
     const size_t r = c->recs.size();
     if (c->timing) check(hipEventRecord(c->event(2 * r), c->stream), "hipEventRecord");
-    if (full) {
-        static const int cap = resident_blocks((const void*)k_elem_ins_em<P, true>);
-        hipLaunchKernelGGL((k_elem_ins_em<P, true>), dim3(persistent_grid(nlogical, cap)), dim3(256), 0, c->stream,
-                           a, c->eres);
+    auto go = [&](auto kern, T* eres, T* eout, int cap) {
+        hipLaunchKernelGGL(kern, dim3(persistent_grid(nlogical, cap) + eblk), dim3(256), 0, c->stream, a, eres, e, eout, eblk);
+    };
+    if constexpr (F64) {
+        static const int cf = resident_blocks((const void*)k_elem_ins_em<P, true>);
+        static const int ci = resident_blocks((const void*)k_elem_ins_em<P, false>);
+        if (full) go(k_elem_ins_em<P, true>, c->eres, c->eout, cf);
+        else go(k_elem_ins_em<P, false>, c->eres, c->eout, ci);
     } else {
-        static const int cap = resident_blocks((const void*)k_elem_ins_em<P, false>);
-        hipLaunchKernelGGL((k_elem_ins_em<P, false>), dim3(persistent_grid(nlogical, cap)), dim3(256), 0, c->stream,
-                           a, c->eres);
+        static const int cf = resident_blocks((const void*)k_elem_ins32_em<P, true>);
+        static const int ci = resident_blocks((const void*)k_elem_ins32_em<P, false>);
+        if (full) go(k_elem_ins32_em<P, true>, c->eres32, c->eout32, cf);
+        else go(k_elem_ins32_em<P, false>, c->eres32, c->eout32, ci);
     }
     if (c->timing) {
         check(hipEventRecord(c->event(2 * r + 1), c->stream), "hipEventRecord");
-        c->recs.push_back({full ? 1 : 0, a.end - a.begin});
+        c->recs.push_back({(full ? 1 : 0) + (F64 ? 0 : 2), a.end - a.begin});
     }
 }
 
-template <int P>
-void launch_elem32_em(hpg_ctx* c, const ElemArgs32& a, bool full) {
-    const int nlogical = (a.end - a.begin + 63) / 64;
-    if (nlogical == 0) return;
-    const size_t r = c->recs.size();
-    if (c->timing) check(hipEventRecord(c->event(2 * r), c->stream), "hipEventRecord");
-    if (full) {
-        static const int cap = resident_blocks((const void*)k_elem_ins32_em<P, true>);
-        hipLaunchKernelGGL((k_elem_ins32_em<P, true>), dim3(persistent_grid(nlogical, cap)), dim3(256), 0,
-                           c->stream, a, c->eres32);
-    } else {
-        static const int cap = resident_blocks((const void*)k_elem_ins32_em<P, false>);
-        hipLaunchKernelGGL((k_elem_ins32_em<P, false>), dim3(persistent_grid(nlogical, cap)), dim3(256), 0,
-                           c->stream, a, c->eres32);
-    }
-    if (c->timing) {
-        check(hipEventRecord(c->event(2 * r + 1), c->stream), "hipEventRecord");
-        c->recs.push_back({full ? 3 : 2, a.end - a.begin});
-    }
-}
-
-// FP32 element residual of the defect-correction inner solve, colour by colour (timing
-// records 3 / 2 like the linearised kernel)
-template <int P>
-void launch_elem32(hpg_ctx* c, const ElemArgs32& a0, bool full) {
-    for (size_t col = 0; col + 1 < c->coff.size(); ++col) {
-        ElemArgs32 a = a0;
-        a.colour = (int)col;
-        a.begin = c->coff[col];
-        a.end = c->coff[col + 1];
-        a.gbase = 0;
-        const int nlogical = (a.end - a.begin + 63) / 64;
-        if (nlogical == 0) continue;
-        const size_t r = c->recs.size();
-        if (c->timing) check(hipEventRecord(c->event(2 * r), c->stream), "hipEventRecord");
-        if (full) {
-            static const int cap = resident_blocks((const void*)k_elem_ins32<P, true>);
-            hipLaunchKernelGGL((k_elem_ins32<P, true>), dim3(persistent_grid(nlogical, cap)), dim3(256), 0, c->stream,
-                               a);
+// the curved elements' launch after it
+template <typename T>
+void launch_elem_curved(hpg_ctx* c, ElemArgsT<T> b, int p, bool full) {
+    if (c->ncurv == 0) return;
+    b.order = c->clist; b.end = c->ncurv; b.crv = c->crv;
+    const dim3 grid(persistent_grid((c->ncurv + 63) / 64, 1 << 20)), th(256);
+    if constexpr (sizeof(T) == 8) {
+        if (p == 2) {
+            if (full) hipLaunchKernelGGL((k_elem_ins_em_curved<2, true>), grid, th, 0, c->stream, b, c->eres);
+            else hipLaunchKernelGGL((k_elem_ins_em_curved<2, false>), grid, th, 0, c->stream, b, c->eres);
         } else {
-            static const int cap = resident_blocks((const void*)k_elem_ins32<P, false>);
-            hipLaunchKernelGGL((k_elem_ins32<P, false>), dim3(persistent_grid(nlogical, cap)), dim3(256), 0,
-                               c->stream, a);
+            if (full) hipLaunchKernelGGL((k_elem_ins_em_curved<4, true>), grid, th, 0, c->stream, b, c->eres);
+            else hipLaunchKernelGGL((k_elem_ins_em_curved<4, false>), grid, th, 0, c->stream, b, c->eres);
         }
-        if (c->timing) {
-            check(hipEventRecord(c->event(2 * r + 1), c->stream), "hipEventRecord");
-            c->recs.push_back({full ? 3 : 2, a.end - a.begin});
+    } else {
+        if (p == 2) {
+            if (full) hipLaunchKernelGGL((k_elem_ins32_em_curved<2, true>), grid, th, 0, c->stream, b, c->eres32);
+            else hipLaunchKernelGGL((k_elem_ins32_em_curved<2, false>), grid, th, 0, c->stream, b, c->eres32);
+        } else {
+            if (full) hipLaunchKernelGGL((k_elem_ins32_em_curved<4, true>), grid, th, 0, c->stream, b, c->eres32);
+            else hipLaunchKernelGGL((k_elem_ins32_em_curved<4, false>), grid, th, 0, c->stream, b, c->eres32);
         }
     }
+}
+
+// boundary-edge flux arguments on the state (ugv, ugs)
+template <typename T>
+EdgeArgsT<T> edge_args(hpg_ctx* c, const T* ugv, const T* ugs) {
+    const Level& L = c->lv[c->log2p];
+    const LevelDims d(L.p);
+    EdgeArgsT<T> e{};
+    e.eseg = c->eseg; e.seg_pnt = c->seg_pnt; e.pnts = c->pnts; e.ugv = ugv; e.ugs = ugs;
+    e.g1 = L.edge; e.dg1 = L.edge + (d.p + 1) * (d.sm + 2); e.w1 = L.edge + 2 * (d.p + 1) * (d.sm + 2);
+    e.gpx = d.p + 1; e.sm = d.sm; e.sm0 = c->sm0; e.rho = c->prm.rho; e.bc_pressure = c->prm.bc_pressure;
+    if (d.p >= 2) { e.ecrv = c->ecrv; e.scrd = c->scrd; }
+    e.etype = c->etype; e.ub0 = c->ibc_u[0]; e.ub1 = c->ibc_u[1]; e.mu = c->prm.mu;
+    e.begin = 0; e.end = c->neseg;
+    return e;
+}
+
+// the mesh part of the gathers' arguments at the current level
+template <typename T, typename E = T>
+GatherArgsT<T, E> gather_args(hpg_ctx* c) {
+    const LevelDims d(c->lv[c->log2p].p);
+    GatherArgsT<T, E> g{};
+    g.npnt = c->npnt; g.nseg = c->nseg; g.sm = d.sm; g.sm0 = c->sm0; g.bm = d.bm;
+    g.vt_ptr = c->vt_ptr; g.vt_tri = c->vt_tri; g.vt_loc = c->vt_loc;
+    g.st_tri = c->st_tri; g.st_loc = c->st_loc;
+    g.vb_ptr = c->vb_ptr; g.vb_ent = c->vb_ent; g.sedge = c->sedge; g.enext = c->enext;
+    return g;
 }
 
 template <int P>
@@ -576,14 +587,7 @@ void vstage_p1(hpg_ctx* c, int stage, double cfa, bool save_u0) {
     a.ops = L.pack; a.sm0 = c->sm0; a.im0 = c->im0;
     a.rho = c->prm.rho; a.mu = c->prm.mu; a.adis = c->prm.adis; a.beta = beta;
     a.fcv = c->fcv; a.fcs = c->fcs; a.colour = 0; a.keep = f;
-    const LevelDims d(1);
-    EdgeArgs e{};
-    e.eseg = c->eseg; e.seg_pnt = c->seg_pnt; e.pnts = c->pnts; e.ugv = c->ugv; e.ugs = c->ugs;
-    e.resv = c->resv; e.ress = c->ress;
-    e.g1 = L.edge; e.dg1 = L.edge + (d.p + 1) * (d.sm + 2); e.w1 = L.edge + 2 * (d.p + 1) * (d.sm + 2);
-    e.gpx = d.p + 1; e.sm = d.sm; e.sm0 = c->sm0; e.rho = c->prm.rho; e.bc_pressure = c->prm.bc_pressure;
-    e.etype = c->etype; e.ub0 = c->ibc_u[0]; e.ub1 = c->ibc_u[1]; e.mu = c->prm.mu;
-    e.begin = 0; e.end = c->neseg;
+    const EdgeArgs e = edge_args<double>(c, c->ugv, c->ugs);
     // element blocks (one thread per element, mesh order) followed by the boundary-edge
     // blocks
     const int eg = (int)nblk(c->ntri, 256);
@@ -648,31 +652,18 @@ void do_rsdl(hpg_ctx* c, int stage, bool store_lin = false) {
         // element-major over all elements in mesh order (the straight ones, then the
         // curved ones, when there are curved boundary sides), then the fixed-order gather
         a.order = c->ncurv ? c->slist : nullptr; a.begin = 0; a.end = c->ntri - c->ncurv;
+        const EdgeArgs e = edge_args<double>(c, c->ugv, c->ugs);
         switch (L.p) {
-            case 2: launch_elem_em<2>(c, a, full); break;
-            case 4: launch_elem_em<4>(c, a, full); break;
+            case 2: launch_elem_em<2, double>(c, a, e, full); break;
+            case 4: launch_elem_em<4, double>(c, a, e, full); break;
             default: throw std::runtime_error("unsupported p");
         }
-        if (c->ncurv) {
-            ElemArgs b = a;
-            b.order = c->clist; b.end = c->ncurv; b.crv = c->crv;
-            const dim3 grid(persistent_grid((c->ncurv + 63) / 64, 1 << 20));
-            if (L.p == 2) {
-                if (full) hipLaunchKernelGGL((k_elem_ins_em_curved<2, true>), grid, dim3(256), 0, c->stream, b, c->eres);
-                else hipLaunchKernelGGL((k_elem_ins_em_curved<2, false>), grid, dim3(256), 0, c->stream, b, c->eres);
-            } else {
-                if (full) hipLaunchKernelGGL((k_elem_ins_em_curved<4, true>), grid, dim3(256), 0, c->stream, b, c->eres);
-                else hipLaunchKernelGGL((k_elem_ins_em_curved<4, false>), grid, dim3(256), 0, c->stream, b, c->eres);
-            }
-        }
-        const LevelDims dd(L.p);
-        GatherArgsT<double> ga{};
-        ga.npnt = c->npnt; ga.nseg = c->nseg; ga.sm = dd.sm; ga.sm0 = c->sm0; ga.bm = dd.bm;
-        ga.vt_ptr = c->vt_ptr; ga.vt_tri = c->vt_tri; ga.vt_loc = c->vt_loc;
-        ga.st_tri = c->st_tri; ga.st_loc = c->st_loc; ga.eres = c->eres;
+        launch_elem_curved<double>(c, a, L.p, full);
+        GatherArgsT<double> ga = gather_args<double>(c);
+        ga.eres = c->eres; ga.eout = c->eout;
         ga.resv = c->resv; ga.rrv = c->rrv; ga.ress = c->ress; ga.rrs = c->rrs;
         ga.keep = f; ga.full = full ? 1 : 0;
-        const long lanes = ((long)c->npnt + (long)c->nseg * dd.sm) * NV;
+        const long lanes = ((long)c->npnt + (long)c->nseg * ga.sm) * NV;
         hipLaunchKernelGGL((k_gather_vs<double, NV>), dim3(nblk(lanes)), dim3(256), 0, c->stream, ga);
     } else {
         switch (L.p) {
@@ -681,23 +672,17 @@ void do_rsdl(hpg_ctx* c, int stage, bool store_lin = false) {
             case 4: launch_elem<4>(c, a, full); break;
             default: throw std::runtime_error("unsupported p");
         }
-    }
-    const LevelDims d(L.p);
-    EdgeArgs e{};
-    e.eseg = c->eseg; e.seg_pnt = c->seg_pnt; e.pnts = c->pnts; e.ugv = c->ugv; e.ugs = c->ugs;
-    e.resv = c->resv; e.ress = c->ress;
-    e.g1 = L.edge; e.dg1 = L.edge + (d.p + 1) * (d.sm + 2); e.w1 = L.edge + 2 * (d.p + 1) * (d.sm + 2);
-    e.gpx = d.p + 1; e.sm = d.sm; e.sm0 = c->sm0; e.rho = c->prm.rho; e.bc_pressure = c->prm.bc_pressure;
-    e.ecrv = c->ecrv; e.scrd = c->scrd;
-    e.etype = c->etype; e.ub0 = c->ibc_u[0]; e.ub1 = c->ibc_u[1]; e.mu = c->prm.mu;
-    for (size_t col = 0; col + 1 < c->eoff.size(); ++col) {
-        e.begin = c->eoff[col];
-        e.end = c->eoff[col + 1];
-        if (e.end > e.begin) {
-            const dim3 be(nblk(e.end - e.begin, 64)), te(64);
-            if (L.p == 1) hipLaunchKernelGGL(k_edge_ins<1>, be, te, 0, c->stream, e);
-            else if (L.p == 2) hipLaunchKernelGGL(k_edge_ins<2>, be, te, 0, c->stream, e);
-            else hipLaunchKernelGGL(k_edge_ins<4>, be, te, 0, c->stream, e);
+        EdgeArgs e = edge_args<double>(c, c->ugv, c->ugs);
+        e.resv = c->resv; e.ress = c->ress;
+        for (size_t col = 0; col + 1 < c->eoff.size(); ++col) {
+            e.begin = c->eoff[col];
+            e.end = c->eoff[col + 1];
+            if (e.end > e.begin) {
+                const dim3 be(nblk(e.end - e.begin, 64)), te(64);
+                if (L.p == 1) hipLaunchKernelGGL(k_edge_ins<1>, be, te, 0, c->stream, e);
+                else if (L.p == 2) hipLaunchKernelGGL(k_edge_ins<2>, be, te, 0, c->stream, e);
+                else hipLaunchKernelGGL(k_edge_ins<4>, be, te, 0, c->stream, e);
+            }
         }
     }
     periodic_combine<double>(c, c->resv);
@@ -725,56 +710,25 @@ void do_rsdl32(hpg_ctx* c, int stage) {
     // periodic: the vertex source enters after the copies are summed (once per group)
     a.srcv = c->periodic ? nullptr : c->resv; a.srcs = c->ress; a.srci = c->resi; a.sfac = c->fd_scal + 1;
     const bool full = beta > 0.0;
-    if (L.p >= 2) {
-        // element-major over all elements in mesh order, then the fixed-order gather
-        // (which adds the source of the vertex and side modes)
-        a.order = c->ncurv ? c->slist : nullptr; a.begin = 0; a.end = c->ntri - c->ncurv;
-        if (L.p == 2) launch_elem32_em<2>(c, a, full);
-        else launch_elem32_em<4>(c, a, full);
-        if (c->ncurv) {
-            ElemArgs32 b = a;
-            b.order = c->clist; b.end = c->ncurv; b.crv = c->crv;
-            const dim3 grid(persistent_grid((c->ncurv + 63) / 64, 1 << 20));
-            if (L.p == 2) {
-                if (full) hipLaunchKernelGGL((k_elem_ins32_em_curved<2, true>), grid, dim3(256), 0, c->stream, b, c->eres32);
-                else hipLaunchKernelGGL((k_elem_ins32_em_curved<2, false>), grid, dim3(256), 0, c->stream, b, c->eres32);
-            } else {
-                if (full) hipLaunchKernelGGL((k_elem_ins32_em_curved<4, true>), grid, dim3(256), 0, c->stream, b, c->eres32);
-                else hipLaunchKernelGGL((k_elem_ins32_em_curved<4, false>), grid, dim3(256), 0, c->stream, b, c->eres32);
-            }
-        }
-        const LevelDims dd(L.p);
-        GatherArgsT<float> ga{};
-        ga.npnt = c->npnt; ga.nseg = c->nseg; ga.sm = dd.sm; ga.sm0 = c->sm0; ga.bm = dd.bm;
-        ga.vt_ptr = c->vt_ptr; ga.vt_tri = c->vt_tri; ga.vt_loc = c->vt_loc;
-        ga.st_tri = c->st_tri; ga.st_loc = c->st_loc; ga.eres = c->eres32;
-        ga.resv = c->r32v; ga.rrv = c->rr32v; ga.ress = c->r32s; ga.rrs = c->rr32s;
-        ga.keep = (float)f; ga.full = full ? 1 : 0;
-        // periodic: the vertex source enters after the copies are summed (once per group)
-        ga.srcv = c->periodic ? nullptr : c->resv; ga.srcs = c->ress; ga.sfac = c->fd_scal + 1;
-        const long lanes = ((long)c->npnt + (long)c->nseg * dd.sm) * NV;
-        hipLaunchKernelGGL((k_gather_vs<float, NV>), dim3(nblk(lanes)), dim3(256), 0, c->stream, ga);
-    } else {
-        launch_elem32<1>(c, a, full);
+    // element-major over all elements in mesh order, then the fixed-order gather (which
+    // adds the source of the vertex and side modes); elements are straight at p = 1
+    const bool curv = c->ncurv && L.p >= 2;
+    a.order = curv ? c->slist : nullptr; a.begin = 0; a.end = c->ntri - (curv ? c->ncurv : 0);
+    const EdgeArgsT<float> e = edge_args<float>(c, c->dlv, c->dls);
+    switch (L.p) {
+        case 1: launch_elem_em<1, float>(c, a, e, full); break;
+        case 2: launch_elem_em<2, float>(c, a, e, full); break;
+        default: launch_elem_em<4, float>(c, a, e, full); break;
     }
-    const LevelDims d(L.p);
-    EdgeArgsT<float> e{};
-    e.eseg = c->eseg; e.seg_pnt = c->seg_pnt; e.pnts = c->pnts; e.ugv = c->dlv; e.ugs = c->dls;
-    e.resv = c->r32v; e.ress = c->r32s;
-    e.g1 = L.edge; e.dg1 = L.edge + (d.p + 1) * (d.sm + 2); e.w1 = L.edge + 2 * (d.p + 1) * (d.sm + 2);
-    e.gpx = d.p + 1; e.sm = d.sm; e.sm0 = c->sm0; e.rho = c->prm.rho; e.bc_pressure = c->prm.bc_pressure;
-    e.ecrv = c->ecrv; e.scrd = c->scrd;
-    e.etype = c->etype; e.ub0 = c->ibc_u[0]; e.ub1 = c->ibc_u[1]; e.mu = c->prm.mu;
-    for (size_t col = 0; col + 1 < c->eoff.size(); ++col) {
-        e.begin = c->eoff[col];
-        e.end = c->eoff[col + 1];
-        if (e.end > e.begin) {
-            const dim3 be(nblk(e.end - e.begin, 64)), te(64);
-            if (L.p == 1) hipLaunchKernelGGL((k_edge_ins<1, float>), be, te, 0, c->stream, e);
-            else if (L.p == 2) hipLaunchKernelGGL((k_edge_ins<2, float>), be, te, 0, c->stream, e);
-            else hipLaunchKernelGGL((k_edge_ins<4, float>), be, te, 0, c->stream, e);
-        }
-    }
+    if (curv) launch_elem_curved<float>(c, a, L.p, full);
+    GatherArgsT<float> ga = gather_args<float>(c);
+    ga.eres = c->eres32; ga.eout = c->eout32;
+    ga.resv = c->r32v; ga.rrv = c->rr32v; ga.ress = c->r32s; ga.rrs = c->rr32s;
+    ga.keep = (float)f; ga.full = full ? 1 : 0;
+    // periodic: the vertex source enters after the copies are summed (once per group)
+    ga.srcv = c->periodic ? nullptr : c->resv; ga.srcs = c->ress; ga.sfac = c->fd_scal + 1;
+    const long lanes = ((long)c->npnt + (long)c->nseg * ga.sm) * NV;
+    hipLaunchKernelGGL((k_gather_vs<float, NV>), dim3(nblk(lanes)), dim3(256), 0, c->stream, ga);
     if (c->periodic) {
         periodic_combine<float>(c, c->r32v);
         hipLaunchKernelGGL(k_add_src32, dim3(nblk((long)c->npnt * NV)), dim3(256), 0, c->stream, (long)c->npnt * NV,
@@ -1329,6 +1283,14 @@ void build_edges(hpg_ctx* c, const int* seg_pnt, int np, const std::vector<int>&
         for (int k = 0; k < 2; ++k) vb_ent[f[seg_pnt[2 * eseg[j] + k]]++] = 2 * j + k;
     c->vb_ptr = c->upload(vb_ptr.data(), vb_ptr.size());
     c->vb_ent = c->upload(vb_ent.data(), vb_ent.size());
+    // edges of each side, ascending
+    std::vector<int> sedge(c->nseg, -1), enext(neseg, -1);
+    for (int j = neseg - 1; j >= 0; --j) {
+        enext[j] = sedge[eseg[j]];
+        sedge[eseg[j]] = j;
+    }
+    c->sedge = c->upload(sedge.data(), sedge.size());
+    c->enext = c->upload(enext.data(), enext.size());
 }
 }  // namespace
 
@@ -1544,7 +1506,8 @@ int hpg_create(const hpg_tri_mesh* m, const hpg_params* prm, hpg_ctx** out) {
             // element-major vertex and side modes of the finest level (3p per element)
             c->eres = c->alloc<double>((size_t)nt * 3 * (1 << c->log2pmax) * 2 * NV);
             c->eres32 = c->alloc<float>((size_t)nt * 3 * (1 << c->log2pmax) * 2 * NV);
-            c->eout = c->alloc<double>((size_t)neseg * 2 * NV);
+            c->eout = c->alloc<double>((size_t)neseg * (p0 + 1) * NV);
+            c->eout32 = c->alloc<float>((size_t)neseg * (p0 + 1) * NV);
             c->tprcn_vx = c->alloc<double>((size_t)nt * NV);
             c->tprcn_sd = c->alloc<double>((size_t)nt * NV);
             c->tprcn_in = c->alloc<double>((size_t)nt * NV);

@@ -98,7 +98,7 @@ __device__ __forceinline__ ElemConn elem_conn(const A& a, int t) {
     return c;
 }
 
-template <int P, class A>
+template <int P, int NVn = NV, class A>
 __device__ __forceinline__ ElemSlots<P> elem_slots(const A& a, const ElemConn& c, int q) {
     using D = Dims<P>;
     constexpr int SMD = D::SM > 0 ? D::SM : 1;
@@ -116,7 +116,7 @@ __device__ __forceinline__ ElemSlots<P> elem_slots(const A& a, const ElemConn& c
         const int k = 4 * s + q;
         int kind;
         double sg;
-        const int off = mode_offset<P>(k, valid ? c.t : 0, c.vtx, c.seg, c.sgn, a.sm0, a.im0, kind, sg);
+        const int off = mode_offset<P, NVn>(k, valid ? c.t : 0, c.vtx, c.seg, c.sgn, a.sm0, a.im0, kind, sg);
         S.off[s] = sg < 0.0 ? ~off : off;
         const bool live = valid && k < D::TM;
         const bool first = live && (kind == 2 || (kind == 0 ? a.fcv[sel3(c.vtx, k)]
@@ -143,8 +143,7 @@ __device__ __forceinline__ ElemSlots<P> elem_slots(const A& a, const ElemConn& c
 // the element order[idx / jcols] with its own copy of column idx % jcols's coefficient
 // moved by dw, so the columns of all elements are independent entries of one launch.
 template <typename T, int P, bool FULL, bool EM = false, bool CURV = false, bool JAC = false>
-__device__ __forceinline__ void elem_ins_body(const ElemArgsT<T>& a, T* __restrict__ eres = nullptr,
-                                              int egrid = 0) {
+__device__ __forceinline__ void elem_ins_body(const ElemArgsT<T>& a, T* __restrict__ eres = nullptr, int eblk = 0) {
     using D = Dims<P>;
     using V4 = typename Vec4<T>::type;
     constexpr int GT = D::GT, KT = D::KT;
@@ -156,9 +155,9 @@ __device__ __forceinline__ void elem_ins_body(const ElemArgsT<T>& a, T* __restri
     const int e = lane & 15, q = lane >> 4;
     // XCD-aware split: hardware deals consecutive blocks round-robin to the 8 XCDs;
     // XCD x owns groups [x*gpx, (x+1)*gpx) so neighbouring elements share its L2
-    // egrid: blocks of the launch that walk elements (the rest do other work)
-    const int WX = ((egrid ? egrid : (int)gridDim.x) >> 3) * 4;
-    const int rank = (blockIdx.x >> 3) * 4 + w;
+    // eblk: leading blocks of the launch that do other work (a multiple of 8)
+    const int WX = (((int)gridDim.x - eblk) >> 3) * 4;
+    const int rank = (((int)blockIdx.x - eblk) >> 3) * 4 + w;
     const int xcd = blockIdx.x & 7;
     const int ng = (a.end - a.begin + 15) >> 4;
     const int gpx = (ng + 7) >> 3;
@@ -595,14 +594,6 @@ __global__ __launch_bounds__(256) void k_elem_ins(ElemArgs a) {
     elem_ins_body<double, P, FULL>(a);
 }
 
-// FP32 instantiation (the inner solve of the FP32 defect correction): the same
-// residual in single precision on v_mfma_f32_16x16x4f32; its operator pack permutes
-// the output rows of Ir/Is so that register s of lane group q again holds mode 4s + q
-template <int P, bool FULL>
-__global__ __launch_bounds__(256, 2) void k_elem_ins32(ElemArgs32 a) {
-    elem_ins_body<float, P, FULL>(a);
-}
-
 // ---------------------------------------------------------------------------------
 // Mode-array helpers over v(nent, mstride, NV) with the first nm modes active.
 // op 0: x = 0, y *= c           (rsdl start, tri_hp/nstage.cpp:21-49)
@@ -708,8 +699,8 @@ __device__ __forceinline__ void edge_flux_ins(int type, const double* u, double 
 
 // P fixes the edge's mode count (p + 1) and Gauss points (p + 1), so the per-lane
 // arrays stay in registers
-// EM: element-major output eout[(idx*2 + k)*NV + n] for endpoint k of boundary edge
-// idx (p = 1, summed into the vertices by k_vstage1) instead of the RMW scatter
+// EM: element-major output eout[(idx*(SM+2) + k)*NV + n], k the two ends then the side
+// modes, summed by the gathers, instead of the RMW scatter (the linearisation's path)
 template <int P, typename S, bool EM>
 __device__ __forceinline__ void edge_ins_body(const EdgeArgsT<S>& a, S* __restrict__ eout, int idx) {
     constexpr int SM = P - 1, N1 = SM + 2, GPX = P + 1;
@@ -774,10 +765,9 @@ __device__ __forceinline__ void edge_ins_body(const EdgeArgsT<S>& a, S* __restri
     }
     if constexpr (EM) {
 #pragma unroll
-        for (int n = 0; n < NV; ++n) {
-            eout[(2 * idx) * NV + n] = (S)lf[n][0];
-            eout[(2 * idx + 1) * NV + n] = (S)lf[n][1];
-        }
+        for (int n = 0; n < NV; ++n)
+#pragma unroll
+            for (int k = 0; k < N1; ++k) eout[((long)idx * N1 + k) * NV + n] = (S)lf[n][k];
         return;
     }
 #pragma unroll
@@ -789,24 +779,39 @@ __device__ __forceinline__ void edge_ins_body(const EdgeArgsT<S>& a, S* __restri
     }
 }
 
-template <int P, typename S = double>
-__global__ __launch_bounds__(64) void k_edge_ins(EdgeArgsT<S> a) {
-    edge_ins_body<P, S, false>(a, nullptr, a.begin + blockIdx.x * blockDim.x + threadIdx.x);
+template <int P>
+__global__ __launch_bounds__(64) void k_edge_ins(EdgeArgs a) {
+    edge_ins_body<P, double, false>(a, nullptr, a.begin + blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // Element-major residual (no colouring, mesh order): the element body with its EM
 // output, persistent over all elements; k_gather_vs then sums the vertex and side
 // modes in a fixed order.  At p = 2 the bound of 256 registers keeps two waves per
 // SIMD without spilling (272 otherwise, one wave).
+// The first eblk blocks (a multiple of 8) compute the boundary-edge fluxes into eout: one
+// launch instead of three, and on small meshes the edges' latency hides behind the
+// elements' (two edge launches were 10 us of a 31 us stage at 33 x 33, p = 2).
 template <int P, bool FULL>
-__global__ __launch_bounds__(256, P == 2 ? 2 : 1) void k_elem_ins_em(ElemArgs a, double* eres) {
-    elem_ins_body<double, P, FULL, true>(a, eres);
+__global__ __launch_bounds__(256, P == 2 ? 2 : 1) void k_elem_ins_em(ElemArgs a, double* eres, EdgeArgs e,
+                                                                     double* eout, int eblk) {
+    if ((int)blockIdx.x < eblk) {
+        edge_ins_body<P, double, true>(e, eout, blockIdx.x * 256 + threadIdx.x);
+        return;
+    }
+    elem_ins_body<double, P, FULL, true>(a, eres, eblk);
 }
 
-// the FP32 inner solve's element residual in element-major form (as k_elem_ins32)
+// FP32 (the inner solve of the defect correction): the same residual in single precision
+// on v_mfma_f32_16x16x4f32; its operator pack permutes the output rows of Ir/Is so that
+// register s of lane group q again holds mode 4s + q
 template <int P, bool FULL>
-__global__ __launch_bounds__(256, 2) void k_elem_ins32_em(ElemArgs32 a, float* eres) {
-    elem_ins_body<float, P, FULL, true>(a, eres);
+__global__ __launch_bounds__(256, 2) void k_elem_ins32_em(ElemArgs32 a, float* eres, EdgeArgsT<float> e, float* eout,
+                                                          int eblk) {
+    if ((int)blockIdx.x < eblk) {
+        edge_ins_body<P, float, true>(e, eout, blockIdx.x * 256 + threadIdx.x);
+        return;
+    }
+    elem_ins_body<float, P, FULL, true>(a, eres, eblk);
 }
 
 // Element Jacobians of a batch: every (element, column) pair is an entry of one launch,
@@ -838,7 +843,10 @@ __global__ __launch_bounds__(256) void k_elem_ins32_em_curved(ElemArgs32 a, floa
 // colour and the later colours of the scatter do.  FP32 (the defect correction's inner
 // solve): the constant source sfac[0] * src enters with the first element, as on the
 // scatter's first visit.
-template <typename T>
+// E: type of the element results (float under FP64 sums in the cns inner solve).  The
+// boundary-edge results follow the elements (eout, written by the element launch's edge
+// blocks): a vertex adds its edges' end entries in list order, a boundary side its own.
+template <typename T, typename E = T>
 struct GatherArgsT {
     int npnt, nseg, sm, sm0, bm;
     const int* vt_ptr;
@@ -846,23 +854,28 @@ struct GatherArgsT {
     const int* vt_loc;
     const int* st_tri;
     const int* st_loc;
-    const T* eres;
+    const E* eres;
+    const int* vb_ptr;   // boundary-edge ends at each vertex: 2 * edge + end
+    const int* vb_ent;
+    const int* sedge;    // first edge of a side in the boundary lists (-1: none) and
+    const int* enext;    // the edge's next entry for the same side
+    const T* eout;       // (edge, 2 ends then the side modes, NV)
     T* resv;
     T* rrv;
     T* ress;
     T* rrs;
     T keep;
     int full;
-    const double* srcv;  // FP32 only, may be null
+    const double* srcv;  // defect source, may be null
     const double* srcs;
     const double* sfac;
 };
 
-template <typename T, int NVn>
-__device__ __forceinline__ void gather_sum(const GatherArgsT<T>& a, const T* e, int n, T& acc, T& accr) {
-    const T li = e[n];
+template <typename T, int NVn, typename E>
+__device__ __forceinline__ void gather_sum(const GatherArgsT<T, E>& a, const E* e, int n, T sign, T& acc, T& accr) {
+    const T li = sign * T(e[n]);
     if (a.full) {
-        const T lr = e[NVn + n];
+        const T lr = sign * T(e[NVn + n]);
         accr += lr;
         acc = (acc + lr) + li;
     } else {
@@ -870,30 +883,23 @@ __device__ __forceinline__ void gather_sum(const GatherArgsT<T>& a, const T* e, 
     }
 }
 
-template <typename T, int NVn>
-__device__ __forceinline__ void gather_sum_neg(const GatherArgsT<T>& a, const T* e, int n, T& acc, T& accr) {
-    const T li = -e[n];
-    if (a.full) {
-        const T lr = -e[NVn + n];
-        accr += lr;
-        acc = (acc + lr) + li;
-    } else {
-        acc = acc + li;
-    }
-}
-
-template <typename T, int NVn>
-__global__ __launch_bounds__(256) void k_gather_vs(GatherArgsT<T> a) {
+template <typename T, int NVn, typename E = T>
+__global__ __launch_bounds__(256) void k_gather_vs(GatherArgsT<T, E> a) {
     const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long nvl = (long)a.npnt * NVn;
     const T keep = a.keep;
+    const int ne = a.sm + 2;  // entries of a boundary edge
     if (g < nvl) {
         const int v = (int)(g / NVn), n = (int)(g - (long)v * NVn);
         const T r0 = keep == T(0) ? T(0) : keep * a.rrv[g];
         T acc = r0, accr = r0;
         for (int k = a.vt_ptr[v]; k < a.vt_ptr[v + 1]; ++k) {
-            gather_sum<T, NVn>(a, a.eres + ((long)a.vt_tri[k] * a.bm + a.vt_loc[k]) * (2 * NVn), n, acc, accr);
+            gather_sum<T, NVn, E>(a, a.eres + ((long)a.vt_tri[k] * a.bm + a.vt_loc[k]) * (2 * NVn), n, T(1), acc, accr);
             if (k == a.vt_ptr[v] && a.srcv) acc = acc + T(a.srcv[g] * a.sfac[0]);
+        }
+        for (int k = a.vb_ptr[v]; k < a.vb_ptr[v + 1]; ++k) {
+            const int ent = a.vb_ent[k];
+            acc += a.eout[((long)(ent >> 1) * ne + (ent & 1)) * NVn + n];
         }
         if (a.full || keep != T(1)) a.rrv[g] = accr;
         a.resv[g] = acc;
@@ -916,13 +922,12 @@ __global__ __launch_bounds__(256) void k_gather_vs(GatherArgsT<T> a) {
         // way: its odd modes change sign in this side's frame
         const int sl = a.st_loc[2 * s + slot];
         const int mode = 3 + (sl & 3) * a.sm + m;
-        if ((sl & 4) && (m & 1))
-            gather_sum_neg<T, NVn>(a, a.eres + ((long)t * a.bm + mode) * (2 * NVn), n, acc, accr);
-        else
-            gather_sum<T, NVn>(a, a.eres + ((long)t * a.bm + mode) * (2 * NVn), n, acc, accr);
+        gather_sum<T, NVn, E>(a, a.eres + ((long)t * a.bm + mode) * (2 * NVn), n, ((sl & 4) && (m & 1)) ? T(-1) : T(1),
+                              acc, accr);
         if (first && a.srcs) acc = acc + T(a.srcs[o] * a.sfac[0]);
         first = false;
     }
+    for (int ed = a.sedge[s]; ed >= 0; ed = a.enext[ed]) acc += a.eout[((long)ed * ne + 2 + m) * NVn + n];
     if (a.full || keep != T(1)) a.rrs[o] = accr;
     a.ress[o] = acc;
 }
@@ -1824,12 +1829,6 @@ template __global__ void k_elem_ins<2, true>(ElemArgs);
 template __global__ void k_elem_ins<2, false>(ElemArgs);
 template __global__ void k_elem_ins<4, true>(ElemArgs);
 template __global__ void k_elem_ins<4, false>(ElemArgs);
-template __global__ void k_elem_ins32<1, true>(ElemArgs32);
-template __global__ void k_elem_ins32<1, false>(ElemArgs32);
-template __global__ void k_elem_ins32<2, true>(ElemArgs32);
-template __global__ void k_elem_ins32<2, false>(ElemArgs32);
-template __global__ void k_elem_ins32<4, true>(ElemArgs32);
-template __global__ void k_elem_ins32<4, false>(ElemArgs32);
 
 
 // grid-stride copy of n 4-byte words (device-to-device copies inside the solver)
