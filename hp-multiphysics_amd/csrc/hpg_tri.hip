@@ -18,7 +18,6 @@
 #include "tri_kernels.hip"
 #include "tri_kernels_lin.hip"
 #include "tri_kernels_cns.hip"
-#include "tri_jacobian.hip"
 #include "tri_ops.h"
 #include "mlp.h"
 
@@ -123,9 +122,11 @@ struct Level {
     float* packn32 = nullptr;  // FP32 element residual (output rows permuted to the FP64 layout)
     float* lump32 = nullptr;
     int o_sfmv, o_ifmb, o_vfms, o_sdiag, o_sfms, o_bfmi, o_idiag;
-    // cns: point-per-lane operator pack (CDims layout), edge side-mass and interior band factors
+    // cns: point-per-lane operators (CDims layout: project_new_variables in FP64, the element
+    // residual of the defect-correction inner solve in FP32), edge side-mass and interior
+    // band factors
     double* cpack = nullptr;
-    float* cpack32 = nullptr;  // the same operators in FP32 (defect-correction inner solve)
+    float* cpack32 = nullptr;
     double* sdiag1d = nullptr;
     double* idiag = nullptr;
 };
@@ -184,7 +185,6 @@ struct hpg_ctx {
     int *tri_pnt = nullptr, *tri_seg = nullptr, *tri_sgn = nullptr, *seg_pnt = nullptr;
     int* order = nullptr;
     std::vector<int> coff;
-    std::vector<int> tcol;  // colour of each element (host)
     int* eseg = nullptr;
     std::vector<int> eoff;
     int neseg = 0;
@@ -221,6 +221,7 @@ struct hpg_ctx {
     int *vs_ptr, *vs_side, *vs_end, *vt_ptr, *vt_tri, *vt_loc, *st_tri, *st_loc;
     unsigned char *vess, *sess;
     unsigned char *fcv, *fcs;  // first colour touching each vertex / side
+    unsigned char* tcol = nullptr;  // cns: colour of each element
     double *ugv, *ugs, *ugi, *ug0v, *ug0s, *ug0i;
     double *resv, *ress, *resi, *rrv, *rrs, *rri, *r0v, *r0s, *r0i;
     double *dresv[3], *dress[3], *dresi[3];
@@ -362,15 +363,14 @@ static int resident_blocks(const void* kernel) {
 static int persistent_grid(int want, int cap) { return std::min((want + 7) / 8 * 8, cap); }
 
 template <int P>
-void launch_elem(hpg_ctx* c, const ElemArgs& a0, bool full, const std::vector<int>* offs = nullptr) {
-    // offs: colour offsets into a0.order (default: every element, c->order)
-    const std::vector<int>& off = offs ? *offs : c->coff;
+void launch_elem(hpg_ctx* c, const ElemArgs& a0, bool full) {
+    const std::vector<int>& off = c->coff;
     for (size_t col = 0; col + 1 < off.size(); ++col) {
         ElemArgs a = a0;
         a.colour = (int)col;
         a.begin = off[col];
         a.end = off[col + 1];
-        a.gbase = offs ? 0 : c->gbase[col];
+        a.gbase = c->gbase[col];
         const int nlogical = (a.end - a.begin + 63) / 64;
         if (nlogical == 0) continue;
         const size_t r = c->recs.size();
@@ -462,10 +462,10 @@ EdgeArgsT<T> edge_args(hpg_ctx* c, const T* ugv, const T* ugs) {
 }
 
 // the mesh part of the gathers' arguments at the current level
-template <typename T, typename E = T>
-GatherArgsT<T, E> gather_args(hpg_ctx* c) {
+template <typename T>
+GatherArgsT<T> gather_args(hpg_ctx* c) {
     const LevelDims d(c->lv[c->log2p].p);
-    GatherArgsT<T, E> g{};
+    GatherArgsT<T> g{};
     g.npnt = c->npnt; g.nseg = c->nseg; g.sm = d.sm; g.sm0 = c->sm0; g.bm = d.bm;
     g.vt_ptr = c->vt_ptr; g.vt_tri = c->vt_tri; g.vt_loc = c->vt_loc;
     g.st_tri = c->st_tri; g.st_loc = c->st_loc;
@@ -838,51 +838,78 @@ void do_minvrt32(hpg_ctx* c, float cfa) {
 }
 
 // ---- tri_hp_cns drivers ------------------------------------------------------------
-template <int P>
-void launch_elem_cns(hpg_ctx* c, const CnsElemArgs& a0, bool full, const std::vector<int>* offs = nullptr) {
-    const std::vector<int>& off = offs ? *offs : c->coff;
-    for (size_t col = 0; col + 1 < off.size(); ++col) {
-        CnsElemArgs a = a0;
-        a.colour = (int)col;
-        a.begin = off[col];
-        a.end = off[col + 1];
+// element residuals (mesh order) and boundary-edge fluxes in one persistent launch
+template <int P, typename T>
+void launch_elem_cns(hpg_ctx* c, const CnsElemArgsT<T>& a, const CnsEdgeArgs& e, bool full) {
+    constexpr bool F64 = sizeof(T) == 8;
+    const int nlogical = (a.end - a.begin + 63) / 64, eblk = e.end > 0 ? (int)nblk8(e.end) : 0;
+    const size_t r = c->recs.size();
+    if (c->timing) check(hipEventRecord(c->event(2 * r), c->stream), "hipEventRecord");
+    auto go = [&](auto kern, int cap) {
+        hipLaunchKernelGGL(kern, dim3(persistent_grid(nlogical, cap) + eblk), dim3(256), 0, c->stream, a, e, eblk);
+    };
+    if constexpr (F64) {
+        static const int cf = resident_blocks((const void*)k_elem_cns<P, true>);
+        static const int ci = resident_blocks((const void*)k_elem_cns<P, false>);
+        if (full) go(k_elem_cns<P, true>, cf);
+        else go(k_elem_cns<P, false>, ci);
+    } else {
+        // eight elements (half-waves) per block and pass
         const int noct = (a.end - a.begin + 7) / 8;
-        if (noct == 0) continue;
-        const int nb = std::min(((noct + 7) / 8) * 8, 1024);
-        const size_t r = c->recs.size();
-        if (c->timing) check(hipEventRecord(c->event(2 * r), c->stream), "hipEventRecord");
-        if (full)
-            hipLaunchKernelGGL((k_elem_cns<P, true>), dim3(nb), dim3(256), 0, c->stream, a, noct);
-        else
-            hipLaunchKernelGGL((k_elem_cns<P, false>), dim3(nb), dim3(256), 0, c->stream, a, noct);
-        if (c->timing) {
-            check(hipEventRecord(c->event(2 * r + 1), c->stream), "hipEventRecord");
-            c->recs.push_back({full ? 1 : 0, a.end - a.begin});
-        }
+        auto go32 = [&](auto kern, int cap) {
+            hipLaunchKernelGGL(kern, dim3(persistent_grid(noct, cap) + eblk), dim3(256), 0, c->stream, a, e, eblk);
+        };
+        static const int cf = resident_blocks((const void*)k_elem_cns32<P, true>);
+        static const int ci = resident_blocks((const void*)k_elem_cns32<P, false>);
+        if (full) go32(k_elem_cns32<P, true>, cf);
+        else go32(k_elem_cns32<P, false>, ci);
+    }
+    if (c->timing) {
+        check(hipEventRecord(c->event(2 * r + 1), c->stream), "hipEventRecord");
+        c->recs.push_back({(full ? 1 : 0) + (F64 ? 0 : 2), a.end - a.begin});
     }
 }
 
-template <int P>
-void launch_elem_cns32(hpg_ctx* c, const CnsElemArgs32& a0, bool full) {
-    for (size_t col = 0; col + 1 < c->coff.size(); ++col) {
-        CnsElemArgs32 a = a0;
-        a.colour = (int)col;
-        a.begin = c->coff[col];
-        a.end = c->coff[col + 1];
-        const int noct = (a.end - a.begin + 7) / 8;
-        if (noct == 0) continue;
-        const int nb = std::min(((noct + 7) / 8) * 8, 1024);
-        const size_t r = c->recs.size();
-        if (c->timing) check(hipEventRecord(c->event(2 * r), c->stream), "hipEventRecord");
-        if (full)
-            hipLaunchKernelGGL((k_elem_cns32<P, true>), dim3(nb), dim3(256), 0, c->stream, a, noct);
-        else
-            hipLaunchKernelGGL((k_elem_cns32<P, false>), dim3(nb), dim3(256), 0, c->stream, a, noct);
-        if (c->timing) {
-            check(hipEventRecord(c->event(2 * r + 1), c->stream), "hipEventRecord");
-            c->recs.push_back({full ? 3 : 2, a.end - a.begin});
-        }
+// the element, edge and gather launches of a cns residual in arithmetic type T: stage's
+// lf_im and blended lf_re; src (FP32): the defect source srcv, srcs, srci
+template <typename T>
+void cns_residual(hpg_ctx* c, int stage, bool src) {
+    const int nst = c->prm.nstage;
+    const double beta = stage < nst ? c->prm.beta[stage] : 1.0;
+    const double f = stage < nst ? 1.0 - beta : 0.0;
+    const Level& L = c->lv[c->log2p];
+    const LevelDims d(L.p);
+    CnsElemArgsT<T> a{};
+    a.pnts = c->pnts; a.tri_pnt = c->tri_pnt; a.tri_seg = c->tri_seg; a.tri_sgn = c->tri_sgn;
+    a.order = nullptr; a.begin = 0; a.end = c->ntri;
+    a.ugv = c->ugv; a.ugs = c->ugs; a.ugi = c->ugi;
+    a.resi = c->resi; a.rri = c->rri;
+    if constexpr (sizeof(T) == 8) a.ops = L.pack;
+    else a.ops = L.cpack32;
+    a.eres = c->eres; a.tcol = c->tcol;
+    a.sm0 = c->sm0; a.im0 = c->im0;
+    a.ph = c->cph; a.beta = beta; a.keep = f;
+    a.fcv = c->fcv; a.fcs = c->fcs;
+    if (src) { a.srci = c->srci; a.sfac = c->fd_scal + 1; }
+    CnsEdgeArgs e{};
+    e.eseg = c->eseg; e.end = c->neseg; e.seg_pnt = c->seg_pnt; e.pnts = c->pnts; e.ugv = c->ugv; e.ugs = c->ugs;
+    e.eout = c->eout;
+    e.g1 = L.edge; e.dg1 = L.edge + (d.p + 1) * (d.sm + 2); e.w1 = L.edge + 2 * (d.p + 1) * (d.sm + 2);
+    e.sm0 = c->sm0; e.gamma = c->cph.gamma; e.pbc = c->cbc[0];
+    const bool full = beta > 0.0;
+    switch (L.p) {
+        case 1: launch_elem_cns<1, T>(c, a, e, full); break;
+        case 2: launch_elem_cns<2, T>(c, a, e, full); break;
+        case 4: launch_elem_cns<4, T>(c, a, e, full); break;
+        default: throw std::runtime_error("unsupported p");
     }
+    GatherArgsT<double> ga = gather_args<double>(c);
+    ga.eres = c->eres; ga.summed = sizeof(T) == 4; ga.eout = c->eout;
+    ga.resv = c->resv; ga.rrv = c->rrv; ga.ress = c->ress; ga.rrs = c->rrs;
+    ga.keep = f; ga.full = full ? 1 : 0;
+    if (src) { ga.srcv = c->srcv; ga.srcs = c->srcs; ga.sfac = c->fd_scal + 1; }
+    const long lanes = ((long)c->npnt + (long)c->nseg * ga.sm) * NVC;
+    hipLaunchKernelGGL((k_gather_vs<double, NVC>), dim3(nblk(lanes)), dim3(256), 0, c->stream, ga);
 }
 
 // coarse p-level source (tri_hp/nstage.cpp:113-129)
@@ -899,39 +926,7 @@ void mg_source(hpg_ctx* c) {
 }
 
 void do_rsdl_cns(hpg_ctx* c, int stage) {
-    const int nst = c->prm.nstage;
-    const double beta = stage < nst ? c->prm.beta[stage] : 1.0;
-    const double f = stage < nst ? 1.0 - beta : 0.0;
-    const Level& L = c->lv[c->log2p];
-    CnsElemArgs a;
-    a.pnts = c->pnts; a.tri_pnt = c->tri_pnt; a.tri_seg = c->tri_seg; a.tri_sgn = c->tri_sgn;
-    a.order = c->order; a.begin = 0; a.end = 0;
-    a.ugv = c->ugv; a.ugs = c->ugs; a.ugi = c->ugi;
-    a.resv = c->resv; a.ress = c->ress; a.resi = c->resi;
-    a.rrv = c->rrv; a.rrs = c->rrs; a.rri = c->rri;
-    a.ops = L.cpack; a.sm0 = c->sm0; a.im0 = c->im0;
-    a.ph = c->cph; a.beta = beta; a.keep = f;
-    a.fcv = c->fcv; a.fcs = c->fcs; a.colour = 0;
-    const bool full = beta > 0.0;
-    const LevelDims d(L.p);
-    CnsEdgeArgs e;
-    e.eseg = c->eseg; e.seg_pnt = c->seg_pnt; e.pnts = c->pnts; e.ugv = c->ugv; e.ugs = c->ugs;
-    e.resv = c->resv; e.ress = c->ress;
-    e.g1 = L.edge; e.dg1 = L.edge + (d.p + 1) * (d.sm + 2); e.w1 = L.edge + 2 * (d.p + 1) * (d.sm + 2);
-    e.sm0 = c->sm0; e.gamma = c->cph.gamma; e.pbc = c->cbc[0];
-    auto edges = [&](auto kern) {
-        for (size_t col = 0; col + 1 < c->eoff.size(); ++col) {
-            e.begin = c->eoff[col];
-            e.end = c->eoff[col + 1];
-            if (e.end > e.begin) hipLaunchKernelGGL(kern, dim3(nblk(e.end - e.begin, 64)), dim3(64), 0, c->stream, e);
-        }
-    };
-    switch (L.p) {
-        case 1: launch_elem_cns<1>(c, a, full); edges(k_edge_cns<1>); break;
-        case 2: launch_elem_cns<2>(c, a, full); edges(k_edge_cns<2>); break;
-        case 4: launch_elem_cns<4>(c, a, full); edges(k_edge_cns<4>); break;
-        default: throw std::runtime_error("unsupported p");
-    }
+    cns_residual<double>(c, stage, false);
     if (c->coarse_flag) mg_source(c);
     check(hipGetLastError(), "cns rsdl launch");
 }
@@ -940,40 +935,7 @@ void do_rsdl_cns(hpg_ctx* c, int stage) {
 // element residual in FP32 plus the scaled defect source (1/c - 1) R64(u0) (srcv...),
 // the boundary fluxes in FP64
 void do_rsdl_cns32(hpg_ctx* c, int stage) {
-    const int nst = c->prm.nstage;
-    const double beta = stage < nst ? c->prm.beta[stage] : 1.0;
-    const double f = stage < nst ? 1.0 - beta : 0.0;
-    const Level& L = c->lv[c->log2p];
-    CnsElemArgs32 a{};
-    a.pnts = c->pnts; a.tri_pnt = c->tri_pnt; a.tri_seg = c->tri_seg; a.tri_sgn = c->tri_sgn;
-    a.order = c->order; a.begin = 0; a.end = 0;
-    a.ugv = c->ugv; a.ugs = c->ugs; a.ugi = c->ugi;
-    a.resv = c->resv; a.ress = c->ress; a.resi = c->resi;
-    a.rrv = c->rrv; a.rrs = c->rrs; a.rri = c->rri;
-    a.ops = L.cpack32; a.sm0 = c->sm0; a.im0 = c->im0;
-    a.ph = c->cph; a.beta = beta; a.keep = f;
-    a.fcv = c->fcv; a.fcs = c->fcs; a.colour = 0;
-    a.srcv = c->srcv; a.srcs = c->srcs; a.srci = c->srci; a.sfac = c->fd_scal + 1;
-    const bool full = beta > 0.0;
-    const LevelDims d(L.p);
-    CnsEdgeArgs e;
-    e.eseg = c->eseg; e.seg_pnt = c->seg_pnt; e.pnts = c->pnts; e.ugv = c->ugv; e.ugs = c->ugs;
-    e.resv = c->resv; e.ress = c->ress;
-    e.g1 = L.edge; e.dg1 = L.edge + (d.p + 1) * (d.sm + 2); e.w1 = L.edge + 2 * (d.p + 1) * (d.sm + 2);
-    e.sm0 = c->sm0; e.gamma = c->cph.gamma; e.pbc = c->cbc[0];
-    auto edges = [&](auto kern) {
-        for (size_t col = 0; col + 1 < c->eoff.size(); ++col) {
-            e.begin = c->eoff[col];
-            e.end = c->eoff[col + 1];
-            if (e.end > e.begin) hipLaunchKernelGGL(kern, dim3(nblk(e.end - e.begin, 64)), dim3(64), 0, c->stream, e);
-        }
-    };
-    switch (L.p) {
-        case 1: launch_elem_cns32<1>(c, a, full); edges(k_edge_cns<1>); break;
-        case 2: launch_elem_cns32<2>(c, a, full); edges(k_edge_cns<2>); break;
-        case 4: launch_elem_cns32<4>(c, a, full); edges(k_edge_cns<4>); break;
-        default: throw std::runtime_error("unsupported p");
-    }
+    cns_residual<float>(c, stage, c->srcv != nullptr);
     check(hipGetLastError(), "cns rsdl32 launch");
 }
 
@@ -1187,66 +1149,46 @@ struct CallBuffers {
     }
 };
 
-// cns: one column of a colour's batch elements at a time, through the global state
+// the unperturbed residuals of the batch elements, then all their columns in one launch
+// (entries are independent: no colours, no scatter, the state is only read)
 template <int P>
-void jacobian_colour_cns(hpg_ctx* c, const JacArgs& ja, int N) {
-    const int nel = ja.end - ja.begin;
-    const dim3 b1(nblk(nel, 64)), t1(64), bN(nblk((long)nel * N)), tN(256);
+void element_jacobians(hpg_ctx* c, const int* d_tind, int nel, int N, double eps_r, double eps_a, double* base, double* K) {
     const Level& L = c->lv[c->log2p];
     const double beta = c->prm.beta[0];
     const bool full = beta > 0.0;
-    // one launch over the colour's batch elements.  The kernel's first-visit flags are
-    // keyed to colour 0 here, not to the elements' own colour; that does not matter:
-    // every scratch entry starts at zero, so both lftog paths store lf_re + lf_im
-    const std::vector<int> offs = {ja.begin, ja.end};
-    hipLaunchKernelGGL(k_jac_dw<NVC>, b1, t1, 0, c->stream, ja);
-    for (int col = -1; col < N; ++col) {
-        JacArgs a = ja;
-        a.mode = col < 0 ? -1 : col / NVC;
-        a.var = col < 0 ? 0 : col % NVC;
-        if (col >= 0) hipLaunchKernelGGL((k_jac_perturb<P, NVC>), b1, t1, 0, c->stream, a);
-        CnsElemArgs e;
+    auto mesh = [&](auto& e) {
         e.pnts = c->pnts; e.tri_pnt = c->tri_pnt; e.tri_seg = c->tri_seg; e.tri_sgn = c->tri_sgn;
-        e.order = ja.jel; e.begin = 0; e.end = 0;
+        e.order = d_tind;
         e.ugv = c->ugv; e.ugs = c->ugs; e.ugi = c->ugi;
-        e.resv = ja.jrv; e.ress = ja.jrs; e.resi = ja.jri;
-        e.rrv = ja.jqv; e.rrs = ja.jqs; e.rri = ja.jqi;
-        e.ops = L.cpack; e.sm0 = c->sm0; e.im0 = c->im0;
-        e.ph = c->cph; e.beta = beta; e.keep = 0.0;
-        e.fcv = c->fcv; e.fcs = c->fcs; e.colour = 0;
-        launch_elem_cns<P>(c, e, full, &offs);
-        hipLaunchKernelGGL((k_jac_collect<P, NVC>), bN, tN, 0, c->stream, a);
-    }
-    check(hipGetLastError(), "jacobian launch");
-}
-
-// ins: the unperturbed residuals of the batch elements, then all their columns in one
-// launch (entries are independent: no colours, no scatter, the state is only read)
-template <int P>
-void jacobian_ins(hpg_ctx* c, const int* d_tind, int nel, int N, double eps_r, double eps_a, double* base, double* K) {
-    const Level& L = c->lv[c->log2p];
-    ElemArgs e{};
-    e.pnts = c->pnts; e.tri_pnt = c->tri_pnt; e.tri_seg = c->tri_seg; e.tri_sgn = c->tri_sgn;
-    e.order = d_tind;
-    e.ugv = c->ugv; e.ugs = c->ugs; e.ugi = c->ugi;
-    e.ops = L.pack; e.sm0 = c->sm0; e.im0 = c->im0;
-    e.rho = c->prm.rho; e.mu = c->prm.mu; e.adis = c->prm.adis; e.beta = c->prm.beta[0];
-    e.fcv = c->fcv; e.fcs = c->fcs;
-    e.jeps_r = eps_r; e.jeps_a = eps_a; e.jbase = base;
-    const bool full = e.beta > 0.0;
-    auto launch = [&](int cols, double* k) {
-        e.jcols = cols; e.jK = k; e.begin = 0; e.end = nel * cols;
-        const int nlogical = (e.end + 63) / 64;
-        if (full) {
-            static const int cap = resident_blocks((const void*)k_elem_ins_jac<P, true>);
-            hipLaunchKernelGGL((k_elem_ins_jac<P, true>), dim3(persistent_grid(nlogical, cap)), dim3(256), 0, c->stream, e);
-        } else {
-            static const int cap = resident_blocks((const void*)k_elem_ins_jac<P, false>);
-            hipLaunchKernelGGL((k_elem_ins_jac<P, false>), dim3(persistent_grid(nlogical, cap)), dim3(256), 0, c->stream, e);
-        }
+        e.ops = L.pack; e.sm0 = c->sm0; e.im0 = c->im0; e.beta = beta;
+        e.fcv = c->fcv; e.fcs = c->fcs;
+        e.jeps_r = eps_r; e.jeps_a = eps_a; e.jbase = base;
     };
-    launch(1, nullptr);
-    launch(N, K);
+    auto launch = [&](auto e, auto kern, int cap, int cols, double* k) {
+        e.jcols = cols; e.jK = k; e.begin = 0; e.end = nel * cols;
+        hipLaunchKernelGGL(kern, dim3(persistent_grid((e.end + 63) / 64, cap)), dim3(256), 0, c->stream, e);
+    };
+    auto both = [&](const auto& e, auto kern, int cap) {
+        launch(e, kern, cap, 1, nullptr);
+        launch(e, kern, cap, N, K);
+    };
+    if (c->physics == HPG_PHYSICS_CNS) {
+        CnsElemArgs e{};
+        mesh(e);
+        e.ph = c->cph;
+        static const int cf = resident_blocks((const void*)k_elem_cns_jac<P, true>);
+        static const int ci = resident_blocks((const void*)k_elem_cns_jac<P, false>);
+        if (full) both(e, k_elem_cns_jac<P, true>, cf);
+        else both(e, k_elem_cns_jac<P, false>, ci);
+    } else {
+        ElemArgs e{};
+        mesh(e);
+        e.rho = c->prm.rho; e.mu = c->prm.mu; e.adis = c->prm.adis;
+        static const int cf = resident_blocks((const void*)k_elem_ins_jac<P, true>);
+        static const int ci = resident_blocks((const void*)k_elem_ins_jac<P, false>);
+        if (full) both(e, k_elem_ins_jac<P, true>, cf);
+        else both(e, k_elem_ins_jac<P, false>, ci);
+    }
     check(hipGetLastError(), "jacobian launch");
 }
 
@@ -1366,7 +1308,6 @@ int hpg_create(const hpg_tri_mesh* m, const hpg_params* prm, hpg_ctx** out) {
         c->fcs = c->upload(fcs.data(), fcs.size());
         c->order = c->upload(order.data(), order.size());
         c->coff = off;
-        c->tcol = tcol;
         {
             std::vector<int> sides, bid(neseg, 0);
             if (neseg > 0) sides.assign(m->ebdry_seg, m->ebdry_seg + neseg);
@@ -1456,6 +1397,8 @@ int hpg_create(const hpg_tri_mesh* m, const hpg_params* prm, hpg_ctx** out) {
             c->vpc = c->alloc<double>((size_t)np * 16);
             c->spc = c->alloc<double>((size_t)ns * 16);
             c->tpc = c->alloc<double>((size_t)nt * 16);
+            const std::vector<unsigned char> tc(tcol.begin(), tcol.end());
+            c->tcol = c->upload(tc.data(), tc.size());
             c->rtv = c->alloc<double>(nv);
             c->rts = c->alloc<double>(nsz);
             // inflow boundaries (essential u, v, RT): their vertices (once each) and sides
@@ -1502,11 +1445,11 @@ int hpg_create(const hpg_tri_mesh* m, const hpg_params* prm, hpg_ctx** out) {
         c->featX = c->alloc<float>((size_t)nt * MLP_IN);
         c->mlpY = c->alloc<float>((size_t)nt * MLP_OUT);
         c->jdiag = c->alloc<double>((size_t)nt * 3 * NV);
+        // element-major vertex and side modes of the finest level (3p per element)
+        c->eres = c->alloc<double>((size_t)nt * 3 * p0 * 2 * NVX);
+        c->eout = c->alloc<double>((size_t)neseg * (p0 + 1) * NVX);
         if (c->physics == HPG_PHYSICS_INS) {
-            // element-major vertex and side modes of the finest level (3p per element)
-            c->eres = c->alloc<double>((size_t)nt * 3 * (1 << c->log2pmax) * 2 * NV);
-            c->eres32 = c->alloc<float>((size_t)nt * 3 * (1 << c->log2pmax) * 2 * NV);
-            c->eout = c->alloc<double>((size_t)neseg * (p0 + 1) * NV);
+            c->eres32 = c->alloc<float>((size_t)nt * 3 * p0 * 2 * NV);
             c->eout32 = c->alloc<float>((size_t)neseg * (p0 + 1) * NV);
             c->tprcn_vx = c->alloc<double>((size_t)nt * NV);
             c->tprcn_sd = c->alloc<double>((size_t)nt * NV);
@@ -1880,68 +1823,24 @@ int hpg_element_jacobian(hpg_ctx* c, const int* tind, int nel, double eps_r, dou
             seen[tind[j]] = 1;
         }
         CallBuffers B(c->stream);
-        if (c->physics == HPG_PHYSICS_INS) {
-            int* d_tind = B.get<int>(nel);
-            check(hipMemcpyAsync(d_tind, tind, (size_t)nel * 4, hipMemcpyHostToDevice, c->stream), "H2D");
-            // a slice of the batch at a time: the entry index of a launch is a 32-bit int
-            // and the scratch for K stays within 256 MiB however large the batch is
-            const int slice = (int)std::min<size_t>(nel, std::max<size_t>(1, (size_t)(1 << 25) / ((size_t)N * N)));
-            double* base = B.get<double>((size_t)slice * N);
-            double* dK = B.get<double>((size_t)slice * N * N);
-            for (int j0 = 0; j0 < nel; j0 += slice) {
-                const int nj = std::min(slice, nel - j0);
-                switch (L.p) {
-                    case 1: jacobian_ins<1>(c, d_tind + j0, nj, N, eps_r, eps_a, base, dK); break;
-                    case 2: jacobian_ins<2>(c, d_tind + j0, nj, N, eps_r, eps_a, base, dK); break;
-                    case 4: jacobian_ins<4>(c, d_tind + j0, nj, N, eps_r, eps_a, base, dK); break;
-                    default: throw std::runtime_error("unsupported p");
-                }
-                check(hipMemcpyAsync(K + (size_t)j0 * N * N, dK, (size_t)nj * N * N * 8, hipMemcpyDeviceToHost, c->stream), "D2H");
-                check(hipStreamSynchronize(c->stream), "sync");
-            }
-            return 0;
-        }
-        // cns: group the batch by colour (stable in the caller's order)
-        const int ncol = (int)c->coff.size() - 1;
-        std::vector<int> cnt(ncol + 1, 0), jel(nel), jpos(nel);
-        for (int j = 0; j < nel; ++j) ++cnt[c->tcol[tind[j]] + 1];
-        for (int k = 0; k < ncol; ++k) cnt[k + 1] += cnt[k];
-        const std::vector<int> joff = cnt;
-        for (int j = 0; j < nel; ++j) {
-            const int q = cnt[c->tcol[tind[j]]]++;
-            jel[q] = tind[j];
-            jpos[q] = j;
-        }
-        JacArgs ja{};
-        ja.jel = B.get<int>(nel);
-        ja.jpos = B.get<int>(nel);
-        check(hipMemcpyAsync((void*)ja.jel, jel.data(), (size_t)nel * 4, hipMemcpyHostToDevice, c->stream), "H2D");
-        check(hipMemcpyAsync((void*)ja.jpos, jpos.data(), (size_t)nel * 4, hipMemcpyHostToDevice, c->stream), "H2D");
-        ja.tri_pnt = c->tri_pnt; ja.tri_seg = c->tri_seg; ja.tri_sgn = c->tri_sgn;
-        ja.sm0 = c->sm0; ja.im0 = c->im0;
-        ja.ugv = c->ugv; ja.ugs = c->ugs; ja.ugi = c->ugi;
-        const size_t nv = (size_t)c->npnt * nvv, ns = (size_t)c->nseg * c->sm0 * nvv, ni = (size_t)c->ntri * c->im0 * nvv;
-        ja.jrv = B.get<double>(nv, true); ja.jrs = B.get<double>(ns, true); ja.jri = B.get<double>(ni, true);
-        ja.jqv = B.get<double>(nv, true); ja.jqs = B.get<double>(ns, true); ja.jqi = B.get<double>(ni, true);
-        ja.dw = B.get<double>((size_t)nel * nvv);
-        ja.save = B.get<double>(nel);
-        ja.base = B.get<double>((size_t)nel * N);
-        ja.K = B.get<double>((size_t)nel * N * N);
-        ja.eps_r = eps_r; ja.eps_a = eps_a;
-        for (int col = 0; col < ncol; ++col) {
-            if (joff[col + 1] == joff[col]) continue;
-            JacArgs a = ja;
-            a.begin = joff[col];
-            a.end = joff[col + 1];
+        int* d_tind = B.get<int>(nel);
+        check(hipMemcpyAsync(d_tind, tind, (size_t)nel * 4, hipMemcpyHostToDevice, c->stream), "H2D");
+        // a slice of the batch at a time: the entry index of a launch is a 32-bit int
+        // and the scratch for K stays within 256 MiB however large the batch is
+        const int slice = (int)std::min<size_t>(nel, std::max<size_t>(1, (size_t)(1 << 25) / ((size_t)N * N)));
+        double* base = B.get<double>((size_t)slice * N);
+        double* dK = B.get<double>((size_t)slice * N * N);
+        for (int j0 = 0; j0 < nel; j0 += slice) {
+            const int nj = std::min(slice, nel - j0);
             switch (L.p) {
-                case 1: jacobian_colour_cns<1>(c, a, N); break;
-                case 2: jacobian_colour_cns<2>(c, a, N); break;
-                case 4: jacobian_colour_cns<4>(c, a, N); break;
+                case 1: element_jacobians<1>(c, d_tind + j0, nj, N, eps_r, eps_a, base, dK); break;
+                case 2: element_jacobians<2>(c, d_tind + j0, nj, N, eps_r, eps_a, base, dK); break;
+                case 4: element_jacobians<4>(c, d_tind + j0, nj, N, eps_r, eps_a, base, dK); break;
                 default: throw std::runtime_error("unsupported p");
             }
+            check(hipMemcpyAsync(K + (size_t)j0 * N * N, dK, (size_t)nj * N * N * 8, hipMemcpyDeviceToHost, c->stream), "D2H");
+            check(hipStreamSynchronize(c->stream), "sync");
         }
-        check(hipMemcpyAsync(K, ja.K, (size_t)nel * N * N * 8, hipMemcpyDeviceToHost, c->stream), "D2H");
-        check(hipStreamSynchronize(c->stream), "sync");
     });
     return 0;
 }

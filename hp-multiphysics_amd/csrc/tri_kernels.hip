@@ -843,10 +843,10 @@ __global__ __launch_bounds__(256) void k_elem_ins32_em_curved(ElemArgs32 a, floa
 // colour and the later colours of the scatter do.  FP32 (the defect correction's inner
 // solve): the constant source sfac[0] * src enters with the first element, as on the
 // scatter's first visit.
-// E: type of the element results (float under FP64 sums in the cns inner solve).  The
-// boundary-edge results follow the elements (eout, written by the element launch's edge
+// summed: the elements' first entry already is lf_im + beta lf_re.  The boundary-edge
+// results follow the elements (eout, written by the element launch's edge
 // blocks): a vertex adds its edges' end entries in list order, a boundary side its own.
-template <typename T, typename E = T>
+template <typename T>
 struct GatherArgsT {
     int npnt, nseg, sm, sm0, bm;
     const int* vt_ptr;
@@ -854,7 +854,7 @@ struct GatherArgsT {
     const int* vt_loc;
     const int* st_tri;
     const int* st_loc;
-    const E* eres;
+    const T* eres;
     const int* vb_ptr;   // boundary-edge ends at each vertex: 2 * edge + end
     const int* vb_ent;
     const int* sedge;    // first edge of a side in the boundary lists (-1: none) and
@@ -865,26 +865,26 @@ struct GatherArgsT {
     T* ress;
     T* rrs;
     T keep;
-    int full;
+    int full, summed;
     const double* srcv;  // defect source, may be null
     const double* srcs;
     const double* sfac;
 };
 
-template <typename T, int NVn, typename E>
-__device__ __forceinline__ void gather_sum(const GatherArgsT<T, E>& a, const E* e, int n, T sign, T& acc, T& accr) {
-    const T li = sign * T(e[n]);
+template <typename T, int NVn>
+__device__ __forceinline__ void gather_sum(const GatherArgsT<T>& a, const T* e, int n, T sign, T& acc, T& accr) {
+    const T li = sign * e[n];
     if (a.full) {
-        const T lr = sign * T(e[NVn + n]);
+        const T lr = sign * e[NVn + n];
         accr += lr;
-        acc = (acc + lr) + li;
+        acc = (a.summed ? acc : acc + lr) + li;
     } else {
         acc = acc + li;
     }
 }
 
-template <typename T, int NVn, typename E = T>
-__global__ __launch_bounds__(256) void k_gather_vs(GatherArgsT<T, E> a) {
+template <typename T, int NVn>
+__global__ __launch_bounds__(256) void k_gather_vs(GatherArgsT<T> a) {
     const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long nvl = (long)a.npnt * NVn;
     const T keep = a.keep;
@@ -894,7 +894,7 @@ __global__ __launch_bounds__(256) void k_gather_vs(GatherArgsT<T, E> a) {
         const T r0 = keep == T(0) ? T(0) : keep * a.rrv[g];
         T acc = r0, accr = r0;
         for (int k = a.vt_ptr[v]; k < a.vt_ptr[v + 1]; ++k) {
-            gather_sum<T, NVn, E>(a, a.eres + ((long)a.vt_tri[k] * a.bm + a.vt_loc[k]) * (2 * NVn), n, T(1), acc, accr);
+            gather_sum<T, NVn>(a, a.eres + ((long)a.vt_tri[k] * a.bm + a.vt_loc[k]) * (2 * NVn), n, T(1), acc, accr);
             if (k == a.vt_ptr[v] && a.srcv) acc = acc + T(a.srcv[g] * a.sfac[0]);
         }
         for (int k = a.vb_ptr[v]; k < a.vb_ptr[v + 1]; ++k) {
@@ -922,7 +922,7 @@ __global__ __launch_bounds__(256) void k_gather_vs(GatherArgsT<T, E> a) {
         // way: its odd modes change sign in this side's frame
         const int sl = a.st_loc[2 * s + slot];
         const int mode = 3 + (sl & 3) * a.sm + m;
-        gather_sum<T, NVn, E>(a, a.eres + ((long)t * a.bm + mode) * (2 * NVn), n, ((sl & 4) && (m & 1)) ? T(-1) : T(1),
+        gather_sum<T, NVn>(a, a.eres + ((long)t * a.bm + mode) * (2 * NVn), n, ((sl & 4) && (m & 1)) ? T(-1) : T(1),
                               acc, accr);
         if (first && a.srcs) acc = acc + T(a.srcs[o] * a.sfac[0]);
         first = false;

@@ -3,15 +3,11 @@
 // elements, diagonal preconditioner with the per-vertex 4x4 block preconditioner of
 // the primitive-variable projection.
 //
-// The element residual is dominated by pointwise work: a 4x4 stabilisation matrix
-// (eigen-decomposed flux Jacobians, an LU solve) at every Gauss point.  One element
-// therefore maps to 32 lanes (half a wave), one Gauss point per lane (G <= 25):
-// modal transforms are per-lane dot products against operator rows staged in LDS
-// (stored point-contiguous, so the 32 lanes of a half-wave read consecutive words),
-// and the derivative and integration contractions exchange point values through
-// LDS.  The element loop is persistent: each workgroup stages the operators once
-// and walks a contiguous range of 8-element octets of one colour, the ranges laid
-// out so that each XCD works on a contiguous part of the colour.
+// Element residual: the matrix-core layout of tri_kernels.hip (16 elements per wave, every
+// transform a contraction on v_mfma_f64_16x16x4f64 or v_mfma_f32_16x16x4f32), with the
+// pointwise physics -- the stabilisation solve at every Gauss point above all -- in the
+// lane that holds the point.  project_new_variables keeps a half-wave per element, one
+// Gauss point per lane, and exchanges point values through LDS.
 #include <hip/hip_runtime.h>
 #include "tri_kernels.h"
 
@@ -253,41 +249,40 @@ __device__ __forceinline__ void lower4(const double L[16], double r[4]) {
 }
 
 // ---------------------------------------------------------------------------------
-// tri_hp_cns::element_rsdl, straight branch (tri_hp/cns/rsdl.cpp:312-530), steady,
-// source "zero", CALC_TAU2 (tau at every Gauss point), for the elements
-// order[begin:end) of one colour.
-// T: arithmetic type of the kernel (double, or float in the FP32 inner solve of the
-// defect correction); state and residual arrays are FP64 in both
+// T: arithmetic type of the element kernel (double, or float in the FP32 inner solve of
+// the defect correction); the state and residual arrays are FP64 in both
 template <typename T>
 struct CnsElemArgsT {
     const double* pnts;
     const int* tri_pnt;
     const int* tri_seg;
     const int* tri_sgn;
-    const int* order;
+    const int* order;  // null: mesh order
     int begin, end;
     const double* ugv;
     const double* ugs;
     const double* ugi;
-    double* resv;
-    double* ress;
     double* resi;
-    double* rrv;
-    double* rrs;
     double* rri;
-    const T* ops;  // CDims<P> pack
+    double* eres;  // element-major vertex and side modes, (element, 3p, im | re, 4)
+    const T* ops;  // double: the operator pack of the ins element kernel; float: CDims pack
     int sm0, im0;
     CnsPhys ph;
     double beta, keep;
+    // FP32 kernel: constant source sfac[0] * srci of the interior modes (the scaled FP64
+    // residual of the defect correction); null otherwise
+    const double* srci;
+    const double* sfac;
+    // FP32 kernel: each element's colour and the first colour at each vertex and side
+    const unsigned char* tcol;
     const unsigned char* fcv;
     const unsigned char* fcs;
     int colour;
-    // FP32 kernel: constant source sfac[0] * src added on the first visit of every
-    // coefficient (the scaled FP64 residual of the defect correction); null otherwise
-    const double* srcv;
-    const double* srcs;
-    const double* srci;
-    const double* sfac;
+    // element Jacobians: as ElemArgsT
+    int jcols;
+    double jeps_r, jeps_a;
+    double* jbase;
+    double* jK;
 };
 typedef CnsElemArgsT<double> CnsElemArgs;
 typedef CnsElemArgsT<float> CnsElemArgs32;
@@ -304,14 +299,458 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-#define HPG_OCTET_LOOP(noct, oc)                                                          \
-    const int nbx_ = gridDim.x >> 3, xcd_ = blockIdx.x & 7, jb_ = blockIdx.x >> 3;       \
+#define HPG_OCTET_LOOP_OF(noct, oc, blk, nblk)                                            \
+    const int nbx_ = (nblk) >> 3, xcd_ = (blk) & 7, jb_ = (blk) >> 3;                      \
     const int per_ = ((noct) + 7) / 8;                                                     \
     const int oend_ = min((xcd_ + 1) * per_, (noct));                                      \
     for (int oc = xcd_ * per_ + jb_; oc < oend_; oc += nbx_)
+#define HPG_OCTET_LOOP(noct, oc) HPG_OCTET_LOOP_OF(noct, oc, (int)blockIdx.x, (int)gridDim.x)
 
+// Stabilised residual Tau res at one Gauss point, Tau = Tinv^-1 P dpdc with
+// Tinv = 2 (|A| + |B| + h S) / h (tri_hp/cns/setup_preconditioner.cpp:241-515, alph = 0,
+// hdt = 0; the full matrices are cns_tau).  Only one right-hand side is needed here, and
+// the closed forms leave few entries: with |A| = V |L| W written out, Tinv couples u and v
+// to p alone, so rows 1 and 2 are eliminated by their own positive pivots and a 2 x 2
+// system in (p, RT) remains.  About 200 operations against about 700 for the general
+// products and a four-column solve.
+struct CnsStab {
+    double gam, gm1, gogm1, kg, mu, acp, h, ih, hh;
+};
+
+__device__ __forceinline__ void cns_stab(const CnsStab& k, double pr, double u, double v, double rt, const double* res, double* x) {
+    const double irho = rt / pr, rho = pr / rt;
+    const double qq = u * u + v * v, ke = 0.5 * qq, c2 = k.gam * rt;
+    const double ic = 1.0 / sqrt(c2);  // NaN for RT < 0, as every quantity below
+    const double nu = k.mu * irho, al = k.acp * irho;
+    const double m2u = qq * ic * ic;
+    const double m2 = m2u > 1e-10 ? m2u : 1e-10;
+    double b2 = 1.0;
+    if (m2 < 0.64) {
+        const double hc = k.ih * ic, a = 4.0 * nu * hc, b = 2.0 * al * hc;
+        const double s = m2 / (1.0 - m2) + a * a + b * b;
+        b2 = s < 1.0 ? s : 1.0;
+    }
+    const double bm = b2 - 1.0, c3 = bm * irho / k.gogm1;
+    const double f4 = 4.0 * b2 * c2, bb = 1.0 - 2.0 * b2 + b2 * b2;
+    // |A|: eigenvalues e0, e1, |u| with p, m the roots of the acoustic pair
+    const double t1 = sqrt(u * u * bb + f4), it1 = 1.0 / t1;
+    const double p1 = 0.5 * (u * bm + t1), m1 = 0.5 * (u * bm - t1);
+    const double e0 = fabs(0.5 * (u + u * b2 + t1)) * it1, e1 = fabs(0.5 * (u + u * b2 - t1)) * it1;
+    const double au = fabs(u), av = fabs(v);
+    const double A00 = p1 * e0 - m1 * e1, A01 = p1 * m1 * (e1 - e0), A10 = irho * (e0 - e1), A11 = p1 * e1 - m1 * e0;
+    const double t2 = sqrt(v * v * bb + f4), it2 = 1.0 / t2;
+    const double p2 = 0.5 * (v * bm + t2), n2 = 0.5 * (v * bm - t2);
+    const double g0 = fabs(0.5 * (v + v * b2 + t2)) * it2, g1 = fabs(0.5 * (v + v * b2 - t2)) * it2;
+    const double B00 = p2 * g0 - n2 * g1, B02 = p2 * n2 * (g1 - g0), B20 = irho * (g0 - g1), B22 = p2 * g1 - n2 * g0;
+    // h S = h (P dpdc) diag(0, nu, nu, alpha) / h^2
+    const double Dn = nu * k.ih, Da = al * k.ih, w = k.gm1 * (irho + c3), kr = k.kg * irho;
+    const double M00 = A00 + B00, M01 = rho * A01 - b2 * k.gm1 * u * Dn, M02 = rho * B02 - b2 * k.gm1 * v * Dn;
+    const double M03 = b2 * k.gm1 * Da;
+    const double M11 = A11 + av + irho * Dn, M22 = au + B22 + irho * Dn;
+    const double M30 = kr * (A00 - au) + kr * (B00 - av), M31 = k.kg * A01 - w * u * Dn, M32 = k.kg * B02 - w * v * Dn;
+    const double M33 = au + av + w * Da;
+    // P dpdc res
+    const double z = k.gm1 * (ke * res[0] - u * res[1] - v * res[2] + res[3]);
+    const double r0 = b2 * z, r1 = irho * (res[1] - u * res[0]), r2 = irho * (res[2] - v * res[0]);
+    const double r3 = irho * (z - rt * res[0]) + c3 * z;
+    const double i1 = 1.0 / M11, i2 = 1.0 / M22;
+    const double a1 = A10 * i1, a2 = B20 * i2, y1 = r1 * i1, y2 = r2 * i2;
+    const double d00 = M00 - M01 * a1 - M02 * a2, d30 = M30 - M31 * a1 - M32 * a2;
+    const double s0 = r0 - M01 * y1 - M02 * y2, s3 = r3 - M31 * y1 - M32 * y2;
+    const double q = d30 / d00;
+    const double x3 = (s3 - q * s0) / (M33 - q * M03);
+    const double x0 = (s0 - M03 * x3) / d00;
+    x[0] = k.hh * x0;
+    x[1] = k.hh * (y1 - a1 * x0);
+    x[2] = k.hh * (y2 - a2 * x0);
+    x[3] = k.hh * x3;
+}
+
+// tri_hp_cns::element_rsdl, straight branch (tri_hp/cns/rsdl.cpp:312-530), steady, source
+// "zero", CALC_TAU2 (tau at every Gauss point), 16 elements per wave in the layout of
+// elem_ins_body: operators of the ins pack, accumulators fed back as operands, element-major
+// output.  Fluxes are formed right before the matrix instructions that consume them; the
+// values (U), the viscous fluxes (F) and the strong residual (R) of the element's points
+// stay in registers.  JAC: entries are (element, column) pairs as in elem_ins_body.
+template <int P, bool FULL, bool JAC = false>
+__device__ __forceinline__ void elem_cns_body(const CnsElemArgs& a, int eblk = 0) {
+    using D = Dims<P>;
+    using T = double;
+    using V4 = d4;
+    constexpr int GT = D::GT, KT = D::KT;
+    __shared__ T sops[D::PACK];
+    for (int k = threadIdx.x; k < D::PACK; k += blockDim.x) sops[k] = a.ops[k];
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int e = lane & 15, q = lane >> 4;
+    const int WX = (((int)gridDim.x - eblk) >> 3) * 4;
+    const int rank = (((int)blockIdx.x - eblk) >> 3) * 4 + wv;
+    const int xcd = blockIdx.x & 7;
+    const int ng = (a.end - a.begin + 15) >> 4;
+    const int gpx = (ng + 7) >> 3;
+    const int g0 = xcd * gpx + rank;
+    const int gend = min(ng, (xcd + 1) * gpx);
+    if (g0 >= gend) return;
+
+    CnsStab ks;
+    ks.gam = T(a.ph.gamma);
+    ks.gm1 = ks.gam - T(1);
+    ks.gogm1 = ks.gam / ks.gm1;
+    ks.kg = ks.gm1 / ks.gam;
+    ks.mu = T(a.ph.mu);
+    ks.acp = T(a.ph.kcond) / (ks.gogm1 * T(a.ph.Rgas));
+    const T igm1 = T(1) / ks.gm1;
+    // a K-step (tile kt, register i; points 16 kt + 4 i + q) of padding points adds nothing
+    auto dead = [](int kt, int i) { return 16 * kt + 4 * i >= D::G; };
+
+    ElemSlots<P> S = elem_slots<P, NVC>(a, elem_conn(a, elem_of_group<JAC>(a, g0, gend, e)), q);
+    ElemConn cnext = elem_conn(a, elem_of_group<JAC>(a, g0 + WX, gend, e));
+    int tnext2 = elem_of_group<JAC>(a, g0 + 2 * WX, gend, e);
+    for (int g = g0; g < gend; g += WX) {
+        const ElemSlots<P> Sn = elem_slots<P, NVC>(a, cnext, q);
+        const ElemConn cn2 = elem_conn(a, tnext2);
+        const int tn3 = elem_of_group<JAC>(a, g + 3 * WX, gend, e);
+
+        // modal coefficients: K-step s of lane l is mode 4s + l/16; padding elements carry
+        // p = RT = 1 in their vertex modes
+        T b[NVC][KT];
+#pragma unroll
+        for (int s = 0; s < KT; ++s) {
+            const int k = 4 * s + q, kind = mode_kind<P>(k);
+            const bool live = S.t >= 0 && k < D::TM;
+            const int off = S.off[s] < 0 ? ~S.off[s] : S.off[s];
+            const T sg = S.off[s] < 0 ? T(-1) : T(1);
+            const double* src = kind == 0 ? a.ugv : (kind == 1 ? a.ugs : a.ugi);
+#pragma unroll
+            for (int n = 0; n < NVC; ++n)
+                b[n][s] = live ? sg * T(src[off + n]) : ((k < 3 && (n == 0 || n == 3)) ? T(1) : T(0));
+        }
+        int jcol = 0, jel = 0;
+        T jdw = T(1);
+        if constexpr (JAC) {
+            const int idx = a.begin + g * 16 + e;
+            jel = idx / a.jcols;
+            jcol = idx - jel * a.jcols;
+            if (a.jK) {
+                const int jm = jcol / NVC, jn = jcol - jm * NVC;
+#pragma unroll
+                for (int n = 0; n < NVC; ++n) {
+                    T v = T(0);
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) v = v + fabs(__shfl(b[n][0], 16 * k + e, 64));
+                    const T dw = v * T(a.jeps_r) + T(a.jeps_a);
+                    if (n != jn) continue;
+                    jdw = dw;
+#pragma unroll
+                    for (int s = 0; s < KT; ++s)
+                        if (4 * s + q == jm && S.t >= 0) b[n][s] += dw;
+                }
+            }
+        }
+        const double x0 = S.x[0], y0 = S.y[0], x1 = S.x[1], y1 = S.y[1], x2 = S.x[2], y2 = S.y[2];
+        // ldcrd(n,0) = dx_n/dr, ldcrd(n,1) = dx_n/ds (rsdl.cpp:56-59)
+        const T l00 = T(0.5 * (x2 - x1)), l01 = T(0.5 * (x0 - x1));
+        const T l10 = T(0.5 * (y2 - y1)), l11 = T(0.5 * (y0 - y1));
+
+        const V4 zz = {T(0), T(0), T(0), T(0)};
+        V4 U[NVC][GT];
+#pragma unroll
+        for (int mt = 0; mt < GT; ++mt) {
+            V4 c[NVC] = {zz, zz, zz, zz};
+#pragma unroll
+            for (int s = 0; s < KT; ++s) {
+                const T av = sops[D::OFF_P + (mt * KT + s) * 64 + lane];
+#pragma unroll
+                for (int n = 0; n < NVC; ++n) c[n] = mfma(av, b[n][s], c[n]);
+            }
+            // padding rows of the point tiles: p = u = v = RT = 1, where the pointwise work
+            // is finite also for mu = 0 (a zero operator column does not cancel a NaN)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (16 * mt + 4 * i + q >= D::G) { c[0][i] = T(1); c[1][i] = T(1); c[2][i] = T(1); c[3][i] = T(1); }
+#pragma unroll
+            for (int n = 0; n < NVC; ++n) U[n][mt] = c[n];
+        }
+        // convective fluxes of point (kt, i) (rsdl.cpp:315-351)
+        auto conv = [&](int kt, int i, T* cv) {
+            const T pr = U[0][kt][i], u = U[1][kt][i], v = U[2][kt][i], rt = U[3][kt][i];
+            const T rho = pr / rt, fx = rho * u, fy = rho * v;
+            cv[0] = l11 * fx - l01 * fy;
+            cv[1] = -l10 * fx + l00 * fy;
+            cv[2] = u * cv[0] + l11 * pr;
+            cv[3] = u * cv[1] - l10 * pr;
+            cv[4] = v * cv[0] - l01 * pr;
+            cv[5] = v * cv[1] + l00 * pr;
+            const T E = rt * igm1 + T(0.5) * (u * u + v * v);
+            const T nx = E * fx + pr * u, ny = E * fy + pr * v;
+            cv[6] = l11 * nx - l01 * ny;
+            cv[7] = -l10 * nx + l00 * ny;
+        };
+
+        V4 LI[NVC] = {zz, zz, zz, zz}, LR[NVC] = {zz, zz, zz, zz};
+        if constexpr (!FULL) {
+#pragma unroll
+            for (int kt = 0; kt < GT; ++kt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (dead(kt, i)) continue;
+                    T cv[8];
+                    conv(kt, i, cv);
+                    const T ar = sops[D::OFF_IR + (kt * 4 + i) * 64 + lane];
+                    const T as = sops[D::OFF_IS + (kt * 4 + i) * 64 + lane];
+#pragma unroll
+                    for (int n = 0; n < NVC; ++n) {
+                        LI[n] = mfma(ar, cv[2 * n], LI[n]);
+                        LI[n] = mfma(as, cv[2 * n + 1], LI[n]);
+                    }
+                }
+        } else {
+            // viscous stress and heat flux coefficients (rsdl.cpp:355-380), rhorbd0 = 0
+            const T cjcb = l00 * l11 - l10 * l01;
+            const T mj = ks.mu / cjcb, kj = T(a.ph.kcond) / cjcb / T(a.ph.Rgas);
+            const T f43 = T(4.) / T(3.), f23 = T(2.) / T(3.), f13 = T(1.) / T(3.);
+            const T v0000 = -mj * (f43 * l11 * l11 + l01 * l01), v0011 = -mj * (f43 * l10 * l10 + l00 * l00);
+            const T v0001 = mj * (f43 * l11 * l10 + l01 * l00);
+            const T v1100 = -mj * (l11 * l11 + f43 * l01 * l01), v1111 = -mj * (l10 * l10 + f43 * l00 * l00);
+            const T v1101 = mj * (l11 * l10 + f43 * l01 * l00);
+            const T v0100 = mj * f13 * l01 * l11, v0111 = mj * f13 * l00 * l10;
+            const T v0101 = -mj * (l01 * l10 - f23 * l00 * l11), v0110 = -mj * (l00 * l11 - f23 * l01 * l10);
+            const T k00 = -kj * (l11 * l11 + l01 * l01), k11 = -kj * (l10 * l10 + l00 * l00);
+            const T k01 = kj * (l11 * l10 + l01 * l00);
+            T F[GT][4][6];
+            V4 R[NVC][GT];
+#pragma unroll
+            for (int mt = 0; mt < GT; ++mt)
+#pragma unroll
+                for (int n = 0; n < NVC; ++n) R[n][mt] = zz;
+#pragma unroll
+            for (int kt = 0; kt < GT; ++kt) {
+                V4 dr[3] = {zz, zz, zz}, ds[3] = {zz, zz, zz};  // of u, v, RT on point tile kt
+#pragma unroll
+                for (int s = 0; s < KT; ++s) {
+                    const T ar = sops[D::OFF_PR + (kt * KT + s) * 64 + lane];
+                    const T as = sops[D::OFF_PS + (kt * KT + s) * 64 + lane];
+#pragma unroll
+                    for (int n = 0; n < 3; ++n) {
+                        dr[n] = mfma(ar, b[n + 1][s], dr[n]);
+                        ds[n] = mfma(as, b[n + 1][s], ds[n]);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (dead(kt, i)) continue;
+                    if (GT > 1) __builtin_amdgcn_sched_barrier(0);
+                    T cv[8];
+                    conv(kt, i, cv);
+                    const T ar = sops[D::OFF_IR + (kt * 4 + i) * 64 + lane];
+                    const T as = sops[D::OFF_IS + (kt * 4 + i) * 64 + lane];
+#pragma unroll
+                    for (int n = 0; n < NVC; ++n) {
+                        LI[n] = mfma(ar, cv[2 * n], LI[n]);
+                        LI[n] = mfma(as, cv[2 * n + 1], LI[n]);
+                    }
+                    const T ur = dr[0][i], vr = dr[1][i], tr = dr[2][i], us = ds[0][i], vs = ds[1][i], ts = ds[2][i];
+                    const T u = U[1][kt][i], v = U[2][kt][i];
+                    T* f = F[kt][i];
+                    f[0] = v0000 * ur + v0100 * vr + v0001 * us + v0101 * vs;
+                    f[1] = v0001 * ur + v0110 * vr + v0011 * us + v0111 * vs;
+                    f[2] = v0100 * ur + v1100 * vr + v0110 * us + v1101 * vs;
+                    f[3] = v0101 * ur + v1101 * vr + v0111 * us + v1111 * vs;
+                    f[4] = k00 * tr + k01 * ts + f[0] * u + f[2] * v;
+                    f[5] = k01 * tr + k11 * ts + f[1] * u + f[3] * v;
+#pragma unroll
+                    for (int j = 0; j < 6; ++j) cv[j + 2] += f[j];
+                    // strong residual: derivr/derivs of the total fluxes (rsdl.cpp:425-429)
+#pragma unroll
+                    for (int mt = 0; mt < GT; ++mt) {
+                        const T odr = sops[D::OFF_DR + ((mt * GT + kt) * 4 + i) * 64 + lane];
+                        const T ods = sops[D::OFF_DS + ((mt * GT + kt) * 4 + i) * 64 + lane];
+#pragma unroll
+                        for (int n = 0; n < NVC; ++n) {
+                            R[n][mt] = mfma(odr, cv[2 * n], R[n][mt]);
+                            R[n][mt] = mfma(ods, cv[2 * n + 1], R[n][mt]);
+                        }
+                    }
+                }
+            }
+            // CALC_TAU2 (rsdl.cpp:431-452), the stabilisation (:454-488) and
+            // lf_re = intgrtrs(viscous - stabilisation fluxes) (:490-497)
+            const T dx1 = T(x0 - x2), dy1 = T(y0 - y2), dx2 = T(x1 - x0), dy2 = T(y1 - y0);
+            const T ar2 = dx1 * dy2 - dy1 * dx2;
+            const T perim = sqrt(dx1 * dx1 + dy1 * dy1) + sqrt(dx2 * dx2 + dy2 * dy2) +
+                            sqrt((dx1 + dx2) * (dx1 + dx2) + (dy1 + dy2) * (dy1 + dy2));
+            ks.h = T(0.25) * ar2 / ((ar2 / perim) * (T(0.25) * (P + 1) * (P + 1)));
+            ks.ih = T(1) / ks.h;
+            ks.hh = T(0.5) * ks.h * (T(a.ph.adis) / cjcb);
+#pragma unroll
+            for (int kt = 0; kt < GT; ++kt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (dead(kt, i)) continue;
+                    const T pr = U[0][kt][i], u = U[1][kt][i], v = U[2][kt][i], rt = U[3][kt][i];
+                    const T res[4] = {R[0][kt][i], R[1][kt][i], R[2][kt][i], R[3][kt][i]};
+                    if (GT > 1) __builtin_amdgcn_sched_barrier(0);  // one point's solve at a time (registers)
+                    T x[4];
+                    cns_stab(ks, pr, u, v, rt, res, x);
+                    // the primitive flux Jacobians A, B times x
+                    const T rho = pr / rt, H = ks.gogm1 * rt + T(0.5) * (u * u + v * v);
+                    const T dr = (x[0] - rho * x[3]) / rt;
+                    const T fa0 = u * dr + rho * x[1], fb0 = v * dr + rho * x[2];
+                    const T ru = rho * u, rv = rho * v;
+                    const T fa1 = u * fa0 + ru * x[1] + x[0], fb2 = v * fb0 + rv * x[2] + x[0];
+                    const T fab = u * fb0 + rv * x[1];
+                    const T en = u * x[1] + v * x[2] + ks.gogm1 * x[3];
+                    const T fa3 = H * fa0 + ru * en, fb3 = H * fb0 + rv * en;
+                    const T* f = F[kt][i];
+                    const T w[8] = {-(l11 * fa0 - l01 * fb0),        -(l00 * fb0 - l10 * fa0),
+                                    f[0] - (l11 * fa1 - l01 * fab), f[1] - (l00 * fab - l10 * fa1),
+                                    f[2] - (l11 * fab - l01 * fb2), f[3] - (l00 * fb2 - l10 * fab),
+                                    f[4] - (l11 * fa3 - l01 * fb3), f[5] - (l00 * fb3 - l10 * fa3)};
+                    const T ar = sops[D::OFF_IR + (kt * 4 + i) * 64 + lane];
+                    const T as = sops[D::OFF_IS + (kt * 4 + i) * 64 + lane];
+#pragma unroll
+                    for (int n = 0; n < NVC; ++n) {
+                        LR[n] = mfma(ar, w[2 * n], LR[n]);
+                        LR[n] = mfma(as, w[2 * n + 1], LR[n]);
+                    }
+                }
+        }
+
+        const T bt = T(a.beta);
+#pragma unroll
+        for (int s = 0; s < KT; ++s) {
+            const int k = 4 * s + q, kind = mode_kind<P>(k);
+            if (S.t < 0 || k >= D::TM) continue;
+            const T sg = S.off[s] < 0 ? T(-1) : T(1);
+            if constexpr (JAC) {
+                constexpr int N = D::TM * NVC;
+#pragma unroll
+                for (int n = 0; n < NVC; ++n) {
+                    const T rr = FULL ? LR[n][s] * bt + LI[n][s] : LI[n][s];
+                    const size_t r = (size_t)jel * N + (k * NVC + n);
+                    if (a.jK) a.jK[r * N + jcol] = (rr - a.jbase[r]) / jdw;
+                    else a.jbase[r] = rr;
+                }
+            } else if (kind < 2) {
+                double* o = a.eres + ((size_t)S.t * D::BM + k) * (2 * NVC);
+#pragma unroll
+                for (int n = 0; n < NVC; ++n) {
+                    o[n] = sg * LI[n][s];
+                    if constexpr (FULL) o[NVC + n] = sg * (LR[n][s] * bt);
+                }
+            } else {
+                const int off = S.off[s];
+#pragma unroll
+                for (int n = 0; n < NVC; ++n) {
+                    const double r0 = a.keep == 0.0 ? 0.0 : a.keep * a.rri[off + n];
+                    const double lr = FULL ? LR[n][s] * bt : 0.0;
+                    if (FULL || a.keep != 1.0) a.rri[off + n] = r0 + lr;
+                    a.resi[off + n] = r0 + lr + LI[n][s];
+                }
+            }
+        }
+        S = Sn;
+        cnext = cn2;
+        tnext2 = tn3;
+    }
+}
+
+// ---------------------------------------------------------------------------------
+// edge-boundary flux residual (tri_hp/hp_boundary.cpp:973-1049) with the
+// bdry_cns::generic flux (tri_hp/cns/bdry.cpp:192-245); p_bc = boundary pressure
+struct CnsEdgeArgs {
+    const int* eseg;
+    int end;
+    const int* seg_pnt;
+    const double* pnts;
+    const double* ugv;
+    const double* ugs;
+    double* eout;  // (edge, 2 ends then the side modes, 4), added by the gathers
+    const double* g1;
+    const double* dg1;
+    const double* w1;
+    int sm0;
+    double gamma, pbc;
+};
+
+template <int P>
+__device__ __forceinline__ void edge_cns_body(const CnsEdgeArgs& a, int idx) {
+    constexpr int SM = Dims<P>::SM, N1 = SM + 2, GPX = P + 1;
+    if (idx >= a.end) return;
+    const int sind = a.eseg[idx];
+    const int v0 = a.seg_pnt[2 * sind], v1 = a.seg_pnt[2 * sind + 1];
+    double uh[NVC][N1];
+#pragma unroll
+    for (int n = 0; n < NVC; ++n) {
+        uh[n][0] = a.ugv[v0 * NVC + n];
+        uh[n][1] = a.ugv[v1 * NVC + n];
+#pragma unroll
+        for (int m = 0; m < SM; ++m) uh[n][m + 2] = a.ugs[(sind * a.sm0 + m) * NVC + n];
+    }
+    const double X0 = a.pnts[2 * v0], Y0 = a.pnts[2 * v0 + 1], X1 = a.pnts[2 * v1], Y1 = a.pnts[2 * v1 + 1];
+    const double gm1 = a.gamma - 1.0, pbc = a.pbc;
+    double lf[NVC][N1];
+#pragma unroll
+    for (int n = 0; n < NVC; ++n)
+#pragma unroll
+        for (int k = 0; k < N1; ++k) lf[n][k] = 0.0;
+#pragma unroll
+    for (int ip = 0; ip < GPX; ++ip) {
+        const double* g = a.g1 + ip * N1;
+        const double* dg = a.dg1 + ip * N1;
+        const double dxc = X0 * dg[0] + X1 * dg[1];
+        const double dyc = Y0 * dg[0] + Y1 * dg[1];
+        double u[NVC];
+#pragma unroll
+        for (int n = 0; n < NVC; ++n) {
+            double s = 0.0;
+#pragma unroll
+            for (int k = 0; k < N1; ++k) s += uh[n][k] * g[k];
+            u[n] = s;
+        }
+        double nx = dyc, ny = -dxc;
+        const double jcb = sqrt(nx * nx + ny * ny);
+        nx /= jcb; ny /= jcb;
+        const double un = u[1] * nx + u[2] * ny;
+        const double f0 = pbc / u[3] * un;
+        const double rho = u[0] / u[3];
+        const double E = pbc / (rho * gm1) + 0.5 * (u[1] * u[1] + u[2] * u[2]);
+        const double fl[NVC] = {f0, f0 * u[1] + pbc * nx, f0 * u[2] + pbc * ny, rho * E * un + pbc * un};
+#pragma unroll
+        for (int n = 0; n < NVC; ++n) {
+            const double r = fl[n] * jcb * a.w1[ip];
+#pragma unroll
+            for (int k = 0; k < N1; ++k) lf[n][k] += g[k] * r;
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < NVC; ++n)
+#pragma unroll
+        for (int k = 0; k < N1; ++k) a.eout[((long)idx * N1 + k) * NVC + n] = lf[n][k];
+}
+
+// The element launch (persistent over every element in mesh order after the first eblk
+// blocks, which compute the boundary-edge fluxes).  Bound: the FP64 matrix cores and the
+// pointwise solves, one wave per SIMD.  105 800 elements, p = 4: 177 us full and 71 us
+// inviscid, against 7 x 114 us and 7 x 35 us for colour launches with an element per 32
+// lanes (a general 4 x 4 product and solve per point, 25 of 32 lanes in use).
+template <int P, bool FULL>
+__global__ __launch_bounds__(256) void k_elem_cns(CnsElemArgs a, CnsEdgeArgs e, int eblk) {
+    if ((int)blockIdx.x < eblk) {
+        edge_cns_body<P>(e, blockIdx.x * 256 + threadIdx.x);
+        return;
+    }
+    elem_cns_body<P, FULL>(a, eblk);
+}
+
+// FP32 arithmetic (the inner solve of the defect correction), FP64 state and residual: one
+// element per 32 lanes, one Gauss point per lane; transforms are per-lane dot products
+// against operator rows in LDS (point-contiguous), derivative and integration
+// contractions exchange point values through LDS.  It keeps the order of every FP32
+// operation: the residual of a near-uniform stream is a small difference of FP32 fluxes,
+// and another order, as accurate against FP64, moves the mixed iterates by up to 1e-2.
 template <typename T, int P, bool FULL>
-__device__ __forceinline__ void elem_cns_body(const CnsElemArgsT<T>& a, int noct) {
+__device__ __forceinline__ void elem_cns_lane_body(const CnsElemArgsT<T>& a, int noct, int blk, int nblk) {
     using D = CDims<P>;
     constexpr int TM = D::TM, G = D::G, NO = NVC * TM;
     constexpr int SMD = D::SM > 0 ? D::SM : 1;
@@ -326,11 +765,11 @@ __device__ __forceinline__ void elem_cns_body(const CnsElemArgsT<T>& a, int noct
     const T gm1 = T(a.ph.gamma) - T(1.0), gogm1 = T(a.ph.gamma) / gm1;
     __syncthreads();  // operators staged
 
-    HPG_OCTET_LOOP(noct, oc) {
+    HPG_OCTET_LOOP_OF(noct, oc, blk, nblk) {
         wave_lds_sync();  // previous octet done with this half-wave's LDS buffers
         const int idx = a.begin + oc * 8 + hw;
         const bool valid = idx < a.end;
-        const int t = valid ? a.order[idx] : a.order[a.begin];
+        const int t = valid ? idx : a.begin;
         int vtx[3], seg[3], sgn[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
@@ -509,8 +948,11 @@ __device__ __forceinline__ void elem_cns_body(const CnsElemArgsT<T>& a, int noct
             }
         }
 
-        // lftog with the first-colour initialisation of res / res_r (tri_hp/nstage.cpp:21-82)
+        // element-major: the sum lf_im + beta lf_re and beta lf_re, in FP64.  The element
+        // whose colour touches a coefficient first adds the two parts one by one, the
+        // others their FP32 sum (the rounding that this mixed iteration has always had)
         if (valid) {
+            const int col = a.tcol[t];
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
                 const int o = g + 32 * r;
@@ -519,118 +961,35 @@ __device__ __forceinline__ void elem_cns_body(const CnsElemArgsT<T>& a, int noct
                 int kind;
                 double sg;
                 const int off = mode_offset<P, NVC>(k, t, vtx, seg, sgn, a.sm0, a.im0, kind, sg) + n;
-                double* di = kind == 0 ? a.resv : (kind == 1 ? a.ress : a.resi);
-                double* dr = kind == 0 ? a.rrv : (kind == 1 ? a.rrs : a.rri);
-                const bool first = kind == 2 || (kind == 0 ? a.fcv[sel3(vtx, k)] : a.fcs[sel3(seg, (k - 3) / SMD)]) == a.colour;
                 const T vli = T(sg) * li[r], vlr = T(sg) * lr[r];
-                if (first) {
-                    const double r0 = a.keep == 0.0 ? 0.0 : a.keep * dr[off];
-                    if (FULL || a.keep != 1.0) dr[off] = r0 + vlr;
-                    if constexpr (sizeof(T) == 4) {
-                        const double* sr = kind == 0 ? a.srcv : (kind == 1 ? a.srcs : a.srci);
-                        di[off] = r0 + vlr + vli + (sr ? sr[off] * a.sfac[0] : 0.0);
-                    } else {
-                        di[off] = r0 + vlr + vli;
-                    }
+                if (kind < 2) {
+                    const bool first = (kind == 0 ? a.fcv[sel3(vtx, k)] : a.fcs[sel3(seg, (k - 3) / SMD)]) == col;
+                    double* d = a.eres + ((size_t)t * D::BM + k) * (2 * NVC) + n;
+                    d[0] = first ? (double)vlr + (double)vli : (double)(vlr + vli);
+                    if constexpr (FULL) d[NVC] = vlr;
                 } else {
-                    if constexpr (FULL) dr[off] += vlr;
-                    di[off] += vlr + vli;
+                    const double r0 = a.keep == 0.0 ? 0.0 : a.keep * a.rri[off];
+                    if (FULL || a.keep != 1.0) a.rri[off] = r0 + vlr;
+                    a.resi[off] = r0 + vlr + vli + (a.srci ? a.srci[off] * a.sfac[0] : 0.0);
                 }
             }
         }
     }
 }
 
-// two waves per SIMD: at p = 4 the full residual needs 295 registers unbounded (one wave
-// per SIMD, its LDS round trips unhidden); bounded to 256 it spills 172 bytes per lane
 template <int P, bool FULL>
-__global__ __launch_bounds__(256, 2) void k_elem_cns(CnsElemArgs a, int noct) {
-    elem_cns_body<double, P, FULL>(a, noct);
+__global__ __launch_bounds__(256) void k_elem_cns32(CnsElemArgs32 a, CnsEdgeArgs e, int eblk) {
+    if ((int)blockIdx.x < eblk) {
+        edge_cns_body<P>(e, blockIdx.x * 256 + threadIdx.x);
+        return;
+    }
+    elem_cns_lane_body<float, P, FULL>(a, (a.end - a.begin + 7) / 8, (int)blockIdx.x - eblk, (int)gridDim.x - eblk);
 }
 
-// FP32 arithmetic (the inner solve of the defect correction); FP64 state and residual
+// Element Jacobians of a batch, as k_elem_ins_jac
 template <int P, bool FULL>
-__global__ __launch_bounds__(256) void k_elem_cns32(CnsElemArgs32 a, int noct) {
-    elem_cns_body<float, P, FULL>(a, noct);
-}
-
-// ---------------------------------------------------------------------------------
-// edge-boundary flux residual (tri_hp/hp_boundary.cpp:973-1049) with the
-// bdry_cns::generic flux (tri_hp/cns/bdry.cpp:192-245); p_bc = boundary pressure
-struct CnsEdgeArgs {
-    const int* eseg;
-    int begin, end;
-    const int* seg_pnt;
-    const double* pnts;
-    const double* ugv;
-    const double* ugs;
-    double* resv;
-    double* ress;
-    const double* g1;
-    const double* dg1;
-    const double* w1;
-    int sm0;
-    double gamma, pbc;
-};
-
-template <int P>
-__global__ __launch_bounds__(64) void k_edge_cns(CnsEdgeArgs a) {
-    constexpr int SM = Dims<P>::SM, N1 = SM + 2, GPX = P + 1;
-    const int idx = a.begin + blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= a.end) return;
-    const int sind = a.eseg[idx];
-    const int v0 = a.seg_pnt[2 * sind], v1 = a.seg_pnt[2 * sind + 1];
-    double uh[NVC][N1];
-#pragma unroll
-    for (int n = 0; n < NVC; ++n) {
-        uh[n][0] = a.ugv[v0 * NVC + n];
-        uh[n][1] = a.ugv[v1 * NVC + n];
-#pragma unroll
-        for (int m = 0; m < SM; ++m) uh[n][m + 2] = a.ugs[(sind * a.sm0 + m) * NVC + n];
-    }
-    const double X0 = a.pnts[2 * v0], Y0 = a.pnts[2 * v0 + 1], X1 = a.pnts[2 * v1], Y1 = a.pnts[2 * v1 + 1];
-    const double gm1 = a.gamma - 1.0, pbc = a.pbc;
-    double lf[NVC][N1];
-#pragma unroll
-    for (int n = 0; n < NVC; ++n)
-#pragma unroll
-        for (int k = 0; k < N1; ++k) lf[n][k] = 0.0;
-#pragma unroll
-    for (int ip = 0; ip < GPX; ++ip) {
-        const double* g = a.g1 + ip * N1;
-        const double* dg = a.dg1 + ip * N1;
-        const double dxc = X0 * dg[0] + X1 * dg[1];
-        const double dyc = Y0 * dg[0] + Y1 * dg[1];
-        double u[NVC];
-#pragma unroll
-        for (int n = 0; n < NVC; ++n) {
-            double s = 0.0;
-#pragma unroll
-            for (int k = 0; k < N1; ++k) s += uh[n][k] * g[k];
-            u[n] = s;
-        }
-        double nx = dyc, ny = -dxc;
-        const double jcb = sqrt(nx * nx + ny * ny);
-        nx /= jcb; ny /= jcb;
-        const double un = u[1] * nx + u[2] * ny;
-        const double f0 = pbc / u[3] * un;
-        const double rho = u[0] / u[3];
-        const double E = pbc / (rho * gm1) + 0.5 * (u[1] * u[1] + u[2] * u[2]);
-        const double fl[NVC] = {f0, f0 * u[1] + pbc * nx, f0 * u[2] + pbc * ny, rho * E * un + pbc * un};
-#pragma unroll
-        for (int n = 0; n < NVC; ++n) {
-            const double r = fl[n] * jcb * a.w1[ip];
-#pragma unroll
-            for (int k = 0; k < N1; ++k) lf[n][k] += g[k] * r;
-        }
-    }
-#pragma unroll
-    for (int n = 0; n < NVC; ++n) {
-        a.resv[v0 * NVC + n] += lf[n][0];
-        a.resv[v1 * NVC + n] += lf[n][1];
-#pragma unroll
-        for (int m = 0; m < SM; ++m) a.ress[(sind * a.sm0 + m) * NVC + n] += lf[n][m + 2];
-    }
+__global__ __launch_bounds__(256) void k_elem_cns_jac(CnsElemArgs a) {
+    elem_cns_body<P, FULL, true>(a);
 }
 
 // ---------------------------------------------------------------------------------
@@ -972,7 +1331,8 @@ __global__ __launch_bounds__(256) void k_pnv_int(CnsProjArgs a, int noct) {
     constexpr int TM = D::TM, G = D::G, IM = D::IM, BM = D::BM, SM = D::SM;
     __shared__ double sP[TM * 32];
     __shared__ double sI[G * 16];
-    // rows padded by one word (LDS banks: see elem_cns_body)
+    // rows padded by one word: the half-waves' buffers unpadded sit a multiple of the LDS bank
+    // period apart
     __shared__ double sc[8][3][NVC][17];  // u, conservative correction, primitive boundary correction
     __shared__ double sf[8][NVC][33];
     __shared__ double so[8][NVC][IM];
