@@ -122,13 +122,11 @@ struct Level {
     float* packn32 = nullptr;  // FP32 element residual (output rows permuted to the FP64 layout)
     float* lump32 = nullptr;
     int o_sfmv, o_ifmb, o_vfms, o_sdiag, o_sfms, o_bfmi, o_idiag;
-    // cns: point-per-lane operators (CDims layout: project_new_variables in FP64, the element
-    // residual of the defect-correction inner solve in FP32), edge side-mass and interior
-    // band factors
-    double* cpack = nullptr;
+    // cns: point-per-lane operators of the defect-correction inner solve (CDims layout), the
+    // interior projection's operators (PDims layout), edge side-mass band factor
     float* cpack32 = nullptr;
+    double* ppack = nullptr;
     double* sdiag1d = nullptr;
-    double* idiag = nullptr;
 };
 
 // cns operator pack of one level: P, Pr, Ps as [mode][32], Dr, Ds as [point'][32],
@@ -155,6 +153,35 @@ std::vector<double> build_cns_pack(const TriOps& o) {
             pk[OP_IS + q * 16 + k] = o.Is[k * G + q];
             pk[OP_I + q * 16 + k] = o.I[k * G + q];
         }
+    return pk;
+}
+
+// operators of the interior projection (PDims layout): lane-ready P (the first block of the
+// element pack), vertex functions per point, the interior band solve applied to the
+// integration rows and to their products with P
+std::vector<double> build_pnv_pack(const TriOps& o, const std::vector<double>& elem_pack) {
+    const LevelDims d(o.p);
+    const int im = o.im, tm = o.tm, G = o.G, OP_V = d.PROJ, OP_I = OP_V + 96, OP_IP = OP_I + 96;
+    std::vector<double> pk(OP_IP + 48, 0.0);
+    std::copy(elem_pack.begin(), elem_pack.begin() + d.PROJ, pk.begin());
+    for (int g = 0; g < G; ++g) {
+        for (int k = 0; k < 3; ++k) pk[OP_V + g * 3 + k] = o.P[g * tm + k];
+        // rows j of the band factor: U(j-1,j), U(j,j); U^T U x = I(:, g)
+        std::vector<double> x(im);
+        for (int j = 0; j < im; ++j) {
+            x[j] = o.I[(o.bm + j) * G + g];
+            if (j) x[j] -= o.idiag[2 * j] * x[j - 1];
+            x[j] /= o.idiag[2 * j + 1];
+        }
+        for (int j = im - 1; j >= 0; --j) {
+            x[j] /= o.idiag[2 * j + 1];
+            if (j) x[j - 1] -= o.idiag[2 * j] * x[j];
+        }
+        for (int m = 0; m < im; ++m) {
+            pk[OP_I + g * 3 + m] = x[m];
+            for (int k = 0; k < o.bm; ++k) pk[OP_IP + k * 3 + m] += x[m] * o.P[g * tm + k];
+        }
+    }
     return pk;
 }
 
@@ -967,8 +994,9 @@ int do_setup_cns(hpg_ctx* c, bool sync = true) {
     return herr;
 }
 
-// inflow modify_boundary_residual, then project_new_variables (tri_hp/cns/update.cpp:276-357)
-void cns_boundary_and_projection(hpg_ctx* c) {
+// inflow modify_boundary_residual, project_new_variables and the stage update
+// ug = ug0 - cfa * correction (tri_hp/cns/update.cpp:276-357)
+void cns_boundary_and_projection(hpg_ctx* c, double cfa) {
     const Level& L = c->lv[c->log2p];
     const LevelDims d(L.p);
     const double* g1 = L.edge;
@@ -988,7 +1016,8 @@ void cns_boundary_and_projection(hpg_ctx* c) {
     a.ugv = c->ugv; a.ugs = c->ugs; a.ugi = c->ugi; a.resv = c->resv; a.ress = c->ress; a.resi = c->resi;
     a.rtv = c->rtv; a.rts = c->rts; a.vpc = c->vpc; a.vess = c->vess; a.sess = c->sess;
     a.seg_pnt = c->seg_pnt; a.tri_pnt = c->tri_pnt; a.tri_seg = c->tri_seg; a.tri_sgn = c->tri_sgn;
-    a.order = c->order; a.g1 = g1; a.w1 = w1; a.sdiag1d = L.sdiag1d; a.idiag = L.idiag; a.ops = L.cpack;
+    a.ug0i = c->ug0i; a.cfa = cfa;
+    a.g1 = g1; a.w1 = w1; a.sdiag1d = L.sdiag1d; a.ops = L.ppack;
     a.npnt = c->npnt; a.nseg = c->nseg; a.ntri = c->ntri; a.sm0 = c->sm0; a.im0 = c->im0; a.gamma = c->cph.gamma;
     hipLaunchKernelGGL(k_pnv_vrtx, dim3(nblk8(c->npnt)), dim3(256), 0, c->stream, a);
     if (d.sm > 0) {
@@ -996,10 +1025,11 @@ void cns_boundary_and_projection(hpg_ctx* c) {
         else hipLaunchKernelGGL(k_pnv_side<4>, dim3(nblk8(c->nseg)), dim3(256), 0, c->stream, a);
     }
     if (d.im > 0) {
-        const int noct = (c->ntri + 7) / 8;
         static const int cap = resident_blocks((const void*)k_pnv_int<4>);
-        hipLaunchKernelGGL(k_pnv_int<4>, dim3(persistent_grid(noct, cap)), dim3(256), 0, c->stream, a, noct);
+        hipLaunchKernelGGL(k_pnv_int<4>, dim3(persistent_grid((c->ntri + 63) / 64, cap)), dim3(256), 0, c->stream, a);
     }
+    launch_modes(c, 4, c->npnt, 1, 1, c->ugv, c->ug0v, c->resv, cfa);
+    launch_modes(c, 4, c->nseg, d.sm, c->sm0, c->ugs, c->ug0s, c->ress, cfa);
     check(hipGetLastError(), "cns projection launch");
 }
 
@@ -1012,9 +1042,7 @@ void update_cns(hpg_ctx* c) {
     for (int stage = 0; stage < c->prm.nstage; ++stage) {
         do_rsdl_cns(c, stage);
         do_minvrt(c);
-        cns_boundary_and_projection(c);
-        modes_vsi(c, 4, c->ugv, c->ugs, c->ugi, c->ug0v, c->ug0s, c->ug0i, c->resv, c->ress, c->resi,
-                  c->prm.alpha[stage] * c->prm.cfl[c->log2p]);
+        cns_boundary_and_projection(c, c->prm.alpha[stage] * c->prm.cfl[c->log2p]);
     }
     check(hipGetLastError(), "cns update launch");
 }
@@ -1049,9 +1077,7 @@ void mixed_update_cns(hpg_ctx* c) {
                 do_rsdl_cns32(c, stage);
             }
             do_minvrt(c);
-            cns_boundary_and_projection(c);
-            modes_vsi(c, 4, c->ugv, c->ugs, c->ugi, c->ug0v, c->ug0s, c->ug0i, c->resv, c->ress, c->resi,
-                      c->prm.alpha[stage] * c->prm.cfl[c->log2p]);
+            cns_boundary_and_projection(c, c->prm.alpha[stage] * c->prm.cfl[c->log2p]);
         }
     }
     hipLaunchKernelGGL(k_fd_final64, dim3(std::min<unsigned>(nblk(nv), RED_BLOCKS)), dim3(256), 0, c->stream, nv, c->ugv, c->u0cv, c->fd_scal, c->fd_max + 1);
@@ -1499,12 +1525,13 @@ int hpg_create(const hpg_tri_mesh* m, const hpg_params* prm, hpg_ctx** out) {
             L.edge = c->upload(ed.data(), ed.size());
             if (c->physics == HPG_PHYSICS_CNS) {
                 const std::vector<double> cp = build_cns_pack(o);
-                L.cpack = c->upload(cp.data(), cp.size());
                 const std::vector<float> cp32(cp.begin(), cp.end());
                 L.cpack32 = c->upload(cp32.data(), cp32.size());
                 L.sdiag1d = c->upload(o.sdiag1d.data(), o.sdiag1d.size());
-                const std::vector<double> idg = o.idiag.empty() ? std::vector<double>(2, 1.0) : o.idiag;
-                L.idiag = c->upload(idg.data(), idg.size());
+                if (o.im > 0) {
+                    const std::vector<double> pp = build_pnv_pack(o, pk);
+                    L.ppack = c->upload(pp.data(), pp.size());
+                }
             }
         }
         check(hipStreamSynchronize(c->stream), "create sync");

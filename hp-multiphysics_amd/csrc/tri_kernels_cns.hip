@@ -6,8 +6,7 @@
 // Element residual: the matrix-core layout of tri_kernels.hip (16 elements per wave, every
 // transform a contraction on v_mfma_f64_16x16x4f64 or v_mfma_f32_16x16x4f32), with the
 // pointwise physics -- the stabilisation solve at every Gauss point above all -- in the
-// lane that holds the point.  project_new_variables keeps a half-wave per element, one
-// Gauss point per lane, and exchanges point values through LDS.
+// lane that holds the point; project_new_variables' interior sweep likewise.
 #include <hip/hip_runtime.h>
 #include "tri_kernels.h"
 
@@ -217,24 +216,16 @@ __device__ __forceinline__ void cns_tau(const CnsPhys& ph, T pr, T u, T v, T rt,
     solve4(Tinv, Tau);
 }
 
-// conservative -> primitive change at state (p, u, v, RT) (tri_hp/cns/update.cpp:247-271)
+// conservative -> primitive change at state (p, u, v, RT) (tri_hp/cns/update.cpp:247-271);
+// written with one division (the matrix form has ten, and the projections are bound by
+// their pointwise FP64 work)
 __device__ __forceinline__ void switch_vars(const double w[4], double a[4], double gm1) {
-    const double pr = w[0], u = w[1], v = w[2], rt = w[3];
-    const double rho = pr / rt, ke = 0.5 * (u * u + v * v);
-    const double d[4][4] = {{ke * gm1, -u * gm1, -v * gm1, gm1},
-                            {-u / rho, 1.0 / rho, 0.0, 0.0},
-                            {-v / rho, 0.0, 1.0 / rho, 0.0},
-                            {(gm1 * ke - rt) / rho, -u * gm1 / rho, -v * gm1 / rho, gm1 / rho}};
-    double t[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        double s = 0.0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) s += d[i][j] * a[j];
-        t[i] = s;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) a[i] = t[i];
+    const double u = w[1], v = w[2], rt = w[3], irho = rt / w[0];
+    const double z = gm1 * (0.5 * (u * u + v * v) * a[0] - u * a[1] - v * a[2] + a[3]);
+    a[1] = irho * (a[1] - u * a[0]);
+    a[2] = irho * (a[2] - v * a[0]);
+    a[3] = irho * (z - rt * a[0]);
+    a[0] = z;
 }
 
 // forward substitution with the lower triangle (diagonal included) of a row-major 4x4
@@ -1219,7 +1210,9 @@ __global__ __launch_bounds__(256) void k_mbr_side(CnsBcArgs a) {
 struct CnsProjArgs {
     const double* ugv;
     const double* ugs;
-    const double* ugi;
+    double* ugi;          // interiors: the stage update ug = ug0 - cfa * correction included
+    const double* ug0i;
+    double cfa;
     double* resv;
     double* ress;
     double* resi;
@@ -1232,12 +1225,10 @@ struct CnsProjArgs {
     const int* tri_pnt;
     const int* tri_seg;
     const int* tri_sgn;
-    const int* order;
     const double* g1;
     const double* w1;
     const double* sdiag1d;
-    const double* idiag;  // interior band factor: row j = U(j-1,j), U(j,j)
-    const double* ops;    // CDims<P> pack
+    const double* ops;    // PDims<P> pack
     int npnt, nseg, ntri, sm0, im0;
     double gamma;
 };
@@ -1324,111 +1315,133 @@ __global__ __launch_bounds__(256) void k_pnv_side(CnsProjArgs a) {
     }
 }
 
-// interiors: one element per half-wave, one Gauss point per lane
+// operators of the interior projection: P as lane-ready K-steps, then per Gauss point the
+// three vertex functions and the three interior rows of S I (S the interior band solve, I
+// the integration), then per mode the interior rows of S I P
 template <int P>
-__global__ __launch_bounds__(256) void k_pnv_int(CnsProjArgs a, int noct) {
-    using D = CDims<P>;
-    constexpr int TM = D::TM, G = D::G, IM = D::IM, BM = D::BM, SM = D::SM;
-    __shared__ double sP[TM * 32];
-    __shared__ double sI[G * 16];
-    // rows padded by one word: the half-waves' buffers unpadded sit a multiple of the LDS bank
-    // period apart
-    __shared__ double sc[8][3][NVC][17];  // u, conservative correction, primitive boundary correction
-    __shared__ double sf[8][NVC][33];
-    __shared__ double so[8][NVC][IM];
-    __shared__ double sL[8][3][16];   // the vertices' 4x4 blocks, loaded once per element
-    __shared__ double sid[2 * (IM > 0 ? IM : 1)];
-    for (int k = threadIdx.x; k < TM * 32; k += blockDim.x) sP[k] = a.ops[D::OP_P + k];
-    for (int k = threadIdx.x; k < G * 16; k += blockDim.x) sI[k] = a.ops[D::OP_I + k];
-    for (int k = threadIdx.x; k < 2 * IM; k += blockDim.x) sid[k] = a.idiag[k];
-    const int hw = threadIdx.x >> 5, g = threadIdx.x & 31;
+struct PDims {
+    static constexpr int PROJ = Dims<P>::PROJ, OP_V = PROJ, OP_I = OP_V + 32 * 3, OP_IP = OP_I + 32 * 3;
+    static constexpr int SIZE = OP_IP + 16 * 3;
+};
+
+// interiors (IM = 3, p = 4): r <- S I (tt - L^-1 dpdc(u) r) with tt the primitive correction
+// of the element's vertices and sides.  16 elements per wave: u and r are projected on the
+// FP64 matrix cores, the lower-triangular solve runs in the lane that holds the point, and
+// the integration, with the band solve and the projection of tt folded into its operators,
+// is 33 products per lane and variable, summed over the four lanes of an element.
+// Stage update of the interior state included (only this element reads it).  105 800
+// elements: 77 us, against 154 us with an element per half-wave and its transforms
+// through LDS.
+template <int P>
+__global__ __launch_bounds__(256, 2) void k_pnv_int(CnsProjArgs a) {
+    using D = Dims<P>;
+    using Q = PDims<P>;
+    constexpr int GT = D::GT, KT = D::KT, IM = D::IM;
+    static_assert(IM == 3, "interior modes of an element: one per lane group");
+    __shared__ double so[Q::SIZE];
+    for (int k = threadIdx.x; k < Q::SIZE; k += blockDim.x) so[k] = a.ops[k];
+    __syncthreads();
+    const int lane = threadIdx.x & 63, e = lane & 15, q = lane >> 4;
+    const int WX = ((int)gridDim.x >> 3) * 4, rank = ((int)blockIdx.x >> 3) * 4 + (threadIdx.x >> 6);
+    const int xcd = blockIdx.x & 7, ng = (a.ntri + 15) >> 4, gpx = (ng + 7) >> 3;
+    const int g0 = xcd * gpx + rank, gend = min(ng, (xcd + 1) * gpx);
+    if (g0 >= gend) return;
     const double gm1 = a.gamma - 1.0;
-    __syncthreads();  // operators staged
-    HPG_OCTET_LOOP(noct, oc) {
-        wave_lds_sync();  // previous octet done with this half-wave's LDS buffers
-        const int idx = oc * 8 + hw;
-        const bool valid = idx < a.ntri;
-        const int t = valid ? idx : 0;
-        int vtx[3], seg[3], sgn[3];
+    auto elem = [&](int g) { const int t = g * 16 + e; return g < gend && t < a.ntri ? t : -1; };
+    ElemConn cn = elem_conn(a, elem(g0));
+    for (int g = g0; g < gend; g += WX) {
+        const ElemConn c = cn;
+        cn = elem_conn(a, elem(g + WX));
+        const bool valid = c.t >= 0;
+        double u[NVC][KT], r[NVC][KT], x[IM][NVC];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            vtx[k] = a.tri_pnt[3 * t + k];
-            seg[k] = a.tri_seg[3 * t + k];
-            sgn[k] = a.tri_sgn[3 * t + k];
-        }
-        if (g < TM) {
-            const int k = g;
+        for (int m = 0; m < IM; ++m)
+#pragma unroll
+            for (int n = 0; n < NVC; ++n) x[m][n] = 0.0;
+#pragma unroll
+        for (int s = 0; s < KT; ++s) {
+            const int k = 4 * s + q;
+            const bool live = valid && k < D::TM;
+            int kind;
+            double sg;
+            const int off = mode_offset<P, NVC>(k, valid ? c.t : 0, c.vtx, c.seg, c.sgn, a.sm0, a.im0, kind, sg);
+            const double* pu = kind == 0 ? a.ugv : (kind == 1 ? a.ugs : a.ugi);
+            const double* pr = kind == 0 ? a.rtv : (kind == 1 ? a.rts : a.resi);
+            const double* pt = kind == 0 ? a.resv : a.ress;
+            double ip[IM];
+#pragma unroll
+            for (int m = 0; m < IM; ++m) ip[m] = so[Q::OP_IP + k * 3 + m];
 #pragma unroll
             for (int n = 0; n < NVC; ++n) {
-                double u, rr, tt;
-                if (k < 3) {
-                    const int ix = sel3(vtx, k) * NVC + n;
-                    u = a.ugv[ix]; rr = a.rtv[ix]; tt = a.resv[ix];
-                } else if (k < BM) {
-                    const int i = (k - 3) / SM, m = (k - 3) - i * SM;
-                    const double sg = ((m & 1) && sel3(sgn, i) < 0) ? -1.0 : 1.0;
-                    const int ix = (sel3(seg, i) * a.sm0 + m) * NVC + n;
-                    u = sg * a.ugs[ix]; rr = sg * a.rts[ix]; tt = sg * a.ress[ix];
-                } else {
-                    const int ix = (t * a.im0 + (k - BM)) * NVC + n;
-                    u = a.ugi[ix]; rr = a.resi[ix]; tt = 0.0;
+                u[n][s] = live ? sg * pu[off + n] : 0.0;
+                r[n][s] = live ? sg * pr[off + n] : 0.0;
+                const double t = live && kind < 2 ? sg * pt[off + n] : 0.0;
+#pragma unroll
+                for (int m = 0; m < IM; ++m) x[m][n] += ip[m] * t;
+            }
+        }
+        // lower triangles of the vertices' 4 x 4 blocks
+        double L[3][10];
+#pragma unroll
+        for (int v = 0; v < 3; ++v)
+#pragma unroll
+            for (int i = 0, o = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j <= i; ++j, ++o) L[v][o] = valid ? a.vpc[(long)16 * c.vtx[v] + 4 * i + j] : (i == j ? 1.0 : 0.0);
+#pragma unroll
+        for (int kt = 0; kt < GT; ++kt) {
+            const d4 z = {0.0, 0.0, 0.0, 0.0};
+            d4 cu[NVC] = {z, z, z, z}, cr[NVC] = {z, z, z, z};
+#pragma unroll
+            for (int s = 0; s < KT; ++s) {
+                const double av = so[(kt * KT + s) * 64 + lane];
+#pragma unroll
+                for (int n = 0; n < NVC; ++n) {
+                    cu[n] = mfma(av, u[n][s], cu[n]);
+                    cr[n] = mfma(av, r[n][s], cr[n]);
                 }
-                sc[hw][0][n][k] = u;
-                sc[hw][1][n][k] = rr;
-                sc[hw][2][n][k] = tt;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (16 * kt + 4 * i >= D::G) continue;
+                __builtin_amdgcn_sched_barrier(0);  // one point at a time (registers)
+                const int pt = 16 * kt + 4 * i + q;
+                const bool in = valid && pt < D::G;
+                const double b0 = so[Q::OP_V + pt * 3], b1 = so[Q::OP_V + pt * 3 + 1], b2 = so[Q::OP_V + pt * 3 + 2];
+                double w[NVC], f[NVC], M[16];
+#pragma unroll
+                for (int n = 0; n < NVC; ++n) { w[n] = in ? cu[n][i] : 1.0; f[n] = cr[n][i]; }
+#pragma unroll
+                for (int ii = 0, o = 0; ii < 4; ++ii)
+#pragma unroll
+                    for (int j = 0; j <= ii; ++j, ++o)
+                        M[4 * ii + j] = in ? L[0][o] * b0 + L[1][o] * b1 + L[2][o] * b2 : (ii == j ? 1.0 : 0.0);
+                switch_vars(w, f, gm1);
+                lower4(M, f);
+#pragma unroll
+                for (int m = 0; m < IM; ++m) {
+                    const double wi = so[Q::OP_I + pt * 3 + m];
+#pragma unroll
+                    for (int n = 0; n < NVC; ++n) x[m][n] -= wi * (in ? f[n] : 0.0);
+                }
             }
         }
-        for (int e = g; e < 48; e += 32) sL[hw][e >> 4][e & 15] = a.vpc[16 * sel3(vtx, e >> 4) + (e & 15)];
-        wave_lds_sync();
-        double w[NVC], r[NVC], tp[NVC];
+        // sum over the element's four lanes; lane group m stores interior mode m
 #pragma unroll
-        for (int n = 0; n < NVC; ++n) { w[n] = 0.0; r[n] = 0.0; tp[n] = 0.0; }
-#pragma unroll 3
-        for (int k = 0; k < TM; ++k) {
-            const double pk = sP[k * 32 + g];
+        for (int m = 0; m < IM; ++m)
 #pragma unroll
             for (int n = 0; n < NVC; ++n) {
-                w[n] += pk * sc[hw][0][n][k];
-                r[n] += pk * sc[hw][1][n][k];
-                tp[n] += pk * sc[hw][2][n][k];
+                x[m][n] += __shfl_xor(x[m][n], 16, 64);
+                x[m][n] += __shfl_xor(x[m][n], 32, 64);
             }
-        }
-        if (g >= G) { w[0] = 1.0; w[3] = 1.0; }
-        double L[16];
-        {
-            const double b0 = sP[0 * 32 + g], b1 = sP[1 * 32 + g], b2 = sP[2 * 32 + g];
+        if (valid && q < IM) {
+            const long o = ((long)c.t * a.im0 + q) * NVC;
 #pragma unroll
-            for (int k = 0; k < 16; ++k)
-                L[k] = (k % 5 == 0 && g >= G) ? 1.0 : sL[hw][0][k] * b0 + sL[hw][1][k] * b1 + sL[hw][2][k] * b2;
-        }
-        switch_vars(w, r, gm1);
-        lower4(L, r);
-#pragma unroll
-        for (int n = 0; n < NVC; ++n) sf[hw][n][g] = tp[n] - r[n];
-        wave_lds_sync();
-        // intgrt onto the interior modes, then the interior banded solve (dpbtrs)
-        if (g < NVC * IM) {
-            const int n = g / IM, m = g - n * IM, k = BM + m;
-            double s = 0.0;
-#pragma unroll 5
-            for (int q = 0; q < G; ++q) s += sI[q * 16 + k] * sf[hw][n][q];
-            so[hw][n][m] = s;
-        }
-        wave_lds_sync();
-        if (valid && g < NVC) {
-            const int n = g;
-            double x[IM];
-#pragma unroll
-            for (int m = 0; m < IM; ++m) x[m] = so[hw][n][m];
-#pragma unroll
-            for (int j = 0; j < IM; ++j) x[j] = (x[j] - (j ? sid[j * 2] * x[j - 1] : 0.0)) / sid[j * 2 + 1];
-#pragma unroll
-            for (int j = IM - 1; j >= 0; --j) {
-                x[j] /= sid[j * 2 + 1];
-                if (j) x[j - 1] -= sid[j * 2] * x[j];
+            for (int n = 0; n < NVC; ++n) {
+                const double d = -(q == 0 ? x[0][n] : (q == 1 ? x[1][n] : x[2][n]));
+                a.resi[o + n] = d;
+                a.ugi[o + n] = a.ug0i[o + n] - a.cfa * d;
             }
-#pragma unroll
-            for (int m = 0; m < IM; ++m) a.resi[(t * a.im0 + m) * NVC + n] = -x[m];
         }
     }
 }
