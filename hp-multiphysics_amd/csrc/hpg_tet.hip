@@ -98,7 +98,8 @@ void csr(int nent, const std::vector<std::pair<int, int>>& pairs, std::vector<in
 
 struct hpg_tet_ctx {
     hipStream_t stream = nullptr;
-    std::vector<void*> allocs;
+    DeviceArrays arrays;
+    HostCopyUser staging;
     std::string err;
     int npnt = 0, nseg = 0, ntet = 0, nbf = 0, log2pmax = 0, log2p = 0, em0 = 0;
     int nv = TNV;            // 4 (ins: u, v, w, p) or 5 (cns: p, u, v, w, RT)
@@ -140,23 +141,12 @@ struct hpg_tet_ctx {
         return events[k];
     }
     template <class T>
-    T* alloc(size_t n) {
-        void* p = nullptr;
-        if (n == 0) n = 1;
-        if (hipMalloc(&p, n * sizeof(T)) != hipSuccess) throw std::runtime_error("hipMalloc failed");
-        allocs.push_back(p);
-        check(hipMemsetAsync(p, 0, n * sizeof(T), stream), "memset");
-        return static_cast<T*>(p);
-    }
+    T* alloc(size_t n) { return arrays.alloc<T>(stream, n); }
     template <class T>
-    T* upload(const T* h, size_t n) {
-        T* d = alloc<T>(n);
-        if (n) check(hipMemcpyAsync(d, h, n * sizeof(T), hipMemcpyHostToDevice, stream), "H2D");
-        return d;
-    }
+    T* upload(const T* h, size_t n) { return arrays.upload(stream, h, n); }
     ~hpg_tet_ctx() {
         if (stream) hipStreamSynchronize(stream);
-        for (void* p : allocs) hipFree(p);
+        arrays.release();
         for (hipEvent_t e : events) hipEventDestroy(e);
         if (stream) hipStreamDestroy(stream);
     }
@@ -445,8 +435,15 @@ void launch_setup_tetc(hpg_tet_ctx* c) {
     hipLaunchKernelGGL(k_setup_tetc<P>, dim3(nblk8(c->ntet)), dim3(256), 0, c->stream, a);
 }
 
+int read_error(hpg_tet_ctx* c) {  // as for tri contexts
+    int herr = 0;
+    const HostSeg seg{&herr, c->d_err, sizeof(int)};
+    copy_to_host(c->stream, &seg, 1);
+    if (herr) hipLaunchKernelGGL(k_clear_u32, dim3(1), dim3(64), 0, c->stream, 1, (unsigned*)c->d_err);
+    return herr;
+}
+
 int do_setup_tetc(hpg_tet_ctx* c) {
-    check(hipMemsetAsync(c->d_err, 0, sizeof(int), c->stream), "memset");
     if (c->lv[c->log2p].p == 1) launch_setup_tetc<1>(c); else launch_setup_tetc<2>(c);
     hipLaunchKernelGGL(k_setup_gather_tetc, dim3(nblk8(c->npnt)), dim3(256), 0, c->stream, c->npnt, c->vt_ptr,
                        c->vt_code, c->iprcn, c->tpc, c->vprcn, c->vpc);
@@ -454,10 +451,7 @@ int do_setup_tetc(hpg_tet_ctx* c) {
         hipLaunchKernelGGL(k_setup_gather_tetc, dim3(nblk8(c->nseg)), dim3(256), 0, c->stream, c->nseg, c->et_ptr,
                            c->et_code, c->iprcn, c->tpc, c->eprcn, c->epc);
     check(hipGetLastError(), "tet cns setup launch");
-    int h = 0;
-    check(hipMemcpyAsync(&h, c->d_err, sizeof(int), hipMemcpyDeviceToHost, c->stream), "D2H");
-    check(hipStreamSynchronize(c->stream), "sync");
-    return h;
+    return read_error(c);
 }
 
 int do_setup_tet(hpg_tet_ctx* c) {
@@ -465,7 +459,6 @@ int do_setup_tet(hpg_tet_ctx* c) {
     TetSetupArgs a;
     a.pnts = c->pnts; a.tet_pnt = c->tet_pnt; a.ugv = c->ugv; a.ntet = c->ntet; a.p = c->lv[c->log2p].p;
     a.rho = c->prm.rho; a.mu = c->prm.mu; a.adis = c->prm.adis; a.iprcn = c->iprcn; a.tau = c->tau; a.err = c->d_err;
-    check(hipMemsetAsync(c->d_err, 0, sizeof(int), c->stream), "memset");
     hipLaunchKernelGGL(k_setup_tet, dim3(nblk8(c->ntet)), dim3(256), 0, c->stream, a);
     hipLaunchKernelGGL(k_setup_gather_tet, dim3(nblk8(c->npnt)), dim3(256), 0, c->stream, c->npnt, c->vt_ptr,
                        c->vt_code, c->iprcn, c->vprcn);
@@ -473,10 +466,7 @@ int do_setup_tet(hpg_tet_ctx* c) {
         hipLaunchKernelGGL(k_setup_gather_tet, dim3(nblk8(c->nseg)), dim3(256), 0, c->stream, c->nseg, c->et_ptr,
                            c->et_code, c->iprcn, c->eprcn);
     check(hipGetLastError(), "tet setup launch");
-    int h = 0;
-    check(hipMemcpyAsync(&h, c->d_err, sizeof(int), hipMemcpyDeviceToHost, c->stream), "D2H");
-    check(hipStreamSynchronize(c->stream), "sync");
-    return h;
+    return read_error(c);
 }
 
 // y += sfac[0] x (the scaled defect source of the inner solve)
@@ -665,7 +655,7 @@ int hpg_tet_create(const hpg_tet_mesh* m, const hpg_params* prm, hpg_tet_ctx** o
                 L.vfms = c->upload(o.vfms.data(), o.vfms.size());
             }
         }
-        check(hipStreamSynchronize(c->stream), "sync");
+        c->arrays.flush(c->stream);
     } catch (const std::exception&) {
         return -1;
     }
@@ -678,18 +668,12 @@ int hpg_tet_destroy(hpg_tet_ctx* c) {
     return 0;
 }
 
-static int tet_copy(hpg_tet_ctx* c, bool h2d, double* dv, double* de, const double* hv, const double* he, double* ov,
-                    double* oe) {
+static int tet_copy(hpg_tet_ctx* c, bool h2d, double* dv, double* de, const double* v, const double* e) {
     HPG_TRY(c, {
-        const size_t nv = (size_t)c->npnt * c->nv * 8, ne = (size_t)c->nseg * c->em0 * c->nv * 8;
-        if (h2d) {
-            check(hipMemcpyAsync(dv, hv, nv, hipMemcpyHostToDevice, c->stream), "H2D");
-            if (ne) check(hipMemcpyAsync(de, he, ne, hipMemcpyHostToDevice, c->stream), "H2D");
-        } else {
-            check(hipMemcpyAsync(ov, dv, nv, hipMemcpyDeviceToHost, c->stream), "D2H");
-            if (ne) check(hipMemcpyAsync(oe, de, ne, hipMemcpyDeviceToHost, c->stream), "D2H");
-        }
-        check(hipStreamSynchronize(c->stream), "sync");
+        const HostSeg seg[2] = {{const_cast<double*>(v), dv, (size_t)c->npnt * c->nv * 8},
+                                {const_cast<double*>(e), de, (size_t)c->nseg * c->em0 * c->nv * 8}};
+        if (h2d) copy_to_device(c->stream, seg, 2);
+        else copy_to_host(c->stream, seg, 2);
     });
     return 0;
 }
@@ -697,19 +681,19 @@ static int tet_copy(hpg_tet_ctx* c, bool h2d, double* dv, double* de, const doub
 int hpg_tet_set_state(hpg_tet_ctx* c, const double* v, const double* e) {
     if (!c || !v || (c->em0 && !e)) return -2;
     c->fd_reset = true;
-    return tet_copy(c, true, c->ugv, c->uge, v, e, nullptr, nullptr);
+    return tet_copy(c, true, c->ugv, c->uge, v, e);
 }
 int hpg_tet_get_state(hpg_tet_ctx* c, double* v, double* e) {
     if (!c || !v || (c->em0 && !e)) return -2;
-    return tet_copy(c, false, c->ugv, c->uge, nullptr, nullptr, v, e);
+    return tet_copy(c, false, c->ugv, c->uge, v, e);
 }
 int hpg_tet_get_residual(hpg_tet_ctx* c, double* v, double* e) {
     if (!c || !v || (c->em0 && !e)) return -2;
-    return tet_copy(c, false, c->resv, c->rese, nullptr, nullptr, v, e);
+    return tet_copy(c, false, c->resv, c->rese, v, e);
 }
 int hpg_tet_set_residual(hpg_tet_ctx* c, const double* v, const double* e) {
     if (!c || !v || (c->em0 && !e)) return -2;
-    return tet_copy(c, true, c->resv, c->rese, v, e, nullptr, nullptr);
+    return tet_copy(c, true, c->resv, c->rese, v, e);
 }
 int hpg_tet_get_preconditioner(hpg_tet_ctx* c, double* vprcn, double* eprcn, double* iprcn, double* tau) {
     if (!c || !vprcn || !eprcn || !iprcn || !tau) return -2;
@@ -839,8 +823,8 @@ int hpg_tet_element_jacobian(hpg_tet_ctx* c, const int* tind, int nel, double ep
             }
         }
         check(hipGetLastError(), "tet jacobian launch");
-        check(hipMemcpyAsync(K, a.K, (size_t)nel * N * N * 8, hipMemcpyDeviceToHost, c->stream), "D2H");
-        check(hipStreamSynchronize(c->stream), "sync");
+        const HostSeg seg{K, a.K, (size_t)nel * N * N * 8};
+        copy_to_host(c->stream, &seg, 1);
     });
     return 0;
 }

@@ -20,6 +20,7 @@
 #include "tri_kernels_cns.hip"
 #include "tri_ops.h"
 #include "mlp.h"
+#include "host_copy.h"
 
 using namespace hpg;
 
@@ -207,7 +208,8 @@ struct hpg_ctx {
     hipEvent_t xev = nullptr;  // orders this context's stream against a neighbour level's
     int *hr_ptr = nullptr, *hr_fidx = nullptr, *hi_fv = nullptr, *hp_cv = nullptr;
     double *hr_wt = nullptr, *hi_wt = nullptr, *hp_wt = nullptr, *vug_frst = nullptr;
-    std::vector<void*> allocs;
+    DeviceArrays arrays;
+    HostCopyUser staging;
     double* pnts = nullptr;
     int *tri_pnt = nullptr, *tri_seg = nullptr, *tri_sgn = nullptr, *seg_pnt = nullptr;
     int* order = nullptr;
@@ -306,25 +308,41 @@ struct hpg_ctx {
     }
 
     template <class T>
-    T* alloc(size_t n) {
-        void* p = nullptr;
-        if (n == 0) n = 1;
-        if (hipMalloc(&p, n * sizeof(T)) != hipSuccess) throw std::runtime_error("hipMalloc failed");
-        allocs.push_back(p);
-        hipMemsetAsync(p, 0, n * sizeof(T), stream);
-        return static_cast<T*>(p);
-    }
+    T* alloc(size_t n) { return arrays.alloc<T>(stream, n); }
     template <class T>
-    T* upload(const T* h, size_t n) {
-        T* d = alloc<T>(n);
-        if (n && hipMemcpyAsync(d, h, n * sizeof(T), hipMemcpyHostToDevice, stream) != hipSuccess)
-            throw std::runtime_error("hipMemcpy H2D failed");
-        return d;
+    T* upload(const T* h, size_t n) { return arrays.upload(stream, h, n); }
+
+    // arrays of options, allocated by the call that first selects the option (not by every
+    // context): the FP32 inner solve and linearisation (ins), the linearisation data, the
+    // learned preconditioner
+    int neseg_max = 0;
+    void need_inner() {
+        if (d0v) return;
+        const size_t nvx = (size_t)npnt * NV, nsx = (size_t)nseg * sm0 * NV, nix = (size_t)ntri * im0 * NV;
+        for (float** p : {&dlv, &r32v, &rr32v, &b32v, &vp32}) *p = alloc<float>(nvx);
+        for (float** p : {&dls, &d0s, &r32s, &rr32s, &b32s}) *p = alloc<float>(nsx);
+        for (float** p : {&dli, &d0i, &r32i, &rr32i, &b32i}) *p = alloc<float>(nix);
+        sp32 = alloc<float>((size_t)nseg * NV);
+        for (float** p : {&tp32, &tp32s, &tp32i}) *p = alloc<float>((size_t)ntri * NV);
+        eres32 = alloc<float>((size_t)ntri * 3 * (sm0 + 1) * 2 * NV);
+        eout32 = alloc<float>((size_t)neseg_max * (sm0 + 2) * NV);
+        d0v = alloc<float>(nvx);  // last: marks the set complete
+    }
+    void need_lin() {
+        if (!lin) lin = alloc<float>((size_t)ngroups * 5 * LevelDims(sm0 + 1).GT * 4 * 64);
+    }
+    void need_learned() {
+        if (tprcn_in) return;
+        featX = alloc<float>((size_t)ntri * MLP_IN);
+        mlpY = alloc<float>((size_t)ntri * MLP_OUT);
+        tprcn_vx = alloc<double>((size_t)ntri * NV);
+        tprcn_sd = alloc<double>((size_t)ntri * NV);
+        tprcn_in = alloc<double>((size_t)ntri * NV);
     }
     ~hpg_ctx() {
         if (stream) hipStreamSynchronize(stream);
         if (cg_exec) hipGraphExecDestroy(cg_exec);
-        for (void* p : allocs) hipFree(p);
+        arrays.release();
         for (hipEvent_t e : events) hipEventDestroy(e);
         if (xev) hipEventDestroy(xev);
         if (stream) hipStreamDestroy(stream);
@@ -966,12 +984,21 @@ void do_rsdl_cns32(hpg_ctx* c, int stage) {
     check(hipGetLastError(), "cns rsdl32 launch");
 }
 
+// the error flag of the kernels enqueued so far (waits for them).  The flag is zero between
+// calls: whoever reads it set clears it
+int read_error(hpg_ctx* c) {
+    int herr = 0;
+    const HostSeg seg{&herr, c->d_err, sizeof(int)};
+    copy_to_host(c->stream, &seg, 1);
+    if (herr) hipLaunchKernelGGL(k_clear_u32, dim3(1), dim3(64), 0, c->stream, 1, (unsigned*)c->d_err);
+    return herr;
+}
+
 // sync = false (the fused multigrid cycle): the error flag accumulates on the device and
 // is read once after the cycle; nothing waits for the device here
 int do_setup_cns(hpg_ctx* c, bool sync = true) {
     const Level& L = c->lv[c->log2p];
     const LevelDims d(L.p);
-    if (sync) check(hipMemsetAsync(c->d_err, 0, sizeof(int), c->stream), "memset");
     CnsSetupArgs s;
     s.pnts = c->pnts; s.tri_pnt = c->tri_pnt; s.tri_seg = c->tri_seg; s.tri_sgn = c->tri_sgn;
     s.ugv = c->ugv; s.ugs = c->ugs; s.ugi = c->ugi; s.Pmat = L.Pmat; s.tprcn = c->tprcn; s.tpc = c->tpc;
@@ -988,10 +1015,7 @@ int do_setup_cns(hpg_ctx* c, bool sync = true) {
         hipLaunchKernelGGL(k_setup_side_cns, dim3(nblk8(c->nseg)), dim3(256), 0, c->stream, c->nseg, c->st_tri,
                            c->tprcn, c->tpc, c->sprcn, c->spc);
     if (!sync) return 0;
-    int herr = 0;
-    check(hipMemcpyAsync(&herr, c->d_err, sizeof(int), hipMemcpyDeviceToHost, c->stream), "memcpy err");
-    check(hipStreamSynchronize(c->stream), "sync");
-    return herr;
+    return read_error(c);
 }
 
 // inflow modify_boundary_residual, project_new_variables and the stage update
@@ -1090,7 +1114,6 @@ int do_setup(hpg_ctx* c, bool sync = true) {
     if (c->physics == HPG_PHYSICS_CNS) return do_setup_cns(c, sync);
     const Level& L = c->lv[c->log2p];
     const LevelDims d(L.p);
-    if (sync) check(hipMemsetAsync(c->d_err, 0, sizeof(int), c->stream), "memset");
     SetupArgs s{};
     s.pnts = c->pnts; s.tri_pnt = c->tri_pnt; s.tri_seg = c->tri_seg; s.tri_sgn = c->tri_sgn;
     s.ugv = c->ugv; s.ugs = c->ugs; s.ugi = c->ugi; s.Pmat = L.Pmat; s.tprcn = c->tprcn; s.err = c->d_err;
@@ -1127,10 +1150,7 @@ int do_setup(hpg_ctx* c, bool sync = true) {
         hipLaunchKernelGGL(k_setup_side, dim3(nblk(c->nseg)), dim3(256), 0, c->stream, c->nseg, c->st_tri,
                            c->typed_prcn ? c->tprcn_sd : c->tprcn, c->sprcn);
     if (!sync) return 0;
-    int herr = 0;
-    check(hipMemcpyAsync(&herr, c->d_err, sizeof(int), hipMemcpyDeviceToHost, c->stream), "memcpy err");
-    check(hipStreamSynchronize(c->stream), "sync");
-    return herr;
+    return read_error(c);
 }
 
 // max over (nent, nm of mstride, NV) of |x|, per variable
@@ -1452,38 +1472,12 @@ int hpg_create(const hpg_tri_mesh* m, const hpg_params* prm, hpg_ctx** out) {
         for (size_t col = 0; col + 1 < c->coff.size(); ++col)
             c->gbase[col + 1] = c->gbase[col] + ((c->coff[col + 1] - c->coff[col] + 63) / 64) * 4;
         c->ngroups = c->gbase.back();
-        const LevelDims dmax(p0);
-        c->lin = c->alloc<float>((size_t)c->ngroups * 5 * dmax.GT * 4 * 64);
-        float** f32v[] = {&c->dlv, &c->d0v, &c->r32v, &c->rr32v};
-        float** f32s[] = {&c->dls, &c->d0s, &c->r32s, &c->rr32s};
-        float** f32i[] = {&c->dli, &c->d0i, &c->r32i, &c->rr32i};
-        for (auto p : f32v) *p = c->alloc<float>(nv);
-        for (auto p : f32s) *p = c->alloc<float>(nsz);
-        for (auto p : f32i) *p = c->alloc<float>(ni);
-        c->b32v = c->alloc<float>(nv);
-        c->b32s = c->alloc<float>(nsz);
-        c->b32i = c->alloc<float>(ni);
+        c->neseg_max = neseg;
         c->fd_scal = c->alloc<double>(2);
         c->fd_max = c->alloc<unsigned>(2);
-        c->vp32 = c->alloc<float>(nv);
-        c->sp32 = c->alloc<float>((size_t)ns * NV);
-        c->tp32 = c->alloc<float>((size_t)nt * NV);
-        c->featX = c->alloc<float>((size_t)nt * MLP_IN);
-        c->mlpY = c->alloc<float>((size_t)nt * MLP_OUT);
-        c->jdiag = c->alloc<double>((size_t)nt * 3 * NV);
         // element-major vertex and side modes of the finest level (3p per element)
         c->eres = c->alloc<double>((size_t)nt * 3 * p0 * 2 * NVX);
         c->eout = c->alloc<double>((size_t)neseg * (p0 + 1) * NVX);
-        if (c->physics == HPG_PHYSICS_INS) {
-            c->eres32 = c->alloc<float>((size_t)nt * 3 * p0 * 2 * NV);
-            c->eout32 = c->alloc<float>((size_t)neseg * (p0 + 1) * NV);
-            c->tprcn_vx = c->alloc<double>((size_t)nt * NV);
-            c->tprcn_sd = c->alloc<double>((size_t)nt * NV);
-            c->tprcn_in = c->alloc<double>((size_t)nt * NV);
-            c->tp32s = c->alloc<float>((size_t)nt * NV);
-            c->tp32i = c->alloc<float>((size_t)nt * NV);
-        }
-
         for (int l = 0; l <= c->log2pmax; ++l) {
             Level& L = c->lv[l];
             L.p = 1 << l;
@@ -1534,7 +1528,7 @@ int hpg_create(const hpg_tri_mesh* m, const hpg_params* prm, hpg_ctx** out) {
                 }
             }
         }
-        check(hipStreamSynchronize(c->stream), "create sync");
+        c->arrays.flush(c->stream);
     } catch (const std::exception& ex) {
         return -1;
     }
@@ -1547,21 +1541,14 @@ int hpg_destroy(hpg_ctx* c) {
     return 0;
 }
 
-static int copy3(hpg_ctx* c, bool h2d, double* dv, double* ds, double* di, const double* hv, const double* hs,
-                 const double* hi, double* ov, double* os, double* oi) {
+static int copy3(hpg_ctx* c, bool h2d, double* dv, double* ds, double* di, const double* v, const double* s,
+                 const double* i) {
     HPG_TRY(c, {
-        const size_t nv = (size_t)c->npnt * c->nv * 8, ns = (size_t)c->nseg * c->sm0 * c->nv * 8,
-                     ni = (size_t)c->ntri * c->im0 * c->nv * 8;
-        if (h2d) {
-            check(hipMemcpyAsync(dv, hv, nv, hipMemcpyHostToDevice, c->stream), "H2D");
-            if (ns) check(hipMemcpyAsync(ds, hs, ns, hipMemcpyHostToDevice, c->stream), "H2D");
-            if (ni) check(hipMemcpyAsync(di, hi, ni, hipMemcpyHostToDevice, c->stream), "H2D");
-        } else {
-            check(hipMemcpyAsync(ov, dv, nv, hipMemcpyDeviceToHost, c->stream), "D2H");
-            if (ns) check(hipMemcpyAsync(os, ds, ns, hipMemcpyDeviceToHost, c->stream), "D2H");
-            if (ni) check(hipMemcpyAsync(oi, di, ni, hipMemcpyDeviceToHost, c->stream), "D2H");
-        }
-        check(hipStreamSynchronize(c->stream), "sync");
+        const HostSeg seg[3] = {{const_cast<double*>(v), dv, (size_t)c->npnt * c->nv * 8},
+                                {const_cast<double*>(s), ds, (size_t)c->nseg * c->sm0 * c->nv * 8},
+                                {const_cast<double*>(i), di, (size_t)c->ntri * c->im0 * c->nv * 8}};
+        if (h2d) copy_to_device(c->stream, seg, 3);
+        else copy_to_host(c->stream, seg, 3);
     });
     return 0;
 }
@@ -1569,29 +1556,28 @@ static int copy3(hpg_ctx* c, bool h2d, double* dv, double* ds, double* di, const
 int hpg_set_state(hpg_ctx* c, const double* v, const double* s, const double* i) {
     if (!c) return -2;
     c->fd_reset = true;
-    const int rc = copy3(c, true, c->ugv, c->ugs, c->ugi, v, s, i, nullptr, nullptr, nullptr);
+    const int rc = copy3(c, true, c->ugv, c->ugs, c->ugi, v, s, i);
     if (rc == 0 && c->periodic) HPG_TRY(c, periodic_sync(c));
     return rc;
 }
 int hpg_get_state(hpg_ctx* c, double* v, double* s, double* i) {
     if (!c) return -2;
-    return copy3(c, false, c->ugv, c->ugs, c->ugi, nullptr, nullptr, nullptr, v, s, i);
+    return copy3(c, false, c->ugv, c->ugs, c->ugi, v, s, i);
 }
 int hpg_get_residual(hpg_ctx* c, double* v, double* s, double* i) {
     if (!c) return -2;
-    return copy3(c, false, c->resv, c->ress, c->resi, nullptr, nullptr, nullptr, v, s, i);
+    return copy3(c, false, c->resv, c->ress, c->resi, v, s, i);
 }
 int hpg_set_residual(hpg_ctx* c, const double* v, const double* s, const double* i) {
     if (!c) return -2;
-    return copy3(c, true, c->resv, c->ress, c->resi, v, s, i, nullptr, nullptr, nullptr);
+    return copy3(c, true, c->resv, c->ress, c->resi, v, s, i);
 }
 int hpg_get_preconditioner(hpg_ctx* c, double* vp, double* sp, double* tp) {
     if (!c) return -2;
     HPG_TRY(c, {
-        check(hipMemcpyAsync(vp, c->vprcn, (size_t)c->npnt * c->nv * 8, hipMemcpyDeviceToHost, c->stream), "D2H");
-        check(hipMemcpyAsync(sp, c->sprcn, (size_t)c->nseg * c->nv * 8, hipMemcpyDeviceToHost, c->stream), "D2H");
-        check(hipMemcpyAsync(tp, c->tprcn, (size_t)c->ntri * c->nv * 8, hipMemcpyDeviceToHost, c->stream), "D2H");
-        check(hipStreamSynchronize(c->stream), "sync");
+        const HostSeg seg[3] = {{vp, c->vprcn, (size_t)c->npnt * c->nv * 8}, {sp, c->sprcn, (size_t)c->nseg * c->nv * 8},
+                                {tp, c->tprcn, (size_t)c->ntri * c->nv * 8}};
+        copy_to_host(c->stream, seg, 3);
     });
     return 0;
 }
@@ -1709,6 +1695,7 @@ int hpg_residual_fp32(hpg_ctx* c, double* ov, double* os, double* oi) {
         return hpg_get_residual(c, ov, os, oi);
     }
     HPG_TRY(c, {
+        c->need_inner();
         const long nv = (long)c->npnt * NV, nsz = (long)c->nseg * c->sm0 * NV, ni = (long)c->ntri * c->im0 * NV;
         hipLaunchKernelGGL(k_base32, dim3(std::min<unsigned>(nblk(nv), RED_BLOCKS)), dim3(256), 0, c->stream, nv, c->ugv, c->b32v, c->dlv, c->fd_max);
         if (nsz) hipLaunchKernelGGL(k_base32, dim3(std::min<unsigned>(nblk(nsz), RED_BLOCKS)), dim3(256), 0, c->stream, nsz, c->ugs, c->b32s, c->dls, c->fd_max);
@@ -1746,6 +1733,8 @@ int hpg_apply_jacobian(hpg_ctx* c, const double* dv, const double* ds, const dou
     if (c->log2p != c->log2pmax) { c->err = "apply_jacobian runs on the finest level"; return -2; }
     HPG_TRY(c, {
         const size_t nv = (size_t)c->npnt * NV, nsz = (size_t)c->nseg * c->sm0 * NV, ni = (size_t)c->ntri * c->im0 * NV;
+        c->need_inner();
+        c->need_lin();
         do_rsdl(c, c->prm.nstage, true);
         std::vector<float> hv(dv, dv + nv), hs(nsz), hi(ni);
         for (size_t k = 0; k < nsz; ++k) hs[k] = (float)ds[k];
@@ -1775,6 +1764,7 @@ int hpg_set_prcn_log_scalings(hpg_ctx* c, const float* y) {
     if (!c || c->physics != HPG_PHYSICS_INS) return -2;
     if (!y) { c->user_y = false; return 0; }
     HPG_TRY(c, {
+        c->need_learned();
         check(hipMemcpyAsync(c->mlpY, y, (size_t)c->ntri * MLP_OUT * 4, hipMemcpyHostToDevice, c->stream), "H2D");
         check(hipStreamSynchronize(c->stream), "sync");
         c->user_y = true;
@@ -1786,6 +1776,7 @@ int hpg_mlp_features(hpg_ctx* c, float* out) {
     if (!c || !out) return -2;
     if (c->physics != HPG_PHYSICS_INS) { c->err = "ins only"; return -2; }
     HPG_TRY(c, {
+        c->need_learned();
         hipLaunchKernelGGL(k_mlp_features, dim3(nblk(c->ntri)), dim3(256), 0, c->stream, c->ntri, c->pnts, c->tri_pnt,
                            c->ugv, c->tprcn, c->prm.mu, c->prm.rho, c->featX);
         check(hipMemcpyAsync(out, c->featX, (size_t)c->ntri * MLP_IN * 4, hipMemcpyDeviceToHost, c->stream), "D2H");
@@ -1801,6 +1792,8 @@ int hpg_measure_jacobian_diag(hpg_ctx* c, double* out) {
     if (c->physics != HPG_PHYSICS_INS) { c->err = "ins only"; return -2; }
     if (c->log2p != c->log2pmax) { c->err = "measure_jacobian_diag runs on the finest level"; return -2; }
     HPG_TRY(c, {
+        c->need_lin();
+        if (!c->jdiag) c->jdiag = c->alloc<double>((size_t)c->ntri * 3 * NV);
         do_rsdl(c, c->prm.nstage, true);
         check(hipMemsetAsync(c->jdiag, 0, (size_t)c->ntri * 3 * NV * 8, c->stream), "memset");
         const Level& L = c->lv[c->log2p];
@@ -1865,8 +1858,8 @@ int hpg_element_jacobian(hpg_ctx* c, const int* tind, int nel, double eps_r, dou
                 case 4: element_jacobians<4>(c, d_tind + j0, nj, N, eps_r, eps_a, base, dK); break;
                 default: throw std::runtime_error("unsupported p");
             }
-            check(hipMemcpyAsync(K + (size_t)j0 * N * N, dK, (size_t)nj * N * N * 8, hipMemcpyDeviceToHost, c->stream), "D2H");
-            check(hipStreamSynchronize(c->stream), "sync");
+            const HostSeg seg{K + (size_t)j0 * N * N, dK, (size_t)nj * N * N * 8};
+            copy_to_host(c->stream, &seg, 1);
         }
     });
     return 0;
@@ -2192,10 +2185,7 @@ int hpg_mg_cycle(hpg_ctx* const* grids, int ngrid, int extra_finest_levels, int 
         unsigned long long mx[NVC] = {0, 0, 0, 0};
         check(hipMemcpyAsync(mx, f->d_max, sizeof(mx), hipMemcpyDeviceToHost, f->stream), "D2H");
         for (int k = 0; k < ngrid; ++k) {
-            int e = 0;
-            check(hipMemcpyAsync(&e, grids[k]->d_err, sizeof(int), hipMemcpyDeviceToHost, grids[k]->stream), "D2H");
-            check(hipStreamSynchronize(grids[k]->stream), "sync");
-            nerr += e != 0;
+            nerr += read_error(grids[k]) != 0;
         }
         double m = 0.0;
         for (int n = 0; n < f->nv; ++n) {
@@ -2233,6 +2223,7 @@ int hpg_set_precision(hpg_ctx* c, int mode) {
             check(hipStreamSynchronize(c->stream), "sync");
         });
     }
+    if (c->physics == HPG_PHYSICS_INS && mode == HPG_FP32_DEFECT) HPG_TRY(c, c->need_inner());
     c->precision = mode;
     c->fd_reset = true;
     return 0;
@@ -2241,6 +2232,7 @@ int hpg_set_precision(hpg_ctx* c, int mode) {
 int hpg_set_preconditioner(hpg_ctx* c, int mode) {
     if (!c || (mode != HPG_PRCN_ANALYTIC && mode != HPG_PRCN_LEARNED)) return -2;
     if (c->physics != HPG_PHYSICS_INS && mode != HPG_PRCN_ANALYTIC) { c->err = "the learned preconditioner is built for ins"; return -2; }
+    if (mode == HPG_PRCN_LEARNED) HPG_TRY(c, c->need_learned());
     c->prcn_mode = mode;
     return 0;
 }

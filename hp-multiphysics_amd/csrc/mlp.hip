@@ -20,6 +20,7 @@
 
 #include "../../include/hpgpu.h"
 #include "mlp.h"
+#include "host_copy.h"
 
 namespace hpg {
 
@@ -530,6 +531,7 @@ using namespace hpg;
 
 struct hpg_mlp {
     hipStream_t stream = nullptr;
+    HostCopyUser staging;
     float *master = nullptr, *wq = nullptr, *m1 = nullptr, *m2 = nullptr, *grad = nullptr;
     float *partial = nullptr, *lossp = nullptr, *X = nullptr, *T = nullptr, *Y = nullptr;
     double* lsum = nullptr;  // loss sum of a training run's last epoch
@@ -566,6 +568,12 @@ void ensure_n(hpg_mlp* m, int n) {
     ck(hipMalloc(&m->T, (size_t)n * MO * 4), "hipMalloc");
     ck(hipMalloc(&m->Y, (size_t)n * MO * 4), "hipMalloc");
     m->cap_n = n;
+}
+// the caller's samples (and targets) into X (and T)
+void send_batch(hpg_mlp* m, const float* X, const float* T, int n) {
+    const HostSeg seg[2] = {{const_cast<float*>(X), m->X, (size_t)n * MI * 4},
+                            {const_cast<float*>(T), m->T, T ? (size_t)n * MO * 4 : 0}};
+    copy_to_device(m->stream, seg, 2);
 }
 // device address of `scratch` per GPU, resolved once per device with that device
 // current (each GPU holds its own copy of the array at its own address)
@@ -698,10 +706,10 @@ int hpg_mlp_forward(hpg_mlp* m, const float* X, int n, float* Y) {
     if (!m || !X || !Y || n < 0) return -2;
     try {
         ensure_n(m, n);
-        ck(hipMemcpyAsync(m->X, X, (size_t)n * MI * 4, hipMemcpyHostToDevice, m->stream), "H2D");
+        send_batch(m, X, nullptr, n);
         mlp_forward_device(m, m->X, n, m->Y, m->stream);
-        ck(hipMemcpyAsync(Y, m->Y, (size_t)n * MO * 4, hipMemcpyDeviceToHost, m->stream), "D2H");
-        ck(hipStreamSynchronize(m->stream), "sync");
+        const HostSeg seg{Y, m->Y, (size_t)n * MO * 4};
+        copy_to_host(m->stream, &seg, 1);
     } catch (const std::exception& e) { m->err = e.what(); return -1; }
     return 0;
 }
@@ -713,8 +721,7 @@ int hpg_mlp_loss_grad(hpg_mlp* m, const float* X, const float* T, int n, float* 
         ensure_n(m, n);
         const int nb = train_blocks(n);
         ensure_blocks(m, nb);
-        ck(hipMemcpyAsync(m->X, X, (size_t)n * MI * 4, hipMemcpyHostToDevice, m->stream), "H2D");
-        ck(hipMemcpyAsync(m->T, T, (size_t)n * MO * 4, hipMemcpyHostToDevice, m->stream), "H2D");
+        send_batch(m, X, T, n);
         enqueue_loss_grad(m, m->X, m->T, n, m->partial, m->lossp, m->grad);
         std::vector<float> lp(nb);
         ck(hipMemcpyAsync(lp.data(), m->lossp, nb * 4, hipMemcpyDeviceToHost, m->stream), "D2H");
@@ -759,8 +766,7 @@ int hpg_mlp_train(hpg_mlp* m, const float* X, const float* T, int n, int epochs,
         ensure_n(m, n);
         batch = ((batch + 63) / 64) * 64;
         ensure_blocks(m, train_blocks(std::min(batch, n)));
-        ck(hipMemcpyAsync(m->X, X, (size_t)n * MI * 4, hipMemcpyHostToDevice, m->stream), "H2D");
-        ck(hipMemcpyAsync(m->T, T, (size_t)n * MO * 4, hipMemcpyHostToDevice, m->stream), "H2D");
+        send_batch(m, X, T, n);
         double lsum = 0.0;
         ck(hipMemcpyAsync(m->lsum, &lsum, sizeof(double), hipMemcpyHostToDevice, m->stream), "H2D");
         for (int ep = 0; ep < epochs; ++ep) {
