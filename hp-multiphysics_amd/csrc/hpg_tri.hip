@@ -248,6 +248,7 @@ struct hpg_ctx {
     int *sedge = nullptr, *enext = nullptr;  // each side's first edge in eseg, each edge's next one
     float* eout32 = nullptr;
     int *vs_ptr, *vs_side, *vs_end, *vt_ptr, *vt_tri, *vt_loc, *st_tri, *st_loc;
+    double* mplane = nullptr;  // p = 4: work planes of the side sweeps of minvrt
     unsigned char *vess, *sess;
     unsigned char *fcv, *fcs;  // first colour touching each vertex / side
     unsigned char* tcol = nullptr;  // cns: colour of each element
@@ -577,6 +578,8 @@ MinvArgsT<T> minv_args(hpg_ctx* c) {
     a.ugv = a.ugs = a.ugi = nullptr;
     a.ug0v = a.ug0s = a.ug0i = nullptr;
     a.cfa = T(0);
+    a.pl = reinterpret_cast<T*>(c->mplane);
+    a.store = 1;
     return a;
 }
 
@@ -829,9 +832,9 @@ void do_lin_rsdl(hpg_ctx* c, int stage, bool with_source) {
 
 template <typename T, int NVn>
 void launch_minv_nv(hpg_ctx* c, const MinvArgsT<T>& a) {
-    // one lane per (entity, variable); k_minv_sscale one lane per (side, mode, variable)
+    // one lane per (entity, variable); the mode sweeps take 64 sides per block
     const dim3 bv(nblk8((long)c->npnt * NVn)), bs(nblk8((long)c->nseg * NVn)), bt(nblk8((long)c->ntri * NVn));
-    const dim3 bq(nblk8((long)c->nseg * a.sm * NVn)), th(256);
+    const dim3 b64(nblk8(c->nseg, 64)), th(256), t64(64 * NVn);
     switch (a.sm + 1) {
         case 1:
             hipLaunchKernelGGL((k_minv_vrtx<T, 1, NVn>), bv, th, 0, c->stream, a);
@@ -839,14 +842,12 @@ void launch_minv_nv(hpg_ctx* c, const MinvArgsT<T>& a) {
         case 2:
             hipLaunchKernelGGL((k_minv_vrtx<T, 2, NVn>), bv, th, 0, c->stream, a);
             hipLaunchKernelGGL((k_minv_side<T, 2, NVn>), bs, th, 0, c->stream, a);
-            hipLaunchKernelGGL((k_minv_sscale<T, 2, NVn>), bq, th, 0, c->stream, a);
             break;
         case 4:
             hipLaunchKernelGGL((k_minv_vrtx<T, 4, NVn>), bv, th, 0, c->stream, a);
             hipLaunchKernelGGL((k_minv_side<T, 4, NVn>), bs, th, 0, c->stream, a);
-            hipLaunchKernelGGL((k_minv_sub<T, 4, 0, NVn>), bs, th, 0, c->stream, a);
-            hipLaunchKernelGGL((k_minv_sub<T, 4, 1, NVn>), bs, th, 0, c->stream, a);
-            hipLaunchKernelGGL((k_minv_sscale<T, 4, NVn>), bq, th, 0, c->stream, a);
+            hipLaunchKernelGGL((k_minv_sub<T, 4, 0, NVn>), b64, t64, 0, c->stream, a);
+            hipLaunchKernelGGL((k_minv_sub<T, 4, 1, NVn>), b64, t64, 0, c->stream, a);
             hipLaunchKernelGGL((k_minv_int<T, 4, NVn>), bt, th, 0, c->stream, a);
             break;
         default:
@@ -862,9 +863,11 @@ void launch_minv(hpg_ctx* c, const MinvArgsT<T>& a) {
 }
 
 // minvrt; with update_cfa >= 0 the stage update ug = ug0 - update_cfa*res is fused
-// into the sweeps that produce the final vertex, side and interior values
-void do_minvrt(hpg_ctx* c, double update_cfa = -1.0) {
+// into the sweeps that produce the final vertex, side and interior values; last = false:
+// another stage follows, which overwrites the residual arrays unread
+void do_minvrt(hpg_ctx* c, double update_cfa = -1.0, bool last = true) {
     MinvArgsT<double> a = minv_args<double>(c);
+    a.store = last ? 1 : 0;
     if (update_cfa >= 0.0) {
         a.ugv = c->ugv; a.ug0v = c->ug0v; a.cfa = update_cfa;
         if (a.sm > 0) { a.ugs = c->ugs; a.ug0s = c->ug0s; }
@@ -876,6 +879,7 @@ void do_minvrt(hpg_ctx* c, double update_cfa = -1.0) {
 // FP32 minvrt of the inner residual with the fused delta update
 void do_minvrt32(hpg_ctx* c, float cfa) {
     MinvArgsT<float> a = minv_args<float>(c);
+    a.store = 0;  // nothing reads the corrections of the FP32 stages
     a.ugv = c->dlv; a.ug0v = c->d0v; a.cfa = cfa;
     if (a.sm > 0) { a.ugs = c->dls; a.ug0s = c->d0s; }
     if (a.im > 0) { a.ugi = c->dli; a.ug0i = c->d0i; }
@@ -1477,6 +1481,7 @@ int hpg_create(const hpg_tri_mesh* m, const hpg_params* prm, hpg_ctx** out) {
         c->fd_max = c->alloc<unsigned>(2);
         // element-major vertex and side modes of the finest level (3p per element)
         c->eres = c->alloc<double>((size_t)nt * 3 * p0 * 2 * NVX);
+        if (p0 == 4) c->mplane = c->alloc<double>((size_t)ns * c->sm0 * NVX);
         c->eout = c->alloc<double>((size_t)neseg * (p0 + 1) * NVX);
         for (int l = 0; l <= c->log2pmax; ++l) {
             Level& L = c->lv[l];
@@ -1891,7 +1896,7 @@ void do_update(hpg_ctx* c) {
     if (ni) dcopy(c, c->ug0i, c->ugi, ni);
     for (int stage = 0; stage < c->prm.nstage; ++stage) {
         do_rsdl(c, stage);
-        do_minvrt(c, c->prm.alpha[stage] * c->prm.cfl[c->log2p]);
+        do_minvrt(c, c->prm.alpha[stage] * c->prm.cfl[c->log2p], stage + 1 == c->prm.nstage);
     }
     check(hipGetLastError(), "update launch");
 }

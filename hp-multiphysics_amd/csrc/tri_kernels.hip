@@ -1396,6 +1396,13 @@ struct MinvArgsT {
     const T* lump;  // sfmv | ifmb | vfms | sdiag | sfms | bfmi | idiag
     int npnt, nseg, ntri, sm, im, bm, sm0, im0;
     int o_sfmv, o_ifmb, o_vfms, o_sdiag, o_sfms, o_bfmi, o_idiag;
+    // p = 4: work planes of the side sweeps, one per mode, (mode, side, variable).  A sweep
+    // reads one mode of four neighbouring sides: from the (side, mode, variable) records it
+    // would fetch all three
+    T* pl;
+    // the solved side and interior values go to ress / resi (always, unless another stage
+    // of the same update overwrites them unread)
+    int store;
     // fused stage update ug = ug0 - cfa * res (tri_hp/nstage.cpp:387-409) when ug != null
     T* ugv;
     T* ugs;
@@ -1518,7 +1525,15 @@ __global__ __launch_bounds__(256) void k_vstage1(VStageArgs a) {
     }
 }
 
-// sides: subtract interior couplings (:137-148), then the vertex solution (:192-214)
+// solved value of side mode `mode` from its residual r (:245-267, :331-343): scale, sdirichlet
+template <typename T, int NVn>
+__device__ __forceinline__ T side_solved(const MinvArgsT<T>& a, int s, int mode, int n, T r) {
+    if ((a.sess[s] >> n) & 1) return T(0);
+    return r * (a.sprcn[s * NVn + n] * a.lump[a.o_sdiag + mode]);
+}
+
+// sides: subtract interior couplings (:137-148), then the vertex solution (:192-214), and
+// solve mode 0 (p = 2: the only one, stored with its stage update)
 template <typename T, int P, int NVn>
 __global__ __launch_bounds__(256) void k_minv_side(MinvArgsT<T> a) {
     constexpr int SM = Dims<P>::SM, IM = Dims<P>::IM;
@@ -1567,75 +1582,85 @@ __global__ __launch_bounds__(256) void k_minv_side(MinvArgsT<T> a) {
             }
         }
     }
+    const T x0 = side_solved<T, NVn>(a, s, 0, n, r[0]);
+    if constexpr (SM == 1) {
+        const int ix = s * a.sm0 * NVn + n;
+        const T u0 = a.ugs ? a.ug0s[ix] : T(0);
+        if (a.store) a.ress[ix] = x0;
+        if (a.ugs) a.ugs[ix] = u0 - a.cfa * x0;
+    } else {
+        a.pl[s * NVn + n] = x0;
 #pragma unroll
-    for (int m = 0; m < SM; ++m) a.ress[(s * a.sm0 + m) * NVn + n] = r[m];
+        for (int m = 1; m < SM; ++m) a.pl[((long)m * a.nseg + s) * NVn + n] = r[m];
+    }
 }
 
-template <typename T, int NVn>
-__device__ __forceinline__ T side_scaled(const MinvArgsT<T>& a, int s, int mode, int n) {
-    if ((a.sess[s] >> n) & 1) return T(0);
-    return a.ress[(s * a.sm0 + mode) * NVn + n] * (a.sprcn[s * NVn + n] * a.lump[a.o_sdiag + mode]);
-}
-
-// remove solved side mode `MODE` from the higher modes (:244-328); the solved value
-// sprcn*sdiag*res with sdirichlet is formed on the fly, stored later by k_minv_sscale
+// remove solved side mode MODE from the higher modes (:244-328) and solve mode MODE + 1.
+// The last mode's sweep also stores the solved values and the stage update: 64 sides per
+// block go through LDS so that the (side, mode, variable) records are read and written as
+// one contiguous stream.  512 x 512, p = 4, FP64: MEASURED_SUB
 template <typename T, int P, int MODE, int NVn>
-__global__ __launch_bounds__(256) void k_minv_sub(MinvArgsT<T> a) {
+__global__ __launch_bounds__(64 * NVn) void k_minv_sub(MinvArgsT<T> a) {
     constexpr int SM = Dims<P>::SM;
-    int s, n;
-    if (!minv_lane<T, NVn>(a.nseg, s, n)) return;
-    T r[SM];
+    constexpr bool LAST = MODE == SM - 2;
+    __shared__ T sx[LAST ? 64 * SM * NVn : 1];
+    const int blk = xcd_block();
+    const int ls = threadIdx.x / NVn, n = threadIdx.x - ls * NVn;
+    const int s = blk * 64 + ls;
+    if (s < a.nseg) {
+        T r[SM];
 #pragma unroll
-    for (int m = MODE + 1; m < SM; ++m) r[m] = a.ress[(s * a.sm0 + m) * NVn + n];
-    for (int k = 0; k < 2; ++k) {
-        const int t = a.st_tri[2 * s + k];
-        if (t < 0) continue;
-        const int sl = a.st_loc[2 * s + k], i = sl & 3;
-        const T tp = a.tprcn_s[NVn * t + n];
-        T uh[3];
-        int sign[3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const int jj = (i + j) % 3;
-            const int sj = a.tri_seg[3 * t + jj];
-            sign[j] = a.tri_sgn[3 * t + jj];
-            const T sg = (MODE % 2) ? T(sign[j]) : T(1);
-            uh[j] = sg * side_scaled<T, NVn>(a, sj, MODE, n) * tp;
-        }
-        // into this side's frame: a periodic partner's element (st_loc bit 2) has its
-        // own copy of the side running the other way
-        const int s0 = (sl & 4) ? -sign[0] : sign[0];
-        T ms = ((MODE + 1) % 2) ? T(s0) : T(1);
-#pragma unroll
-        for (int m = MODE + 1; m < SM; ++m) {
+        for (int m = MODE + 1; m < SM; ++m) r[m] = a.pl[((long)m * a.nseg + s) * NVn + n];
+        for (int k = 0; k < 2; ++k) {
+            const int t = a.st_tri[2 * s + k];
+            if (t < 0) continue;
+            const int sl = a.st_loc[2 * s + k], i = sl & 3;
+            const T tp = a.tprcn_s[NVn * t + n];
+            T uh[3];
+            int sign[3];
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
-                const T c = ms * a.lump[a.o_sfms + (MODE * SM + m) * 3 + j];
-                r[m] -= c * uh[j];
+                const int jj = (i + j) % 3;
+                const int sj = a.tri_seg[3 * t + jj];
+                sign[j] = a.tri_sgn[3 * t + jj];
+                const T sg = (MODE % 2) ? T(sign[j]) : T(1);
+                uh[j] = sg * a.pl[((long)MODE * a.nseg + sj) * NVn + n] * tp;
             }
-            ms *= s0;
+            // into this side's frame: a periodic partner's element (st_loc bit 2) has its
+            // own copy of the side running the other way
+            const int s0 = (sl & 4) ? -sign[0] : sign[0];
+            T ms = ((MODE + 1) % 2) ? T(s0) : T(1);
+#pragma unroll
+            for (int m = MODE + 1; m < SM; ++m) {
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    const T c = ms * a.lump[a.o_sfms + (MODE * SM + m) * 3 + j];
+                    r[m] -= c * uh[j];
+                }
+                ms *= s0;
+            }
+        }
+        const T x = side_solved<T, NVn>(a, s, MODE + 1, n, r[MODE + 1]);
+        a.pl[((long)(MODE + 1) * a.nseg + s) * NVn + n] = x;
+        if constexpr (LAST) {
+#pragma unroll
+            for (int m = 0; m < SM - 1; ++m) sx[(ls * SM + m) * NVn + n] = a.pl[((long)m * a.nseg + s) * NVn + n];
+            sx[(ls * SM + SM - 1) * NVn + n] = x;
+        } else {
+#pragma unroll
+            for (int m = MODE + 2; m < SM; ++m) a.pl[((long)m * a.nseg + s) * NVn + n] = r[m];
         }
     }
-#pragma unroll
-    for (int m = MODE + 1; m < SM; ++m) a.ress[(s * a.sm0 + m) * NVn + n] = r[m];
-}
-
-// store the solved side modes: res.s *= sprcn*sdiag(mode), sdirichlet (:245-267, :331-343);
-// one lane per (side, mode, variable), so on the finest level the sweep is a plain
-// contiguous stream
-template <typename T, int P, int NVn>
-__global__ __launch_bounds__(256) void k_minv_sscale(MinvArgsT<T> a) {
-    constexpr int SM = Dims<P>::SM;
-    const long g = (long)xcd_block() * blockDim.x + threadIdx.x;
-    const int s = (int)(g / (SM * NVn));
-    if (s >= a.nseg) return;
-    const int mn = (int)(g - (long)s * (SM * NVn)), m = mn / NVn, n = mn - m * NVn;
-    const int ix = (s * a.sm0 + m) * NVn + n;
-    // every load before the first store: the stores could alias later loads
-    const T x = side_scaled<T, NVn>(a, s, m, n);
-    const T u0 = a.ugs ? a.ug0s[ix] : T(0);
-    a.ress[ix] = x;
-    if (a.ugs) a.ugs[ix] = u0 - a.cfa * x;
+    if constexpr (LAST) {
+        __syncthreads();
+        const long o = (long)blk * 64 * SM * NVn;
+        const int cnt = min(64, a.nseg - blk * 64) * SM * NVn;
+        for (int k = threadIdx.x; k < cnt; k += 64 * NVn) {
+            const T u0 = a.ugs ? a.ug0s[o + k] : T(0);
+            if (a.store) a.ress[o + k] = sx[k];
+            if (a.ugs) a.ugs[o + k] = u0 - a.cfa * sx[k];
+        }
+    }
 }
 
 // interiors: banded solve with the literal DPBTRSNU2 indexing (utilities/myblas.c:91-122),
@@ -1672,7 +1697,7 @@ __global__ __launch_bounds__(256) void k_minv_int(MinvArgsT<T> a) {
         T ms = T(1);
 #pragma unroll
         for (int m = 0; m < SM; ++m) {
-            uh[3 + i * SM + m] = ms * a.ress[(sd * a.sm0 + m) * NVn + n];
+            uh[3 + i * SM + m] = ms * a.pl[((long)m * a.nseg + sd) * NVn + n];
             ms *= sgn;
         }
     }
@@ -1689,7 +1714,7 @@ __global__ __launch_bounds__(256) void k_minv_int(MinvArgsT<T> a) {
 #pragma unroll
     for (int k = 0; k < IM; ++k) {
         const int ix = (t * a.im0 + k) * NVn + n;
-        a.resi[ix] = b[k];
+        if (a.store) a.resi[ix] = b[k];
         if (a.ugi) a.ugi[ix] = u0[k] - a.cfa * b[k];
     }
 }
