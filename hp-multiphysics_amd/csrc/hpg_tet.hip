@@ -300,23 +300,18 @@ void launch_elem_tet32(hpg_tet_ctx* c, int stage) {
     }
 }
 
-template <int NVn>
-void tet_modes_nv(hpg_tet_ctx* c, int op, double* xv, double* xe, double* yv, double* ye, const double* zv,
-                  const double* ze, double k) {
-    const long nv = (long)c->npnt * NVn;
-    hipLaunchKernelGGL(k_modes<NVn>, dim3(nblk(nv)), dim3(256), 0, c->stream, op, (long)c->npnt, 1, 1, xv, yv, zv, k);
-    const int em = c->em();
-    if (em > 0) {
-        const long ne = (long)c->nseg * em * NVn;
-        hipLaunchKernelGGL(k_modes<NVn>, dim3(nblk(ne)), dim3(256), 0, c->stream, op, (long)c->nseg, em, c->em0, xe, ye,
-                           ze, k);
-    }
-}
-
 void tet_modes(hpg_tet_ctx* c, int op, double* xv, double* xe, double* yv, double* ye, const double* zv,
                const double* ze, double k) {
-    if (c->cns()) tet_modes_nv<CNV>(c, op, xv, xe, yv, ye, zv, ze, k);
-    else tet_modes_nv<TNV>(c, op, xv, xe, yv, ye, zv, ze, k);
+    launch_modes(c->stream, c->nv, op, {{c->npnt, 1, 1, xv, yv, zv}, {c->nseg, c->em(), c->em0, xe, ye, ze}}, k);
+}
+
+Span3 tet_span(const hpg_tet_ctx* c) { return span3((long)c->npnt * c->nv, (long)c->nseg * c->em0 * c->nv); }
+
+// ug0 = ug
+void save_state_tet(hpg_tet_ctx* c) {
+    const Span3 n = tet_span(c);
+    hipLaunchKernelGGL(k_span_copy<double>, span_grid(n), dim3(256), 0, c->stream, n,
+                       Ptr3<const double>{{c->ugv, c->uge, nullptr}}, Ptr3<double>{{c->ug0v, c->ug0e, nullptr}});
 }
 
 // tet_hp::rsdl (tet_hp/update.cpp:9-131).  fp32: the element residual in FP32 arithmetic
@@ -401,11 +396,7 @@ void do_minvrt_tetc(hpg_tet_ctx* c, double cfa) {
     if (a.em > 0) {
         if (upd) { a.uge_out = c->uge; a.ug0e = c->ug0e; }
         hipLaunchKernelGGL(k_minv_edge_tetc, dim3(nblk8(c->nseg)), dim3(256), 0, c->stream, a);
-        if (upd) {
-            const long n = (long)c->npnt * CNV;
-            hipLaunchKernelGGL(k_modes<CNV>, dim3(nblk(n)), dim3(256), 0, c->stream, 4, (long)c->npnt, 1, 1, c->ugv,
-                               c->ug0v, c->resv, cfa);
-        }
+        if (upd) launch_modes(c->stream, CNV, 4, {{c->npnt, 1, 1, c->ugv, c->ug0v, c->resv}}, cfa);
     }
     check(hipGetLastError(), "tet cns minvrt launch");
 }
@@ -469,46 +460,36 @@ int do_setup_tet(hpg_tet_ctx* c) {
     return read_error(c);
 }
 
-// y += sfac[0] x (the scaled defect source of the inner solve)
-__global__ void k_axpy_dev(long n, const double* __restrict__ x, const double* __restrict__ sfac, double* __restrict__ y) {
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) y[k] += sfac[0] * x[k];
-}
-
 // FP32 defect correction of tet_hp::update / tet_hp_cns::update with FP64 storage: the
 // outer iteration of the tri cns form (mixed_update_cns).  R64(u0) is kept in src; the
 // inner state v = fl32(u0) + dhat lives in ug, so minvrt and the stage update run as
 // in the FP64 update; stage 0 is R64(u0)/c, the later stages evaluate the element
 // residual in FP32 and add (1/c - 1) R64(u0); finally u = u0 + c (v - fl32(u0)).
 void mixed_update_tet(hpg_tet_ctx* c) {
-    const long nv = (long)c->npnt * c->nv, ne = (long)c->nseg * c->em0 * c->nv;
+    const Span3 n = tet_span(c);
+    const dim3 th(256), all = span_grid(n), red = span_grid_reduce(n);
+    const Ptr3<double> u{{c->ugv, c->uge, nullptr}}, res{{c->resv, c->rese, nullptr}};
     do_rsdl_tet(c, c->prm.nstage);
-    auto copy = [&](double* dst, const double* src, long n) {
-        if (n) check(hipMemcpyAsync(dst, src, n * 8, hipMemcpyDeviceToDevice, c->stream), "D2D");
-    };
-    auto grid = [](long n) { return dim3(std::min<unsigned>(nblk(n), RED_BLOCKS)); };
-    copy(c->srcv, c->resv, nv); copy(c->srce, c->rese, ne);
-    copy(c->u0cv, c->ugv, nv); copy(c->u0ce, c->uge, ne);
-    hipLaunchKernelGGL(k_round32, grid(nv), dim3(256), 0, c->stream, nv, c->ugv, c->fd_max);
-    if (ne) hipLaunchKernelGGL(k_round32, grid(ne), dim3(256), 0, c->stream, ne, c->uge, c->fd_max);
+    hipLaunchKernelGGL(k_fd_open64, red, th, 0, c->stream, n, Ptr3<const double>{{c->resv, c->rese, nullptr}},
+                       Ptr3<double>{{c->srcv, c->srce, nullptr}}, u, Ptr3<double>{{c->u0cv, c->u0ce, nullptr}},
+                       Ptr3<double>{{c->ug0v, c->ug0e, nullptr}}, c->fd_max);
     hipLaunchKernelGGL(k_fd_scale, dim3(1), dim3(1), 0, c->stream, c->fd_scal, c->fd_max, c->fd_reset ? 1 : 0, FD_H);
     c->fd_reset = false;
     for (int it = 0; it < c->ninner; ++it) {
-        copy(c->ug0v, c->ugv, nv); copy(c->ug0e, c->uge, ne);
+        if (it) save_state_tet(c);
         for (int s = 0; s < c->prm.nstage; ++s) {
             if (it == 0 && s == 0) {
-                hipLaunchKernelGGL(k_scale64, dim3(nblk(nv)), dim3(256), 0, c->stream, nv, c->resv, c->fd_scal);
-                if (ne) hipLaunchKernelGGL(k_scale64, dim3(nblk(ne)), dim3(256), 0, c->stream, ne, c->rese, c->fd_scal);
+                hipLaunchKernelGGL(k_fd_first64, all, th, 0, c->stream, n, res, c->fd_scal);
             } else {
                 do_rsdl_tet(c, s, true);
-                hipLaunchKernelGGL(k_axpy_dev, dim3(nblk(nv)), dim3(256), 0, c->stream, nv, c->srcv, c->fd_scal + 1, c->resv);
-                if (ne) hipLaunchKernelGGL(k_axpy_dev, dim3(nblk(ne)), dim3(256), 0, c->stream, ne, c->srce, c->fd_scal + 1, c->rese);
+                hipLaunchKernelGGL(k_span_axpy, all, th, 0, c->stream, n, c->fd_scal + 1,
+                                   Ptr3<const double>{{c->srcv, c->srce, nullptr}}, res);
             }
             do_minvrt_tet(c, !c->cns(), c->prm.alpha[s] * c->prm.cfl[c->log2p]);
         }
     }
-    hipLaunchKernelGGL(k_fd_final64, grid(nv), dim3(256), 0, c->stream, nv, c->ugv, c->u0cv, c->fd_scal, c->fd_max + 1);
-    if (ne) hipLaunchKernelGGL(k_fd_final64, grid(ne), dim3(256), 0, c->stream, ne, c->uge, c->u0ce, c->fd_scal, c->fd_max + 1);
+    hipLaunchKernelGGL(k_fd_close64, red, th, 0, c->stream, n, u, Ptr3<const double>{{c->u0cv, c->u0ce, nullptr}},
+                       c->fd_scal, c->fd_max + 1);
     check(hipGetLastError(), "tet mixed update launch");
 }
 
@@ -742,10 +723,7 @@ int hpg_tet_update(hpg_tet_ctx* c) {
     HPG_TRY(c, {
         // tet_hp::update (update.cpp:181-417) and tet_hp_cns::update (cns/update.cpp:18-143,
         // no Dirichlet pass before minvrt)
-        check(hipMemcpyAsync(c->ug0v, c->ugv, (size_t)c->npnt * c->nv * 8, hipMemcpyDeviceToDevice, c->stream), "D2D");
-        if (c->em0)
-            check(hipMemcpyAsync(c->ug0e, c->uge, (size_t)c->nseg * c->em0 * c->nv * 8, hipMemcpyDeviceToDevice,
-                                 c->stream), "D2D");
+        save_state_tet(c);
         for (int s = 0; s < c->prm.nstage; ++s) {
             do_rsdl_tet(c, s);
             do_minvrt_tet(c, !c->cns(), c->prm.alpha[s] * c->prm.cfl[c->log2p]);

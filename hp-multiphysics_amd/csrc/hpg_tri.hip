@@ -4,6 +4,7 @@
 // block's mesh and solution arrays, the per-level operator packs, the element
 // colouring used for the deterministic scatter, and one HIP stream.  Everything
 // between hpg_set_state and hpg_get_state stays resident in HBM.
+#include <initializer_list>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -368,31 +369,44 @@ static inline unsigned nblk8(long n, int bs = 256) { return ((nblk(n, bs) + 7u) 
 
 namespace {
 
-// device-to-device copy of `bytes` (a multiple of 4) as a kernel launch, so that a
-// captured cycle holds kernel nodes only
-void dcopy(hpg_ctx* c, void* dst, const void* src, size_t bytes) {
-    const long n = (long)(bytes / 4);
-    if (n <= 0) return;
-    const unsigned nb = std::min<unsigned>(nblk(n), 4096u);
-    hipLaunchKernelGGL(k_copy_words, dim3(nb), dim3(256), 0, c->stream, n, (const unsigned*)src, (unsigned*)dst);
+// spans over the vertex, side and interior parts of a context's arrays (one kernel launch
+// each: a captured cycle holds kernel nodes only)
+Span3 span3(long n0, long n1 = 0, long n2 = 0) { return Span3{{n0, n0 + n1, n0 + n1 + n2}}; }
+Span3 state_span(const hpg_ctx* c) {
+    return span3((long)c->npnt * c->nv, (long)c->nseg * c->sm0 * c->nv, (long)c->ntri * c->im0 * c->nv);
+}
+dim3 span_grid(const Span3& n) { return dim3(nblk(n.end[2])); }
+dim3 span_grid_reduce(const Span3& n) { return dim3(std::min<unsigned>(nblk(n.end[2]), RED_BLOCKS)); }
+
+// ug0 = ug
+void save_state(hpg_ctx* c) {
+    const Span3 n = state_span(c);
+    hipLaunchKernelGGL(k_span_copy<double>, span_grid(n), dim3(256), 0, c->stream, n,
+                       Ptr3<const double>{{c->ugv, c->ugs, c->ugi}}, Ptr3<double>{{c->ug0v, c->ug0s, c->ug0i}});
 }
 
-void launch_modes(hpg_ctx* c, int op, long nent, int nm, int mstride, double* x, double* y, const double* z, double k) {
-    if (nent <= 0 || nm <= 0) return;
-    const long n = nent * nm * c->nv;
-    if (c->nv == NVC)
-        hipLaunchKernelGGL(k_modes<NVC>, dim3(nblk(n)), dim3(256), 0, c->stream, op, nent, nm, mstride, x, y, z, k);
-    else
-        hipLaunchKernelGGL(k_modes<NV>, dim3(nblk(n)), dim3(256), 0, c->stream, op, nent, nm, mstride, x, y, z, k);
+// one part of a k_modes launch: entities, active modes, modes in memory, the arrays
+struct ModePart { long nent; int nm, mstride; double *x, *y; const double* z; };
+void launch_modes(hipStream_t stream, int nv, int op, std::initializer_list<ModePart> parts, double k) {
+    ModeSpan m{};
+    long end = 0;
+    int i = 0;
+    for (const ModePart& q : parts) {
+        end += q.nent * q.nm * nv;
+        m.end[i] = end; m.per[i] = std::max(1, q.nm * nv); m.stride[i] = q.mstride * nv;
+        m.x[i] = q.x; m.y[i] = q.y; m.z[i] = q.z;
+        ++i;
+    }
+    for (; i < 3; ++i) { m.end[i] = end; m.per[i] = 1; }
+    if (end > 0) hipLaunchKernelGGL(k_modes, dim3(nblk(end)), dim3(256), 0, stream, op, m, k);
 }
 
 // apply a k_modes op over the active v/s/i modes of the current level
 void modes_vsi(hpg_ctx* c, int op, double* xv, double* xs, double* xi, double* yv, double* ys, double* yi,
                const double* zv, const double* zs, const double* zi, double k) {
     const LevelDims d(1 << c->log2p);
-    launch_modes(c, op, c->npnt, 1, 1, xv, yv, zv, k);
-    if (d.sm > 0) launch_modes(c, op, c->nseg, d.sm, c->sm0, xs, ys, zs, k);
-    if (d.im > 0) launch_modes(c, op, c->ntri, d.im, c->im0, xi, yi, zi, k);
+    launch_modes(c->stream, c->nv, op, {{c->npnt, 1, 1, xv, yv, zv}, {c->nseg, d.sm, c->sm0, xs, ys, zs},
+                                        {c->ntri, d.im, c->im0, xi, yi, zi}}, k);
 }
 
 // blocks of 256 threads of `kernel` that the whole device holds at once (a multiple
@@ -1056,17 +1070,13 @@ void cns_boundary_and_projection(hpg_ctx* c, double cfa) {
         static const int cap = resident_blocks((const void*)k_pnv_int<4>);
         hipLaunchKernelGGL(k_pnv_int<4>, dim3(persistent_grid((c->ntri + 63) / 64, cap)), dim3(256), 0, c->stream, a);
     }
-    launch_modes(c, 4, c->npnt, 1, 1, c->ugv, c->ug0v, c->resv, cfa);
-    launch_modes(c, 4, c->nseg, d.sm, c->sm0, c->ugs, c->ug0s, c->ress, cfa);
+    launch_modes(c->stream, c->nv, 4, {{c->npnt, 1, 1, c->ugv, c->ug0v, c->resv},
+                                       {c->nseg, d.sm, c->sm0, c->ugs, c->ug0s, c->ress}}, cfa);
     check(hipGetLastError(), "cns projection launch");
 }
 
 void update_cns(hpg_ctx* c) {
-    const size_t nv = (size_t)c->npnt * c->nv * 8, ns = (size_t)c->nseg * c->sm0 * c->nv * 8,
-                 ni = (size_t)c->ntri * c->im0 * c->nv * 8;
-    dcopy(c, c->ug0v, c->ugv, nv);
-    if (ns) dcopy(c, c->ug0s, c->ugs, ns);
-    if (ni) dcopy(c, c->ug0i, c->ugi, ni);
+    save_state(c);
     for (int stage = 0; stage < c->prm.nstage; ++stage) {
         do_rsdl_cns(c, stage);
         do_minvrt(c);
@@ -1081,36 +1091,28 @@ void update_cns(hpg_ctx* c) {
 // and the stage update run as in update_cns; stage 0 is F(b) = R64(u0)/c and the later
 // stages evaluate the element residual in FP32; finally u = u0 + c (v - fl32(u0)).
 void mixed_update_cns(hpg_ctx* c) {
-    const long nv = (long)c->npnt * c->nv, ns = (long)c->nseg * c->sm0 * c->nv, ni = (long)c->ntri * c->im0 * c->nv;
+    const Span3 n = state_span(c);
+    const dim3 th(256), all = span_grid(n), red = span_grid_reduce(n);
+    const Ptr3<double> u{{c->ugv, c->ugs, c->ugi}}, res{{c->resv, c->ress, c->resi}}, u0{{c->u0cv, c->u0cs, c->u0ci}};
     do_rsdl_cns(c, c->prm.nstage);
-    auto copy = [&](double* dst, const double* src, long n) {
-        if (n) dcopy(c, dst, src, n * 8);
-    };
-    copy(c->srcv, c->resv, nv); copy(c->srcs, c->ress, ns); copy(c->srci, c->resi, ni);
-    copy(c->u0cv, c->ugv, nv); copy(c->u0cs, c->ugs, ns); copy(c->u0ci, c->ugi, ni);
-    hipLaunchKernelGGL(k_round32, dim3(std::min<unsigned>(nblk(nv), RED_BLOCKS)), dim3(256), 0, c->stream, nv, c->ugv, c->fd_max);
-    if (ns) hipLaunchKernelGGL(k_round32, dim3(std::min<unsigned>(nblk(ns), RED_BLOCKS)), dim3(256), 0, c->stream, ns, c->ugs, c->fd_max);
-    if (ni) hipLaunchKernelGGL(k_round32, dim3(std::min<unsigned>(nblk(ni), RED_BLOCKS)), dim3(256), 0, c->stream, ni, c->ugi, c->fd_max);
+    hipLaunchKernelGGL(k_fd_open64, red, th, 0, c->stream, n, Ptr3<const double>{{c->resv, c->ress, c->resi}},
+                       Ptr3<double>{{c->srcv, c->srcs, c->srci}}, u, u0, Ptr3<double>{{c->ug0v, c->ug0s, c->ug0i}}, c->fd_max);
     hipLaunchKernelGGL(k_fd_scale, dim3(1), dim3(1), 0, c->stream, c->fd_scal, c->fd_max, c->fd_reset ? 1 : 0, FD_H);
     c->fd_reset = false;
     for (int it = 0; it < c->ninner; ++it) {
-        copy(c->ug0v, c->ugv, nv); copy(c->ug0s, c->ugs, ns); copy(c->ug0i, c->ugi, ni);
+        if (it) save_state(c);
         for (int stage = 0; stage < c->prm.nstage; ++stage) {
-            if (it == 0 && stage == 0) {
+            if (it == 0 && stage == 0)
                 // res and res_r hold R64(u0) and its viscous part: the residual at v = b
-                hipLaunchKernelGGL(k_scale64, dim3(nblk(nv)), dim3(256), 0, c->stream, nv, c->resv, c->fd_scal);
-                if (ns) hipLaunchKernelGGL(k_scale64, dim3(nblk(ns)), dim3(256), 0, c->stream, ns, c->ress, c->fd_scal);
-                if (ni) hipLaunchKernelGGL(k_scale64, dim3(nblk(ni)), dim3(256), 0, c->stream, ni, c->resi, c->fd_scal);
-            } else {
+                hipLaunchKernelGGL(k_fd_first64, all, th, 0, c->stream, n, res, c->fd_scal);
+            else
                 do_rsdl_cns32(c, stage);
-            }
             do_minvrt(c);
             cns_boundary_and_projection(c, c->prm.alpha[stage] * c->prm.cfl[c->log2p]);
         }
     }
-    hipLaunchKernelGGL(k_fd_final64, dim3(std::min<unsigned>(nblk(nv), RED_BLOCKS)), dim3(256), 0, c->stream, nv, c->ugv, c->u0cv, c->fd_scal, c->fd_max + 1);
-    if (ns) hipLaunchKernelGGL(k_fd_final64, dim3(std::min<unsigned>(nblk(ns), RED_BLOCKS)), dim3(256), 0, c->stream, ns, c->ugs, c->u0cs, c->fd_scal, c->fd_max + 1);
-    if (ni) hipLaunchKernelGGL(k_fd_final64, dim3(std::min<unsigned>(nblk(ni), RED_BLOCKS)), dim3(256), 0, c->stream, ni, c->ugi, c->u0ci, c->fd_scal, c->fd_max + 1);
+    hipLaunchKernelGGL(k_fd_close64, red, th, 0, c->stream, n, u, Ptr3<const double>{{c->u0cv, c->u0cs, c->u0ci}},
+                       c->fd_scal, c->fd_max + 1);
     check(hipGetLastError(), "cns mixed update launch");
 }
 
@@ -1627,10 +1629,6 @@ int hpg_minvrt(hpg_ctx* c) {
 
 namespace {
 
-void launch_f32(hpg_ctx* c, long n, const double* x, float* y) {
-    if (n > 0) hipLaunchKernelGGL(k_to_f32, dim3(nblk(n)), dim3(256), 0, c->stream, n, x, y);
-}
-
 // One outer defect-correction iteration: the FP64 residual R64(u0) (the judge and the
 // defect), then `ninner` multistage iterations of the reference's scheme in FP32 on
 // F(v) = R32(v) + (1/c - 1) R64(u0) from v = b = fl32(u0) with the FP32 minvrt, then
@@ -1640,45 +1638,38 @@ void launch_f32(hpg_ctx* c, long n, const double* x, float* y) {
 // FP64 viscous part carried into the stage blend, so it costs no FP32 evaluation: an
 // update evaluates one FP64 and nstage - 1 FP32 residuals, as many as the FP64 scheme.
 void mixed_update(hpg_ctx* c) {
-    const long nv = (long)c->npnt * NV, nsz = (long)c->nseg * c->sm0 * NV, ni = (long)c->ntri * c->im0 * NV;
+    const Span3 n = state_span(c);
+    const dim3 th(256), all = span_grid(n), red = span_grid_reduce(n);
+    const Ptr3<float> v{{c->dlv, c->dls, c->dli}}, v0{{c->d0v, c->d0s, c->d0i}};
     do_rsdl(c, c->prm.nstage);
-    launch_f32(c, nv, c->vprcn, c->vp32);
-    launch_f32(c, (long)c->nseg * NV, c->sprcn, c->sp32);
-    launch_f32(c, (long)c->ntri * NV, c->tprcn, c->tp32);
-    if (c->typed_prcn) {
-        launch_f32(c, (long)c->ntri * NV, c->tprcn_sd, c->tp32s);
-        launch_f32(c, (long)c->ntri * NV, c->tprcn_in, c->tp32i);
-    }
-    hipLaunchKernelGGL(k_base32, dim3(std::min<unsigned>(nblk(nv), RED_BLOCKS)), dim3(256), 0, c->stream, nv, c->ugv, c->b32v, c->dlv, c->fd_max);
-    if (nsz) hipLaunchKernelGGL(k_base32, dim3(std::min<unsigned>(nblk(nsz), RED_BLOCKS)), dim3(256), 0, c->stream, nsz, c->ugs, c->b32s, c->dls, c->fd_max);
-    if (ni) hipLaunchKernelGGL(k_base32, dim3(std::min<unsigned>(nblk(ni), RED_BLOCKS)), dim3(256), 0, c->stream, ni, c->ugi, c->b32i, c->dli, c->fd_max);
+    auto to32 = [&](const Span3& m, Ptr3<const double> x, Ptr3<float> y) {
+        hipLaunchKernelGGL(k_span_to_f32, span_grid(m), th, 0, c->stream, m, x, y);
+    };
+    const long nt = (long)c->ntri * NV;
+    to32(span3((long)c->npnt * NV, (long)c->nseg * NV, nt), {{c->vprcn, c->sprcn, c->tprcn}}, {{c->vp32, c->sp32, c->tp32}});
+    if (c->typed_prcn) to32(span3(nt, nt), {{c->tprcn_sd, c->tprcn_in, nullptr}}, {{c->tp32s, c->tp32i, nullptr}});
+    hipLaunchKernelGGL(k_fd_open32, red, th, 0, c->stream, n, Ptr3<const double>{{c->ugv, c->ugs, c->ugi}},
+                       Ptr3<float>{{c->b32v, c->b32s, c->b32i}}, v, v0, c->fd_max);
     hipLaunchKernelGGL(k_fd_scale, dim3(1), dim3(1), 0, c->stream, c->fd_scal, c->fd_max, c->fd_reset ? 1 : 0, FD_H);
     c->fd_reset = false;
     for (int it = 0; it < c->ninner; ++it) {
-        dcopy(c, c->d0v, c->dlv, nv * 4);
-        if (nsz) dcopy(c, c->d0s, c->dls, nsz * 4);
-        if (ni) dcopy(c, c->d0i, c->dli, ni * 4);
+        if (it)
+            hipLaunchKernelGGL(k_span_copy<float>, all, th, 0, c->stream, n,
+                               Ptr3<const float>{{c->dlv, c->dls, c->dli}}, v0);
         for (int stage = 0; stage < c->prm.nstage; ++stage) {
-            if (it == 0 && stage == 0) {
-                hipLaunchKernelGGL(k_scale_f32, dim3(nblk(nv)), dim3(256), 0, c->stream, nv, c->resv, c->fd_scal, c->r32v);
-                if (nsz) hipLaunchKernelGGL(k_scale_f32, dim3(nblk(nsz)), dim3(256), 0, c->stream, nsz, c->ress, c->fd_scal, c->r32s);
-                if (ni) hipLaunchKernelGGL(k_scale_f32, dim3(nblk(ni)), dim3(256), 0, c->stream, ni, c->resi, c->fd_scal, c->r32i);
-                launch_f32(c, nv, c->rrv, c->rr32v);
-                launch_f32(c, nsz, c->rrs, c->rr32s);
-                launch_f32(c, ni, c->rri, c->rr32i);
-            } else {
+            if (it == 0 && stage == 0)
+                hipLaunchKernelGGL(k_fd_first32, all, th, 0, c->stream, n, Ptr3<const double>{{c->resv, c->ress, c->resi}},
+                                   Ptr3<const double>{{c->rrv, c->rrs, c->rri}}, c->fd_scal,
+                                   Ptr3<float>{{c->r32v, c->r32s, c->r32i}}, Ptr3<float>{{c->rr32v, c->rr32s, c->rr32i}});
+            else
                 do_rsdl32(c, stage);
-            }
             do_minvrt32(c, (float)(c->prm.alpha[stage] * c->prm.cfl[c->log2p]));
         }
     }
-    // |dhat| of this iteration (read by the next k_fd_scale), then the FP64 update
-    hipLaunchKernelGGL(k_diffmax32, dim3(std::min<unsigned>(nblk(nv), RED_BLOCKS)), dim3(256), 0, c->stream, nv, c->dlv, c->b32v, c->fd_max + 1);
-    if (nsz) hipLaunchKernelGGL(k_diffmax32, dim3(std::min<unsigned>(nblk(nsz), RED_BLOCKS)), dim3(256), 0, c->stream, nsz, c->dls, c->b32s, c->fd_max + 1);
-    if (ni) hipLaunchKernelGGL(k_diffmax32, dim3(std::min<unsigned>(nblk(ni), RED_BLOCKS)), dim3(256), 0, c->stream, ni, c->dli, c->b32i, c->fd_max + 1);
-    hipLaunchKernelGGL(k_add_scaled, dim3(nblk(nv)), dim3(256), 0, c->stream, nv, c->ugv, c->dlv, c->b32v, c->fd_scal);
-    if (nsz) hipLaunchKernelGGL(k_add_scaled, dim3(nblk(nsz)), dim3(256), 0, c->stream, nsz, c->ugs, c->dls, c->b32s, c->fd_scal);
-    if (ni) hipLaunchKernelGGL(k_add_scaled, dim3(nblk(ni)), dim3(256), 0, c->stream, ni, c->ugi, c->dli, c->b32i, c->fd_scal);
+    // |dhat| of this iteration (read by the next k_fd_scale) and the FP64 update
+    hipLaunchKernelGGL(k_fd_close32, red, th, 0, c->stream, n, Ptr3<double>{{c->ugv, c->ugs, c->ugi}},
+                       Ptr3<const float>{{c->dlv, c->dls, c->dli}}, Ptr3<const float>{{c->b32v, c->b32s, c->b32i}},
+                       c->fd_scal, c->fd_max + 1);
     check(hipGetLastError(), "mixed update launch");
 }
 
@@ -1702,9 +1693,10 @@ int hpg_residual_fp32(hpg_ctx* c, double* ov, double* os, double* oi) {
     HPG_TRY(c, {
         c->need_inner();
         const long nv = (long)c->npnt * NV, nsz = (long)c->nseg * c->sm0 * NV, ni = (long)c->ntri * c->im0 * NV;
-        hipLaunchKernelGGL(k_base32, dim3(std::min<unsigned>(nblk(nv), RED_BLOCKS)), dim3(256), 0, c->stream, nv, c->ugv, c->b32v, c->dlv, c->fd_max);
-        if (nsz) hipLaunchKernelGGL(k_base32, dim3(std::min<unsigned>(nblk(nsz), RED_BLOCKS)), dim3(256), 0, c->stream, nsz, c->ugs, c->b32s, c->dls, c->fd_max);
-        if (ni) hipLaunchKernelGGL(k_base32, dim3(std::min<unsigned>(nblk(ni), RED_BLOCKS)), dim3(256), 0, c->stream, ni, c->ugi, c->b32i, c->dli, c->fd_max);
+        const Span3 sp = state_span(c);
+        hipLaunchKernelGGL(k_fd_open32, span_grid_reduce(sp), dim3(256), 0, c->stream, sp,
+                           Ptr3<const double>{{c->ugv, c->ugs, c->ugi}}, Ptr3<float>{{c->b32v, c->b32s, c->b32i}},
+                           Ptr3<float>{{c->dlv, c->dls, c->dli}}, Ptr3<float>{{c->d0v, c->d0s, c->d0i}}, c->fd_max);
         // scale 1: the source factor 1/c - 1 is zero
         hipLaunchKernelGGL(k_fd_scale, dim3(1), dim3(1), 0, c->stream, c->fd_scal, c->fd_max, 1, 1.0);
         c->fd_reset = true;
@@ -1889,11 +1881,7 @@ void do_update(hpg_ctx* c) {
             vstage_p1(c, stage, c->prm.alpha[stage] * c->prm.cfl[c->log2p], stage == 0);
         return;
     }
-    const size_t nv = (size_t)c->npnt * NV * 8, ns = (size_t)c->nseg * c->sm0 * NV * 8,
-                 ni = (size_t)c->ntri * c->im0 * NV * 8;
-    dcopy(c, c->ug0v, c->ugv, nv);
-    if (ns) dcopy(c, c->ug0s, c->ugs, ns);
-    if (ni) dcopy(c, c->ug0i, c->ugi, ni);
+    save_state(c);
     for (int stage = 0; stage < c->prm.nstage; ++stage) {
         do_rsdl(c, stage);
         do_minvrt(c, c->prm.alpha[stage] * c->prm.cfl[c->log2p], stage + 1 == c->prm.nstage);

@@ -601,20 +601,31 @@ __global__ __launch_bounds__(256) void k_elem_ins(ElemArgs a) {
 // op 2: y = c*z - x, x += y     (mg_source first visit, nstage.cpp:113-128)
 // op 3: y = x                   (mg_restrict, movco.cpp:18-37)
 // op 4: x = y - c*z             (update, nstage.cpp:387-409)
-template <int NVn>
-__global__ void k_modes(int op, long nent, int nm, int mstride, double* __restrict__ x, double* __restrict__ y,
-                        const double* __restrict__ zz, double c) {
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long span = (long)nm * NVn;
-    if (k >= nent * span) return;
-    const long ent = k / span, r = k - ent * span;
-    const long ix = ent * (long)mstride * NVn + r;
+// Up to three arrays (vertex, side, interior modes) as one index range, one launch.
+struct ModeSpan {
+    long end[3];      // running counts of active values
+    int per[3];       // active values per entity: nm * NV
+    int stride[3];    // values per entity in memory: mstride * NV
+    double *x[3], *y[3];
+    const double* z[3];
+};
+__global__ __launch_bounds__(256) void k_modes(int op, ModeSpan m, double c) {
+    long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= m.end[2]) return;
+    const int i = k < m.end[0] ? 0 : (k < m.end[1] ? 1 : 2);
+    if (i) k -= i == 1 ? m.end[0] : m.end[1];
+    const int per = i == 0 ? m.per[0] : (i == 1 ? m.per[1] : m.per[2]);
+    const int stride = i == 0 ? m.stride[0] : (i == 1 ? m.stride[1] : m.stride[2]);
+    double* x = i == 0 ? m.x[0] : (i == 1 ? m.x[1] : m.x[2]);
+    double* y = i == 0 ? m.y[0] : (i == 1 ? m.y[1] : m.y[2]);
+    const double* z = i == 0 ? m.z[0] : (i == 1 ? m.z[1] : m.z[2]);
+    const long ent = k / per, ix = ent * stride + (k - ent * per);
     switch (op) {
         case 0: x[ix] = 0.0; y[ix] *= c; break;
         case 1: x[ix] += y[ix]; break;
-        case 2: { const double d = c * zz[ix] - x[ix]; y[ix] = d; x[ix] += d; } break;
+        case 2: { const double d = c * z[ix] - x[ix]; y[ix] = d; x[ix] += d; } break;
         case 3: y[ix] = x[ix]; break;
-        case 4: x[ix] = y[ix] - c * zz[ix]; break;
+        case 4: x[ix] = y[ix] - c * z[ix]; break;
     }
 }
 
@@ -1855,11 +1866,6 @@ template __global__ void k_elem_ins<2, false>(ElemArgs);
 template __global__ void k_elem_ins<4, true>(ElemArgs);
 template __global__ void k_elem_ins<4, false>(ElemArgs);
 
-
-// grid-stride copy of n 4-byte words (device-to-device copies inside the solver)
-__global__ void k_copy_words(long n, const unsigned* __restrict__ src, unsigned* __restrict__ dst) {
-    for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (long)gridDim.x * blockDim.x) dst[k] = src[k];
-}
 
 // grid-stride 16-byte copy (reference kernel for traffic counters)
 __global__ void k_copy16(const uint4* __restrict__ src, uint4* __restrict__ dst, long long n16) {
