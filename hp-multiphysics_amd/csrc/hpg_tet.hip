@@ -13,6 +13,8 @@ struct TetLevel {
     int p = 0;
     double* ops = nullptr;   // TDims<p>::SIZE
     double* opsm = nullptr;  // TMDims<p>::SIZE, the matrix-core kernel's operators (p = 2)
+    double* ops4 = nullptr;  // TM4::COUNT blocks, the 4x4x4 kernel's operators (p = 2)
+    TetLines lines{};        // and its line factors
     float* opsm32 = nullptr;  // the same for the FP32 matrix-core kernel (its K order)
     float* ops32 = nullptr;  // the same operators in FP32 (defect-correction inner solve)
     double* P2 = nullptr;    // face values GF x tm2d
@@ -82,6 +84,40 @@ std::vector<double> build_tet_mfma_pack(const TetOps& o, bool f32 = false) {
                 if (m < D::TM && h < D::G) pk[M::OFF_INT + (op * M::QK + k) * 64 + l] = (*integ[op])[m * D::G + h];
             }
     return pk;
+}
+
+// operators of the 4x4x4 kernels (TM4): block element [column k][row i] at 4 k + i.  Gauss
+// point (i, j, k) is register 3 i + j, row k; row 3 is padding.
+std::vector<double> build_tet4_pack(const TetOps& o) {
+    std::vector<double> pk(TM4::COUNT * 16, 0.0);
+    const int tm = o.tm, G = o.G;
+    auto at = [&](int blk, int row, int col) -> double& { return pk[16 * blk + 4 * col + row]; };
+    const std::vector<double>* V[3] = {&o.Vr, &o.Vs, &o.Vt};
+    for (int i = 0; i < 4; ++i)
+        for (int k = 0; k < 4; ++k) {
+            for (int r = 0; r < 9; ++r) {
+                for (int s = 0; s < 3; ++s)
+                    if (i < 3 && 4 * s + k < tm) at(TM4::P + 3 * r + s, i, k) = o.P[(3 * r + i) * tm + 4 * s + k];
+                if (k < 3) at(TM4::W + r, i, k) = -o.W[3 * r + k] * o.P[(3 * r + k) * tm + i];
+            }
+            for (int x = 0; x < 3; ++x) {
+                for (int s = 0; s < 3; ++s) {
+                    if (4 * s + k < tm) at(TM4::GV + 3 * x + s, i, k) = (*V[x])[i * tm + 4 * s + k];
+                    if (4 * s + i < tm) at(TM4::GX + 3 * x + s, i, k) = (*V[x])[k * tm + 4 * s + i];
+                }
+                at(TM4::DL + x, i, k) = (*V[x])[k];
+            }
+            for (int g = 0; g < G; ++g) at(TM4::MASS, i, k) -= o.W[g] * o.P[g * tm + i] * o.P[g * tm + k];
+            if (i < 3 && k < 3) at(TM4::LZ, i, k) = o.Lz[3 * i + k];
+        }
+    return pk;
+}
+TetLines tet_lines(const TetOps& o) {
+    TetLines l;
+    std::copy(o.Lx.begin(), o.Lx.end(), l.lx); std::copy(o.Ly.begin(), o.Ly.end(), l.ly);
+    std::copy(o.x0.begin(), o.x0.end(), l.x0); std::copy(o.y0.begin(), o.y0.end(), l.y0);
+    std::copy(o.y1.begin(), o.y1.end(), l.y1); std::copy(o.z0.begin(), o.z0.end(), l.z0);
+    return l;
 }
 
 // CSR of entity -> codes, built from (entity, code) pairs in ascending code order
@@ -212,16 +248,17 @@ void launch_elem_tet(hpg_tet_ctx* c, int stage, const int* elist = nullptr, int 
     if (c->timing) check(hipEventRecord(c->event(2 * r), c->stream), "hipEventRecord");
     if (P == 2) {
         // matrix-core form: groups of 16 elements, four groups per block
-        a.ops = c->lv[c->log2p].opsm;
+        a.ops = c->lv[c->log2p].ops4;
+        const TetLines& ln = c->lv[c->log2p].lines;
         const int ngrp = (count + 15) / 16;
         if (beta > 0.0) {
             static const int cap = resident_blocks((const void*)k_elem_tet_mfma<2, true>);
             hipLaunchKernelGGL((k_elem_tet_mfma<2, true>), dim3(persistent_grid((ngrp + 3) / 4, cap)), dim3(256), 0,
-                               c->stream, a, ngrp);
+                               c->stream, a, ln, ngrp);
         } else {
             static const int cap = resident_blocks((const void*)k_elem_tet_mfma<2, false>);
             hipLaunchKernelGGL((k_elem_tet_mfma<2, false>), dim3(persistent_grid((ngrp + 3) / 4, cap)), dim3(256), 0,
-                               c->stream, a, ngrp);
+                               c->stream, a, ln, ngrp);
         }
     } else if (beta > 0.0) {
         static const int cap = resident_blocks((const void*)k_elem_tet<P, true>);
@@ -343,6 +380,7 @@ void do_rsdl_tet(hpg_tet_ctx* c, int stage, bool fp32 = false) {
     const int tm = L.p == 1 ? 4 : 10, tm2 = L.p == 1 ? 3 : 6;
     TetGatherArgs g;
     const int nvv = c->nv;
+    g.re = beta > 0.0 ? 1 : 0;
     g.tm = tm; g.tm2 = tm2; g.lf = c->lf; g.flf = c->flf; g.omb = 1.0 - beta; g.fnv = c->cns() ? CNV : 1;
     g.nent = c->npnt; g.mbase = 0; g.fbase = 0; g.stride = nvv; g.ptr = c->vt_ptr; g.code = c->vt_code;
     g.fptr = c->vf_ptr; g.fcode = c->vf_code; g.res = c->resv; g.rr = c->rrv;
@@ -623,6 +661,9 @@ int hpg_tet_create(const hpg_tet_mesh* m, const hpg_params* prm, hpg_tet_ctx** o
             if (o.p == 2) {
                 const std::vector<double> pm = build_tet_mfma_pack<2>(o);
                 L.opsm = c->upload(pm.data(), pm.size());
+                const std::vector<double> p4 = build_tet4_pack(o);
+                L.ops4 = c->upload(p4.data(), p4.size());
+                L.lines = tet_lines(o);
                 const std::vector<double> pm32d = build_tet_mfma_pack<2>(o, true);
                 const std::vector<float> pm32(pm32d.begin(), pm32d.end());
                 L.opsm32 = c->upload(pm32.data(), pm32.size());
@@ -772,7 +813,7 @@ int hpg_tet_element_jacobian(hpg_tet_ctx* c, const int* tind, int nel, double ep
         check(hipMemcpyAsync((void*)a.jel, jel.data(), (size_t)nel * 4, hipMemcpyHostToDevice, c->stream), "H2D");
         check(hipMemcpyAsync((void*)a.jpos, jpos.data(), (size_t)nel * 4, hipMemcpyHostToDevice, c->stream), "H2D");
         a.tet_pnt = c->tet_pnt; a.tet_seg = c->tet_seg; a.em0 = c->em0; a.tm = tm; a.nv = nvv;
-        a.ugv = c->ugv; a.uge = c->uge; a.lf = c->lf;
+        a.ugv = c->ugv; a.uge = c->uge; a.lf = c->lf; a.re = c->prm.beta[0] > 0.0 ? 1 : 0;
         a.dw = (double*)get((size_t)nel * 8);
         a.save = (double*)get((size_t)nel * 8);
         a.base = (double*)get((size_t)nel * N * 8);

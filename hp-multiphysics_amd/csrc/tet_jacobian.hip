@@ -20,7 +20,8 @@ struct TetJacArgs {
     const int *tet_pnt, *tet_seg;
     int em0, tm, nv;   // edge-mode stride, modes and variables of the level
     double *ugv, *uge;
-    const double* lf;  // element records [t][m][0 = im, 1 = re][n]
+    const double* lf;  // element records [t][m][0 = im, 1 = re][n], [t][m][n] when re == 0
+    int re;
     double* dw;        // batch
     double* save;      // batch
     double* base;      // batch x tm x nv: Rbar
@@ -64,8 +65,8 @@ __global__ void k_tjac_collect(TetJacArgs a) {
     const int j = a.begin + (int)(g / N), r = (int)(g % N);
     const int i = r / a.nv, n = r - i * a.nv;
     const int t = a.jel[j], jp = a.jpos[j];
-    const double* rec = a.lf + ((size_t)t * a.tm + i) * (2 * a.nv);
-    const double R = rec[a.nv + n] + rec[n];
+    const double* rec = a.lf + ((size_t)t * a.tm + i) * (a.re ? 2 * a.nv : a.nv);
+    const double R = (a.re ? rec[a.nv + n] : 0.0) + rec[n];
     double* rb = a.base + (size_t)jp * N + r;
     if (a.mode < 0) {
         *rb = R;

@@ -51,7 +51,8 @@ struct TetElemArgsT {
     const double* ugv;
     const double* uge;
     const double* tau;  // ntet x 4 (0: momentum, 3: continuity)
-    double* lf;         // ntet x TM x 2 x 4: [t][m][0 = imaginary, 1 = real][n]
+    double* lf;         // element records [t][m][0 = imaginary, 1 = real][n]; without viscous terms
+                        // (FULL = false) [t][m][n], the imaginary part only
     const T* ops;
     double rho, mu, beta;
 };
@@ -222,14 +223,15 @@ __device__ __forceinline__ void elem_tet_body(const TetElemArgsT<T>& a, int noct
         for (int c = 0; c < 3; ++c) sf[hw][9 + c][g] = c3[c];
         wave_lds_sync();
         // lf_im = intgrtrst of the fluxes (rsdl.cpp:509-511); mode g / 3 lands in lane g
-        double* lfo = a.lf + (size_t)tt * (2 * TNV * TM);
+        constexpr int REC = FULL ? 2 * TNV : TNV;
+        double* lfo = a.lf + (size_t)tt * (REC * TM);
         const bool owner = valid && g < 3 * TM && g % 3 == 0;
         {
             T li[TNV];
             tet_intgrtrst<D, TNV, D::FROW, T>(sops, sf[hw], g, li);
             if (owner)
 #pragma unroll
-                for (int n = 0; n < TNV; ++n) lfo[(g / 3) * (2 * TNV) + n] = li[n];
+                for (int n = 0; n < TNV; ++n) lfo[(g / 3) * REC + n] = li[n];
         }
         if constexpr (FULL) {
             // viscous fluxes (rsdl.cpp:518-674): visc(n,m)(a,b) = -mu/cjcb (delta_nm
@@ -284,11 +286,7 @@ __device__ __forceinline__ void elem_tet_body(const TetElemArgsT<T>& a, int noct
             tet_intgrtrst<D, TNV, D::FROW, T>(sops, sf[hw], g, lr);
             if (owner)
 #pragma unroll
-                for (int n = 0; n < TNV; ++n) lfo[(g / 3) * (2 * TNV) + TNV + n] = lr[n] * T(a.beta);
-        } else {
-            if (owner)
-#pragma unroll
-                for (int n = 0; n < TNV; ++n) lfo[(g / 3) * (2 * TNV) + TNV + n] = T(0.0);
+                for (int n = 0; n < TNV; ++n) lfo[(g / 3) * REC + TNV + n] = lr[n] * T(a.beta);
         }
     }
 }
@@ -449,14 +447,14 @@ __device__ __forceinline__ void elem_tet_mfma_body(const TetElemArgsT<T>& a, int
                     }
                 }
             // register i holds mode 4 i + l / 16 (f64) or 4 (l / 16) + i (f32) of element e
-            double* lfo = a.lf + (size_t)tt * (2 * TNV * TM);
+            constexpr int REC = FULL ? 2 * TNV : TNV;
+            double* lfo = a.lf + (size_t)tt * (REC * TM);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int m = F64 ? 4 * i + q : 4 * q + i;
                 if (valid && m < TM) {
-                    double* o = lfo + m * (2 * TNV);
+                    double* o = lfo + m * REC;
                     o[0] = double(L0[i]); o[1] = double(L1[i]); o[2] = double(L2[i]); o[3] = double(L3[i]);
-                    if constexpr (!FULL) { o[4] = 0.0; o[5] = 0.0; o[6] = 0.0; o[7] = 0.0; }
                 }
             }
         }
@@ -576,9 +574,333 @@ __device__ __forceinline__ void elem_tet_mfma_body(const TetElemArgsT<T>& a, int
     }
 }
 
+// ---------------------------------------------------------------------------------
+// FP64 form at p = 2: 16 tetrahedra per wave64 on v_mfma_f64_4x4x4f64 (lane l: element
+// l % 16; operands' K index and results' row l / 16; 4 cycles a step against 16 for the
+// 16x16x4 form, the same rate per product), so that a contraction pays for its products in
+// tiles of 4 x 4 and not of 16 x 4.  FP64 vector and matrix instructions share one unit at
+// one rate, and the kernel is bound by it: what counts is the number of products.
+//  - Points: accumulator register 3 i + j of lane row k is the Gauss point (i, j, k) (row 3 is
+//    padding), so the x and y lines of the collapsed grid lie in a lane's registers: the
+//    derivatives along them are 3-term sums on the vector unit, and only z is a contraction.
+//    Dense 27 x 27 operators would be 42 products per point and direction pair against 15.
+//  - Tests: the p = 2 modes have linear gradients, so intgrtrst is four moments per
+//    direction, M[v] = -sum_g w_g lambda_v(g) F(g), and grad phi_m at the four vertices.
+//  - Viscous fluxes are linear on the (straight) element: they are formed at its four
+//    vertices; their moments are one 4 x 4 mass product, their divergence a constant.
+// Operands (TM4 offsets) are 4 x 4 blocks in LDS, lane l reads row l % 4, column l / 16.
+// 384 000 tetrahedra: full 519 -> 234 us, inviscid 149 -> 95 us against the 16x16x4 form with
+// dense operators (one wave per SIMD, 512 registers; this one fits two waves).  The inviscid
+// stages write and gather records of the imaginary part only, half the bytes.
+struct TM4 {
+    static constexpr int P = 0;        // 27: values at register r of K-step s, [3 r + s]
+    static constexpr int GV = 27;      // 9: gradients at the vertices, [3 x + s]
+    static constexpr int GX = 36;      // 9: d phi_m / dx at the vertices, [3 x + row block]
+    static constexpr int W = 45;       // 9: -w_g lambda_v(g), register r
+    static constexpr int MASS = 54;    // -sum_g w_g lambda_v lambda_v'
+    static constexpr int DL = 55;      // 3: gradients of the barycentrics, every row
+    static constexpr int LZ = 58;      // z derivative
+    static constexpr int COUNT = 59;
+};
+// line factors of the collapsed grid (kernel argument: scalar registers)
+struct TetLines {
+    double lx[9], ly[9], x0[3], y0[3], y1[3], z0[3];
+};
+__device__ __forceinline__ double mfma4(double a, double b, double c) {
+    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+// keeps the compiler from moving operand loads (all loop invariants) and flux sums across the
+// phases of an element group: hoisted, they spill
+__device__ __forceinline__ void tet_phase() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+// the same for values: what is computed from d after this is computed anew (81 fluxes kept
+// from the pass before would not fit the registers)
+__device__ __forceinline__ void tet_opaque(double d[3][3]) {
+    tet_phase();
+#pragma unroll
+    for (int k = 0; k < 9; ++k) asm volatile("" : "+v"(d[k / 3][k % 3]));
+}
+// x, y and z derivative sums of one variable, one direction of its fluxes at a time (f:
+// the nine registers of a lane): acc = y0 (Lx f_r + x0 Lx (f_s + f_t)), then
+// acc = z0 (acc + Ly f_s + y1 Ly f_t), then acc += Lz f_t
+__device__ __forceinline__ void tet_line_r(const TetLines& ln, const double f[9], double acc[9]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            acc[3 * i + j] = ln.lx[3 * i] * f[j] + ln.lx[3 * i + 1] * f[3 + j] + ln.lx[3 * i + 2] * f[6 + j];
+}
+__device__ __forceinline__ void tet_line_st(const TetLines& ln, const double f[9], double acc[9]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const double d = ln.lx[3 * i] * f[j] + ln.lx[3 * i + 1] * f[3 + j] + ln.lx[3 * i + 2] * f[6 + j];
+            acc[3 * i + j] = ln.y0[j] * (acc[3 * i + j] + ln.x0[i] * d);
+        }
+}
+__device__ __forceinline__ void tet_line_s(const TetLines& ln, const double f[9], double acc[9]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            acc[3 * i + j] += ln.ly[3 * j] * f[3 * i] + ln.ly[3 * j + 1] * f[3 * i + 1] + ln.ly[3 * j + 2] * f[3 * i + 2];
+}
+__device__ __forceinline__ void tet_line_t(const TetLines& ln, double z0, double lz, const double f[9], double acc[9]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const double d = ln.ly[3 * j] * f[3 * i] + ln.ly[3 * j + 1] * f[3 * i + 1] + ln.ly[3 * j + 2] * f[3 * i + 2];
+            acc[3 * i + j] = mfma4(lz, f[3 * i + j], z0 * (acc[3 * i + j] + ln.y1[j] * d));
+        }
+}
+
+// geometry of a straight element: cofactors d (rsdl.cpp:58-62, 449-458) and the Jacobian;
+// padding elements take the reference tetrahedron
+__device__ __forceinline__ double tet_cofactors(const double* __restrict__ pnts, const int* __restrict__ tet_pnt, int tt,
+                                                bool valid, double d[3][3]) {
+    double X[4][3];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int v = tet_pnt[4 * tt + k];
+#pragma unroll
+        for (int n = 0; n < 3; ++n)
+            X[k][n] = valid ? pnts[3 * v + n] : ((k == 0 && n == 2) || (k == 1 && n == 1) || (k == 3 && n == 0) ? 1.0 : -1.0);
+    }
+    double ld[3][3];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+        ld[n][0] = 0.5 * (X[3][n] - X[2][n]);
+        ld[n][1] = 0.5 * (X[1][n] - X[2][n]);
+        ld[n][2] = 0.5 * (X[0][n] - X[2][n]);
+    }
+    d[0][0] = ld[1][1] * ld[2][2] - ld[1][2] * ld[2][1];
+    d[0][1] = -ld[0][1] * ld[2][2] + ld[0][2] * ld[2][1];
+    d[0][2] = ld[0][1] * ld[1][2] - ld[0][2] * ld[1][1];
+    d[1][0] = -ld[1][0] * ld[2][2] + ld[1][2] * ld[2][0];
+    d[1][1] = ld[0][0] * ld[2][2] - ld[0][2] * ld[2][0];
+    d[1][2] = -ld[0][0] * ld[1][2] + ld[0][2] * ld[1][0];
+    d[2][0] = ld[1][0] * ld[2][1] - ld[1][1] * ld[2][0];
+    d[2][1] = -ld[0][0] * ld[2][1] + ld[0][1] * ld[2][0];
+    d[2][2] = ld[0][0] * ld[1][1] - ld[0][1] * ld[1][0];
+    return ld[0][0] * (ld[1][1] * ld[2][2] - ld[1][2] * ld[2][1]) - ld[0][1] * (ld[1][0] * ld[2][2] - ld[2][0] * ld[1][2]) +
+           ld[0][2] * (ld[1][0] * ld[2][1] - ld[2][0] * ld[1][1]);
+}
+
+// tet_hp_ins::element_rsdl as in elem_tet_mfma_body
+template <bool FULL>
+__device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetLines& ln, int ngrp) {
+    constexpr int TM = TDims<2>::TM, REC = FULL ? 2 * TNV : TNV;
+    __shared__ double sops[TM4::COUNT * 16];
+    __shared__ double sv[FULL ? 12 : 1][256];  // each lane's own viscous results
+    for (int k = threadIdx.x; k < TM4::COUNT * 16; k += blockDim.x) sops[k] = a.ops[k];
+    __syncthreads();
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int e = lane & 15, q = lane >> 4;
+    const double* op = sops + (lane & 3) + 4 * q;  // this lane's element of block b: op[16 b]
+    const int WX = ((int)gridDim.x >> 3) * 4;
+    const int rank = ((int)blockIdx.x >> 3) * 4 + w;
+    const int xcd = (int)blockIdx.x & 7;
+    const int gpx = (ngrp + 7) >> 3;
+    const int gend = min(ngrp, (xcd + 1) * gpx);
+    for (int grp = xcd * gpx + rank; grp < gend; grp += WX) {
+        tet_phase();
+        const int slot = grp * 16 + e;
+        const bool valid = slot < a.ntet;
+        const int tt = valid ? (a.elist ? a.elist[slot] : slot) : 0;
+        // modal coefficients: K-step s of lane l is mode 4 s + l / 16; padding elements zero
+        double b[TNV][3];
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            const int k = 4 * s + q;
+            const double* src = nullptr;
+            if (valid && k < TM)
+                src = k < 4 ? a.ugv + (size_t)a.tet_pnt[4 * tt + k] * TNV
+                            : a.uge + (size_t)a.tet_seg[6 * tt + (k - 4)] * a.em0 * TNV;
+#pragma unroll
+            for (int n = 0; n < TNV; ++n) b[n][s] = src ? src[n] : 0.0;
+        }
+        double d[3][3];
+        const double cjcb = tet_cofactors(a.pnts, a.tet_pnt, tt, valid, d);
+        const double rho = a.rho;
+        tet_phase();
+        // values at the Gauss points
+        double U[TNV][9];
+#pragma unroll
+        for (int r = 0; r < 9; ++r) {
+#pragma unroll
+            for (int n = 0; n < TNV; ++n) U[n][r] = 0.0;
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+                const double av = op[16 * (TM4::P + 3 * r + s)];
+#pragma unroll
+                for (int n = 0; n < TNV; ++n) U[n][r] = mfma4(av, b[n][s], U[n][r]);
+            }
+        }
+        tet_phase();
+        if constexpr (FULL) {
+            // velocity gradients at vertex q, then (rsdl.cpp:518-674) the fluxes
+            // -mu/cjcb (sum_b dd(x,b) du(n,b) + sum_m d(x)(m) sum_b d(b)(n) du(m,b))
+            double du[3][3], df[3][3], gm[3][3];
+#pragma unroll
+            for (int x = 0; x < 3; ++x) {
+#pragma unroll
+                for (int n = 0; n < 3; ++n) du[n][x] = 0.0;
+#pragma unroll
+                for (int s = 0; s < 3; ++s) {
+                    const double av = op[16 * (TM4::GV + 3 * x + s)];
+#pragma unroll
+                    for (int n = 0; n < 3; ++n) du[n][x] = mfma4(av, b[n][s], du[n][x]);
+                }
+            }
+            const double nuj = -a.mu / cjcb;
+#pragma unroll
+            for (int m = 0; m < 3; ++m)
+#pragma unroll
+                for (int n = 0; n < 3; ++n) gm[m][n] = d[0][n] * du[m][0] + d[1][n] * du[m][1] + d[2][n] * du[m][2];
+#pragma unroll
+            for (int n = 0; n < 3; ++n)
+#pragma unroll
+                for (int x = 0; x < 3; ++x)
+                    df[n][x] = nuj * (d[x][0] * (gm[n][0] + gm[0][n]) + d[x][1] * (gm[n][1] + gm[1][n]) +
+                                      d[x][2] * (gm[n][2] + gm[2][n]));
+            const double am = op[16 * TM4::MASS];
+#pragma unroll
+            for (int n = 0; n < 3; ++n)
+#pragma unroll
+                for (int x = 0; x < 3; ++x) sv[3 * x + n][threadIdx.x] = mfma4(am, df[n][x], 0.0);  // moments
+            double dv[3] = {0.0, 0.0, 0.0};  // flux divergence
+#pragma unroll
+            for (int x = 0; x < 3; ++x) {
+                const double al = op[16 * (TM4::DL + x)];
+#pragma unroll
+                for (int n = 0; n < 3; ++n) dv[n] = mfma4(al, df[n][x], dv[n]);
+            }
+#pragma unroll
+            for (int n = 0; n < 3; ++n) sv[9 + n][threadIdx.x] = dv[n];
+        }
+        // L[n][rb] (mode 4 rb + q) += sum_v d phi_m/dx(v) M[n]
+        auto expand = [&](int x, const double M[TNV], double L[TNV][3]) {
+#pragma unroll
+            for (int rb = 0; rb < 3; ++rb) {
+                const double ag = op[16 * (TM4::GX + 3 * x + rb)];
+#pragma unroll
+                for (int n = 0; n < TNV; ++n) L[n][rb] = mfma4(ag, M[n], L[n][rb]);
+            }
+        };
+        double* lfo = a.lf + (size_t)tt * (REC * TM);
+        auto store = [&](const double L[TNV][3], int off, double f) {
+#pragma unroll
+            for (int rb = 0; rb < 3; ++rb) {
+                const int m = 4 * rb + q;
+                if (valid && m < TM) {
+                    double* o = lfo + m * REC + off;
+#pragma unroll
+                    for (int n = 0; n < TNV; ++n) o[n] = f * L[n][rb];
+                }
+            }
+        };
+        tet_phase();
+        // lf_im = intgrtrst of the convective and pressure fluxes (rsdl.cpp:461-511)
+        {
+            double L[TNV][3];
+#pragma unroll
+            for (int n = 0; n < TNV; ++n)
+#pragma unroll
+                for (int rb = 0; rb < 3; ++rb) L[n][rb] = 0.0;
+#pragma unroll
+            for (int x = 0; x < 3; ++x) {
+                tet_phase();
+                double M[TNV] = {0.0, 0.0, 0.0, 0.0};
+                const double rx = rho * d[x][0], ry = rho * d[x][1], rz = rho * d[x][2];
+#pragma unroll
+                for (int r = 0; r < 9; ++r) {
+                    const double aw = op[16 * (TM4::W + r)];
+                    const double c = rx * U[0][r] + ry * U[1][r] + rz * U[2][r];
+#pragma unroll
+                    for (int n = 0; n < 3; ++n) M[n] = mfma4(aw, U[n][r] * c + d[x][n] * U[3][r], M[n]);
+                    M[3] = mfma4(aw, c, M[3]);
+                }
+                expand(x, M, L);
+            }
+            store(L, 0, 1.0);
+        }
+        if constexpr (FULL) {
+            tet_opaque(d);
+            // strong residual: derivr/derivs/derivt of the total fluxes (rsdl.cpp:683-692)
+            double R[TNV][9];
+            const double z0 = ln.z0[q < 3 ? q : 2], lz = op[16 * TM4::LZ];
+            // fluxes of variable n in the (combined) direction with cofactors g and mass flux c
+            auto flux = [&](int n, const double g[3], const double c[9], double f[9]) {
+#pragma unroll
+                for (int r = 0; r < 9; ++r) f[r] = n < 3 ? U[n][r] * c[r] + g[n] * U[3][r] : c[r];
+            };
+            auto mass = [&](const double g[3], double c[9]) {
+                const double gx = rho * g[0], gy = rho * g[1], gz = rho * g[2];
+#pragma unroll
+                for (int r = 0; r < 9; ++r) c[r] = gx * U[0][r] + gy * U[1][r] + gz * U[2][r];
+            };
+            double c[9], f[9];
+            mass(d[0], c);
+#pragma unroll
+            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, d[0], c, f); tet_line_r(ln, f, R[n]); }
+            const double g[3] = {d[1][0] + d[2][0], d[1][1] + d[2][1], d[1][2] + d[2][2]};
+            mass(g, c);
+#pragma unroll
+            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, g, c, f); tet_line_st(ln, f, R[n]); }
+            mass(d[1], c);
+#pragma unroll
+            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, d[1], c, f); tet_line_s(ln, f, R[n]); }
+            mass(d[2], c);
+#pragma unroll
+            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, d[2], c, f); tet_line_t(ln, z0, lz, f, R[n]); }
+            // stabilisation (rsdl.cpp:695-767) into lf_re, with t = tau (residual):
+            // -((d.u) t_n + u_n (d.t) + d_n t_3) for n < 3 and -(d.t)
+            const double tm = -a.tau[4 * tt], tc = -a.tau[4 * tt + 3];
+            const double dv[3] = {sv[9][threadIdx.x], sv[10][threadIdx.x], sv[11][threadIdx.x]};
+            double M[3][TNV];
+#pragma unroll
+            for (int x = 0; x < 3; ++x) {
+#pragma unroll
+                for (int n = 0; n < 3; ++n) M[x][n] = sv[3 * x + n][threadIdx.x];
+                M[x][3] = 0.0;
+            }
+#pragma unroll
+            for (int r = 0; r < 9; ++r) {
+                tet_phase();
+                const double aw = op[16 * (TM4::W + r)];
+                const double t0 = tm * (R[0][r] + dv[0]), t1 = tm * (R[1][r] + dv[1]), t2 = tm * (R[2][r] + dv[2]),
+                             t3 = tc * R[3][r];
+#pragma unroll
+                for (int x = 0; x < 3; ++x) {
+                    const double su = d[x][0] * U[0][r] + d[x][1] * U[1][r] + d[x][2] * U[2][r];
+                    const double st = d[x][0] * t0 + d[x][1] * t1 + d[x][2] * t2;
+                    M[x][0] = mfma4(aw, su * t0 + U[0][r] * st + d[x][0] * t3, M[x][0]);
+                    M[x][1] = mfma4(aw, su * t1 + U[1][r] * st + d[x][1] * t3, M[x][1]);
+                    M[x][2] = mfma4(aw, su * t2 + U[2][r] * st + d[x][2] * t3, M[x][2]);
+                    M[x][3] = mfma4(aw, st, M[x][3]);
+                }
+            }
+            tet_phase();
+            double L[TNV][3];
+#pragma unroll
+            for (int n = 0; n < TNV; ++n)
+#pragma unroll
+                for (int rb = 0; rb < 3; ++rb) L[n][rb] = 0.0;
+#pragma unroll
+            for (int x = 0; x < 3; ++x) expand(x, M[x], L);
+            store(L, TNV, a.beta);
+        }
+    }
+}
+
 template <int P, bool FULL>
-__global__ __launch_bounds__(256) void k_elem_tet_mfma(TetElemArgs a, int ngrp) {
-    elem_tet_mfma_body<double, P, FULL>(a, ngrp);
+__global__ __launch_bounds__(256, FULL ? 2 : 3) void k_elem_tet_mfma(TetElemArgs a, TetLines ln, int ngrp) {
+    static_assert(P == 2, "");
+    elem_tet_body64<FULL>(a, ln, ngrp);
 }
 
 // FP32 arithmetic (the inner solve of the defect correction) on v_mfma_f32_16x16x4f32
@@ -642,6 +964,7 @@ __global__ __launch_bounds__(256) void k_face_tet(int nbf, const int* __restrict
 // (tet_hp/update.cpp:13-31, 45-70, bdry.cpp:16-57); elements and faces ascending
 struct TetGatherArgs {
     int nent, tm, tm2, mbase, fbase, stride;
+    int re;           // 1: records [im/re][n]; 0: [n] only (lf_re = 0)
     int fnv;          // face variables: 1 (continuity into the last variable) or NV, flf[f][fnv][tm2]
     const int* ptr;   // CSR entity -> (element, local index) codes 16*t + i
     const int* code;
@@ -676,13 +999,14 @@ __global__ __launch_bounds__(256) void k_gather_tet(TetGatherArgs a) {
     for (int n = 0; n < NV; ++n) sr[n] = a.omb * RR[n];
     for (int k = a.ptr[v]; k < a.ptr[v + 1]; ++k) {
         const int c = a.code[k], t = c >> 4, i = c & 15;
-        // one contiguous record of 2 NV doubles per (element, mode)
-        const double* L = a.lf + (size_t)t * (2 * NV * a.tm) + (size_t)(a.mbase + i) * (2 * NV);
+        // one contiguous record per (element, mode)
+        const int rec = a.re ? 2 * NV : NV;
+        const double* L = a.lf + ((size_t)t * a.tm + a.mbase + i) * rec;
 #pragma unroll
-        for (int n = 0; n < NV; ++n) {
-            si[n] += L[n];
-            sr[n] += L[NV + n];
-        }
+        for (int n = 0; n < NV; ++n) si[n] += L[n];
+        if (a.re)
+#pragma unroll
+            for (int n = 0; n < NV; ++n) sr[n] += L[NV + n];
     }
 #pragma unroll
     for (int n = 0; n < NV; ++n) {

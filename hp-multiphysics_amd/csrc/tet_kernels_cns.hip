@@ -523,14 +523,15 @@ __device__ __forceinline__ void elem_tetc_body(const TetcElemArgsT<T>& a, int no
             for (int c = 0; c < 3; ++c) sf[hw][3 * n + c][g] = g < G ? cv[n][c] : T(0.0);
         wave_lds_sync();
         // lf_im = intgrtrst of the fluxes (rsdl.cpp:542-543); mode g / 3 lands in lane g
-        double* lfo = a.lf + (size_t)tt * (2 * CNV * TM);
+        constexpr int REC = FULL ? 2 * CNV : CNV;
+        double* lfo = a.lf + (size_t)tt * (REC * TM);
         const bool owner = valid && g < 3 * TM && g % 3 == 0;
         {
             T li[CNV];
             tet_intgrtrst<D, CNV, D::FROW, T>(sops, sf[hw], g, li);
             if (owner)
 #pragma unroll
-                for (int n = 0; n < CNV; ++n) lfo[(g / 3) * (2 * CNV) + n] = li[n];
+                for (int n = 0; n < CNV; ++n) lfo[(g / 3) * REC + n] = li[n];
         }
         if constexpr (FULL) {
             // viscous stress and heat flux (rsdl.cpp:584-755): visc(n,m)(a,b) applied to
@@ -599,11 +600,7 @@ __device__ __forceinline__ void elem_tetc_body(const TetcElemArgsT<T>& a, int no
             tet_intgrtrst<D, CNV, D::FROW, T>(sops, sf[hw], g, lr);
             if (owner)
 #pragma unroll
-                for (int n = 0; n < CNV; ++n) lfo[(g / 3) * (2 * CNV) + CNV + n] = lr[n] * T(a.beta);
-        } else {
-            if (owner)
-#pragma unroll
-                for (int n = 0; n < CNV; ++n) lfo[(g / 3) * (2 * CNV) + CNV + n] = T(0.0);
+                for (int n = 0; n < CNV; ++n) lfo[(g / 3) * REC + CNV + n] = lr[n] * T(a.beta);
         }
     }
 }
@@ -756,17 +753,15 @@ __device__ __forceinline__ void elem_tetc_mfma_body(const TetcElemArgsT<T>& a, i
                     }
                 }
             }
-            double* lfo = a.lf + (size_t)tt * (2 * CNV * TM);
+            constexpr int REC = FULL ? 2 * CNV : CNV;
+            double* lfo = a.lf + (size_t)tt * (REC * TM);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int m = F64 ? 4 * i + q : 4 * q + i;
                 if (valid && m < TM) {
-                    double* o = lfo + m * (2 * CNV);
+                    double* o = lfo + m * REC;
 #pragma unroll
                     for (int n = 0; n < CNV; ++n) o[n] = double(L[n][i]);
-                    if constexpr (!FULL)
-#pragma unroll
-                        for (int n = 0; n < CNV; ++n) o[CNV + n] = 0.0;
                 }
             }
         }

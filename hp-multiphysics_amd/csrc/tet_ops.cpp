@@ -69,7 +69,7 @@ TetOps::TetOps(int p_) : p(p_) {
     for (auto& w : wz) w *= 0.25;
     P.assign(G * tm, 0.0); Pr = Ps = Pt = P;
     Ir.assign(tm * G, 0.0); Is = It = Ir;
-    std::vector<double> W(G);
+    W.assign(G, 0.0);
     double val[10], grad[10][3], l[4];
     for (int i = 0; i < gp; ++i)
         for (int j = 0; j < gp; ++j)
@@ -92,21 +92,30 @@ TetOps::TetOps(int p_) : p(p_) {
     // Gauss-grid derivatives: d/dr = y0 z0 d/dx, d/ds = x0 y0 z0 d/dx + z0 d/dy,
     // d/dt = x0 y0 z0 d/dx + y1 z0 d/dy + d/dz (x0 = (1+x)/2, y0 = 2/(1-y),
     // y1 = (1+y)/2, z0 = 2/(1-z))
-    const std::vector<double> Lx = lagrange_derivative(x), Ly = lagrange_derivative(y), Lz = lagrange_derivative(z);
+    Lx = lagrange_derivative(x); Ly = lagrange_derivative(y); Lz = lagrange_derivative(z);
+    for (int i = 0; i < gp; ++i) {
+        x0.push_back(0.5 * (1 + x[i])); y0.push_back(2.0 / (1 - y[i]));
+        y1.push_back(0.5 * (1 + y[i])); z0.push_back(2.0 / (1 - z[i]));
+    }
+    Vr.assign(4 * tm, 0.0); Vs = Vt = Vr;
+    for (int v = 0; v < 4; ++v) {
+        for (int k = 0; k < 4; ++k) l[k] = k == v ? 1.0 : 0.0;
+        modes(tm, l, val, grad);
+        for (int m = 0; m < tm; ++m) { Vr[v * tm + m] = grad[m][0]; Vs[v * tm + m] = grad[m][1]; Vt[v * tm + m] = grad[m][2]; }
+    }
     Dr.assign(G * G, 0.0); Ds = Dt = Dr;
     for (int i = 0; i < gp; ++i)
         for (int j = 0; j < gp; ++j)
             for (int k = 0; k < gp; ++k) {
                 const int g = (i * gp + j) * gp + k;
-                const double x0 = 0.5 * (1 + x[i]), y0 = 2.0 / (1 - y[j]), y1 = 0.5 * (1 + y[j]), z0 = 2.0 / (1 - z[k]);
                 for (int n = 0; n < gp; ++n) {
                     const int gx = (n * gp + j) * gp + k, gy = (i * gp + n) * gp + k, gz = (i * gp + j) * gp + n;
                     const double dx = Lx[i * gp + n], dy = Ly[j * gp + n], dz = Lz[k * gp + n];
-                    Dr[g * G + gx] += y0 * z0 * dx;
-                    Ds[g * G + gx] += x0 * y0 * z0 * dx;
-                    Ds[g * G + gy] += z0 * dy;
-                    Dt[g * G + gx] += x0 * y0 * z0 * dx;
-                    Dt[g * G + gy] += y1 * z0 * dy;
+                    Dr[g * G + gx] += y0[j] * z0[k] * dx;
+                    Ds[g * G + gx] += x0[i] * y0[j] * z0[k] * dx;
+                    Ds[g * G + gy] += z0[k] * dy;
+                    Dt[g * G + gx] += x0[i] * y0[j] * z0[k] * dx;
+                    Dt[g * G + gy] += y1[j] * z0[k] * dy;
                     Dt[g * G + gz] += dz;
                 }
             }

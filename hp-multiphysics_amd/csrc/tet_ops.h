@@ -12,7 +12,9 @@
 //   P [g][m], Pr/Ps/Pt [g][m]   values and r, s, t derivatives          (proj)
 //   Ir/Is/It [m][g] = -w_g dphi_m/d(r,s,t)                               (intgrtrst)
 //   Dr/Ds/Dt [g][g']  derivatives of the collapsed-coordinate Lagrange interpolant
-//                     (derivr/derivs/derivt)
+//                     (derivr/derivs/derivt); their factors are the 1-D derivatives
+//                     Lx/Ly/Lz [gp][gp] and the line factors x0, y0, y1, z0 [gp]
+//   Vr/Vs/Vt [v][m]   derivatives of the modes at the four vertices
 // Face 0 (tet_basis/proj2d.cpp, intgrt2d.cpp): modes V1, V2, V3, E(V2,V3), E(V1,V3),
 // E(V1,V2) on the (x, y) face grid, P2 [gf][m] and W2 [gf].
 // Lumped-mass factors as tet_basis/initialize.cpp:521-800 and the p = 2 edge
@@ -27,6 +29,10 @@ struct TetOps {
     std::vector<double> P, Pr, Ps, Pt;   // G x tm
     std::vector<double> Ir, Is, It;      // tm x G
     std::vector<double> Dr, Ds, Dt;      // G x G
+    std::vector<double> W;               // G weights
+    std::vector<double> Lx, Ly, Lz;      // gp x gp
+    std::vector<double> x0, y0, y1, z0;  // gp
+    std::vector<double> Vr, Vs, Vt;      // 4 x tm
     std::vector<double> P2, W2;          // GF x tm2d, GF
     std::vector<double> mass;            // tm x tm
     double vdiag;
