@@ -12,10 +12,9 @@ namespace {
 struct TetLevel {
     int p = 0;
     double* ops = nullptr;   // TDims<p>::SIZE
-    double* opsm = nullptr;  // TMDims<p>::SIZE, the matrix-core kernel's operators (p = 2)
-    double* ops4 = nullptr;  // TM4::COUNT blocks, the 4x4x4 kernel's operators (p = 2)
-    TetLines lines{};        // and its line factors
-    float* opsm32 = nullptr;  // the same for the FP32 matrix-core kernel (its K order)
+    double* ops4 = nullptr;  // TM4::COUNT blocks, the FP64 matrix-core kernels' operators (p = 2)
+    TetLines lines{};        // and their line factors
+    float* opsm32 = nullptr;  // TMDims<p>::SIZE, the FP32 matrix-core kernels' operators (p = 2)
     float* ops32 = nullptr;  // the same operators in FP32 (defect-correction inner solve)
     double* P2 = nullptr;    // face values GF x tm2d
     double* W2 = nullptr;    // face weights GF
@@ -44,20 +43,16 @@ std::vector<double> build_tet_pack(const TetOps& o) {
     return pk;
 }
 
-// operators of k_elem_tet_mfma as lane-ready A blocks: block (tile t, K-step k) lane l
+// operators of k_elem_tet32_mfma as lane-ready A blocks: block (tile t, K-step k) lane l
 // holds A[16 t + l % 16][K index of lane l].  The projections' K index is the mode
 // 4 k + l / 16; the derivatives' and integrations' K index is the Gauss point that
-// accumulator register k % 4 of tile k / 4 holds in lane l: 16 (k / 4) + 4 (k % 4) +
-// l / 16 for the f64 matrix cores, 16 (k / 4) + 4 (l / 16) + k % 4 for the f32 ones
-// (f32 = true).  Rows and K indices beyond the G points and TM modes are zero.
+// accumulator register k % 4 of tile k / 4 holds in lane l.  Rows and K indices beyond the G points and TM modes are zero.
 template <int P>
-std::vector<double> build_tet_mfma_pack(const TetOps& o, bool f32 = false) {
+std::vector<double> build_tet_mfma_pack(const TetOps& o) {
     using D = TDims<P>;
     using M = TMDims<P>;
     std::vector<double> pk(M::SIZE, 0.0);
-    auto kpoint = [f32](int k, int l) {
-        return f32 ? 16 * (k / 4) + 4 * (l / 16) + k % 4 : 16 * (k / 4) + 4 * (k % 4) + l / 16;
-    };
+    auto kpoint = [](int k, int l) { return 16 * (k / 4) + 4 * (l / 16) + k % 4; };
     const std::vector<double>* proj[4] = {&o.P, &o.Pr, &o.Ps, &o.Pt};
     for (int op = 0; op < 4; ++op)
         for (int t = 0; t < M::GT; ++t)
@@ -87,7 +82,8 @@ std::vector<double> build_tet_mfma_pack(const TetOps& o, bool f32 = false) {
 }
 
 // operators of the 4x4x4 kernels (TM4): block element [column k][row i] at 4 k + i.  Gauss
-// point (i, j, k) is register 3 i + j, row k; row 3 is padding.
+// point (i, j, k) is register 3 i + j, row k; row 3 is padding: it repeats row 2 (the state
+// there stays one the fluxes can be formed from) with zero weights.
 std::vector<double> build_tet4_pack(const TetOps& o) {
     std::vector<double> pk(TM4::COUNT * 16, 0.0);
     const int tm = o.tm, G = o.G;
@@ -97,7 +93,7 @@ std::vector<double> build_tet4_pack(const TetOps& o) {
         for (int k = 0; k < 4; ++k) {
             for (int r = 0; r < 9; ++r) {
                 for (int s = 0; s < 3; ++s)
-                    if (i < 3 && 4 * s + k < tm) at(TM4::P + 3 * r + s, i, k) = o.P[(3 * r + i) * tm + 4 * s + k];
+                    if (4 * s + k < tm) at(TM4::P + 3 * r + s, i, k) = o.P[(3 * r + std::min(i, 2)) * tm + 4 * s + k];
                 if (k < 3) at(TM4::W + r, i, k) = -o.W[3 * r + k] * o.P[(3 * r + k) * tm + i];
             }
             for (int x = 0; x < 3; ++x) {
@@ -109,6 +105,7 @@ std::vector<double> build_tet4_pack(const TetOps& o) {
             }
             for (int g = 0; g < G; ++g) at(TM4::MASS, i, k) -= o.W[g] * o.P[g * tm + i] * o.P[g * tm + k];
             if (i < 3 && k < 3) at(TM4::LZ, i, k) = o.Lz[3 * i + k];
+            at(TM4::Z0, i, k) = o.z0[std::min(k, 2)];
         }
     return pk;
 }
@@ -116,7 +113,7 @@ TetLines tet_lines(const TetOps& o) {
     TetLines l;
     std::copy(o.Lx.begin(), o.Lx.end(), l.lx); std::copy(o.Ly.begin(), o.Ly.end(), l.ly);
     std::copy(o.x0.begin(), o.x0.end(), l.x0); std::copy(o.y0.begin(), o.y0.end(), l.y0);
-    std::copy(o.y1.begin(), o.y1.end(), l.y1); std::copy(o.z0.begin(), o.z0.end(), l.z0);
+    std::copy(o.y1.begin(), o.y1.end(), l.y1);
     return l;
 }
 
@@ -199,20 +196,21 @@ void launch_elem_tetc(hpg_tet_ctx* c, double beta, const int* elist, int count) 
     a.pnts = c->pnts; a.tet_pnt = c->tet_pnt; a.tet_seg = c->tet_seg;
     a.ntet = count; a.elist = elist; a.em0 = c->em0; a.ugv = c->ugv; a.uge = c->uge; a.tau = c->tau; a.lf = c->lf;
     a.ops = c->lv[c->log2p].ops; a.mu = c->prm.mu; a.kcond = c->kcond; a.R = c->prm.Rgas; a.gamma = c->prm.gamma;
-    a.atm = 0.0; a.beta = beta;
+    a.atm = 0.0; a.beta = beta; a.gogm1 = c->prm.gamma / (c->prm.gamma - 1.0);
     const int noct = (count + 7) / 8;
-    if (P == 2) {
+    if constexpr (P == 2) {
         // matrix-core form: groups of 16 elements, four groups per block
-        a.ops = c->lv[c->log2p].opsm;
+        a.ops = c->lv[c->log2p].ops4;
+        const TetLines& ln = c->lv[c->log2p].lines;
         const int ngrp = (count + 15) / 16;
         if (beta > 0.0) {
             static const int cap = resident_blocks((const void*)k_elem_tetc_mfma<2, true>);
             hipLaunchKernelGGL((k_elem_tetc_mfma<2, true>), dim3(persistent_grid((ngrp + 3) / 4, cap)), dim3(256), 0,
-                               c->stream, a, ngrp);
+                               c->stream, a, ln, ngrp);
         } else {
             static const int cap = resident_blocks((const void*)k_elem_tetc_mfma<2, false>);
             hipLaunchKernelGGL((k_elem_tetc_mfma<2, false>), dim3(persistent_grid((ngrp + 3) / 4, cap)), dim3(256), 0,
-                               c->stream, a, ngrp);
+                               c->stream, a, ln, ngrp);
         }
     } else if (beta > 0.0) {
         static const int cap = resident_blocks((const void*)k_elem_tetc<P, true>);
@@ -246,7 +244,7 @@ void launch_elem_tet(hpg_tet_ctx* c, int stage, const int* elist = nullptr, int 
     const int noct = (count + 7) / 8;
     const size_t r = c->recs.size();
     if (c->timing) check(hipEventRecord(c->event(2 * r), c->stream), "hipEventRecord");
-    if (P == 2) {
+    if constexpr (P == 2) {
         // matrix-core form: groups of 16 elements, four groups per block
         a.ops = c->lv[c->log2p].ops4;
         const TetLines& ln = c->lv[c->log2p].lines;
@@ -286,7 +284,7 @@ void launch_elem_tet32(hpg_tet_ctx* c, int stage) {
         a.ntet = count; a.elist = nullptr; a.em0 = c->em0; a.ugv = c->ugv; a.uge = c->uge; a.tau = c->tau; a.lf = c->lf;
         a.ops = c->lv[c->log2p].ops32; a.mu = c->prm.mu; a.kcond = c->kcond; a.R = c->prm.Rgas;
         a.gamma = c->prm.gamma; a.atm = 0.0; a.beta = beta;
-        if (P == 2) {
+        if constexpr (P == 2) {
             a.ops = c->lv[c->log2p].opsm32;
             const int ngrp = (count + 15) / 16;
             if (beta > 0.0) {
@@ -310,7 +308,7 @@ void launch_elem_tet32(hpg_tet_ctx* c, int stage) {
         a.pnts = c->pnts; a.tet_pnt = c->tet_pnt; a.tet_seg = c->tet_seg; a.tet_sgn = nullptr;
         a.ntet = count; a.elist = nullptr; a.em0 = c->em0; a.ugv = c->ugv; a.uge = c->uge; a.tau = c->tau; a.lf = c->lf;
         a.ops = c->lv[c->log2p].ops32; a.rho = c->prm.rho; a.mu = c->prm.mu; a.beta = beta;
-        if (P == 2) {
+        if constexpr (P == 2) {
             // matrix-core form: groups of 16 elements, four groups per block
             a.ops = c->lv[c->log2p].opsm32;
             const int ngrp = (count + 15) / 16;
@@ -659,12 +657,10 @@ int hpg_tet_create(const hpg_tet_mesh* m, const hpg_params* prm, hpg_tet_ctx** o
             const std::vector<float> pk32(pk.begin(), pk.end());
             L.ops32 = c->upload(pk32.data(), pk32.size());
             if (o.p == 2) {
-                const std::vector<double> pm = build_tet_mfma_pack<2>(o);
-                L.opsm = c->upload(pm.data(), pm.size());
                 const std::vector<double> p4 = build_tet4_pack(o);
                 L.ops4 = c->upload(p4.data(), p4.size());
                 L.lines = tet_lines(o);
-                const std::vector<double> pm32d = build_tet_mfma_pack<2>(o, true);
+                const std::vector<double> pm32d = build_tet_mfma_pack<2>(o);
                 const std::vector<float> pm32(pm32d.begin(), pm32d.end());
                 L.opsm32 = c->upload(pm32.data(), pm32.size());
             }

@@ -303,12 +303,12 @@ __global__ __launch_bounds__(256) void k_elem_tet32(TetElemArgs32 a, int noct) {
 }
 
 // ---------------------------------------------------------------------------------
-// Matrix-core form of the FP64 element residual (p = 2): 16 tetrahedra per wave64,
-// every transform a contraction on v_mfma_f64_16x16x4f64 with the layout of the tri
-// kernels: columns are the wave's 16 elements, rows Gauss points (27 in two 16-row
+// Matrix-core form of the FP32 element residual (p = 2, the inner solve of the defect
+// correction): 16 tetrahedra per wave64, every transform a contraction on
+// v_mfma_f32_16x16x4f32 with the layout of the tri kernels: columns are the wave's 16 elements, rows Gauss points (27 in two 16-row
 // tiles) or modes (10 in one tile), A operands lane-ready from LDS, B operands the
 // accumulator registers of the previous contraction (register i of lane l holds row
-// 4 i + l / 16 of its tile, which is the B operand of K-step 4 tile + i when the
+// 4 (l / 16) + i of its tile, which is the B operand of K-step 4 tile + i when the
 // operator's K index is laid out that way).  Point fluxes are formed in the lane that
 // holds the point, right before the contraction that consumes them, so no field is
 // exchanged between lanes and nothing but the operators sits in LDS.
@@ -337,11 +337,9 @@ __device__ __forceinline__ void elem_tet_mfma_body(const TetElemArgsT<T>& a, int
     using M = TMDims<P>;
     using V4 = typename Vec4<T>::type;
     constexpr int GT = M::GT, KT = M::KT, QK = M::QK, TM = D::TM;
-    // output row of accumulator register i in lane l: 4 i + l / 16 (f64), 4 (l / 16) + i (f32)
-    constexpr bool F64 = sizeof(T) == 8;
-    // first Gauss point of K-step (tile kt, register i): its four points are
-    // 16 kt + 4 i + l / 16 (f64) or 16 kt + 4 (l / 16) + i (f32)
-    auto kfirst = [](int kt, int i) { return F64 ? 16 * kt + 4 * i : 16 * kt + i; };
+    // output row of accumulator register i in lane l: 4 (l / 16) + i
+    // first Gauss point of K-step (tile kt, register i): its four points are 16 kt + 4 (l / 16) + i
+    auto kfirst = [](int kt, int i) { return 16 * kt + i; };
     __shared__ T sops[M::SIZE];
     for (int k = threadIdx.x; k < M::SIZE; k += blockDim.x) sops[k] = a.ops[k];
     __syncthreads();
@@ -451,7 +449,7 @@ __device__ __forceinline__ void elem_tet_mfma_body(const TetElemArgsT<T>& a, int
             double* lfo = a.lf + (size_t)tt * (REC * TM);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int m = F64 ? 4 * i + q : 4 * q + i;
+                const int m = 4 * q + i;
                 if (valid && m < TM) {
                     double* o = lfo + m * REC;
                     o[0] = double(L0[i]); o[1] = double(L1[i]); o[2] = double(L2[i]); o[3] = double(L3[i]);
@@ -564,7 +562,7 @@ __device__ __forceinline__ void elem_tet_mfma_body(const TetElemArgsT<T>& a, int
             const T bt = T(a.beta);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int m = F64 ? 4 * i + q : 4 * q + i;
+                const int m = 4 * q + i;
                 if (valid && m < TM) {
                     double* o = lfo + m * (2 * TNV) + TNV;
                     o[0] = double(L0[i] * bt); o[1] = double(L1[i] * bt); o[2] = double(L2[i] * bt); o[3] = double(L3[i] * bt);
@@ -589,7 +587,7 @@ __device__ __forceinline__ void elem_tet_mfma_body(const TetElemArgsT<T>& a, int
 //  - Viscous fluxes are linear on the (straight) element: they are formed at its four
 //    vertices; their moments are one 4 x 4 mass product, their divergence a constant.
 // Operands (TM4 offsets) are 4 x 4 blocks in LDS, lane l reads row l % 4, column l / 16.
-// 384 000 tetrahedra: full 519 -> 234 us, inviscid 149 -> 95 us against the 16x16x4 form with
+// 384 000 tetrahedra: full 519 -> 219 us, inviscid 149 -> 87 us against the 16x16x4 form with
 // dense operators (one wave per SIMD, 512 registers; this one fits two waves).  The inviscid
 // stages write and gather records of the imaginary part only, half the bytes.
 struct TM4 {
@@ -600,11 +598,12 @@ struct TM4 {
     static constexpr int MASS = 54;    // -sum_g w_g lambda_v lambda_v'
     static constexpr int DL = 55;      // 3: gradients of the barycentrics, every row
     static constexpr int LZ = 58;      // z derivative
-    static constexpr int COUNT = 59;
+    static constexpr int Z0 = 59;      // z0 of the column's points (not an operand)
+    static constexpr int COUNT = 60;
 };
 // line factors of the collapsed grid (kernel argument: scalar registers)
 struct TetLines {
-    double lx[9], ly[9], x0[3], y0[3], y1[3], z0[3];
+    double lx[9], ly[9], x0[3], y0[3], y1[3];
 };
 __device__ __forceinline__ double mfma4(double a, double b, double c) {
     return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
@@ -617,10 +616,10 @@ __device__ __forceinline__ void tet_phase() {
 }
 // the same for values: what is computed from d after this is computed anew (81 fluxes kept
 // from the pass before would not fit the registers)
-__device__ __forceinline__ void tet_opaque(double d[3][3]) {
+__device__ __forceinline__ void tet_opaque9(double x[9]) {
     tet_phase();
 #pragma unroll
-    for (int k = 0; k < 9; ++k) asm volatile("" : "+v"(d[k / 3][k % 3]));
+    for (int k = 0; k < 9; ++k) asm volatile("" : "+v"(x[k]));
 }
 // x, y and z derivative sums of one variable, one direction of its fluxes at a time (f:
 // the nine registers of a lane): acc = y0 (Lx f_r + x0 Lx (f_s + f_t)), then
@@ -658,14 +657,63 @@ __device__ __forceinline__ void tet_line_t(const TetLines& ln, double z0, double
         }
 }
 
+// Indices of an element group (vertices 0-3, edges 4-9, element 10), loaded a group ahead and
+// kept in the wave's LDS rows: the loads of the state and the coordinates then wait for one
+// latency and not for two.  fetch() issues lane (e, q)'s part, put() stores it, get() reads.
+struct TetAhead {
+    int tt, v, s0, s1;
+    template <class Args>
+    __device__ __forceinline__ void fetch(const Args& a, int grp, int e, int q) {
+        const int slot = grp * 16 + e;
+        tt = slot < a.ntet ? (a.elist ? a.elist[slot] : slot) : 0;
+        v = a.tet_pnt[4 * (size_t)tt + q];
+        s0 = a.tet_seg[6 * (size_t)tt + q];
+        s1 = a.tet_seg[6 * (size_t)tt + 4 + (q & 1)];
+    }
+    __device__ __forceinline__ void put(int (*rows)[16], int e, int q) const {
+        wave_lds_sync();
+        rows[q][e] = v;
+        rows[4 + q][e] = s0;
+        if (q < 2) rows[8 + q][e] = s1;
+        else if (q == 2) rows[10][e] = tt;
+        wave_lds_sync();
+    }
+};
+struct TetGroup {
+    int tt, vtx[4], seg[2];  // seg: edges of modes 4 + q and 8 + q
+    bool valid;
+    __device__ __forceinline__ TetGroup(const int (*rows)[16], int grp, int ntet, int e, int q) {
+        valid = grp * 16 + e < ntet;
+        tt = rows[10][e];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) vtx[k] = rows[k][e];
+        seg[0] = rows[4 + q][e];
+        seg[1] = rows[8 + (q & 1)][e];
+    }
+};
+// modal coefficients: K-step s of lane l is mode 4 s + q, q = l / 16 (vertices 0-3, then one
+// mode of edges 0-5); padding elements: `pad` at the vertices, zero elsewhere
+template <int NV, class Args>
+__device__ __forceinline__ void tet_modal(const Args& a, const TetGroup& g, int q, const double pad[NV], double b[NV][3]) {
+    const int v = q == 0 ? g.vtx[0] : (q == 1 ? g.vtx[1] : (q == 2 ? g.vtx[2] : g.vtx[3]));
+    const double* src[3] = {a.ugv + (size_t)v * NV, a.uge + (size_t)g.seg[0] * a.em0 * NV, a.uge + (size_t)g.seg[1] * a.em0 * NV};
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+        for (int n = 0; n < NV; ++n) {
+            const double x = src[s][n];
+            b[n][s] = g.valid && (s < 2 || q < 2) ? x : (s == 0 ? pad[n] : 0.0);
+        }
+}
+
 // geometry of a straight element: cofactors d (rsdl.cpp:58-62, 449-458) and the Jacobian;
 // padding elements take the reference tetrahedron
-__device__ __forceinline__ double tet_cofactors(const double* __restrict__ pnts, const int* __restrict__ tet_pnt, int tt,
-                                                bool valid, double d[3][3]) {
+__device__ __forceinline__ double tet_cofactors(const double* __restrict__ pnts, const int vtx[4], bool valid,
+                                                double d[3][3]) {
     double X[4][3];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        const int v = tet_pnt[4 * tt + k];
+        const int v = vtx[k];
 #pragma unroll
         for (int n = 0; n < 3; ++n)
             X[k][n] = valid ? pnts[3 * v + n] : ((k == 0 && n == 2) || (k == 1 && n == 1) || (k == 3 && n == 0) ? 1.0 : -1.0);
@@ -695,6 +743,8 @@ template <bool FULL>
 __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetLines& ln, int ngrp) {
     constexpr int TM = TDims<2>::TM, REC = FULL ? 2 * TNV : TNV;
     __shared__ double sops[TM4::COUNT * 16];
+    __shared__ int sidx[4][11][16];
+    __shared__ double sd[FULL ? 4 : 1][16][9];  // cofactors, out of the registers of the strong residual
     __shared__ double sv[FULL ? 12 : 1][256];  // each lane's own viscous results
     for (int k = threadIdx.x; k < TM4::COUNT * 16; k += blockDim.x) sops[k] = a.ops[k];
     __syncthreads();
@@ -706,26 +756,23 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
     const int xcd = (int)blockIdx.x & 7;
     const int gpx = (ngrp + 7) >> 3;
     const int gend = min(ngrp, (xcd + 1) * gpx);
+    TetAhead ahead;
+    if (xcd * gpx + rank < gend) {
+        ahead.fetch(a, xcd * gpx + rank, e, q);
+        ahead.put(sidx[w], e, q);
+    }
     for (int grp = xcd * gpx + rank; grp < gend; grp += WX) {
         tet_phase();
-        const int slot = grp * 16 + e;
-        const bool valid = slot < a.ntet;
-        const int tt = valid ? (a.elist ? a.elist[slot] : slot) : 0;
-        // modal coefficients: K-step s of lane l is mode 4 s + l / 16; padding elements zero
+        const TetGroup G(sidx[w], grp, a.ntet, e, q);
+        const bool valid = G.valid;
+        const int tt = G.tt;
+        const double pad[TNV] = {0.0, 0.0, 0.0, 0.0};
         double b[TNV][3];
-#pragma unroll
-        for (int s = 0; s < 3; ++s) {
-            const int k = 4 * s + q;
-            const double* src = nullptr;
-            if (valid && k < TM)
-                src = k < 4 ? a.ugv + (size_t)a.tet_pnt[4 * tt + k] * TNV
-                            : a.uge + (size_t)a.tet_seg[6 * tt + (k - 4)] * a.em0 * TNV;
-#pragma unroll
-            for (int n = 0; n < TNV; ++n) b[n][s] = src ? src[n] : 0.0;
-        }
+        tet_modal<TNV>(a, G, q, pad, b);
         double d[3][3];
-        const double cjcb = tet_cofactors(a.pnts, a.tet_pnt, tt, valid, d);
+        const double cjcb = tet_cofactors(a.pnts, G.vtx, valid, d);
         const double rho = a.rho;
+        ahead.fetch(a, min(grp + WX, gend - 1), e, q);
         tet_phase();
         // values at the Gauss points
         double U[TNV][9];
@@ -740,8 +787,13 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
                 for (int n = 0; n < TNV; ++n) U[n][r] = mfma4(av, b[n][s], U[n][r]);
             }
         }
+        ahead.put(sidx[w], e, q);
         tet_phase();
         if constexpr (FULL) {
+            if (q == 0)
+#pragma unroll
+                for (int k = 0; k < 9; ++k) sd[w][e][k] = d[k / 3][k % 3];
+            wave_lds_sync();
             // velocity gradients at vertex q, then (rsdl.cpp:518-674) the fluxes
             // -mu/cjcb (sum_b dd(x,b) du(n,b) + sum_m d(x)(m) sum_b d(b)(n) du(m,b))
             double du[3][3], df[3][3], gm[3][3];
@@ -829,14 +881,20 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
             store(L, 0, 1.0);
         }
         if constexpr (FULL) {
-            tet_opaque(d);
+            tet_phase();
             // strong residual: derivr/derivs/derivt of the total fluxes (rsdl.cpp:683-692)
             double R[TNV][9];
-            const double z0 = ln.z0[q < 3 ? q : 2], lz = op[16 * TM4::LZ];
+            const double z0 = op[16 * TM4::Z0], lz = op[16 * TM4::LZ];
             // fluxes of variable n in the (combined) direction with cofactors g and mass flux c
             auto flux = [&](int n, const double g[3], const double c[9], double f[9]) {
 #pragma unroll
                 for (int r = 0; r < 9; ++r) f[r] = n < 3 ? U[n][r] * c[r] + g[n] * U[3][r] : c[r];
+            };
+            double g[3];
+            auto cof = [&](int x, double g[3]) {
+                tet_phase();
+#pragma unroll
+                for (int n = 0; n < 3; ++n) g[n] = sd[w][e][3 * x + n];
             };
             auto mass = [&](const double g[3], double c[9]) {
                 const double gx = rho * g[0], gy = rho * g[1], gz = rho * g[2];
@@ -844,19 +902,23 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
                 for (int r = 0; r < 9; ++r) c[r] = gx * U[0][r] + gy * U[1][r] + gz * U[2][r];
             };
             double c[9], f[9];
-            mass(d[0], c);
+            cof(0, g);
+            mass(g, c);
 #pragma unroll
-            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, d[0], c, f); tet_line_r(ln, f, R[n]); }
-            const double g[3] = {d[1][0] + d[2][0], d[1][1] + d[2][1], d[1][2] + d[2][2]};
+            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, g, c, f); tet_line_r(ln, f, R[n]); }
+#pragma unroll
+            for (int n = 0; n < 3; ++n) g[n] = sd[w][e][3 + n] + sd[w][e][6 + n];
             mass(g, c);
 #pragma unroll
             for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, g, c, f); tet_line_st(ln, f, R[n]); }
-            mass(d[1], c);
+            cof(1, g);
+            mass(g, c);
 #pragma unroll
-            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, d[1], c, f); tet_line_s(ln, f, R[n]); }
-            mass(d[2], c);
+            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, g, c, f); tet_line_s(ln, f, R[n]); }
+            cof(2, g);
+            mass(g, c);
 #pragma unroll
-            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, d[2], c, f); tet_line_t(ln, z0, lz, f, R[n]); }
+            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, g, c, f); tet_line_t(ln, z0, lz, f, R[n]); }
             // stabilisation (rsdl.cpp:695-767) into lf_re, with t = tau (residual):
             // -((d.u) t_n + u_n (d.t) + d_n t_3) for n < 3 and -(d.t)
             const double tm = -a.tau[4 * tt], tc = -a.tau[4 * tt + 3];
@@ -876,11 +938,12 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
                              t3 = tc * R[3][r];
 #pragma unroll
                 for (int x = 0; x < 3; ++x) {
-                    const double su = d[x][0] * U[0][r] + d[x][1] * U[1][r] + d[x][2] * U[2][r];
-                    const double st = d[x][0] * t0 + d[x][1] * t1 + d[x][2] * t2;
-                    M[x][0] = mfma4(aw, su * t0 + U[0][r] * st + d[x][0] * t3, M[x][0]);
-                    M[x][1] = mfma4(aw, su * t1 + U[1][r] * st + d[x][1] * t3, M[x][1]);
-                    M[x][2] = mfma4(aw, su * t2 + U[2][r] * st + d[x][2] * t3, M[x][2]);
+                    const double dx[3] = {sd[w][e][3 * x], sd[w][e][3 * x + 1], sd[w][e][3 * x + 2]};
+                    const double su = dx[0] * U[0][r] + dx[1] * U[1][r] + dx[2] * U[2][r];
+                    const double st = dx[0] * t0 + dx[1] * t1 + dx[2] * t2;
+                    M[x][0] = mfma4(aw, su * t0 + U[0][r] * st + dx[0] * t3, M[x][0]);
+                    M[x][1] = mfma4(aw, su * t1 + U[1][r] * st + dx[1] * t3, M[x][1]);
+                    M[x][2] = mfma4(aw, su * t2 + U[2][r] * st + dx[2] * t3, M[x][2]);
                     M[x][3] = mfma4(aw, st, M[x][3]);
                 }
             }

@@ -368,7 +368,7 @@ struct TetcElemArgsT {
     const double* tau;  // ntet x 25
     double* lf;         // ntet x TM x 2 x 5: [t][m][0 = imaginary, 1 = real][n]
     const T* ops;
-    double mu, kcond, R, gamma, atm, beta;
+    double mu, kcond, R, gamma, atm, beta, gogm1;  // gogm1: gamma / (gamma - 1), read by the FP64 matrix-core form
 };
 typedef TetcElemArgsT<double> TetcElemArgs;
 typedef TetcElemArgsT<float> TetcElemArgs32;
@@ -616,7 +616,7 @@ __global__ __launch_bounds__(256) void k_elem_tetc32(TetcElemArgs32 a, int noct)
     elem_tetc_body<float, P, FULL>(a, noct);
 }
 
-// Matrix-core form of the cns element residual (p = 2), the layout of
+// Matrix-core form of the FP32 cns element residual (p = 2), the layout of
 // elem_tet_mfma_body with NV = 5 (p, u, v, w, RT): 16 tetrahedra per wave, Gauss-point
 // rows in two 16-row tiles, accumulators fed back as B operands, point fluxes formed in
 // the lane that holds the point.  The element tau (5 x 5) sits in LDS per wave.
@@ -628,10 +628,8 @@ __device__ __forceinline__ void elem_tetc_mfma_body(const TetcElemArgsT<T>& a, i
     using M = TMDims<P>;
     using V4 = typename Vec4<T>::type;
     constexpr int GT = M::GT, KT = M::KT, QK = M::QK, TM = D::TM, G = D::G;
-    constexpr bool F64 = sizeof(T) == 8;
-    // first Gauss point of K-step (tile kt, register i): its four points are
-    // 16 kt + 4 i + l / 16 (f64) or 16 kt + 4 (l / 16) + i (f32)
-    auto kfirst = [](int kt, int i) { return F64 ? 16 * kt + 4 * i : 16 * kt + i; };
+    // first Gauss point of K-step (tile kt, register i): its four points are 16 kt + 4 (l / 16) + i
+    auto kfirst = [](int kt, int i) { return 16 * kt + i; };
     __shared__ T sops[M::SIZE];
     __shared__ T stau[4][16][25];
     for (int k = threadIdx.x; k < M::SIZE; k += blockDim.x) sops[k] = a.ops[k];
@@ -646,7 +644,7 @@ __device__ __forceinline__ void elem_tetc_mfma_body(const TetcElemArgsT<T>& a, i
     const V4 z = {T(0), T(0), T(0), T(0)};
     const T gm1 = T(a.gamma) - T(1), gogm1 = T(a.gamma) / gm1, atm = T(a.atm);
     // Gauss point of accumulator register i of tile kt in this lane
-    auto point = [&](int kt, int i) { return F64 ? 16 * kt + 4 * i + q : 16 * kt + 4 * q + i; };
+    auto point = [&](int kt, int i) { return 16 * kt + 4 * q + i; };
     for (int grp = xcd * gpx + rank; grp < gend; grp += WX) {
         const int slot = grp * 16 + e;
         const bool valid = slot < a.ntet;
@@ -757,7 +755,7 @@ __device__ __forceinline__ void elem_tetc_mfma_body(const TetcElemArgsT<T>& a, i
             double* lfo = a.lf + (size_t)tt * (REC * TM);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int m = F64 ? 4 * i + q : 4 * q + i;
+                const int m = 4 * q + i;
                 if (valid && m < TM) {
                     double* o = lfo + m * REC;
 #pragma unroll
@@ -885,7 +883,7 @@ __device__ __forceinline__ void elem_tetc_mfma_body(const TetcElemArgsT<T>& a, i
             const T bt = T(a.beta);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int m = F64 ? 4 * i + q : 4 * q + i;
+                const int m = 4 * q + i;
                 if (valid && m < TM) {
                     double* o = lfo + m * (2 * CNV) + CNV;
 #pragma unroll
@@ -896,9 +894,362 @@ __device__ __forceinline__ void elem_tetc_mfma_body(const TetcElemArgsT<T>& a, i
     }
 }
 
+// FP64 form at p = 2 on v_mfma_f64_4x4x4f64, the layout of elem_tet_body64 (points, moments,
+// line derivatives, viscous terms at the vertices).  The state is kept as (rho, u, v, w, RT)
+// so that each point divides once; the stress is linear on the element, its work tau.u is
+// formed at the points from the interpolated stress.  Cofactors, tau, stress and one variable
+// of the strong residual sit in LDS: with them in registers the spills cost more (169 us).
+// Bound by the FP64 unit and the waits of its LDS operands (half the cycles).
+// 118 098 tetrahedra: full 321 -> 150 us, inviscid 69 -> 44 us against the 16x16x4 form.
+template <bool FULL>
+__device__ __forceinline__ void elem_tetc_body64(const TetcElemArgs& a, const TetLines& ln, int ngrp) {
+    constexpr int TM = TDims<2>::TM, REC = FULL ? 2 * CNV : CNV;
+    __shared__ double sops[TM4::COUNT * 16];
+    // each lane's own: strong residual of the energy [r], viscous moments of the energy row
+    // [9 + x], divergences [12 + n], [15], stress at vertex l / 16 [16 + 3 x + n]
+    __shared__ double sv[FULL ? 25 : 1][256];
+    __shared__ int sidx[4][11][16];
+    __shared__ double sd[FULL ? 4 : 1][16][9];  // cofactors, out of the registers of the strong residual
+    __shared__ double stau[FULL ? 4 : 1][16][25];
+    for (int k = threadIdx.x; k < TM4::COUNT * 16; k += blockDim.x) sops[k] = a.ops[k];
+    __syncthreads();
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int e = lane & 15, q = lane >> 4;
+    const double* op = sops + (lane & 3) + 4 * q;
+    const int WX = ((int)gridDim.x >> 3) * 4;
+    const int rank = ((int)blockIdx.x >> 3) * 4 + w;
+    const int xcd = (int)blockIdx.x & 7;
+    const int gpx = (ngrp + 7) >> 3;
+    const int gend = min(ngrp, (xcd + 1) * gpx);
+    const double gogm1 = a.gogm1, atm = a.atm;
+    TetAhead ahead;
+    if (xcd * gpx + rank < gend) {
+        ahead.fetch(a, xcd * gpx + rank, e, q);
+        ahead.put(sidx[w], e, q);
+    }
+    for (int grp = xcd * gpx + rank; grp < gend; grp += WX) {
+        tet_phase();
+        const TetGroup G(sidx[w], grp, a.ntet, e, q);
+        const bool valid = G.valid;
+        const int tt = G.tt;
+        const double pad[CNV] = {1.0, 0.0, 0.0, 0.0, 1.0};
+        double b[CNV][3];
+        tet_modal<CNV>(a, G, q, pad, b);
+        double tau[7];
+        if constexpr (FULL)
+#pragma unroll
+            for (int k = 0; k < 7; ++k) tau[k] = a.tau[25L * tt + min(4 * k + q, 24)];
+        double d[3][3];
+        const double cjcb = tet_cofactors(a.pnts, G.vtx, valid, d);
+        ahead.fetch(a, min(grp + WX, gend - 1), e, q);
+        if constexpr (FULL) {
+            wave_lds_sync();  // the previous group is done with this wave's tau rows
+#pragma unroll
+            for (int k = 0; k < 7; ++k)
+                if (4 * k + q < 25) stau[w][e][4 * k + q] = valid ? tau[k] : 0.0;
+            wave_lds_sync();
+        }
+        tet_phase();
+        // (rho, u, v, w, RT) at the Gauss points; the padding row repeats row 2
+        double U[CNV][9];
+#pragma unroll
+        for (int r = 0; r < 9; ++r) {
+            if (r % 3 == 0) tet_phase();
+#pragma unroll
+            for (int n = 0; n < CNV; ++n) U[n][r] = 0.0;
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+                const double av = op[16 * (TM4::P + 3 * r + s)];
+#pragma unroll
+                for (int n = 0; n < CNV; ++n) U[n][r] = mfma4(av, b[n][s], U[n][r]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 9; ++r) U[0][r] = (U[0][r] + atm) / U[4][r];
+        ahead.put(sidx[w], e, q);
+        tet_phase();
+        if constexpr (FULL) {
+            if (q == 0)
+#pragma unroll
+                for (int k = 0; k < 9; ++k) sd[w][e][k] = d[k / 3][k % 3];
+            wave_lds_sync();
+            // gradients of u, v, w, RT at vertex q; stress and heat flux (rsdl.cpp:584-755):
+            // -mu/cjcb (sum_m d(x)(m) (gm(n,m) + gm(m,n)) - 2/3 d(x)(n) sum_m gm(m,m)) with
+            // gm(m,n) = sum_b d(b)(n) du(m,b), and -kcond/(R cjcb) sum_m d(x)(m) gm(RT,m)
+            double du[4][3], gm[4][3], df[4][3];
+#pragma unroll
+            for (int x = 0; x < 3; ++x) {
+#pragma unroll
+                for (int n = 0; n < 4; ++n) du[n][x] = 0.0;
+#pragma unroll
+                for (int s = 0; s < 3; ++s) {
+                    const double av = op[16 * (TM4::GV + 3 * x + s)];
+#pragma unroll
+                    for (int n = 0; n < 4; ++n) du[n][x] = mfma4(av, b[n + 1][s], du[n][x]);
+                }
+            }
+            const double muj = -a.mu / cjcb, kcj = -a.kcond / cjcb / a.R;
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int n = 0; n < 3; ++n) gm[m][n] = d[0][n] * du[m][0] + d[1][n] * du[m][1] + d[2][n] * du[m][2];
+            const double dil = 2.0 / 3.0 * (gm[0][0] + gm[1][1] + gm[2][2]);
+#pragma unroll
+            for (int x = 0; x < 3; ++x) {
+#pragma unroll
+                for (int n = 0; n < 3; ++n)
+                    df[n][x] = muj * (d[x][0] * (gm[n][0] + gm[0][n]) + d[x][1] * (gm[n][1] + gm[1][n]) +
+                                      d[x][2] * (gm[n][2] + gm[2][n]) - d[x][n] * dil);
+                df[3][x] = kcj * (d[x][0] * gm[3][0] + d[x][1] * gm[3][1] + d[x][2] * gm[3][2]);
+            }
+            const double am = op[16 * TM4::MASS];
+            double dv[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int x = 0; x < 3; ++x) {
+                const double al = op[16 * (TM4::DL + x)];
+#pragma unroll
+                for (int n = 0; n < 4; ++n) {
+                    dv[n] = mfma4(al, df[n][x], dv[n]);
+                    if (n < 3) sv[16 + 3 * x + n][threadIdx.x] = df[n][x];
+                    else sv[9 + x][threadIdx.x] = mfma4(am, df[n][x], 0.0);
+                }
+            }
+#pragma unroll
+            for (int n = 0; n < 4; ++n) sv[12 + n][threadIdx.x] = dv[n];
+        }
+        auto expand = [&](int x, const double M[CNV], double L[CNV][3]) {
+#pragma unroll
+            for (int rb = 0; rb < 3; ++rb) {
+                const double ag = op[16 * (TM4::GX + 3 * x + rb)];
+#pragma unroll
+                for (int n = 0; n < CNV; ++n) L[n][rb] = mfma4(ag, M[n], L[n][rb]);
+            }
+        };
+        double* lfo = a.lf + (size_t)tt * (REC * TM);
+        auto store = [&](const double L[CNV][3], int off, double f) {
+#pragma unroll
+            for (int rb = 0; rb < 3; ++rb) {
+                const int m = 4 * rb + q;
+                if (valid && m < TM) {
+                    double* o = lfo + m * REC + off;
+#pragma unroll
+                    for (int n = 0; n < CNV; ++n) o[n] = f * L[n][rb];
+                }
+            }
+        };
+        auto enthalpy = [&](int r) {
+            return gogm1 * U[4][r] + 0.5 * (U[1][r] * U[1][r] + U[2][r] * U[2][r] + U[3][r] * U[3][r]);
+        };
+        // lf_im = intgrtrst of the fluxes (rsdl.cpp:494-543)
+        {
+            tet_phase();
+            double L[CNV][3];
+#pragma unroll
+            for (int n = 0; n < CNV; ++n)
+#pragma unroll
+                for (int rb = 0; rb < 3; ++rb) L[n][rb] = 0.0;
+#pragma unroll
+            for (int x = 0; x < 3; ++x) {
+                tet_phase();
+                double M[CNV] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int r = 0; r < 9; ++r) {
+                    const double aw = op[16 * (TM4::W + r)];
+                    const double c = U[0][r] * (d[x][0] * U[1][r] + d[x][1] * U[2][r] + d[x][2] * U[3][r]);
+                    const double pr = U[0][r] * U[4][r] - atm;
+                    M[0] = mfma4(aw, c, M[0]);
+#pragma unroll
+                    for (int n = 1; n < 4; ++n) M[n] = mfma4(aw, U[n][r] * c + d[x][n - 1] * pr, M[n]);
+                    M[4] = mfma4(aw, enthalpy(r) * c, M[4]);
+                }
+                expand(x, M, L);
+            }
+            store(L, 0, 1.0);
+        }
+        if constexpr (FULL) {
+            tet_phase();
+            // strong residual: derivr/derivs/derivt of the total fluxes (rsdl.cpp:768-773);
+            // the constant divergences of the stress and the heat flux are added below
+            double R[4][9], c[9], f[9];
+            double g[3];
+            auto cof = [&](int x, double g[3]) {
+                tet_phase();
+#pragma unroll
+                for (int n = 0; n < 3; ++n) g[n] = sd[w][e][3 * x + n];
+            };
+            auto mass = [&](const double g[3]) {
+                tet_phase();
+#pragma unroll
+                for (int r = 0; r < 9; ++r) c[r] = U[0][r] * (g[0] * U[1][r] + g[1] * U[2][r] + g[2] * U[3][r]);
+            };
+            // fluxes of variable n in the (combined) direction with cofactors g and stress t
+            auto flux = [&](int n, const double g[3], const double t[3]) {
+                tet_opaque9(U[4]);
+#pragma unroll
+                for (int r = 0; r < 9; ++r) {
+                    if (n == 0) f[r] = c[r];
+                    else if (n < 4) f[r] = U[n][r] * c[r] + g[n - 1] * (U[0][r] * U[4][r] - atm);
+                    else {
+                        const double av = op[16 * (TM4::P + 3 * r)];  // modes 0-3 are the barycentrics
+                        f[r] = mfma4(av, t[0], 0.0) * U[1][r] + mfma4(av, t[1], 0.0) * U[2][r] + mfma4(av, t[2], 0.0) * U[3][r];
+                    }
+                }
+            };
+            // f holds the work of the stress: its moment joins the energy row's, then the
+            // convective energy flux completes f
+            auto work = [&](int x) {
+                double m = sv[9 + x][threadIdx.x];
+#pragma unroll
+                for (int r = 0; r < 9; ++r) m = mfma4(op[16 * (TM4::W + r)], f[r], m);
+                sv[9 + x][threadIdx.x] = m;
+            };
+            auto energy = [&]() {
+#pragma unroll
+                for (int r = 0; r < 9; ++r) f[r] += enthalpy(r) * c[r];
+            };
+            auto stress = [&](int x, double t[3]) {
+#pragma unroll
+                for (int n = 0; n < 3; ++n) t[n] = sv[16 + 3 * x + n][threadIdx.x];
+            };
+            auto get = [&](double acc[9]) {
+                tet_phase();
+#pragma unroll
+                for (int r = 0; r < 9; ++r) acc[r] = sv[r][threadIdx.x];
+            };
+            auto put = [&](const double acc[9]) {
+#pragma unroll
+                for (int r = 0; r < 9; ++r) sv[r][threadIdx.x] = acc[r];
+            };
+            double t[3];
+            cof(0, g);
+            mass(g);
+            stress(0, t);
+#pragma unroll
+            for (int n = 0; n < CNV; ++n) {
+                flux(n, g, t);
+                if (n < 4) tet_line_r(ln, f, R[n]);
+            }
+            {
+                double acc[9];
+                work(0);
+                energy();
+                tet_line_r(ln, f, acc);
+                put(acc);
+            }
+#pragma unroll
+            for (int n = 0; n < 3; ++n) g[n] = sd[w][e][3 + n] + sd[w][e][6 + n];
+            mass(g);
+            {
+                double t2[3];
+                stress(1, t);
+                stress(2, t2);
+#pragma unroll
+                for (int n = 0; n < 3; ++n) t[n] += t2[n];
+            }
+#pragma unroll
+            for (int n = 0; n < CNV; ++n) {
+                flux(n, g, t);
+                if (n < 4) tet_line_st(ln, f, R[n]);
+            }
+            {
+                double acc[9];
+                energy();
+                get(acc);
+                tet_line_st(ln, f, acc);
+                put(acc);
+            }
+            cof(1, g);
+            mass(g);
+            stress(1, t);
+#pragma unroll
+            for (int n = 0; n < CNV; ++n) {
+                flux(n, g, t);
+                if (n < 4) tet_line_s(ln, f, R[n]);
+            }
+            {
+                double acc[9];
+                work(1);
+                energy();
+                get(acc);
+                tet_line_s(ln, f, acc);
+                put(acc);
+            }
+            cof(2, g);
+            mass(g);
+            stress(2, t);
+#pragma unroll
+            for (int n = 0; n < CNV; ++n) {
+                flux(n, g, t);
+                if (n < 4) tet_line_t(ln, op[16 * TM4::Z0], op[16 * TM4::LZ], f, R[n]);
+            }
+            {
+                double acc[9];
+                work(2);
+                energy();
+                get(acc);
+                tet_line_t(ln, op[16 * TM4::Z0], op[16 * TM4::LZ], f, acc);
+                put(acc);
+            }
+            // stabilisation with the element tau (rsdl.cpp:776-827) into lf_re: the flux
+            // Jacobian of each direction applied to t = tau (residual),
+            // drho = (dp - rho dRT) / RT, dm = drho q + rho dq with q = d.u, dq = d.du,
+            // (dm, dm u_n + m du_n + d_n dp, dm H + m dH)
+            tet_phase();
+            tet_opaque9(U[4]);
+            double M[3][CNV];
+#pragma unroll
+            for (int x = 0; x < 3; ++x) {
+                M[x][0] = 0.0;
+#pragma unroll
+                for (int n = 0; n < 3; ++n) M[x][n + 1] = mfma4(op[16 * TM4::MASS], sv[16 + 3 * x + n][threadIdx.x], 0.0);
+                M[x][4] = sv[9 + x][threadIdx.x];
+            }
+#pragma unroll
+            for (int r = 0; r < 9; ++r) {
+                tet_phase();
+                const double aw = op[16 * (TM4::W + r)];
+                double t5[CNV];
+                const double r4 = sv[r][threadIdx.x];
+#pragma unroll
+                for (int m = 0; m < CNV; ++m) {
+                    double s = stau[w][e][5 * m] * R[0][r];
+#pragma unroll
+                    for (int n = 1; n < CNV; ++n) s += stau[w][e][5 * m + n] * ((n < 4 ? R[n][r] : r4) + sv[11 + n][threadIdx.x]);
+                    t5[m] = -s;
+                }
+                const double dr = (t5[0] - U[0][r] * t5[4]) / U[4][r];
+                const double hh = enthalpy(r);
+                const double dh = gogm1 * t5[4] + U[1][r] * t5[1] + U[2][r] * t5[2] + U[3][r] * t5[3];
+#pragma unroll
+                for (int x = 0; x < 3; ++x) {
+                    const double dx[3] = {sd[w][e][3 * x], sd[w][e][3 * x + 1], sd[w][e][3 * x + 2]};
+                    const double qx = dx[0] * U[1][r] + dx[1] * U[2][r] + dx[2] * U[3][r];
+                    const double dq = dx[0] * t5[1] + dx[1] * t5[2] + dx[2] * t5[3];
+                    const double mx = U[0][r] * qx, dm = dr * qx + U[0][r] * dq;
+                    M[x][0] = mfma4(aw, dm, M[x][0]);
+#pragma unroll
+                    for (int n = 1; n < 4; ++n)
+                        M[x][n] = mfma4(aw, dm * U[n][r] + mx * t5[n] + dx[n - 1] * t5[0], M[x][n]);
+                    M[x][4] = mfma4(aw, dm * hh + mx * dh, M[x][4]);
+                }
+            }
+            tet_phase();
+            double L[CNV][3];
+#pragma unroll
+            for (int n = 0; n < CNV; ++n)
+#pragma unroll
+                for (int rb = 0; rb < 3; ++rb) L[n][rb] = 0.0;
+#pragma unroll
+            for (int x = 0; x < 3; ++x) expand(x, M[x], L);
+            store(L, CNV, a.beta);
+        }
+    }
+}
+
 template <int P, bool FULL>
-__global__ __launch_bounds__(256) void k_elem_tetc_mfma(TetcElemArgs a, int ngrp) {
-    elem_tetc_mfma_body<double, P, FULL>(a, ngrp);
+__global__ __launch_bounds__(256, 2) void k_elem_tetc_mfma(TetcElemArgs a, TetLines ln, int ngrp) {
+    static_assert(P == 2, "");
+    elem_tetc_body64<FULL>(a, ln, ngrp);
 }
 
 template <int P, bool FULL>

@@ -24,3 +24,19 @@ def test_element_residual_sizes(oracle_mod, n, mu):
         err = rel_err(G.get_residual(), O.get_res())
         print("stage", s, "rel err", err, flush=True)
         assert err < RSDL_TOL
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 6])
+@pytest.mark.parametrize("mu", [0.0, 1e-2])
+def test_cns_element_residual_sizes(oracle_mod, n, mu):
+    import test_gpu_tet_cns as C
+    print(f"\n[gpu-case] tet cns elements n={n} mu={mu}", flush=True)
+    m, st, G, O = C._pair(n, 1, mu=mu, seed=n)
+    G.setup_preconditioner()
+    O.setup_preconditioner()
+    for s in (5, 0, 1, 2, 3):
+        G.rsdl(s)
+        O.rsdl(s)
+        err = rel_err(G.get_residual(), O.get_res())
+        print("stage", s, "rel err", err, flush=True)
+        assert err < C.RSDL_TOL
