@@ -501,8 +501,8 @@ __device__ __forceinline__ void elem_ins_body(const ElemArgsT<T>& a, T* __restri
         }
         if constexpr (EM) {
             // element-major output of the vertex and side modes, side sign applied:
-            // eres[(t*BM + k)*2*NV + n] = lf_im, [... + NV + n] = beta lf_re (full
-            // residual only); the gather kernels add the carried real part and sum over
+            // eres[(t*BM + k)*2*NV + n] = lf_im, [... + NV + n] = beta lf_re; without the real
+            // part (FULL = false) eres[(t*BM + k)*NV + n] = lf_im (half the bytes); the gather kernels add the carried real part and sum over
             // the elements.  Interior modes belong to this element: final here, started
             // from keep * res_r as on a first visit.
 #pragma unroll
@@ -519,7 +519,7 @@ __device__ __forceinline__ void elem_ins_body(const ElemArgsT<T>& a, T* __restri
                     lr[2] = sg * (LR2[s] * bt);
                 }
                 if (kind < 2) {
-                    T* o = eres + ((size_t)S.t * D::BM + k) * (2 * NV);
+                    T* o = eres + ((size_t)S.t * D::BM + k) * (FULL ? 2 * NV : NV);
 #pragma unroll
                     for (int n = 0; n < NV; ++n) {
                         o[n] = li[n];
@@ -900,12 +900,13 @@ __global__ __launch_bounds__(256) void k_gather_vs(GatherArgsT<T> a) {
     const long nvl = (long)a.npnt * NVn;
     const T keep = a.keep;
     const int ne = a.sm + 2;  // entries of a boundary edge
+    const int rec = a.full ? 2 * NVn : NVn;  // inviscid stages: records of the imaginary part only
     if (g < nvl) {
         const int v = (int)(g / NVn), n = (int)(g - (long)v * NVn);
         const T r0 = keep == T(0) ? T(0) : keep * a.rrv[g];
         T acc = r0, accr = r0;
         for (int k = a.vt_ptr[v]; k < a.vt_ptr[v + 1]; ++k) {
-            gather_sum<T, NVn>(a, a.eres + ((long)a.vt_tri[k] * a.bm + a.vt_loc[k]) * (2 * NVn), n, T(1), acc, accr);
+            gather_sum<T, NVn>(a, a.eres + ((long)a.vt_tri[k] * a.bm + a.vt_loc[k]) * rec, n, T(1), acc, accr);
             if (k == a.vt_ptr[v] && a.srcv) acc = acc + T(a.srcv[g] * a.sfac[0]);
         }
         for (int k = a.vb_ptr[v]; k < a.vb_ptr[v + 1]; ++k) {
@@ -933,7 +934,7 @@ __global__ __launch_bounds__(256) void k_gather_vs(GatherArgsT<T> a) {
         // way: its odd modes change sign in this side's frame
         const int sl = a.st_loc[2 * s + slot];
         const int mode = 3 + (sl & 3) * a.sm + m;
-        gather_sum<T, NVn>(a, a.eres + ((long)t * a.bm + mode) * (2 * NVn), n, ((sl & 4) && (m & 1)) ? T(-1) : T(1),
+        gather_sum<T, NVn>(a, a.eres + ((long)t * a.bm + mode) * rec, n, ((sl & 4) && (m & 1)) ? T(-1) : T(1),
                               acc, accr);
         if (first && a.srcs) acc = acc + T(a.srcs[o] * a.sfac[0]);
         first = false;
@@ -1016,7 +1017,7 @@ __global__ __launch_bounds__(256) void k_elem_ins1_valu(ElemArgs a, const double
         }
         LI[0][m] = s0; LI[1][m] = s1; LI[2][m] = s2;
     }
-    double* o = eres + (size_t)t * M * (2 * NV);
+    double* o = eres + (size_t)t * M * (FULL ? 2 * NV : NV);
     if constexpr (FULL) {
         double Ur[G], Us[G], Vr[G], Vs[G];
 #pragma unroll
@@ -1108,7 +1109,7 @@ __global__ __launch_bounds__(256) void k_elem_ins1_valu(ElemArgs a, const double
     } else {
 #pragma unroll
         for (int m = 0; m < M; ++m) {
-            double* om = o + m * (2 * NV);
+            double* om = o + m * NV;
             om[0] = LI[0][m]; om[1] = LI[1][m]; om[2] = LI[2][m];
         }
     }
@@ -1479,7 +1480,7 @@ struct VStageArgs {
     const int* vt_loc;
     const int* vb_ptr;  // boundary-edge endpoints at each vertex: entries 2*idx + k of eout
     const int* vb_ent;
-    const double* eres;  // (ntri, 3, 2, NV)
+    const double* eres;  // (ntri, 3, 2, NV), (ntri, 3, NV) without the real part
     const double* eout;  // (neseg, 2, NV)
     double* resv;
     double* rrv;
@@ -1506,7 +1507,7 @@ __global__ __launch_bounds__(256) void k_vstage1(VStageArgs a) {
     const double r0 = (keep == 0.0 || !(a.full || keep != 0.0)) ? 0.0 : keep * a.rrv[o];
     double acc = r0, accr = r0;
     for (int k = a.vt_ptr[v]; k < a.vt_ptr[v + 1]; ++k) {
-        const double* e = a.eres + ((long)a.vt_tri[k] * 3 + a.vt_loc[k]) * (2 * NVn);
+        const double* e = a.eres + ((long)a.vt_tri[k] * 3 + a.vt_loc[k]) * (a.full ? 2 * NVn : NVn);
         const double li = e[n];
         if (a.full) {
             const double lr = e[NVn + n];

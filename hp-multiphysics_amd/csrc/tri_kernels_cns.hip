@@ -623,7 +623,7 @@ __device__ __forceinline__ void elem_cns_body(const CnsElemArgs& a, int eblk = 0
                     else a.jbase[r] = rr;
                 }
             } else if (kind < 2) {
-                double* o = a.eres + ((size_t)S.t * D::BM + k) * (2 * NVC);
+                double* o = a.eres + ((size_t)S.t * D::BM + k) * (FULL ? 2 * NVC : NVC);
 #pragma unroll
                 for (int n = 0; n < NVC; ++n) {
                     o[n] = sg * LI[n][s];
@@ -955,7 +955,7 @@ __device__ __forceinline__ void elem_cns_lane_body(const CnsElemArgsT<T>& a, int
                 const T vli = T(sg) * li[r], vlr = T(sg) * lr[r];
                 if (kind < 2) {
                     const bool first = (kind == 0 ? a.fcv[sel3(vtx, k)] : a.fcs[sel3(seg, (k - 3) / SMD)]) == col;
-                    double* d = a.eres + ((size_t)t * D::BM + k) * (2 * NVC) + n;
+                    double* d = a.eres + ((size_t)t * D::BM + k) * (FULL ? 2 * NVC : NVC) + n;
                     d[0] = first ? (double)vlr + (double)vli : (double)(vlr + vli);
                     if constexpr (FULL) d[NVC] = vlr;
                 } else {
