@@ -112,10 +112,56 @@ void colour(int nitem, int per, const int* verts, int npnt, std::vector<int>& or
 // nonlinearity ~ h)
 constexpr double FD_H = 1e-3;
 
+// operators of k_elem_ins4_em (TI4): block element [column k][row i] at 4 k + i
+std::vector<double> build_ins4_pack(const TriOps& o) {
+    std::vector<double> pk(TI4::COUNT * 16, 0.0);
+    auto at = [&](int blk, int row, int col) -> double& { return pk[16 * blk + 4 * col + row]; };
+    auto point = [](int r, int q) { return r < 5 ? 5 * r + q : (r == 5 ? 5 * q + 4 : 24); };
+    auto xi = [](int reg, int q) { return reg == 0 ? q : 4; };  // x index of registers 5, 6
+    for (int i = 0; i < 4; ++i)
+        for (int k = 0; k < 4; ++k) {
+            for (int r = 0; r < 7; ++r)
+                for (int s = 0; s < 4; ++s) {
+                    const int m = 4 * s + k, g = point(r, i);
+                    if (m < o.tm) {
+                        at(TI4::P + 4 * r + s, i, k) = o.P[g * o.tm + m];
+                        at(TI4::PR + 4 * r + s, i, k) = o.Pr[g * o.tm + m];
+                        at(TI4::PS + 4 * r + s, i, k) = o.Ps[g * o.tm + m];
+                    }
+                    const int mt = 4 * s + i, h = point(r, k);
+                    if (mt < o.tm && (r < 6 || k == 0)) {
+                        at(TI4::IR + 4 * r + s, i, k) = o.Ir[mt * o.G + h];
+                        at(TI4::IS + 4 * r + s, i, k) = o.Is[mt * o.G + h];
+                    }
+                }
+            for (int out = 0; out < 2; ++out)
+                for (int in = 0; in < 2; ++in) {
+                    if (in == 1 && k > 0) continue;
+                    const double lx = o.n0[4] * o.Lx[5 * xi(out, i) + xi(in, k)];
+                    at(TI4::LA + 2 * out + in, i, k) = lx;
+                    at(TI4::LX + 2 * out + in, i, k) = o.x0[xi(out, i)] * lx;
+                }
+            at(TI4::LB, i, k) = o.Ly[5 * i + k];
+            at(TI4::LB4 + k, i, k) = o.Ly[5 * i + 4];
+            at(TI4::LB5 + i, i, k) = o.Ly[5 * 4 + k];
+            at(TI4::N0, i, k) = o.n0[k];
+        }
+    return pk;
+}
+TriLines tri_line_factors(const TriOps& o) {
+    TriLines l;
+    std::copy(o.Lx.begin(), o.Lx.end(), l.lx);
+    std::copy(o.x0.begin(), o.x0.end(), l.x0);
+    l.ly44 = o.Ly[24];
+    return l;
+}
+
 struct Level {
     int p = 0;
     std::unique_ptr<TriOps> ops;
     double* pack = nullptr;
+    double* ops4 = nullptr;  // p = 4: operators of k_elem_ins4_em (TI4) and
+    TriLines lines{};        // its line factors
     double* op1 = nullptr;  // p = 1: dense P, Pr, Ps, Ir, Is, Dr, Ds (k_elem_ins1_valu layout)
     double* Pmat = nullptr;
     double* lump = nullptr;
@@ -464,7 +510,17 @@ void launch_elem_em(hpg_ctx* c, const ElemArgsT<T>& a, const EdgeArgsT<T>& e, bo
     auto go = [&](auto kern, T* eres, T* eout, int cap) {
         hipLaunchKernelGGL(kern, dim3(persistent_grid(nlogical, cap) + eblk), dim3(256), 0, c->stream, a, eres, e, eout, eblk);
     };
-    if constexpr (F64) {
+    if constexpr (F64 && P == 4) {
+        const Level& L = c->lv[c->log2p];
+        auto go4 = [&](auto kern, int cap) {
+            hipLaunchKernelGGL(kern, dim3(persistent_grid(nlogical, cap) + eblk), dim3(256), 0, c->stream, a, L.ops4, L.lines,
+                               c->eres, e, c->eout, eblk);
+        };
+        static const int cf = resident_blocks((const void*)k_elem_ins4_em<true>);
+        static const int ci = resident_blocks((const void*)k_elem_ins4_em<false>);
+        if (full) go4(k_elem_ins4_em<true>, cf);
+        else go4(k_elem_ins4_em<false>, ci);
+    } else if constexpr (F64) {
         static const int cf = resident_blocks((const void*)k_elem_ins_em<P, true>);
         static const int ci = resident_blocks((const void*)k_elem_ins_em<P, false>);
         if (full) go(k_elem_ins_em<P, true>, c->eres, c->eout, cf);
@@ -1504,6 +1560,11 @@ int hpg_create(const hpg_tri_mesh* m, const hpg_params* prm, hpg_ctx** out) {
                 if (o.P.size() != 12 || o.Ir.size() != 12 || o.Dr.size() != 16)
                     throw std::runtime_error("p = 1 operator sizes");
                 L.op1 = c->upload(d1.data(), d1.size());
+            }
+            if (L.p == 4) {
+                const std::vector<double> p4 = build_ins4_pack(o);
+                L.ops4 = c->upload(p4.data(), p4.size());
+                L.lines = tri_line_factors(o);
             }
             const std::vector<double> pk32d = build_pack(o, [](int i, int q) { return f32_row(i, q); });
             const std::vector<float> pk32(pk32d.begin(), pk32d.end());

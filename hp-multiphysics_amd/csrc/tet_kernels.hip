@@ -605,22 +605,6 @@ struct TM4 {
 struct TetLines {
     double lx[9], ly[9], x0[3], y0[3], y1[3];
 };
-__device__ __forceinline__ double mfma4(double a, double b, double c) {
-    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
-}
-// keeps the compiler from moving operand loads (all loop invariants) and flux sums across the
-// phases of an element group: hoisted, they spill
-__device__ __forceinline__ void tet_phase() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-}
-// the same for values: what is computed from d after this is computed anew (81 fluxes kept
-// from the pass before would not fit the registers)
-__device__ __forceinline__ void tet_opaque9(double x[9]) {
-    tet_phase();
-#pragma unroll
-    for (int k = 0; k < 9; ++k) asm volatile("" : "+v"(x[k]));
-}
 // x, y and z derivative sums of one variable, one direction of its fluxes at a time (f:
 // the nine registers of a lane): acc = y0 (Lx f_r + x0 Lx (f_s + f_t)), then
 // acc = z0 (acc + Ly f_s + y1 Ly f_t), then acc += Lz f_t
@@ -762,7 +746,7 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
         ahead.put(sidx[w], e, q);
     }
     for (int grp = xcd * gpx + rank; grp < gend; grp += WX) {
-        tet_phase();
+        group_phase();
         const TetGroup G(sidx[w], grp, a.ntet, e, q);
         const bool valid = G.valid;
         const int tt = G.tt;
@@ -773,7 +757,7 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
         const double cjcb = tet_cofactors(a.pnts, G.vtx, valid, d);
         const double rho = a.rho;
         ahead.fetch(a, min(grp + WX, gend - 1), e, q);
-        tet_phase();
+        group_phase();
         // values at the Gauss points
         double U[TNV][9];
 #pragma unroll
@@ -788,7 +772,7 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
             }
         }
         ahead.put(sidx[w], e, q);
-        tet_phase();
+        group_phase();
         if constexpr (FULL) {
             if (q == 0)
 #pragma unroll
@@ -855,7 +839,7 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
                 }
             }
         };
-        tet_phase();
+        group_phase();
         // lf_im = intgrtrst of the convective and pressure fluxes (rsdl.cpp:461-511)
         {
             double L[TNV][3];
@@ -865,7 +849,7 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
                 for (int rb = 0; rb < 3; ++rb) L[n][rb] = 0.0;
 #pragma unroll
             for (int x = 0; x < 3; ++x) {
-                tet_phase();
+                group_phase();
                 double M[TNV] = {0.0, 0.0, 0.0, 0.0};
                 const double rx = rho * d[x][0], ry = rho * d[x][1], rz = rho * d[x][2];
 #pragma unroll
@@ -881,7 +865,7 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
             store(L, 0, 1.0);
         }
         if constexpr (FULL) {
-            tet_phase();
+            group_phase();
             // strong residual: derivr/derivs/derivt of the total fluxes (rsdl.cpp:683-692)
             double R[TNV][9];
             const double z0 = op[16 * TM4::Z0], lz = op[16 * TM4::LZ];
@@ -892,7 +876,7 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
             };
             double g[3];
             auto cof = [&](int x, double g[3]) {
-                tet_phase();
+                group_phase();
 #pragma unroll
                 for (int n = 0; n < 3; ++n) g[n] = sd[w][e][3 * x + n];
             };
@@ -905,20 +889,20 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
             cof(0, g);
             mass(g, c);
 #pragma unroll
-            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, g, c, f); tet_line_r(ln, f, R[n]); }
+            for (int n = 0; n < TNV; ++n) { group_phase(); flux(n, g, c, f); tet_line_r(ln, f, R[n]); }
 #pragma unroll
             for (int n = 0; n < 3; ++n) g[n] = sd[w][e][3 + n] + sd[w][e][6 + n];
             mass(g, c);
 #pragma unroll
-            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, g, c, f); tet_line_st(ln, f, R[n]); }
+            for (int n = 0; n < TNV; ++n) { group_phase(); flux(n, g, c, f); tet_line_st(ln, f, R[n]); }
             cof(1, g);
             mass(g, c);
 #pragma unroll
-            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, g, c, f); tet_line_s(ln, f, R[n]); }
+            for (int n = 0; n < TNV; ++n) { group_phase(); flux(n, g, c, f); tet_line_s(ln, f, R[n]); }
             cof(2, g);
             mass(g, c);
 #pragma unroll
-            for (int n = 0; n < TNV; ++n) { tet_phase(); flux(n, g, c, f); tet_line_t(ln, z0, lz, f, R[n]); }
+            for (int n = 0; n < TNV; ++n) { group_phase(); flux(n, g, c, f); tet_line_t(ln, z0, lz, f, R[n]); }
             // stabilisation (rsdl.cpp:695-767) into lf_re, with t = tau (residual):
             // -((d.u) t_n + u_n (d.t) + d_n t_3) for n < 3 and -(d.t)
             const double tm = -a.tau[4 * tt], tc = -a.tau[4 * tt + 3];
@@ -932,7 +916,7 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
             }
 #pragma unroll
             for (int r = 0; r < 9; ++r) {
-                tet_phase();
+                group_phase();
                 const double aw = op[16 * (TM4::W + r)];
                 const double t0 = tm * (R[0][r] + dv[0]), t1 = tm * (R[1][r] + dv[1]), t2 = tm * (R[2][r] + dv[2]),
                              t3 = tc * R[3][r];
@@ -947,7 +931,7 @@ __device__ __forceinline__ void elem_tet_body64(const TetElemArgs& a, const TetL
                     M[x][3] = mfma4(aw, st, M[x][3]);
                 }
             }
-            tet_phase();
+            group_phase();
             double L[TNV][3];
 #pragma unroll
             for (int n = 0; n < TNV; ++n)

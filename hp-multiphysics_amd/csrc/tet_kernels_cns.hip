@@ -928,7 +928,7 @@ __device__ __forceinline__ void elem_tetc_body64(const TetcElemArgs& a, const Te
         ahead.put(sidx[w], e, q);
     }
     for (int grp = xcd * gpx + rank; grp < gend; grp += WX) {
-        tet_phase();
+        group_phase();
         const TetGroup G(sidx[w], grp, a.ntet, e, q);
         const bool valid = G.valid;
         const int tt = G.tt;
@@ -949,12 +949,12 @@ __device__ __forceinline__ void elem_tetc_body64(const TetcElemArgs& a, const Te
                 if (4 * k + q < 25) stau[w][e][4 * k + q] = valid ? tau[k] : 0.0;
             wave_lds_sync();
         }
-        tet_phase();
+        group_phase();
         // (rho, u, v, w, RT) at the Gauss points; the padding row repeats row 2
         double U[CNV][9];
 #pragma unroll
         for (int r = 0; r < 9; ++r) {
-            if (r % 3 == 0) tet_phase();
+            if (r % 3 == 0) group_phase();
 #pragma unroll
             for (int n = 0; n < CNV; ++n) U[n][r] = 0.0;
 #pragma unroll
@@ -967,7 +967,7 @@ __device__ __forceinline__ void elem_tetc_body64(const TetcElemArgs& a, const Te
 #pragma unroll
         for (int r = 0; r < 9; ++r) U[0][r] = (U[0][r] + atm) / U[4][r];
         ahead.put(sidx[w], e, q);
-        tet_phase();
+        group_phase();
         if constexpr (FULL) {
             if (q == 0)
 #pragma unroll
@@ -1042,7 +1042,7 @@ __device__ __forceinline__ void elem_tetc_body64(const TetcElemArgs& a, const Te
         };
         // lf_im = intgrtrst of the fluxes (rsdl.cpp:494-543)
         {
-            tet_phase();
+            group_phase();
             double L[CNV][3];
 #pragma unroll
             for (int n = 0; n < CNV; ++n)
@@ -1050,7 +1050,7 @@ __device__ __forceinline__ void elem_tetc_body64(const TetcElemArgs& a, const Te
                 for (int rb = 0; rb < 3; ++rb) L[n][rb] = 0.0;
 #pragma unroll
             for (int x = 0; x < 3; ++x) {
-                tet_phase();
+                group_phase();
                 double M[CNV] = {0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
                 for (int r = 0; r < 9; ++r) {
@@ -1067,24 +1067,24 @@ __device__ __forceinline__ void elem_tetc_body64(const TetcElemArgs& a, const Te
             store(L, 0, 1.0);
         }
         if constexpr (FULL) {
-            tet_phase();
+            group_phase();
             // strong residual: derivr/derivs/derivt of the total fluxes (rsdl.cpp:768-773);
             // the constant divergences of the stress and the heat flux are added below
             double R[4][9], c[9], f[9];
             double g[3];
             auto cof = [&](int x, double g[3]) {
-                tet_phase();
+                group_phase();
 #pragma unroll
                 for (int n = 0; n < 3; ++n) g[n] = sd[w][e][3 * x + n];
             };
             auto mass = [&](const double g[3]) {
-                tet_phase();
+                group_phase();
 #pragma unroll
                 for (int r = 0; r < 9; ++r) c[r] = U[0][r] * (g[0] * U[1][r] + g[1] * U[2][r] + g[2] * U[3][r]);
             };
             // fluxes of variable n in the (combined) direction with cofactors g and stress t
             auto flux = [&](int n, const double g[3], const double t[3]) {
-                tet_opaque9(U[4]);
+                group_opaque(U[4]);
 #pragma unroll
                 for (int r = 0; r < 9; ++r) {
                     if (n == 0) f[r] = c[r];
@@ -1112,7 +1112,7 @@ __device__ __forceinline__ void elem_tetc_body64(const TetcElemArgs& a, const Te
                 for (int n = 0; n < 3; ++n) t[n] = sv[16 + 3 * x + n][threadIdx.x];
             };
             auto get = [&](double acc[9]) {
-                tet_phase();
+                group_phase();
 #pragma unroll
                 for (int r = 0; r < 9; ++r) acc[r] = sv[r][threadIdx.x];
             };
@@ -1194,8 +1194,8 @@ __device__ __forceinline__ void elem_tetc_body64(const TetcElemArgs& a, const Te
             // Jacobian of each direction applied to t = tau (residual),
             // drho = (dp - rho dRT) / RT, dm = drho q + rho dq with q = d.u, dq = d.du,
             // (dm, dm u_n + m du_n + d_n dp, dm H + m dH)
-            tet_phase();
-            tet_opaque9(U[4]);
+            group_phase();
+            group_opaque(U[4]);
             double M[3][CNV];
 #pragma unroll
             for (int x = 0; x < 3; ++x) {
@@ -1206,7 +1206,7 @@ __device__ __forceinline__ void elem_tetc_body64(const TetcElemArgs& a, const Te
             }
 #pragma unroll
             for (int r = 0; r < 9; ++r) {
-                tet_phase();
+                group_phase();
                 const double aw = op[16 * (TM4::W + r)];
                 double t5[CNV];
                 const double r4 = sv[r][threadIdx.x];
@@ -1233,7 +1233,7 @@ __device__ __forceinline__ void elem_tetc_body64(const TetcElemArgs& a, const Te
                     M[x][4] = mfma4(aw, dm * hh + mx * dh, M[x][4]);
                 }
             }
-            tet_phase();
+            group_phase();
             double L[CNV][3];
 #pragma unroll
             for (int n = 0; n < CNV; ++n)

@@ -26,6 +26,28 @@ __device__ __forceinline__ d4 mfma(double a, double b, d4 c) {
 __device__ __forceinline__ f4 mfma(float a, float b, f4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
+// v_mfma_f64_4x4x4f64: four 4 x 4 blocks; lane l holds A[l % 4][l / 16] (the same for the
+// four blocks here), B[l / 16][l % 16] and the result D[l / 16][l % 16].  16 cycles against 64
+// of the 16x16x4 form: the same rate per product without its 16-row tiles.  FP64 vector and
+// matrix instructions share one unit at one rate (measured: neither overlaps the other), so
+// what an FP64 kernel pays for is its number of products, padding included.
+__device__ __forceinline__ double mfma4(double a, double b, double c) {
+    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+// keeps the compiler from moving operand loads (all loop invariants) and flux sums across the
+// phases of an element group: hoisted, they spill
+__device__ __forceinline__ void group_phase() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+// the same for values: what is computed from x after this is computed anew (fluxes kept from
+// the pass before would not fit the registers)
+template <int N>
+__device__ __forceinline__ void group_opaque(double (&x)[N]) {
+    group_phase();
+#pragma unroll
+    for (int k = 0; k < N; ++k) asm volatile("" : "+v"(x[k]));
+}
 template <typename T> struct Vec4;
 template <> struct Vec4<double> { typedef d4 type; };
 template <> struct Vec4<float> { typedef f4 type; };
@@ -803,13 +825,297 @@ __global__ __launch_bounds__(64) void k_edge_ins(EdgeArgs a) {
 // launch instead of three, and on small meshes the edges' latency hides behind the
 // elements' (two edge launches were 10 us of a 31 us stage at 33 x 33, p = 2).
 template <int P, bool FULL>
-__global__ __launch_bounds__(256, P == 2 ? 2 : 1) void k_elem_ins_em(ElemArgs a, double* eres, EdgeArgs e,
+__global__ __launch_bounds__(256, 2) void k_elem_ins_em(ElemArgs a, double* eres, EdgeArgs e,
                                                                      double* eout, int eblk) {
     if ((int)blockIdx.x < eblk) {
         edge_ins_body<P, double, true>(e, eout, blockIdx.x * 256 + threadIdx.x);
         return;
     }
     elem_ins_body<double, P, FULL, true>(a, eres, eblk);
+}
+
+// ---------------------------------------------------------------------------------
+// The FP64 residual of straight elements at p = 4 on v_mfma_f64_4x4x4f64 (see mfma4): 16
+// elements per wave, lane l = 16 q + e.  Point layout, 28 places for the 5 x 5 Gauss grid
+// (i, j): register r < 5 of row q is (r, q), register 5 is (q, 4), register 6 is (4, 4)
+// (rows 1-3 repeat it, their weights are zero).  So the x lines j < 4 lie in a lane's
+// registers, and their derivative is a 5-term sum on the vector unit; only the line j = 4 and
+// the y derivatives are products.  The strong residual of a variable takes 23 blocks and 60
+// multiply-adds, 620 cycles, against 1 792 of the dense 25 x 25 operators in 16-row tiles.
+// Fluxes are formed when they are consumed: 256 registers, two waves per SIMD (the 16x16x4
+// form kept all of them, 482 registers and one wave, and waited for every load).
+// The next group's data are loaded a group ahead (without: 367 and 190 us).
+// Bound by the FP64 unit.  512 x 512: full 482 -> 332 us, inviscid 190 -> 151 us a launch.
+struct TI4 {
+    static constexpr int P = 0;      // 28: values at register r from K-step s, [4 r + s]
+    static constexpr int PR = 28;    // 28: r derivatives
+    static constexpr int PS = 56;    // 28: s derivatives
+    static constexpr int IR = 84;    // 28: tests, [4 r + row block]
+    static constexpr int IS = 112;   // 28
+    static constexpr int LA = 140;   // 4: n0 Lx on the line j = 4, [2 out + in] (registers 5, 6)
+    static constexpr int LX = 144;   // 4: n0 x0 Lx there
+    static constexpr int LB = 148;   // y derivative among j < 4
+    static constexpr int LB4 = 149;  // 4: from (i, 4) to (i, j), column i
+    static constexpr int LB5 = 153;  // 4: from (i, j) to (i, 4), row i
+    static constexpr int N0 = 157;   // n0 of row q (not an operand)
+    static constexpr int COUNT = 158;
+};
+struct TriLines {
+    double lx[25], x0[5], ly44;
+};
+
+// collapsed-coordinate derivatives of one variable's fluxes (derivr of fr + derivs of fs)
+__device__ __forceinline__ void tri_lines(const TriLines& ln, const double* op, const double fr[7], const double fs[7],
+                                          double R[7]) {
+    const double n0 = op[16 * TI4::N0];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        double t = ln.lx[5 * i] * fr[0], t2 = ln.lx[5 * i] * fs[0];
+#pragma unroll
+        for (int n = 1; n < 5; ++n) { t += ln.lx[5 * i + n] * fr[n]; t2 += ln.lx[5 * i + n] * fs[n]; }
+        R[i] = n0 * (t + ln.x0[i] * t2);
+    }
+    const double lb = op[16 * TI4::LB];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) R[i] = mfma4(lb, fs[i], R[i]);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) R[i] = mfma4(op[16 * (TI4::LB4 + (i & 3))], i < 4 ? fs[5] : fs[6], R[i]);
+#pragma unroll
+    for (int o = 0; o < 2; ++o) {
+        double s = ln.ly44 * fs[5 + o];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            s = mfma4(op[16 * (TI4::LA + 2 * o + i)], fr[5 + i], s);
+            s = mfma4(op[16 * (TI4::LX + 2 * o + i)], fs[5 + i], s);
+        }
+        R[5 + o] = s;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) R[5] = mfma4(op[16 * (TI4::LB5 + i)], fs[i], R[5]);
+    R[6] = mfma4(op[16 * TI4::LB5], fs[4], R[6]);
+}
+
+template <bool FULL>
+__device__ __forceinline__ void elem_ins4_body(const ElemArgs& a, const double* __restrict__ ops, const TriLines& ln,
+                                               double* __restrict__ eres, int eblk) {
+    using D = Dims<4>;
+    constexpr int REC = FULL ? 2 * NV : NV;
+    __shared__ double sops[TI4::COUNT * 16];
+    for (int k = threadIdx.x; k < TI4::COUNT * 16; k += blockDim.x) sops[k] = ops[k];
+    __syncthreads();
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int e = lane & 15, q = lane >> 4;
+    const double* op = sops + (lane & 3) + 4 * q;  // this lane's element of block b: op[16 b]
+    // groups of 16 elements per XCD and wave as in elem_ins_body
+    const int WX = (((int)gridDim.x - eblk) >> 3) * 4;
+    const int rank = (((int)blockIdx.x - eblk) >> 3) * 4 + w;
+    const int xcd = blockIdx.x & 7;
+    const int ng = (a.end - a.begin + 15) >> 4;
+    const int gpx = (ng + 7) >> 3;
+    const int g0 = xcd * gpx + rank;
+    const int gend = min(ng, (xcd + 1) * gpx);
+    if (g0 >= gend) return;
+    // the state and coordinates of a group are loaded while the group before it is computed
+    // (ahead of its stores, which the loads would otherwise wait for), its indices one earlier
+    ElemConn cnext = elem_conn(a, elem_of_group(a, g0, gend, e));
+    ElemSlots<4> Sn;
+    double raw[NV][4];
+    auto ahead = [&](int g) {  // g: the group whose indices cnext holds
+        Sn = elem_slots<4>(a, cnext, q);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int k = 4 * s + q, kind = mode_kind<4>(k);
+            const int off = Sn.off[s] < 0 ? ~Sn.off[s] : Sn.off[s];
+            const double* src = kind == 0 ? a.ugv : (kind == 1 ? a.ugs : a.ugi);
+            const bool live = Sn.t >= 0 && k < D::TM;
+#pragma unroll
+            for (int n = 0; n < NV; ++n) raw[n][s] = live ? src[off + n] : 0.0;
+        }
+        cnext = elem_conn(a, elem_of_group(a, g + WX, gend, e));
+    };
+    ahead(g0);
+    for (int g = g0; g < gend; g += WX) {
+        group_phase();
+        const ElemSlots<4> S = Sn;
+        // modal coefficients: K-step s of lane l is mode 4 s + q
+        double b[NV][4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int n = 0; n < NV; ++n) b[n][s] = S.off[s] < 0 ? -raw[n][s] : raw[n][s];
+        // ldcrd(n,0) = dx_n/dr, ldcrd(n,1) = dx_n/ds (rsdl.cpp:44-47): l00, l01, l10, l11
+        double l[4] = {0.5 * (S.x[2] - S.x[1]), 0.5 * (S.x[0] - S.x[1]), 0.5 * (S.y[2] - S.y[1]),
+                       0.5 * (S.y[0] - S.y[1])};
+        const double rho = a.rho;
+        group_phase();
+        if constexpr (!FULL) ahead(g + WX);
+        double U[NV][7];
+#pragma unroll
+        for (int r = 0; r < 7; ++r) {
+            if (r == 3 || r == 5) group_phase();
+#pragma unroll
+            for (int n = 0; n < NV; ++n) U[n][r] = 0.0;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const double av = op[16 * (TI4::P + 4 * r + s)];
+#pragma unroll
+                for (int n = 0; n < NV; ++n) U[n][r] = mfma4(av, b[n][s], U[n][r]);
+            }
+        }
+        // inviscid fluxes at register r (rsdl.cpp:262-291): mass c, momentum f[n], directions r, s
+        auto inviscid = [&](int r, double c[2], double f0[2], double f1[2]) {
+            const double u = U[0][r], v = U[1][r], pr = U[2][r];
+            const double fx = rho * u, fy = rho * v;
+            c[0] = l[3] * fx - l[1] * fy;
+            c[1] = l[0] * fy - l[2] * fx;
+            f0[0] = u * c[0] + l[3] * pr;
+            f0[1] = u * c[1] - l[2] * pr;
+            f1[0] = v * c[0] - l[1] * pr;
+            f1[1] = v * c[1] + l[0] * pr;
+        };
+        auto test = [&](int r, const double f0[2], const double f1[2], const double c[2], double L[NV][4]) {
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb) {
+                const double ar = op[16 * (TI4::IR + 4 * r + rb)], as = op[16 * (TI4::IS + 4 * r + rb)];
+                L[0][rb] = mfma4(ar, f0[0], L[0][rb]); L[1][rb] = mfma4(ar, f1[0], L[1][rb]);
+                L[2][rb] = mfma4(ar, c[0], L[2][rb]);  L[0][rb] = mfma4(as, f0[1], L[0][rb]);
+                L[1][rb] = mfma4(as, f1[1], L[1][rb]); L[2][rb] = mfma4(as, c[1], L[2][rb]);
+            }
+        };
+        auto store = [&](const double L[NV][4], int at, double f) {
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+                const int k = 4 * s + q;
+                if (S.t < 0) continue;
+                const double sg = S.off[s] < 0 ? -f : f;
+                double* o = eres + ((size_t)S.t * D::BM + k) * REC + at;
+#pragma unroll
+                for (int n = 0; n < NV; ++n) o[n] = sg * L[n][s];
+            }
+        };
+        static_assert(D::BM == 12, "row blocks 0-2 hold the vertex and side modes");
+        // lf_im = intgrtrs of the inviscid fluxes (rsdl.cpp:292-294); li: interior modes
+        double li[NV];
+        {
+            double L[NV][4];
+#pragma unroll
+            for (int n = 0; n < NV; ++n)
+#pragma unroll
+                for (int rb = 0; rb < 4; ++rb) L[n][rb] = 0.0;
+#pragma unroll
+            for (int r = 0; r < 7; ++r) {
+                group_phase();
+                double c[2], f0[2], f1[2];
+                inviscid(r, c, f0, f1);
+                test(r, f0, f1, c, L);
+            }
+            store(L, 0, 1.0);
+#pragma unroll
+            for (int n = 0; n < NV; ++n) li[n] = L[n][3];
+        }
+        double lr[NV] = {0.0, 0.0, 0.0};
+        if constexpr (FULL) {
+            group_opaque(l);
+            const double cjcb = l[0] * l[3] - l[2] * l[1];
+            // viscous fluxes (rsdl.cpp:303-326) F[r] = {f00, f01, f10, f11}
+            double F[7][4];
+            {
+                const double cj = a.mu / cjcb;
+                const double v0000 = -cj * (2.0 * l[3] * l[3] + l[1] * l[1]), v0011 = -cj * (2.0 * l[2] * l[2] + l[0] * l[0]);
+                const double v0001 = cj * (2.0 * l[3] * l[2] + l[1] * l[0]);
+                const double v1100 = -cj * (l[3] * l[3] + 2.0 * l[1] * l[1]), v1111 = -cj * (l[2] * l[2] + 2.0 * l[0] * l[0]);
+                const double v1101 = cj * (l[3] * l[2] + 2.0 * l[1] * l[0]);
+                const double v0100 = cj * l[1] * l[3], v0111 = cj * l[0] * l[2];
+                const double v0101 = -cj * l[1] * l[2], v0110 = -cj * l[0] * l[3];
+#pragma unroll
+                for (int r = 0; r < 7; ++r) {
+                    group_phase();
+                    double ur = 0.0, us = 0.0, vr = 0.0, vs = 0.0;
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        const double ar = op[16 * (TI4::PR + 4 * r + s)], as = op[16 * (TI4::PS + 4 * r + s)];
+                        ur = mfma4(ar, b[0][s], ur); us = mfma4(as, b[0][s], us);
+                        vr = mfma4(ar, b[1][s], vr); vs = mfma4(as, b[1][s], vs);
+                    }
+                    F[r][0] = v0000 * ur + v0100 * vr + v0001 * us + v0101 * vs;
+                    F[r][1] = v0001 * ur + v0110 * vr + v0011 * us + v0111 * vs;
+                    F[r][2] = v0100 * ur + v1100 * vr + v0110 * us + v1101 * vs;
+                    F[r][3] = v0101 * ur + v1101 * vr + v0111 * us + v1111 * vs;
+                }
+            }
+            // strong residual: derivr/derivs of the total fluxes (rsdl.cpp:369-375)
+            double R[NV][7], fr[7], fs[7];
+#pragma unroll
+            for (int n = 0; n < NV; ++n) {
+                group_opaque(l);
+#pragma unroll
+                for (int r = 0; r < 7; ++r) {
+                    double c[2], f0[2], f1[2];
+                    inviscid(r, c, f0, f1);
+                    fr[r] = n == 0 ? f0[0] + F[r][0] : (n == 1 ? f1[0] + F[r][2] : c[0]);
+                    fs[r] = n == 0 ? f0[1] + F[r][1] : (n == 1 ? f1[1] + F[r][3] : c[1]);
+                }
+                group_phase();
+                tri_lines(ln, op, fr, fs, R[n]);
+            }
+            ahead(g + WX);
+            // per-point tau (CALC_TAU2, rsdl.cpp:377-395) and the stabilisation (:397-421)
+            group_opaque(l);
+            const double dx1 = -2.0 * (l[0] - l[1]), dy1 = -2.0 * (l[2] - l[3]), dx2 = -2.0 * l[1], dy2 = -2.0 * l[3];
+            const double ar2 = dx1 * dy2 - dy1 * dx2;
+            const double perim = sqrt(dx1 * dx1 + dy1 * dy1) + sqrt(dx2 * dx2 + dy2 * dy2) +
+                                 sqrt((dx1 + dx2) * (dx1 + dx2) + (dy1 + dy2) * (dy1 + dy2));
+            const double h = (ar2 / perim) / (0.25 * 5 * 5);
+            const double gv = 2.0 * (a.mu / rho) / h, gvis = gv * gv, tfac = a.adis * h / cjcb;
+            double L[NV][4];
+#pragma unroll
+            for (int n = 0; n < NV; ++n)
+#pragma unroll
+                for (int rb = 0; rb < 4; ++rb) L[n][rb] = 0.0;
+#pragma unroll
+            for (int r = 0; r < 7; ++r) {
+                group_phase();
+                const double u = U[0][r], v = U[1][r];
+                const double qq = u * u + v * v;
+                double gam = 3.0 * qq + gvis;
+                if (a.mu == 0.0) gam = fmax(gam, 0.1);
+                const double tau0 = tfac / sqrt(gam);
+                const double tau2 = sqrt(qq) * tau0;
+                const double t0 = tau0 * R[0][r], t1 = tau0 * R[1][r], t2 = tau2 * R[2][r];
+                // with q_d = the contravariant velocity and t_d = the contravariant t:
+                // (q_d t_n + u_n t_d + cofactor t2), and t_d
+                const double q0 = l[3] * u - l[1] * v, q1 = l[0] * v - l[2] * u;
+                const double s0 = l[3] * t0 - l[1] * t1, s1 = l[0] * t1 - l[2] * t0;
+                const double c[2] = {-s0, -s1};
+                const double f0[2] = {F[r][0] - (q0 * t0 + u * s0 + l[3] * t2), F[r][1] - (q1 * t0 + u * s1 - l[2] * t2)};
+                const double f1[2] = {F[r][2] - (q0 * t1 + v * s0 - l[1] * t2), F[r][3] - (q1 * t1 + v * s1 + l[0] * t2)};
+                test(r, f0, f1, c, L);
+            }
+            store(L, NV, a.beta);
+#pragma unroll
+            for (int n = 0; n < NV; ++n) lr[n] = a.beta * L[n][3];
+        }
+        // interior modes belong to this element: final here, started from keep * res_r
+        if (S.t >= 0 && q < 3) {
+            const int off = S.off[3];
+#pragma unroll
+            for (int n = 0; n < NV; ++n) {
+                const double r0 = a.keep == 0.0 ? 0.0 : a.keep * a.rri[off + n];
+                if (FULL || a.keep != 1.0) a.rri[off + n] = r0 + lr[n];
+                a.resi[off + n] = r0 + lr[n] + li[n];
+            }
+        }
+    }
+}
+
+template <bool FULL>
+__global__ __launch_bounds__(256, 2) void k_elem_ins4_em(ElemArgs a, const double* __restrict__ ops, TriLines ln,
+                                                                    double* eres, EdgeArgs e, double* eout, int eblk) {
+    if ((int)blockIdx.x < eblk) {
+        edge_ins_body<4, double, true>(e, eout, blockIdx.x * 256 + threadIdx.x);
+        return;
+    }
+    elem_ins4_body<FULL>(a, ops, ln, eres, eblk);
 }
 
 // FP32 (the inner solve of the defect correction): the same residual in single precision

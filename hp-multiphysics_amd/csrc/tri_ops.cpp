@@ -219,14 +219,16 @@ TriOps::TriOps(int p_) : p(p_) {
         return D;
     };
     const std::vector<double> Dx = lagr_deriv(xg), De = lagr_deriv(eg);
+    Lx = Dx; Ly = De;
+    for (double x : xg) x0.push_back(0.5 * (1.0 + x));
+    for (double x : eg) n0.push_back(2.0 / (1.0 - x));
     Dr.assign(G * G, 0.0); Ds = Dr;
     for (int i = 0; i < gpx; ++i)
         for (int j = 0; j < gpn; ++j) {
             const int g = i * gpn + j;
-            const double n0 = 2.0 / (1.0 - eg[j]), x0 = 0.5 * (1.0 + xg[i]);
             for (int i2 = 0; i2 < gpx; ++i2) {
-                Dr[g * G + i2 * gpn + j] += n0 * Dx[i * gpx + i2];
-                Ds[g * G + i2 * gpn + j] += x0 * n0 * Dx[i * gpx + i2];
+                Dr[g * G + i2 * gpn + j] += n0[j] * Dx[i * gpx + i2];
+                Ds[g * G + i2 * gpn + j] += x0[i] * n0[j] * Dx[i * gpx + i2];
             }
             for (int j2 = 0; j2 < gpn; ++j2) Ds[g * G + i * gpn + j2] += De[j * gpn + j2];
         }

@@ -27,6 +27,8 @@ struct TriOps {
     std::vector<double> P, Pr, Ps;   // G x tm
     std::vector<double> I, Ir, Is;   // tm x G
     std::vector<double> Dr, Ds;      // G x G
+    std::vector<double> Lx, Ly;      // their 1-D factors (gpx x gpx, gpn x gpn) and
+    std::vector<double> x0, n0;      // line factors: Dr = n0 Lx, Ds = x0 n0 Lx + Ly
     std::vector<double> g1, dg1, w1; // edge basis: gpx x (sm+2) values / d/dxi, weights
     // upper band (bandwidth 2, row j = column j of U: U(j-2,j), U(j-1,j), U(j,j)) Cholesky
     // factor of the side-mode block of the edge mass matrix (tri_basis/initialize.cpp:1097-1130)
