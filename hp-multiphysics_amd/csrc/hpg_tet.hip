@@ -376,20 +376,19 @@ void do_rsdl_tet(hpg_tet_ctx* c, int stage, bool fp32 = false) {
                                c->pnts, c->ugv, c->uge, c->em0, L.P2, L.W2, c->prm.rho, c->flf);
     }
     const int tm = L.p == 1 ? 4 : 10, tm2 = L.p == 1 ? 3 : 6;
-    TetGatherArgs g;
+    TetGatherArgs g{};
     const int nvv = c->nv;
     g.re = beta > 0.0 ? 1 : 0;
     g.tm = tm; g.tm2 = tm2; g.lf = c->lf; g.flf = c->flf; g.omb = 1.0 - beta; g.fnv = c->cns() ? CNV : 1;
-    g.nent = c->npnt; g.mbase = 0; g.fbase = 0; g.stride = nvv; g.ptr = c->vt_ptr; g.code = c->vt_code;
-    g.fptr = c->vf_ptr; g.fcode = c->vf_code; g.res = c->resv; g.rr = c->rrv;
-    if (c->cns()) hipLaunchKernelGGL(k_gather_tet<CNV>, dim3(nblk8(c->npnt)), dim3(256), 0, c->stream, g);
-    else hipLaunchKernelGGL(k_gather_tet<TNV>, dim3(nblk8(c->npnt)), dim3(256), 0, c->stream, g);
+    g.part[0] = {c->npnt, 0, 0, nvv, c->vt_ptr, c->vt_code, c->vf_ptr, c->vf_code, c->resv, c->rrv};
+    g.vblk = (int)nblk8((long)c->npnt * nvv);
+    unsigned eb = 0;
     if (c->em() > 0) {
-        g.nent = c->nseg; g.mbase = 4; g.fbase = 3; g.stride = c->em0 * nvv; g.ptr = c->et_ptr; g.code = c->et_code;
-        g.fptr = c->ef_ptr; g.fcode = c->ef_code; g.res = c->rese; g.rr = c->rre;
-        if (c->cns()) hipLaunchKernelGGL(k_gather_tet<CNV>, dim3(nblk8(c->nseg)), dim3(256), 0, c->stream, g);
-        else hipLaunchKernelGGL(k_gather_tet<TNV>, dim3(nblk8(c->nseg)), dim3(256), 0, c->stream, g);
+        g.part[1] = {c->nseg, 4, 3, c->em0 * nvv, c->et_ptr, c->et_code, c->ef_ptr, c->ef_code, c->rese, c->rre};
+        eb = nblk8((long)c->nseg * nvv);
     }
+    if (c->cns()) hipLaunchKernelGGL(k_gather_tet<CNV>, dim3(g.vblk + eb), dim3(256), 0, c->stream, g);
+    else hipLaunchKernelGGL(k_gather_tet<TNV>, dim3(g.vblk + eb), dim3(256), 0, c->stream, g);
     if (c->coarse_flag) {
         const int l = c->log2p;
         if (c->isfrst) {
@@ -447,7 +446,7 @@ void do_minvrt_tet(hpg_tet_ctx* c, bool pre_dirichlet, double cfa) {
         a.ugv = c->ugv; a.ug0v = c->ug0v; a.cfa = cfa;
         if (a.em > 0) { a.uge = c->uge; a.ug0e = c->ug0e; }
     }
-    hipLaunchKernelGGL(k_minv_vrtx_tet, dim3(nblk8(c->npnt)), dim3(256), 0, c->stream, a);
+    hipLaunchKernelGGL(k_minv_vrtx_tet, dim3(nblk8((long)c->npnt * TNV)), dim3(256), 0, c->stream, a);
     if (a.em > 0) hipLaunchKernelGGL(k_minv_edge_tet, dim3(nblk8(c->nseg)), dim3(256), 0, c->stream, a);
     check(hipGetLastError(), "tet minvrt launch");
 }
@@ -472,10 +471,10 @@ int read_error(hpg_tet_ctx* c) {  // as for tri contexts
 
 int do_setup_tetc(hpg_tet_ctx* c) {
     if (c->lv[c->log2p].p == 1) launch_setup_tetc<1>(c); else launch_setup_tetc<2>(c);
-    hipLaunchKernelGGL(k_setup_gather_tetc, dim3(nblk8(c->npnt)), dim3(256), 0, c->stream, c->npnt, c->vt_ptr,
+    hipLaunchKernelGGL(k_setup_gather_tetc, dim3(nblk8(25L * c->npnt)), dim3(256), 0, c->stream, c->npnt, c->vt_ptr,
                        c->vt_code, c->iprcn, c->tpc, c->vprcn, c->vpc);
     if (c->em() > 0)
-        hipLaunchKernelGGL(k_setup_gather_tetc, dim3(nblk8(c->nseg)), dim3(256), 0, c->stream, c->nseg, c->et_ptr,
+        hipLaunchKernelGGL(k_setup_gather_tetc, dim3(nblk8(25L * c->nseg)), dim3(256), 0, c->stream, c->nseg, c->et_ptr,
                            c->et_code, c->iprcn, c->tpc, c->eprcn, c->epc);
     check(hipGetLastError(), "tet cns setup launch");
     return read_error(c);

@@ -1006,60 +1006,61 @@ __global__ __launch_bounds__(256) void k_face_tet(int nbf, const int* __restrict
     for (int m = 0; m < D::TM2; ++m) flf[f * D::TM2 + m] = lf[m];
 }
 
-// assembly of one entity kind (vertices: mode = local vertex; edges: mode = 4 + local
-// edge): res_r = omb res_r + sum lf_re; res = face fluxes + sum lf_im + res_r
-// (tet_hp/update.cpp:13-31, 45-70, bdry.cpp:16-57); elements and faces ascending
-struct TetGatherArgs {
-    int nent, tm, tm2, mbase, fbase, stride;
-    int re;           // 1: records [im/re][n]; 0: [n] only (lf_re = 0)
-    int fnv;          // face variables: 1 (continuity into the last variable) or NV, flf[f][fnv][tm2]
+// assembly of the vertices (mode = local vertex) and the edges (mode = 4 + local edge):
+// res_r = omb res_r + sum lf_re; res = face fluxes + sum lf_im + res_r
+// (tet_hp/update.cpp:13-31, 45-70, bdry.cpp:16-57); elements and faces ascending.  One lane
+// per (entity, variable) and one launch for both kinds: bound by the latency of the index
+// and record loads, which NV times the lanes overlap (a lane per entity and a launch per
+// kind: 107 -> 71 us a stage for 384 000 tetrahedra, ins).
+struct TetGatherPart {
+    int nent, mbase, fbase, stride;
     const int* ptr;   // CSR entity -> (element, local index) codes 16*t + i
     const int* code;
     const int* fptr;  // CSR entity -> (face, local index) codes 8*f + j
     const int* fcode;
-    const double* lf;
-    const double* flf;
     double* res;
     double* rr;
+};
+struct TetGatherArgs {
+    TetGatherPart part[2];
+    int vblk;         // blocks of part 0 (a multiple of 8)
+    int tm, tm2;
+    int re;           // 1: records [im/re][n]; 0: [n] only (lf_re = 0)
+    int fnv;          // face variables: 1 (continuity into the last variable) or NV, flf[f][fnv][tm2]
+    const double* lf;
+    const double* flf;
     double omb;
 };
 
 template <int NV>
 __global__ __launch_bounds__(256) void k_gather_tet(TetGatherArgs a) {
-    const int v = xcd_block() * blockDim.x + threadIdx.x;
-    if (v >= a.nent) return;
-    double si[NV], sr[NV];
-#pragma unroll
-    for (int n = 0; n < NV; ++n) si[n] = 0.0;
-    for (int k = a.fptr[v]; k < a.fptr[v + 1]; ++k) {
-        const int c = a.fcode[k], f = c >> 3, j = c & 7;
+    const bool edges = (int)blockIdx.x >= a.vblk;
+    const int nblk = edges ? (int)gridDim.x - a.vblk : a.vblk, blk = (int)blockIdx.x - (edges ? a.vblk : 0);
+    // XCD-aware map as xcd_block(), within the part's blocks
+    const int lane = ((blk & 7) * (nblk >> 3) + (blk >> 3)) * 256 + (int)threadIdx.x;
+    const int v = lane / NV, n = lane - v * NV;
+    const int nent = edges ? a.part[1].nent : a.part[0].nent;
+    if (v >= nent) return;
+    const TetGatherPart& p = edges ? a.part[1] : a.part[0];
+    const size_t o = (size_t)v * p.stride + n;
+    double si = 0.0, sr = a.omb * p.rr[o];
+    for (int k = p.fptr[v]; k < p.fptr[v + 1]; ++k) {
+        const int c = p.fcode[k], f = c >> 3, j = c & 7;
         if (a.fnv == 1) {
-            si[NV - 1] += a.flf[f * a.tm2 + a.fbase + j];
+            if (n == NV - 1) si += a.flf[f * a.tm2 + p.fbase + j];
         } else {
-#pragma unroll
-            for (int n = 0; n < NV; ++n) si[n] += a.flf[(f * NV + n) * a.tm2 + a.fbase + j];
+            si += a.flf[(f * NV + n) * a.tm2 + p.fbase + j];
         }
     }
-    double* R = a.res + (size_t)v * a.stride;
-    double* RR = a.rr + (size_t)v * a.stride;
-#pragma unroll
-    for (int n = 0; n < NV; ++n) sr[n] = a.omb * RR[n];
-    for (int k = a.ptr[v]; k < a.ptr[v + 1]; ++k) {
-        const int c = a.code[k], t = c >> 4, i = c & 15;
-        // one contiguous record per (element, mode)
-        const int rec = a.re ? 2 * NV : NV;
-        const double* L = a.lf + ((size_t)t * a.tm + a.mbase + i) * rec;
-#pragma unroll
-        for (int n = 0; n < NV; ++n) si[n] += L[n];
-        if (a.re)
-#pragma unroll
-            for (int n = 0; n < NV; ++n) sr[n] += L[NV + n];
+    const int rec = a.re ? 2 * NV : NV;
+    for (int k = p.ptr[v]; k < p.ptr[v + 1]; ++k) {
+        const int c = p.code[k], t = c >> 4, i = c & 15;
+        const double* L = a.lf + ((size_t)t * a.tm + p.mbase + i) * rec + n;
+        si += L[0];
+        if (a.re) sr += L[NV];
     }
-#pragma unroll
-    for (int n = 0; n < NV; ++n) {
-        RR[n] = sr[n];
-        R[n] = si[n] + sr[n];
-    }
+    p.rr[o] = sr;
+    p.res[o] = si + sr;
 }
 
 // setup_preconditioner element part (tet_hp/ins/setup_preconditioner.cpp:37-118)
@@ -1175,34 +1176,27 @@ struct TetMinvArgs {
     double cfa;
 };
 
+// one lane per (vertex, variable): 26 -> 16 us for 69 000 vertices against a lane per vertex
 __global__ __launch_bounds__(256) void k_minv_vrtx_tet(TetMinvArgs a) {
-    const int v = xcd_block() * blockDim.x + threadIdx.x;
+    const int lane = xcd_block() * blockDim.x + threadIdx.x, v = lane / TNV, n = lane - v * TNV;
     if (v >= a.npnt) return;
-    double r[TNV];
-    const bool vd = a.vess[v] != 0;
-#pragma unroll
-    for (int n = 0; n < TNV; ++n) r[n] = (a.pre_dirichlet && vd && n < 3) ? 0.0 : a.resv[v * TNV + n];
+    const bool vd = a.vess[v] != 0 && n < 3;
+    double r = (a.pre_dirichlet && vd) ? 0.0 : a.resv[lane];
     if (a.em > 0)
         for (int k = a.ve_ptr[v]; k < a.ve_ptr[v + 1]; ++k) {
             const int c = a.ve_code[k], e = c >> 1;
             const double sf = (c & 1) ? a.sfmv1 : a.sfmv0;
-            const bool ed = a.pre_dirichlet && a.eess[e];
-#pragma unroll
-            for (int n = 0; n < TNV; ++n) r[n] -= sf * ((ed && n < 3) ? 0.0 : a.rese[(e * a.em0) * TNV + n]);
+            const bool ed = a.pre_dirichlet && a.eess[e] && n < 3;
+            r -= sf * (ed ? 0.0 : a.rese[(e * a.em0) * TNV + n]);
         }
-    double x[TNV], u0[TNV];
-#pragma unroll
-    for (int n = 0; n < TNV; ++n) {
-        x[n] = (vd && n < 3) ? 0.0 : r[n] * (a.vprcn[v * TNV + n] * a.vdiag);
-        u0[n] = a.ugv ? a.ug0v[v * TNV + n] : 0.0;
-    }
-#pragma unroll
-    for (int n = 0; n < TNV; ++n) {
-        a.resv[v * TNV + n] = x[n];
-        if (a.ugv) a.ugv[v * TNV + n] = u0[n] - a.cfa * x[n];
-    }
+    const double x = vd ? 0.0 : r * (a.vprcn[lane] * a.vdiag);
+    const double u0 = a.ugv ? a.ug0v[lane] : 0.0;
+    a.resv[lane] = x;
+    if (a.ugv) a.ugv[lane] = u0 - a.cfa * x;
 }
 
+// one lane per edge and all its variables: the solved vertex values come as 32-byte loads (a
+// lane per (edge, variable) took 71 us against 58 for 465 000 edges)
 __global__ __launch_bounds__(256) void k_minv_edge_tet(TetMinvArgs a) {
     const int e = xcd_block() * blockDim.x + threadIdx.x;
     if (e >= a.nseg) return;

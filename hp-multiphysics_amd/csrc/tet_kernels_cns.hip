@@ -331,27 +331,26 @@ __global__ __launch_bounds__(256) void k_setup_tetc(TetcSetupArgs a) {
 }
 
 // per vertex / edge: prcn = 1 / sum of the incident jcb, pc = sum(tpc jcb) / sum(jcb),
-// incident elements ascending (setup_preconditioner.cpp:152-183, tet_hp/setup_preconditioner.cpp:455-476)
+// incident elements ascending (setup_preconditioner.cpp:152-183, tet_hp/setup_preconditioner.cpp:455-476).
+// One lane per (entity, block component): an element's 25 components are one contiguous load
+// of 25 lanes (one lane per entity strode 200 bytes: 65 -> 31 us a launch, 20 000 vertices
+// and 140 000 edges)
 __global__ __launch_bounds__(256) void k_setup_gather_tetc(int nent, const int* __restrict__ ptr,
                                                            const int* __restrict__ code, const double* __restrict__ iprcn,
                                                            const double* __restrict__ tpc, double* __restrict__ prcn,
                                                            double* __restrict__ pc) {
-    const int e = xcd_block() * blockDim.x + threadIdx.x;
+    const long lane = (long)xcd_block() * blockDim.x + threadIdx.x;
+    const int e = (int)(lane / 25), q = (int)(lane - 25L * e);
     if (e >= nent) return;
-    double sj = 0.0, s[25];
-#pragma unroll
-    for (int k = 0; k < 25; ++k) s[k] = 0.0;
+    double sj = 0.0, s = 0.0;
     for (int k = ptr[e]; k < ptr[e + 1]; ++k) {
         const int t = code[k] >> 4;
         const double j = iprcn[CNV * t];
         sj += j;
-#pragma unroll
-        for (int q = 0; q < 25; ++q) s[q] += tpc[25L * t + q] * j;
+        s += tpc[25L * t + q] * j;
     }
-#pragma unroll
-    for (int q = 0; q < 25; ++q) pc[25L * e + q] = s[q] / sj;
-#pragma unroll
-    for (int n = 0; n < CNV; ++n) prcn[CNV * e + n] = 1.0 / sj;
+    pc[25L * e + q] = s / sj;
+    if (q < CNV) prcn[CNV * e + q] = 1.0 / sj;
 }
 
 // T: arithmetic of the element kernel (double, or float in the FP32 inner solve of the
