@@ -56,7 +56,7 @@ MI355X_FP64_MFMA_TFLOPS = 78.6
 # of the reference x 2 + pointwise): full residual (beta > 0) and inviscid-only stage
 FLOP_FULL_P4 = 19250.0
 FLOP_INV_P4 = 7250.0
-# HBM bytes per launch of k_elem_ins_em<4, full> on this workload (one launch over all
+# HBM bytes per launch of k_elem_ins4_em<full> on this workload (one launch over all
 # 524 288 elements per full residual): FETCH_SIZE and WRITE_SIZE counter passes scaled by
 # the same counters over a plain 1 GiB copy; profiles/traffic_ins_p4_512x512_pmc.md
 TRAFFIC_FULL_P4_BYTES_PER_LAUNCH = 545.3e6
@@ -700,7 +700,7 @@ def main() -> int:
         "dof_evals_per_s_without_nv": value / 3,
         "roofline": {
             "bound": "mfma",
-            "kernel": "k_elem_ins_em<4,full>",
+            "kernel": "k_elem_ins4_em<full>",
             "achieved": achieved,
             "peak": MI355X_FP64_MFMA_TFLOPS,
             "unit": "TFLOP/s",
