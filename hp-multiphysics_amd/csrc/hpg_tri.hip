@@ -502,9 +502,13 @@ void launch_elem(hpg_ctx* c, const ElemArgs& a0, bool full) {
 template <int P, typename T>
 void launch_elem_em(hpg_ctx* c, const ElemArgsT<T>& a, const EdgeArgsT<T>& e, bool full) {
     const int nlogical = (a.end - a.begin + 63) / 64;
-    const int eblk = e.end > 0 ? (int)nblk8(e.end) : 0;
-    if (nlogical == 0 && eblk == 0) return;
     constexpr bool F64 = sizeof(T) == 8;
+    // edge blocks of the element launch; FP32 at p = 4: a launch before it
+    constexpr bool OWN = !F64 && P == 4;
+    const int eblk = !OWN && e.end > 0 ? (int)nblk8(e.end) : 0;
+    if constexpr (OWN)
+        if (e.end > 0) hipLaunchKernelGGL(k_edge_ins32_em<P>, dim3(nblk(e.end)), dim3(256), 0, c->stream, e, c->eout32);
+    if (nlogical == 0 && eblk == 0) return;
     const size_t r = c->recs.size();
     if (c->timing) check(hipEventRecord(c->event(2 * r), c->stream), "hipEventRecord");
     auto go = [&](auto kern, T* eres, T* eout, int cap) {

@@ -1121,14 +1121,23 @@ __global__ __launch_bounds__(256, 2) void k_elem_ins4_em(ElemArgs a, const doubl
 // FP32 (the inner solve of the defect correction): the same residual in single precision
 // on v_mfma_f32_16x16x4f32; its operator pack permutes the output rows of Ir/Is so that
 // register s of lane group q again holds mode 4s + q
+// At p = 4 the edges have a launch of their own (k_edge_ins32_em): with their body in the
+// kernel the full residual spills at its 256 registers (255 x 255: 70 -> 81 us, more than the
+// launch saved; the smaller kernels of p <= 2 do not).
 template <int P, bool FULL>
 __global__ __launch_bounds__(256, 2) void k_elem_ins32_em(ElemArgs32 a, float* eres, EdgeArgsT<float> e, float* eout,
                                                           int eblk) {
-    if ((int)blockIdx.x < eblk) {
-        edge_ins_body<P, float, true>(e, eout, blockIdx.x * 256 + threadIdx.x);
-        return;
-    }
+    if constexpr (P < 4)
+        if ((int)blockIdx.x < eblk) {
+            edge_ins_body<P, float, true>(e, eout, blockIdx.x * 256 + threadIdx.x);
+            return;
+        }
     elem_ins_body<float, P, FULL, true>(a, eres, eblk);
+}
+
+template <int P>
+__global__ __launch_bounds__(256) void k_edge_ins32_em(EdgeArgsT<float> e, float* eout) {
+    edge_ins_body<P, float, true>(e, eout, blockIdx.x * 256 + threadIdx.x);
 }
 
 // Element Jacobians of a batch: every (element, column) pair is an entry of one launch,
