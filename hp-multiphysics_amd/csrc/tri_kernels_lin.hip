@@ -424,7 +424,7 @@ constexpr int RED_BLOCKS = 2048;
 
 // The elementwise kernels of the solvers run over up to three arrays (vertex, side, interior
 // parts) as one index range, one launch each (an FP32 defect correction update had 30 of them,
-// one per array; with the merged passes and the guarded maximum below: 2 108 -> 1 880 us an
+// one per array; with the merged passes and the guarded maximum below: 1 054 -> 940 us an
 // update at 255 x 255, p = 4).
 struct Span3 {
     long end[3];  // running lengths
