@@ -37,8 +37,8 @@ struct Slot {
     hipStream_t stream = nullptr;
     void wait() {
         if (!pending) return;
-        pending = false;
         hip(hipEventSynchronize(ev[0]), "staging wait");
+        pending = false;
     }
     ~Slot() {
         if (pending) (void)hipEventSynchronize(ev[0]);
@@ -89,6 +89,12 @@ std::unique_ptr<Slot> take() {
 struct Held {
     std::unique_ptr<Slot> s;
     Held() : s(take()) {}
+    // a copy failed with work of this slot perhaps still queued on the stream: wait for it,
+    // or, where that fails too, keep the slot out of the pool (it stays counted there, so
+    // no more than POOL_SLOTS are ever lost)
+    void settle(hipStream_t st) {
+        if (hipStreamSynchronize(st) != hipSuccess) (void)s.release();
+    }
     ~Held() {
         if (!s) return;
         Pool& q = pool();
@@ -205,10 +211,7 @@ void large(hipStream_t st, const HostSeg* seg, int n, Slot& s, size_t total) {
     work(0);
     for (int j = started; j < nt; ++j) work(j);
     for (std::thread& t : th) t.join();
-    if (failed) {
-        (void)hipStreamSynchronize(st);  // nothing may still use the slot
-        hip((hipError_t)failed.load(), "D2H");
-    }
+    hip((hipError_t)failed.load(), "D2H");
 }
 
 void exchange(hipStream_t st, const HostSeg* seg, int n, bool to_dev) {
@@ -226,9 +229,17 @@ void exchange(hipStream_t st, const HostSeg* seg, int n, bool to_dev) {
         return;
     }
     Held h;
-    if (!h.s) direct(st, seg, n, to_dev);
-    else if (total <= SMALL) small(st, seg, n, to_dev, *h.s);
-    else large(st, seg, n, *h.s, total);
+    if (!h.s) {
+        direct(st, seg, n, to_dev);
+        return;
+    }
+    try {
+        if (total <= SMALL) small(st, seg, n, to_dev, *h.s);
+        else large(st, seg, n, *h.s, total);
+    } catch (...) {
+        h.settle(st);
+        throw;
+    }
 }
 
 }  // namespace
