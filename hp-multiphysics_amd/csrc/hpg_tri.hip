@@ -1621,6 +1621,9 @@ static int copy3(hpg_ctx* c, bool h2d, double* dv, double* ds, double* di, const
                                 {const_cast<double*>(i), di, (size_t)c->ntri * c->im0 * c->nv * 8}};
         if (h2d) copy_to_device(c->stream, seg, 3);
         else copy_to_host(c->stream, seg, 3);
+        // a level of a multigrid stack: its neighbours' streams read and write these arrays
+        // (mg_prolongate, a replayed cycle) and do not wait for this stream's uploads
+        if (h2d && c->xev) check(hipStreamSynchronize(c->stream), "sync");
     });
     return 0;
 }
@@ -2041,7 +2044,9 @@ int hpg_link_fine(hpg_ctx* c, hpg_ctx* f, const int* cc_tri, const double* cc_wt
         c->vug_frst = c->alloc<double>((size_t)nc * c->nv);
         if (!c->xev) check(hipEventCreateWithFlags(&c->xev, hipEventDisableTiming), "hipEventCreate");
         if (!f->xev) check(hipEventCreateWithFlags(&f->xev, hipEventDisableTiming), "hipEventCreate");
+        // uploads from before the two were neighbours
         check(hipStreamSynchronize(c->stream), "sync");
+        check(hipStreamSynchronize(f->stream), "sync");
         c->fine = f;
         c->coarse_level = true;
     });
@@ -2207,6 +2212,12 @@ int hpg_mg_cycle(hpg_ctx* const* grids, int ngrid, int extra_finest_levels, int 
         CycleRun r{grids, ngrid, extra_finest_levels, ngrid + extra_finest_levels, vw, itercrsn, iterrfne};
         bool use_graph = f->graphs;
         for (int k = 0; k < ngrid; ++k) use_graph = use_graph && !grids[k]->timing;
+        // a replay runs every grid's kernels on f's stream: after what the coarse contexts'
+        // own streams still hold
+        for (int k = 1; k < ngrid; ++k) {
+            check(hipEventRecord(grids[k]->xev, grids[k]->stream), "hipEventRecord");
+            check(hipStreamWaitEvent(f->stream, grids[k]->xev, 0), "hipStreamWaitEvent");
+        }
         const std::vector<unsigned long long> sg =
             use_graph ? cycle_signature(grids, ngrid, extra_finest_levels, vw, itercrsn, iterrfne)
                       : std::vector<unsigned long long>();

@@ -72,7 +72,11 @@ typedef struct {
 int hpg_create(const hpg_tri_mesh *mesh, const hpg_params *prm, hpg_ctx **out);
 int hpg_destroy(hpg_ctx *ctx);
 
-/* state exchange with the host-owned ug arrays (tri_hp::ug, tri_hp/tri_hp.h:71-75) */
+/* state exchange with the host-owned ug arrays (tri_hp::ug, tri_hp/tri_hp.h:71-75).  The
+ * arrays handed to a set call (state, residual; tet forms too) may be reused on return; the
+ * device copy of a small one may still be queued on the context's stream, before everything
+ * that the context does afterwards.  On a context that is linked into a multigrid stack
+ * (hpg_link_fine) a set call returns after the device copy. */
 int hpg_set_state(hpg_ctx *ctx, const double *ugv, const double *ugs, const double *ugi);
 int hpg_get_state(hpg_ctx *ctx, double *ugv, double *ugs, double *ugi);
 /* residual exchange (tri_hp::hp_global::res, tri_hp/tri_hp.h:118-121) */
