@@ -151,6 +151,7 @@ struct hpg_tet_ctx {
     double *vprcn = nullptr, *eprcn = nullptr, *iprcn = nullptr, *tau = nullptr, *lf = nullptr, *flf = nullptr;
     double *tpc = nullptr, *vpc = nullptr, *epc = nullptr;  // cns: 5 x 5 blocks per element / vertex / edge
     int* d_err = nullptr;
+    bool err_open = false;  // as for tri contexts
     unsigned long long* d_max = nullptr;
     TetLevel lv[2];
     // FP32 defect correction (hpg_tet_set_precision): device scale scalars and maxima,
@@ -461,15 +462,8 @@ void launch_setup_tetc(hpg_tet_ctx* c) {
     hipLaunchKernelGGL(k_setup_tetc<P>, dim3(nblk8(c->ntet)), dim3(256), 0, c->stream, a);
 }
 
-int read_error(hpg_tet_ctx* c) {  // as for tri contexts
-    int herr = 0;
-    const HostSeg seg{&herr, c->d_err, sizeof(int)};
-    copy_to_host(c->stream, &seg, 1);
-    if (herr) hipLaunchKernelGGL(k_clear_u32, dim3(1), dim3(64), 0, c->stream, 1, (unsigned*)c->d_err);
-    return herr;
-}
-
 int do_setup_tetc(hpg_tet_ctx* c) {
+    open_error(c);
     if (c->lv[c->log2p].p == 1) launch_setup_tetc<1>(c); else launch_setup_tetc<2>(c);
     hipLaunchKernelGGL(k_setup_gather_tetc, dim3(nblk8(25L * c->npnt)), dim3(256), 0, c->stream, c->npnt, c->vt_ptr,
                        c->vt_code, c->iprcn, c->tpc, c->vprcn, c->vpc);
@@ -482,6 +476,7 @@ int do_setup_tetc(hpg_tet_ctx* c) {
 
 int do_setup_tet(hpg_tet_ctx* c) {
     if (c->cns()) return do_setup_tetc(c);
+    open_error(c);
     TetSetupArgs a;
     a.pnts = c->pnts; a.tet_pnt = c->tet_pnt; a.ugv = c->ugv; a.ntet = c->ntet; a.p = c->lv[c->log2p].p;
     a.rho = c->prm.rho; a.mu = c->prm.mu; a.adis = c->prm.adis; a.iprcn = c->iprcn; a.tau = c->tau; a.err = c->d_err;

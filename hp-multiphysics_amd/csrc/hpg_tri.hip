@@ -304,6 +304,7 @@ struct hpg_ctx {
     double *dresv[3], *dress[3], *dresi[3];
     double *vprcn, *sprcn, *tprcn;
     int* d_err;
+    bool err_open = false;  // kernels that may set d_err were enqueued since it was last read
     // mixed precision: per-colour group offsets, linearisation data, FP32 inner arrays
     std::vector<int> gbase;
     int ngroups = 0;
@@ -1062,19 +1063,38 @@ void do_rsdl_cns32(hpg_ctx* c, int stage) {
     check(hipGetLastError(), "cns rsdl32 launch");
 }
 
-// the error flag of the kernels enqueued so far (waits for them).  The flag is zero between
-// calls: whoever reads it set clears it
-int read_error(hpg_ctx* c) {
+// The error flag of a context is zero outside a setup (or cycle): whoever reads it set clears
+// it, and waits for that, so that no later work on another stream (a replayed cycle) meets
+// the clear; a setup that ended before the flag was read leaves err_open, and the next one
+// clears first.
+template <class Ctx>
+void clear_error(Ctx* c) {
+    hipLaunchKernelGGL(k_clear_u32, dim3(1), dim3(64), 0, c->stream, 1, (unsigned*)c->d_err);
+}
+template <class Ctx>
+void open_error(Ctx* c) {
+    if (c->err_open) clear_error(c);
+    c->err_open = true;
+}
+// the flag of the kernels enqueued so far (waits for them)
+template <class Ctx>
+int read_error(Ctx* c) {
     int herr = 0;
     const HostSeg seg{&herr, c->d_err, sizeof(int)};
     copy_to_host(c->stream, &seg, 1);
-    if (herr) hipLaunchKernelGGL(k_clear_u32, dim3(1), dim3(64), 0, c->stream, 1, (unsigned*)c->d_err);
+    if (herr) {
+        clear_error(c);
+        check(hipGetLastError(), "clear launch");
+        check(hipStreamSynchronize(c->stream), "sync");
+    }
+    c->err_open = false;
     return herr;
 }
 
 // sync = false (the fused multigrid cycle): the error flag accumulates on the device and
 // is read once after the cycle; nothing waits for the device here
 int do_setup_cns(hpg_ctx* c, bool sync = true) {
+    if (sync) open_error(c);
     const Level& L = c->lv[c->log2p];
     const LevelDims d(L.p);
     CnsSetupArgs s;
@@ -1178,6 +1198,7 @@ void mixed_update_cns(hpg_ctx* c) {
 
 int do_setup(hpg_ctx* c, bool sync = true) {
     if (c->physics == HPG_PHYSICS_CNS) return do_setup_cns(c, sync);
+    if (sync) open_error(c);
     const Level& L = c->lv[c->log2p];
     const LevelDims d(L.p);
     SetupArgs s{};
@@ -2208,7 +2229,10 @@ int hpg_mg_cycle(hpg_ctx* const* grids, int ngrid, int extra_finest_levels, int 
     HPG_TRY(f, {
         FlagList fl{};
         fl.n = ngrid;
-        for (int k = 0; k < ngrid; ++k) fl.p[k] = (unsigned*)grids[k]->d_err;
+        for (int k = 0; k < ngrid; ++k) {
+            fl.p[k] = (unsigned*)grids[k]->d_err;
+            grids[k]->err_open = true;  // the cycle clears them (k_clear_flags)
+        }
         CycleRun r{grids, ngrid, extra_finest_levels, ngrid + extra_finest_levels, vw, itercrsn, iterrfne};
         bool use_graph = f->graphs;
         for (int k = 0; k < ngrid; ++k) use_graph = use_graph && !grids[k]->timing;

@@ -54,3 +54,53 @@ def test_upload_to_a_coarse_mesh_before_a_replayed_cycle(oracle_mod):
         assert ea == eb
         for x, y in zip(ga[0].get_state(), gb[0].get_state()):
             assert np.array_equal(x, y)
+
+
+def test_error_flags_of_failed_and_good_cycles(oracle_mod):
+    """A cycle on a state without a valid pseudo-time step reports it, enqueued and replayed,
+    as often as it happens and never afterwards."""
+    _case("cycles on good and NaN states, ins 16x16 p=4, 3 grids, graph replay")
+    from hpmp import multigrid as MG
+    _, g, _ = _stacks(oracle_mod, "ins", 16, 2, 3)
+    good = g[0].get_state()
+    nan = [x.copy() for x in good]
+    nan[0][::7] = np.nan
+    want = None
+    for k, st in enumerate((good, nan, nan, good, nan, good, good)):
+        g[0].set_state(*st)
+        if st is nan:
+            with pytest.raises(FloatingPointError, match="setup_preconditioner"):
+                MG.cycle(g, 2, 2, 2, 2, fused=True)
+            continue
+        e = MG.cycle(g, 2, 2, 2, 2, fused=True)
+        assert want is None or e == want
+        want = e
+    for x in g:
+        assert x.setup_preconditioner() == 0
+
+
+def _failing_call(lib, call):
+    """``call`` with an error of an unrelated HIP call pending in this thread: its kernels are
+    enqueued, then it reports that error."""
+    from hpmp import _lib
+    assert lib.hipSetDevice(1 << 20) != 0
+    with pytest.raises(_lib.HpgError):
+        call()
+    lib.hipGetLastError()
+
+
+def test_flag_of_a_setup_that_was_not_read_is_dropped(oracle_mod):
+    _case("setup and cycle that end before their error flag is read")
+    import test_gpu_tet_cns as C
+    from hpmp import multigrid as MG
+    _, g, _ = _stacks(oracle_mod, "ins", 8, 1, 2)
+    good = g[0].get_state()
+    g[0].set_state(np.full_like(good[0], np.nan), *good[1:])
+    _failing_call(g[0].L, lambda: MG.cycle(g, 1, fused=True))
+    g[0].set_state(*good)
+    assert g[0].setup_preconditioner() == 0
+    _, st, G, _ = C._pair(2, 1)
+    G.set_state(np.full_like(st[0], np.nan), st[1])
+    _failing_call(G.L, G.setup_preconditioner)
+    G.set_state(*st)
+    assert G.setup_preconditioner() == 0
