@@ -200,6 +200,7 @@ constexpr int WTILE = 2 * MH * TS + 2 * 16 * TS;                        // h, dz
 constexpr int TRAIN_LDS = LWAVE + 4 * WTILE;
 static_assert(NPARAM <= LWAVE, "the block's gradient sums reuse the weights' LDS");
 static_assert(TRAIN_LDS * 4 <= 160 * 1024, "LDS of one CU");
+static_assert(LWAVE % 2 == 0, "the block's loss is a double there");
 
 // gelu(z) as bfloat16 bits (the B operands of the next layer) and gelu'(z) in place of z
 __device__ inline void gelu_and_slope(f32x4_t z[4], bf16x4_t h[4]) {
@@ -224,7 +225,7 @@ __device__ inline void wave_lds_sync() {
 
 __global__ __launch_bounds__(256) void k_mlp_train_mfma(int n, int nscale, const float* __restrict__ X,
                                                         const float* __restrict__ T, const float* __restrict__ wq,
-                                                        float* __restrict__ partial, float* __restrict__ lossp) {
+                                                        float* __restrict__ partial, double* __restrict__ lossp) {
     __shared__ __align__(16) float sm[TRAIN_LDS];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, q = lane >> 4, c = lane & 15;
     for (int k = threadIdx.x; k < MH * MH; k += 256) {
@@ -265,7 +266,8 @@ __global__ __launch_bounds__(256) void k_mlp_train_mfma(int n, int nscale, const
     float* const sy = sx + 16 * TS;             // output deltas, rows 9.. zero
     const f4_t z0 = {0.f, 0.f, 0.f, 0.f};
     f4_t g2[4][4], g3[4][4], g1[4], g4[4];
-    float gb1[4], gb2[4], gb3[4], gb4 = 0.f, loss = 0.f;
+    float gb1[4], gb2[4], gb3[4], gb4 = 0.f;
+    double loss = 0.0;  // of any number of samples: FP32 would lose a large minibatch's digits
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
         g1[a] = z0; g4[a] = z0; gb1[a] = gb2[a] = gb3[a] = 0.f;
@@ -369,7 +371,7 @@ __global__ __launch_bounds__(256) void k_mlp_train_mfma(int n, int nscale, const
         for (int i = 0; i < 4; ++i) {
             const int o = 4 * q + i;
             const float d = (ok && o < MO) ? y[i] - T[(size_t)s * MO + o] : 0.f;
-            loss += d * d;
+            loss += (double)(d * d);
             dy[i] = 2.f * d / (float)nscale;
             sy[o * TS + c] = dy[i];
         }
@@ -433,6 +435,7 @@ __global__ __launch_bounds__(256) void k_mlp_train_mfma(int n, int nscale, const
     for (int a = 0; a < 4; ++a) { gb1[a] = quarter(gb1[a]); gb2[a] = quarter(gb2[a]); gb3[a] = quarter(gb3[a]); }
     gb4 = quarter(gb4);
     for (int off = 32; off > 0; off >>= 1) loss += __shfl_down(loss, off, 64);
+    double* const lsum = reinterpret_cast<double*>(sm + LWAVE);
     for (int turn = 0; turn < 4; ++turn) {
         __syncthreads();
         if (turn != w) continue;
@@ -457,12 +460,12 @@ __global__ __launch_bounds__(256) void k_mlp_train_mfma(int n, int nscale, const
             }
         }
         if (q == 0 && c < MO) add(O_B4 + c, gb4);
-        if (lane == 0) sm[LWAVE] = w == 0 ? loss : sm[LWAVE] + loss;
+        if (lane == 0) *lsum = w == 0 ? loss : *lsum + loss;
     }
     __syncthreads();
     float* const P = partial + (size_t)blockIdx.x * NPARAM;
     for (int p = threadIdx.x; p < NPARAM; p += 256) P[p] = sm[p];
-    if (threadIdx.x == 0) lossp[blockIdx.x] = sm[LWAVE];
+    if (threadIdx.x == 0) lossp[blockIdx.x] = *lsum;
 }
 
 // gradient = sum of the block partials in a fixed order (four lanes a quarter of the
@@ -473,7 +476,7 @@ __global__ __launch_bounds__(256) void k_mlp_train_mfma(int n, int nscale, const
 __global__ __launch_bounds__(256) void k_mlp_reduce_adam(int nblocks, const float* __restrict__ partial,
                                                          float* __restrict__ grad, float* master, float* wq,
                                                          float* m1, float* m2, float lr, float bc1, float bc2,
-                                                         int do_step, const float* __restrict__ lossp, double* lsum) {
+                                                         int do_step, const double* __restrict__ lossp, double* lsum) {
     __shared__ float part[4][64];
     const int j = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int p = blockIdx.x * 64 + j;
@@ -506,7 +509,7 @@ __global__ __launch_bounds__(256) void k_mlp_reduce_adam(int nblocks, const floa
 
 // mean-square loss from the block losses: the same double sum, in block order, and
 // the same final division as the host side of hpg_mlp_loss_grad
-__global__ void k_mlp_loss_sum(int nblocks, const float* __restrict__ lossp, int nscale, float* __restrict__ loss) {
+__global__ void k_mlp_loss_sum(int nblocks, const double* __restrict__ lossp, int nscale, float* __restrict__ loss) {
     if (blockIdx.x != 0 || threadIdx.x != 0) return;
     double s = 0.0;
     for (int b = 0; b < nblocks; ++b) s += lossp[b];
@@ -515,7 +518,7 @@ __global__ void k_mlp_loss_sum(int nblocks, const float* __restrict__ lossp, int
 
 // Scratch of the allocation-free loss/gradient entry point: the per-block partial
 // gradients (NPARAM floats per block of k_mlp_train_mfma, room for one block per 64
-// samples) followed by the block losses.  One
+// samples) followed by the block losses (doubles, from the next even word).  One
 // copy per GPU, held until the process ends; host code uses the address that
 // hipGetSymbolAddress returns for the current device, never the symbol itself.
 // Every call overwrites what it reads (each block writes all of its partials and
@@ -523,6 +526,7 @@ __global__ void k_mlp_loss_sum(int nblocks, const float* __restrict__ lossp, int
 constexpr int NOALLOC_FLOATS = 4 << 20;  // 16 MiB
 constexpr int NOALLOC_MAX_BLOCKS = NOALLOC_FLOATS / (NPARAM + 1);
 static __device__ __align__(256) float scratch[NOALLOC_FLOATS];
+static_assert((TRAIN_BLOCKS * NPARAM + 1) / 2 * 2 + 2 * TRAIN_BLOCKS <= NOALLOC_FLOATS, "partials and losses of a minibatch");
 static_assert(NOALLOC_MAX_BLOCKS * 64 == HPG_MLP_NOALLOC_MAX_SAMPLES, "header limit out of step with the scratch size");
 
 }  // namespace hpg
@@ -533,15 +537,17 @@ struct hpg_mlp {
     hipStream_t stream = nullptr;
     HostCopyUser staging;
     float *master = nullptr, *wq = nullptr, *m1 = nullptr, *m2 = nullptr, *grad = nullptr;
-    float *partial = nullptr, *lossp = nullptr, *X = nullptr, *T = nullptr, *Y = nullptr;
+    float *partial = nullptr, *X = nullptr, *T = nullptr, *Y = nullptr;
+    double* lossp = nullptr;  // a minibatch's block losses
     double* lsum = nullptr;  // loss sum of a training run's last epoch
     int cap_blocks = 0, cap_n = 0, step = 0;
     int dev = 0;  // device the MLP was created on
     std::string err;
     ~hpg_mlp() {
-        for (float* p : {master, wq, m1, m2, grad, partial, lossp, X, T, Y})
+        for (float* p : {master, wq, m1, m2, grad, partial, X, T, Y})
             if (p) hipFree(p);
-        if (lsum) hipFree(lsum);
+        for (double* p : {lossp, lsum})
+            if (p) hipFree(p);
         if (stream) hipStreamDestroy(stream);
     }
 };
@@ -597,12 +603,12 @@ int train_blocks(int n) { return std::max(1, std::min((n + 63) / 64, TRAIN_BLOCK
 
 // enqueue the backward pass of n samples (block partials and block losses into
 // partial / lossp) and the ordered gradient sum into grad, no weight update
-void enqueue_loss_grad(hpg_mlp* m, const float* X, const float* T, int n, float* partial, float* lossp,
+void enqueue_loss_grad(hpg_mlp* m, const float* X, const float* T, int n, float* partial, double* lossp,
                        float* grad) {
     const int nb = train_blocks(n);
     hipLaunchKernelGGL(k_mlp_train_mfma, dim3(nb), dim3(256), 0, m->stream, n, n * MO, X, T, m->wq, partial, lossp);
     hipLaunchKernelGGL(k_mlp_reduce_adam, dim3((NPARAM + 63) / 64), dim3(256), 0, m->stream, nb, partial, grad,
-                       m->master, m->wq, m->m1, m->m2, 0.f, 1.f, 1.f, 0, (const float*)nullptr, (double*)nullptr);
+                       m->master, m->wq, m->m1, m->m2, 0.f, 1.f, 1.f, 0, (const double*)nullptr, (double*)nullptr);
 }
 
 void ensure_blocks(hpg_mlp* m, int nb) {
@@ -610,7 +616,7 @@ void ensure_blocks(hpg_mlp* m, int nb) {
     if (m->partial) hipFree(m->partial);
     if (m->lossp) hipFree(m->lossp);
     ck(hipMalloc(&m->partial, (size_t)nb * NPARAM * 4), "hipMalloc");
-    ck(hipMalloc(&m->lossp, (size_t)nb * 4), "hipMalloc");
+    ck(hipMalloc(&m->lossp, (size_t)nb * 8), "hipMalloc");
     m->cap_blocks = nb;
 }
 }  // namespace
@@ -723,12 +729,12 @@ int hpg_mlp_loss_grad(hpg_mlp* m, const float* X, const float* T, int n, float* 
         ensure_blocks(m, nb);
         send_batch(m, X, T, n);
         enqueue_loss_grad(m, m->X, m->T, n, m->partial, m->lossp, m->grad);
-        std::vector<float> lp(nb);
-        ck(hipMemcpyAsync(lp.data(), m->lossp, nb * 4, hipMemcpyDeviceToHost, m->stream), "D2H");
+        std::vector<double> lp(nb);
+        ck(hipMemcpyAsync(lp.data(), m->lossp, nb * 8, hipMemcpyDeviceToHost, m->stream), "D2H");
         if (grad) ck(hipMemcpyAsync(grad, m->grad, NPARAM * 4, hipMemcpyDeviceToHost, m->stream), "D2H");
         ck(hipStreamSynchronize(m->stream), "sync");
         double s = 0.0;
-        for (float v : lp) s += v;
+        for (double v : lp) s += v;
         if (loss) *loss = (float)(s / ((double)n * MO));
     } catch (const std::exception& e) { m->err = e.what(); return -1; }
     return 0;
@@ -749,7 +755,7 @@ int hpg_mlp_loss_grad_noalloc(hpg_mlp* m, const float* X, const float* T, int n,
         float* sp = (m->dev >= 0 && m->dev < MAX_DEVICES) ? g_scratch[m->dev] : nullptr;
         if (!sp) throw std::runtime_error("scratch address not resolved for this device");
         const int nb = train_blocks(n);
-        float* lossp = sp + (size_t)nb * NPARAM;
+        double* lossp = reinterpret_cast<double*>(sp + ((size_t)nb * NPARAM + 1) / 2 * 2);
         enqueue_loss_grad(m, X, T, n, sp, lossp, grad);
         hipLaunchKernelGGL(k_mlp_loss_sum, dim3(1), dim3(64), 0, m->stream, nb, lossp, n * MO, loss);
         ck(hipGetLastError(), "loss_grad_noalloc launch");

@@ -41,3 +41,19 @@ def test_epoch_loss_is_the_sample_mean_over_ragged_minibatches():
     assert np.array_equal(net.weights(), w)
     # 128 + 72 samples with a zero step: the epoch loss is the sample mean
     assert abs(net.train(X, T, epochs=2, batch=128, lr=0.0) - lo) <= 2.0 ** -8 * abs(lo)
+
+
+@pytest.mark.parametrize("n", [1 << 18, (1 << 20) + 5])
+def test_loss_of_a_large_minibatch_keeps_its_digits(n):
+    """A network of zeros against one target value: every squared difference is the same
+    FP32 number v, and the mean of n x 9 of them (at most 24 + 24 bits in the sum) is v."""
+    print(f"mlp loss n={n}", flush=True)
+    from hpmp.learned import MLP
+    X = np.random.default_rng(1).standard_normal((n, 11)).astype(np.float32)
+    T = np.full((n, 9), 0.123, np.float32)
+    net = MLP(1)
+    net.set_weights(np.zeros_like(net.weights()))
+    v = float(np.float32(0.123) * np.float32(0.123))
+    loss, _ = net.loss_grad(X, T)
+    assert loss == v
+    assert net.train(X, T, epochs=1, batch=n, lr=0.0) == v
