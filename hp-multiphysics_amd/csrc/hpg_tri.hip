@@ -2213,6 +2213,16 @@ __global__ void k_clear_flags(FlagList f) {
 }
 }  // namespace
 
+// 1 when hpg_mg_cycle runs in this process: the HIP runtime that the library is bound to is
+// at least the release it was compiled for.  A process that loads a package with an older
+// runtime of its own first binds the library to that one; a W cycle of 256 x 256 squares on
+// 5 meshes ended there (7.0 under 7.2) in a segmentation fault on the host whose cause is
+// not known, so the whole-cycle call is refused; the call-by-call cycle runs there.
+int hpg_cycle_available(void) {
+    int v = 0;
+    return hipRuntimeGetVersion(&v) == hipSuccess && v / 100000 >= HIP_VERSION / 100000;  // major, minor
+}
+
 // block::cycle over a stack of grids, enqueued without host round trips inside the cycle.
 // The second call with the same settings captures the cycle into a HIP graph (the
 // coarse contexts' streams join through the restriction and prolongation events);
@@ -2225,6 +2235,11 @@ int hpg_mg_cycle(hpg_ctx* const* grids, int ngrid, int extra_finest_levels, int 
     hpg_ctx* f = grids[0];
     if (f->log2p != f->log2pmax || extra_finest_levels > f->log2pmax) { f->err = "cycle starts on the finest p-level"; return -2; }
     if (ngrid > 16) { f->err = "at most 16 meshes in a cycle"; return -2; }
+    if (!hpg_cycle_available()) {
+        f->err = "the whole-cycle call needs the HIP runtime that the library was built for; another package's older one "
+                 "was loaded first";
+        return -2;
+    }
     int nerr = 0;
     HPG_TRY(f, {
         FlagList fl{};

@@ -35,7 +35,7 @@ EXPORTS = (
     "hpg_mlp_get_weights", "hpg_mlp_set_weights", "hpg_mlp_forward", "hpg_mlp_loss_grad", "hpg_mlp_train",
     "hpg_mlp_loss_grad_noalloc",
     "hpg_set_mlp", "hpg_set_prcn_log_scalings", "hpg_mlp_features", "hpg_measure_jacobian_diag", "hpg_selftest_copy",
-    "hpg_get_block_preconditioner", "hpg_link_fine", "hpg_mg_cycle",
+    "hpg_get_block_preconditioner", "hpg_link_fine", "hpg_mg_cycle", "hpg_cycle_available",
     "hpg_tet_create", "hpg_tet_destroy", "hpg_tet_set_state", "hpg_tet_get_state", "hpg_tet_get_residual",
     "hpg_tet_set_residual", "hpg_tet_get_preconditioner", "hpg_tet_get_cns_blocks", "hpg_tet_rsdl", "hpg_tet_setup_preconditioner",
     "hpg_tet_minvrt", "hpg_tet_update", "hpg_tet_maxres", "hpg_tet_resnorm", "hpg_tet_mg_restrict",
@@ -98,6 +98,7 @@ def load():
     L.hpg_get_block_preconditioner.argtypes = [vp, dp, dp, dp]
     L.hpg_link_fine.argtypes = [vp, vp, dp, dp, dp, dp]
     L.hpg_mg_cycle.argtypes = [C.POINTER(vp), C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_double)]
+    L.hpg_cycle_available.argtypes = []
     L.hpg_tet_create.argtypes = [vp, vp, vp]
     L.hpg_tet_destroy.argtypes = [vp]
     for nm in ("hpg_tet_set_state", "hpg_tet_get_state", "hpg_tet_get_residual", "hpg_tet_set_residual"):

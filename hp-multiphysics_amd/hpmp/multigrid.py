@@ -15,9 +15,12 @@ from . import mesh as M
 
 
 def fused_available(grids) -> bool:
-    """True when every grid is a GPU tri context (hpg_mg_cycle runs the whole cycle)."""
+    """True when every grid is a GPU tri context and hpg_mg_cycle runs in this process (it
+    does not on an older HIP runtime of another package, torch's for one, that was loaded
+    before the library)."""
+    from . import _lib
     from .tri_hp import TriHpIns
-    return all(isinstance(g, TriHpIns) for g in grids)
+    return all(isinstance(g, TriHpIns) for g in grids) and bool(_lib.load().hpg_cycle_available())
 
 
 def cycle(grids, extra_finest_levels: int, vw: int = 1, itercrsn: int = 1, iterrfne: int = 0,
@@ -29,14 +32,15 @@ def cycle(grids, extra_finest_levels: int, vw: int = 1, itercrsn: int = 1, iterr
     (``maxres`` on the entry level), like the reference; raises FloatingPointError on a
     preconditioner error or a residual that is NaN or exactly zero (``throw 1``).
 
-    On GPU contexts (``fused`` None or True) the whole cycle is one call of
+    On GPU contexts (``fused`` None or True; see fused_available) the whole cycle is one call of
     hpg_mg_cycle: the same kernels in the same order, with no host round trip inside the
     cycle, so setup_preconditioner errors are reported after the cycle rather than at
     the failing level.  ``fused=False`` runs the level recursion call by call."""
     if lvl == 0 and mglvls is None and evaluate_preconditioner and fused is not False and fused_available(grids):
         return grids[0].mg_cycle(grids, extra_finest_levels, vw, itercrsn, iterrfne)
     if fused:
-        raise ValueError("the fused cycle needs GPU tri contexts, the entry level and evaluate_preconditioner")
+        raise ValueError("the fused cycle needs GPU tri contexts, the HIP runtime that the library was built for, the "
+                         "entry level and evaluate_preconditioner")
     ngrid = len(grids)
     if mglvls is None:
         mglvls = ngrid + extra_finest_levels

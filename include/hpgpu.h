@@ -133,6 +133,11 @@ int hpg_link_fine(hpg_ctx *coarse, hpg_ctx *fine, const int *cc_tri, const doubl
  * with the same kernels and arguments as the enqueued form. */
 int hpg_mg_cycle(hpg_ctx *const *grids, int ngrid, int extra_finest_levels, int vw, int itercrsn, int iterrfne,
                  double *maxres);
+/* No reference counterpart: 1 when hpg_mg_cycle runs in this process, 0 when the process
+ * has bound the library to a HIP runtime older than the release it was compiled for (a
+ * package that brings its own runtime was loaded first); hpg_mg_cycle then returns -2, and
+ * the cycle is driven call by call. */
+int hpg_cycle_available(void);
 /* No reference counterpart: enable (default) or disable the graph capture of
  * hpg_mg_cycle on this fine context (disabled: every cycle is enqueued call by call). */
 int hpg_set_cycle_graph(hpg_ctx *ctx, int enable);
