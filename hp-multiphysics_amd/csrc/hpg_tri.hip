@@ -497,6 +497,12 @@ void launch_elem(hpg_ctx* c, const ElemArgs& a0, bool full) {
     }
 }
 
+// FP32 at p = 4 (k_elem_ins32_em): the boundary edges as a launch of their own from this many
+// elements.  us per mixed update with blocks of the element launch / with a launch of its
+// own: 4 x 4 177 / 191, 64 x 64 250 / 267, 128 x 128 368 / 389, 208 x 208 593 / 614,
+// 224 x 224 (100 352 elements) 679 / 678, 255 x 255 800 / 787, 512 x 512 2 993 / 2 866
+constexpr int OWN_EDGES = 100000;
+
 // element-major residual over a.order[begin:end) (null order: mesh order) and the
 // boundary-edge fluxes e in one persistent launch (timing records 1 / 0 like the colour
 // launches, 3 / 2 in FP32)
@@ -504,11 +510,11 @@ template <int P, typename T>
 void launch_elem_em(hpg_ctx* c, const ElemArgsT<T>& a, const EdgeArgsT<T>& e, bool full) {
     const int nlogical = (a.end - a.begin + 63) / 64;
     constexpr bool F64 = sizeof(T) == 8;
-    // edge blocks of the element launch; FP32 at p = 4: a launch before it
-    constexpr bool OWN = !F64 && P == 4;
-    const int eblk = !OWN && e.end > 0 ? (int)nblk8(e.end) : 0;
-    if constexpr (OWN)
-        if (e.end > 0) hipLaunchKernelGGL(k_edge_ins32_em<P>, dim3(nblk(e.end)), dim3(256), 0, c->stream, e, c->eout32);
+    // edge blocks of the element launch, or a launch before it
+    const bool own = !F64 && P == 4 && a.end - a.begin >= OWN_EDGES;
+    const int eblk = !own && e.end > 0 ? (int)nblk8(e.end) : 0;
+    if constexpr (!F64 && P == 4)
+        if (own && e.end > 0) hipLaunchKernelGGL(k_edge_ins32_em<P>, dim3(nblk(e.end)), dim3(256), 0, c->stream, e, c->eout32);
     if (nlogical == 0 && eblk == 0) return;
     const size_t r = c->recs.size();
     if (c->timing) check(hipEventRecord(c->event(2 * r), c->stream), "hipEventRecord");
@@ -531,10 +537,16 @@ void launch_elem_em(hpg_ctx* c, const ElemArgsT<T>& a, const EdgeArgsT<T>& e, bo
         if (full) go(k_elem_ins_em<P, true>, c->eres, c->eout, cf);
         else go(k_elem_ins_em<P, false>, c->eres, c->eout, ci);
     } else {
-        static const int cf = resident_blocks((const void*)k_elem_ins32_em<P, true>);
-        static const int ci = resident_blocks((const void*)k_elem_ins32_em<P, false>);
-        if (full) go(k_elem_ins32_em<P, true>, c->eres32, c->eout32, cf);
-        else go(k_elem_ins32_em<P, false>, c->eres32, c->eout32, ci);
+        auto form = [&](auto edges) {
+            constexpr bool E = decltype(edges)::value;
+            static const int cf = resident_blocks((const void*)k_elem_ins32_em<P, true, E>);
+            static const int ci = resident_blocks((const void*)k_elem_ins32_em<P, false, E>);
+            if (full) go(k_elem_ins32_em<P, true, E>, c->eres32, c->eout32, cf);
+            else go(k_elem_ins32_em<P, false, E>, c->eres32, c->eout32, ci);
+        };
+        if constexpr (P == 4)
+            if (own) form(std::false_type{});
+        if (!own) form(std::true_type{});
     }
     if (c->timing) {
         check(hipEventRecord(c->event(2 * r + 1), c->stream), "hipEventRecord");

@@ -1121,13 +1121,14 @@ __global__ __launch_bounds__(256, 2) void k_elem_ins4_em(ElemArgs a, const doubl
 // FP32 (the inner solve of the defect correction): the same residual in single precision
 // on v_mfma_f32_16x16x4f32; its operator pack permutes the output rows of Ir/Is so that
 // register s of lane group q again holds mode 4s + q
-// At p = 4 the edges have a launch of their own (k_edge_ins32_em): with their body in the
-// kernel the full residual spills at its 256 registers (255 x 255: 70 -> 81 us, more than the
-// launch saved; the smaller kernels of p <= 2 do not).
-template <int P, bool FULL>
+// EDGES: the first eblk blocks are the boundary edges, as in k_elem_ins_em.  At p = 4 their
+// body costs registers (104 bytes a lane in scratch against 44 in the full residual, 174
+// registers against 124 in the inviscid one; 255 x 255: 70 -> 81 us and 30 -> 36 us); launches
+// without it take the edges from k_edge_ins32_em (OWN_EDGES says when).
+template <int P, bool FULL, bool EDGES>
 __global__ __launch_bounds__(256, 2) void k_elem_ins32_em(ElemArgs32 a, float* eres, EdgeArgsT<float> e, float* eout,
                                                           int eblk) {
-    if constexpr (P < 4)
+    if constexpr (EDGES)
         if ((int)blockIdx.x < eblk) {
             edge_ins_body<P, float, true>(e, eout, blockIdx.x * 256 + threadIdx.x);
             return;

@@ -50,3 +50,23 @@ def test_side_listed_twice_counts_twice():
         r[k] = g.get_residual()
     want = [a + (b - c) for a, b, c in zip(r["m"], r["only"], r["none"])]
     assert rel_err(r["twice"], want) < 1e-12
+
+
+@pytest.mark.parametrize("n", [223, 224])
+def test_fp32_edges_on_both_sides_of_their_own_launch(n):
+    """p = 4 in FP32: 99 458 elements take the edges in the element launch, 100 352 in one of
+    their own, against the FP64 residual."""
+    print(f"fp32 edges n={n}", flush=True)
+    from hpmp import mesh as M, workloads as W
+    from hpmp.tri_hp import TriHpIns
+    m = M.unit_square(n, 0.2, 3, essential_mask=0)
+    st = W.noisy_freestream(m, 4, seed=n, scale=0.3)
+    g = TriHpIns(m, log2p=2, mu=1e-2)
+    g.set_edge_flux([2] * m.nebd, (1.0, 0.1, 0.2))
+    g.set_state(*st)
+    g.rsdl()
+    r, f = g.get_residual(), g.residual_fp32()
+    b = np.unique(m.ebdry_seg)
+    # FP32 element residual: about 200 roundings of terms of the residual's size
+    assert rel_err([f[1][b]], [r[1][b]]) < 200 * 2.0 ** -23
+    assert rel_err(f, r) < 200 * 2.0 ** -23
