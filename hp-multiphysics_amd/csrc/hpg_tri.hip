@@ -178,11 +178,11 @@ struct Level {
 };
 
 // cns operator pack of one level: P, Pr, Ps as [mode][32], Dr, Ds as [point'][32],
-// Ir, Is, I as [point][16], zero padded
+// Ir, Is as [point][16], zero padded
 std::vector<double> build_cns_pack(const TriOps& o) {
     const int tm = o.tm, G = o.G;
     const int OP_PR = tm * 32, OP_PS = 2 * tm * 32, OP_DR = 3 * tm * 32, OP_DS = OP_DR + G * 32;
-    const int OP_IR = OP_DS + G * 32, OP_IS = OP_IR + G * 16, OP_I = OP_IS + G * 16, SIZE = OP_I + G * 16;
+    const int OP_IR = OP_DS + G * 32, OP_IS = OP_IR + G * 16, SIZE = OP_IS + G * 16;
     std::vector<double> pk(SIZE, 0.0);
     for (int k = 0; k < tm; ++k)
         for (int g = 0; g < G; ++g) {
@@ -199,7 +199,6 @@ std::vector<double> build_cns_pack(const TriOps& o) {
         for (int k = 0; k < tm; ++k) {
             pk[OP_IR + q * 16 + k] = o.Ir[k * G + q];
             pk[OP_IS + q * 16 + k] = o.Is[k * G + q];
-            pk[OP_I + q * 16 + k] = o.I[k * G + q];
         }
     return pk;
 }

@@ -305,8 +305,8 @@ __global__ __launch_bounds__(256) void k_elem_tet32(TetElemArgs32 a, int noct) {
 // ---------------------------------------------------------------------------------
 // Matrix-core form of the FP32 element residual (p = 2, the inner solve of the defect
 // correction): 16 tetrahedra per wave64, every transform a contraction on
-// v_mfma_f32_16x16x4f32 with the layout of the tri kernels: columns are the wave's 16 elements, rows Gauss points (27 in two 16-row
-// tiles) or modes (10 in one tile), A operands lane-ready from LDS, B operands the
+// v_mfma_f32_16x16x4f32 with the layout of the tri kernels: columns are the wave's 16
+// elements, rows Gauss points (27 in two 16-row tiles) or modes (10 in one tile), A operands lane-ready from LDS, B operands the
 // accumulator registers of the previous contraction (register i of lane l holds row
 // 4 (l / 16) + i of its tile, which is the B operand of K-step 4 tile + i when the
 // operator's K index is laid out that way).  Point fluxes are formed in the lane that
@@ -331,8 +331,9 @@ struct TMDims {
 // steady, tau frozen by setup_preconditioner; writes lf like elem_tet_body.  ngrp
 // groups of 16 elements; the grid is a multiple of 8 blocks and XCD x walks the
 // contiguous group range [x * gpx, (x + 1) * gpx) (neighbouring elements share its L2)
-template <typename T, int P, bool FULL>
-__device__ __forceinline__ void elem_tet_mfma_body(const TetElemArgsT<T>& a, int ngrp) {
+template <int P, bool FULL>
+__device__ __forceinline__ void elem_tet_mfma_body(const TetElemArgs32& a, int ngrp) {
+    using T = float;
     using D = TDims<P>;
     using M = TMDims<P>;
     using V4 = typename Vec4<T>::type;
@@ -444,7 +445,7 @@ __device__ __forceinline__ void elem_tet_mfma_body(const TetElemArgsT<T>& a, int
                         L2 = mfma(ad, cv[2][dd], L2); L3 = mfma(ad, c3[dd], L3);
                     }
                 }
-            // register i holds mode 4 i + l / 16 (f64) or 4 (l / 16) + i (f32) of element e
+            // register i holds mode 4 (l / 16) + i of element e
             constexpr int REC = FULL ? 2 * TNV : TNV;
             double* lfo = a.lf + (size_t)tt * (REC * TM);
 #pragma unroll
@@ -574,7 +575,7 @@ __device__ __forceinline__ void elem_tet_mfma_body(const TetElemArgsT<T>& a, int
 
 // ---------------------------------------------------------------------------------
 // FP64 form at p = 2: 16 tetrahedra per wave64 on v_mfma_f64_4x4x4f64 (lane l: element
-// l % 16; operands' K index and results' row l / 16; 4 cycles a step against 16 for the
+// l % 16; operands' K index and results' row l / 16; 16 cycles a step against 64 for the
 // 16x16x4 form, the same rate per product), so that a contraction pays for its products in
 // tiles of 4 x 4 and not of 16 x 4.  FP64 vector and matrix instructions share one unit at
 // one rate, and the kernel is bound by it: what counts is the number of products.
@@ -953,7 +954,7 @@ __global__ __launch_bounds__(256, FULL ? 2 : 3) void k_elem_tet_mfma(TetElemArgs
 // FP32 arithmetic (the inner solve of the defect correction) on v_mfma_f32_16x16x4f32
 template <int P, bool FULL>
 __global__ __launch_bounds__(256, 2) void k_elem_tet32_mfma(TetElemArgs32 a, int ngrp) {
-    elem_tet_mfma_body<float, P, FULL>(a, ngrp);
+    elem_tet_mfma_body<P, FULL>(a, ngrp);
 }
 
 // inflow face flux, continuity only (tet_hp/ins/bdry.cpp:59-102, bdry_ins.h:122-134):

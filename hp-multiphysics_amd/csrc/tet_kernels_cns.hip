@@ -365,7 +365,8 @@ struct TetcElemArgsT {
     const double* ugv;
     const double* uge;
     const double* tau;  // ntet x 25
-    double* lf;         // ntet x TM x 2 x 5: [t][m][0 = imaginary, 1 = real][n]
+    double* lf;         // ntet x TM x 2 x 5: [t][m][0 = imaginary, 1 = real][n]; without viscous
+                        // terms (FULL = false) ntet x TM x 5, the imaginary part only
     const T* ops;
     double mu, kcond, R, gamma, atm, beta, gogm1;  // gogm1: gamma / (gamma - 1), read by the FP64 matrix-core form
 };
@@ -621,8 +622,9 @@ __global__ __launch_bounds__(256) void k_elem_tetc32(TetcElemArgs32 a, int noct)
 // the lane that holds the point.  The element tau (5 x 5) sits in LDS per wave.
 // Padding points and padding elements carry p = RT = 1 so that rho = (p + atm) / RT
 // stays finite (a zero operator column does not cancel an inf in a matrix product).
-template <typename T, int P, bool FULL>
-__device__ __forceinline__ void elem_tetc_mfma_body(const TetcElemArgsT<T>& a, int ngrp) {
+template <int P, bool FULL>
+__device__ __forceinline__ void elem_tetc_mfma_body(const TetcElemArgs32& a, int ngrp) {
+    using T = float;
     using D = TDims<P>;
     using M = TMDims<P>;
     using V4 = typename Vec4<T>::type;
@@ -1253,7 +1255,7 @@ __global__ __launch_bounds__(256, 2) void k_elem_tetc_mfma(TetcElemArgs a, TetLi
 
 template <int P, bool FULL>
 __global__ __launch_bounds__(256) void k_elem_tetc32_mfma(TetcElemArgs32 a, int ngrp) {
-    elem_tetc_mfma_body<float, P, FULL>(a, ngrp);
+    elem_tetc_mfma_body<P, FULL>(a, ngrp);
 }
 
 // inflow face flux (tet_hp/cns/bdry.cpp:58-104, 129-150): pressure from the solution,

