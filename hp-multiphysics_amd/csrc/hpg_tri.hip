@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
 #include <memory>
 #include <string>
@@ -2224,12 +2225,14 @@ __global__ void k_clear_flags(FlagList f) {
 }
 }  // namespace
 
-// 1 when hpg_mg_cycle runs in this process: the HIP runtime that the library is bound to is
-// at least the release it was compiled for.  A process that loads a package with an older
-// runtime of its own first binds the library to that one; a W cycle of 256 x 256 squares on
-// 5 meshes ended there (7.0 under 7.2) in a segmentation fault on the host whose cause is
-// not known, so the whole-cycle call is refused; the call-by-call cycle runs there.
+// 1 when hpg_mg_cycle runs in this process.  Whole W cycles of 256 x 256 squares on 5 meshes
+// and of 512 x 512 on 6 ended in a segmentation fault on the host, inside the runtime, whose
+// cause is not known: the first on a HIP runtime older than the release that the library was
+// compiled for (7.0 under 7.2: a package with a runtime of its own was loaded before it), the
+// second under rocprofv3, which names its tools in ROCP_TOOL_LIBRARIES.  There the whole-cycle
+// call is refused; the call-by-call cycle runs.
 int hpg_cycle_available(void) {
+    if (std::getenv("ROCP_TOOL_LIBRARIES")) return 0;
     int v = 0;
     return hipRuntimeGetVersion(&v) == hipSuccess && v / 100000 >= HIP_VERSION / 100000;  // major, minor
 }
@@ -2247,8 +2250,8 @@ int hpg_mg_cycle(hpg_ctx* const* grids, int ngrid, int extra_finest_levels, int 
     if (f->log2p != f->log2pmax || extra_finest_levels > f->log2pmax) { f->err = "cycle starts on the finest p-level"; return -2; }
     if (ngrid > 16) { f->err = "at most 16 meshes in a cycle"; return -2; }
     if (!hpg_cycle_available()) {
-        f->err = "the whole-cycle call needs the HIP runtime that the library was built for; another package's older one "
-                 "was loaded first";
+        f->err = "the whole-cycle call is off under a profiler and on a HIP runtime older than the library's build (one "
+                 "that another package loaded first)";
         return -2;
     }
     int nerr = 0;

@@ -16,8 +16,8 @@ from . import mesh as M
 
 def fused_available(grids) -> bool:
     """True when every grid is a GPU tri context and hpg_mg_cycle runs in this process (it
-    does not on an older HIP runtime of another package, torch's for one, that was loaded
-    before the library)."""
+    does not under rocprofv3, and on an older HIP runtime of another package, torch's for
+    one, that was loaded before the library)."""
     from . import _lib
     from .tri_hp import TriHpIns
     return all(isinstance(g, TriHpIns) for g in grids) and bool(_lib.load().hpg_cycle_available())
@@ -39,8 +39,8 @@ def cycle(grids, extra_finest_levels: int, vw: int = 1, itercrsn: int = 1, iterr
     if lvl == 0 and mglvls is None and evaluate_preconditioner and fused is not False and fused_available(grids):
         return grids[0].mg_cycle(grids, extra_finest_levels, vw, itercrsn, iterrfne)
     if fused:
-        raise ValueError("the fused cycle needs GPU tri contexts, the HIP runtime that the library was built for, the "
-                         "entry level and evaluate_preconditioner")
+        raise ValueError("the fused cycle needs GPU tri contexts, the HIP runtime that the library was built for, no "
+                         "profiler, the entry level and evaluate_preconditioner")
     ngrid = len(grids)
     if mglvls is None:
         mglvls = ngrid + extra_finest_levels

@@ -133,10 +133,10 @@ int hpg_link_fine(hpg_ctx *coarse, hpg_ctx *fine, const int *cc_tri, const doubl
  * with the same kernels and arguments as the enqueued form. */
 int hpg_mg_cycle(hpg_ctx *const *grids, int ngrid, int extra_finest_levels, int vw, int itercrsn, int iterrfne,
                  double *maxres);
-/* No reference counterpart: 1 when hpg_mg_cycle runs in this process, 0 when the process
- * has bound the library to a HIP runtime older than the release it was compiled for (a
- * package that brings its own runtime was loaded first); hpg_mg_cycle then returns -2, and
- * the cycle is driven call by call. */
+/* No reference counterpart: 1 when hpg_mg_cycle runs in this process, 0 under rocprofv3
+ * (ROCP_TOOL_LIBRARIES set) and when the process has bound the library to a HIP runtime older
+ * than the release it was compiled for (a package that brings its own runtime was loaded
+ * first); hpg_mg_cycle then returns -2, and the cycle is driven call by call. */
 int hpg_cycle_available(void);
 /* No reference counterpart: enable (default) or disable the graph capture of
  * hpg_mg_cycle on this fine context (disabled: every cycle is enqueued call by call). */
@@ -162,7 +162,10 @@ int hpg_get_log2p(hpg_ctx *ctx, int *log2p);
  * in FP64.  F(fl32(u0) + d) ~ R64(u0)/c + J(u0) d, so the inner solve approximates
  * the defect equation for the scaled correction d = delta / c; c keeps |d| near
  * 1e-3 |u0|, where FP32 residual differences resolve J(u0) d.  Coarse p-levels stay
- * FP64.  The FP64 residual stays the judge, so the converged solution is FP64's. */
+ * FP64.  The FP64 residual stays the judge, so the converged solution is FP64's.  It is
+ * the faster mode for ins (0.88 of the FP64 step at 512 x 512, p = 4) and the slower one
+ * for cns (1.3 times the step at 724 x 724, p = 4) and, with hpg_tet_set_precision, for
+ * tetrahedra (1.2 times at 64^3, p = 2), whose FP32 kernels keep their order of operations. */
 int hpg_set_precision(hpg_ctx *ctx, int mode);
 int hpg_set_preconditioner(hpg_ctx *ctx, int mode);
 int hpg_set_defect_inner(hpg_ctx *ctx, int ninner);

@@ -1,5 +1,7 @@
 """The whole-cycle call runs on the HIP runtime that the library was built for, and is neither
-taken by default nor entered on an older one that another package loaded before it."""
+taken by default nor entered on an older one that another package loaded before it, nor under
+a profiler."""
+import os
 import subprocess
 import sys
 
@@ -10,21 +12,27 @@ CODE = """
 import sys
 sys.path.insert(0, {path!r})
 from hpmp import _lib, multigrid
+_lib.load()
+{then}
 print(_lib.load().hpg_cycle_available(), multigrid.fused_available([]))
 """
 
 
-def _run(first):
+def _run(first, then=""):
     import hpmp
-    import os
     path = os.path.dirname(os.path.dirname(os.path.abspath(hpmp.__file__)))
-    r = subprocess.run([sys.executable, "-c", CODE.format(first=first, path=path)], capture_output=True, text=True,
+    r = subprocess.run([sys.executable, "-c", CODE.format(first=first, path=path, then=then)], capture_output=True, text=True,
                        check=True, timeout=300)
     return r.stdout.split()
 
 
 def test_cycle_on_the_runtime_of_the_build():
     assert _run("") == ["1", "True"]
+
+
+def test_no_cycle_under_a_profiler():
+    # set after the runtime is loaded, which would look for the tool
+    assert _run("", "import os; os.environ['ROCP_TOOL_LIBRARIES'] = 'tool'") == ["0", "False"]
 
 
 def test_no_cycle_on_an_older_runtime_loaded_first():
