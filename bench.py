@@ -141,7 +141,7 @@ def cns_throughput(args) -> dict:
            "unknowns": unknowns, "steps": args.cns_steps,
            "ms_per_step": 1e3 * (t1 - t0) / args.cns_steps,
            "dof_evals_per_s": unknowns * 5 * args.cns_steps / (t1 - t0),
-           "roofline": {"bound": "fp64 valu", "kernel": "k_elem_cns<4,full>", "achieved": ach,
+           "roofline": {"bound": "mfma", "kernel": "k_elem_cns<4,full>", "achieved": ach,
                         "peak": MI355X_FP64_MFMA_TFLOPS, "unit": "TFLOP/s", "frac": ach / MI355X_FP64_MFMA_TFLOPS,
                         "avg_launch_ms": tot.value / max(1, nl.value),
                         "elements_per_launch": ne.value / max(1, nl.value), "flop_per_element": FLOP_CNS_FULL_P4}}
@@ -374,8 +374,9 @@ def time_to_tol(args, sols) -> dict:
 
 def cycles_only(args) -> int:
     """Exactly `--cycles-only` W(2,2,2) cycles of the mu = 1e-3 workload (FP64 plain, reference
-    CFL, hierarchy down to 16 x 16), one JSON line with the time per cycle: the run the
-    W-cycle kernel profile is taken from."""
+    CFL, hierarchy down to 16 x 16), one JSON line with the time per cycle: the run a
+    W-cycle kernel profile is taken from (call by call there: the whole-cycle call is off
+    under a profiler)."""
     from hpmp import multigrid as MG
     n = args.tts_n
     ngrid = args.tts_ngrid or max(1, int(np.log2(n // 16)) + 1)

@@ -18,10 +18,13 @@ namespace {
 constexpr int THREADS = 8, HALVES = 2, POOL_SLOTS = 4, MAX_SEG = 4;
 constexpr size_t CHUNK = size_t(1) << 20;                  // staging unit of a large copy
 constexpr size_t SLOT_BYTES = CHUNK * THREADS * HALVES;    // 16 MiB
-// Measured (us; fresh: into pages never touched): 64 KB to the device 16 staged, 36 direct, to
-// the host 27 and 50; 512 KB 38 and 35, 114 and 108; 4 MB to fresh host pages 925 with two
-// threads, 1 109 direct; 64 MB 4 855 with eight, 16 934 direct.  To the device the direct
-// copy is never slower above 256 KB (2 MB: 81 against 95).
+// Measured, staged / direct, us.  To the device (a host array new to the runtime takes what a
+// repeated one does, within 6 us up to 1 MB and 4 % above): 64 KB 14 / 34, 128 KB 16 / 60,
+// 256 KB 20 / 16, 512 KB 28 / 27, 2 MB 96 / 79, 16 MB 571 / 460: direct from 256 KB up.  To
+// the host, into pages touched before: 64 KB 14 / 36, 256 KB 22 / 19, 1 MB 61 / 64, with the
+// threads 2 MB 126 / 127, 4 MB 224 / 251, 64 MB 2 256 / 3 910; into pages never touched (the
+// page faults cost more than the copy): 64 KB 23 / 45, 256 KB 54 / 52, 1 MB 242 / 236, with
+// the threads 2 MB 349 / 471, 4 MB 445 / 967, 64 MB 3 681 / 15 161.
 constexpr size_t SMALL = size_t(1) << 18;
 constexpr size_t LARGE = size_t(2) << 20;
 

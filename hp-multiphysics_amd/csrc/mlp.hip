@@ -177,9 +177,12 @@ __global__ void k_mfma_probe_bf16(const float* A, const float* B, float* out) {
 //            columns, so h and dz go through a transposed copy in LDS (row = unit, 16
 //            samples, padded to 20 words: a lane's four samples are one 16-byte read, no
 //            bank conflicts); v_mfma_f32_16x16x4f32 again.
-// Bound: the FP32 matrix cores (304 instructions of 32 cycles per tile) and, near it, the
-// 48 tanh per lane.  65 536 samples: 1 903 us for the sample-per-lane form with a
-// reduction per parameter before it, 98 us now.
+// A minibatch takes 48 us (the weights and fragments built in LDS from scattered loads, the
+// block sums, 8 us of the update kernel) and 13 us for each tile of a wave: 65 536 samples,
+// four tiles a wave, 100 us (1 903 us for the sample-per-lane form with a reduction per
+// parameter before it).  Of a tile's 13 us the FP32 matrix instructions are 4 (304 of 32
+// cycles); the rest is the 48 tanh a lane and one wave per SIMD (all 512 registers, 108 bytes
+// a lane in scratch) between the LDS round trips of its phases.
 typedef float f4_t __attribute__((ext_vector_type(4)));
 
 __device__ inline f4_t mfma_f32(float a, float b, f4_t c) {

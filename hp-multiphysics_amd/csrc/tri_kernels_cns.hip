@@ -723,7 +723,7 @@ __device__ __forceinline__ void edge_cns_body(const CnsEdgeArgs& a, int idx) {
 
 // The element launch (persistent over every element in mesh order after the first eblk
 // blocks, which compute the boundary-edge fluxes).  Bound: the FP64 matrix cores and the
-// pointwise solves, one wave per SIMD.  105 800 elements, p = 4: 177 us full and 71 us
+// pointwise solves, one wave per SIMD.  105 800 elements, p = 4: 176 us full and 53 us
 // inviscid, against 7 x 114 us and 7 x 35 us for colour launches with an element per 32
 // lanes (a general 4 x 4 product and solve per point, 25 of 32 lanes in use).
 template <int P, bool FULL>
