@@ -253,6 +253,10 @@ struct hpg_ctx {
     hpg_ctx* fine = nullptr;
     bool coarse_level = false;
     hipEvent_t xev = nullptr;  // orders this context's stream against a neighbour level's
+    // library calls on this context, and those on `fine` when this context's stream last
+    // waited for its stream: mg_prolongate waits again if there were more since (an event and
+    // a wait at every prolongation cost a call-by-call W cycle 4 %)
+    long calls = 0, fine_calls = 0;
     int *hr_ptr = nullptr, *hr_fidx = nullptr, *hi_fv = nullptr, *hp_cv = nullptr;
     double *hr_wt = nullptr, *hi_wt = nullptr, *hp_wt = nullptr, *vug_frst = nullptr;
     DeviceArrays arrays;
@@ -398,8 +402,12 @@ struct hpg_ctx {
     }
 };
 
+template <class Ctx>
+static void count_call(Ctx*) {}
+static void count_call(hpg_ctx* c) { ++c->calls; }
 #define HPG_TRY(ctx, ...)                                                      \
     try {                                                                      \
+        count_call(ctx);                                                       \
         __VA_ARGS__;                                                           \
     } catch (const std::exception& ex) {                                       \
         if (ctx) (ctx)->err = ex.what();                                       \
@@ -2086,14 +2094,21 @@ int hpg_link_fine(hpg_ctx* c, hpg_ctx* f, const int* cc_tri, const double* cc_wt
     return 0;
 }
 
+// this context's stream goes on after everything enqueued on the fine context's so far
+static void wait_for_fine(hpg_ctx* c) {
+    hpg_ctx* f = c->fine;
+    check(hipEventRecord(f->xev, f->stream), "hipEventRecord");
+    check(hipStreamWaitEvent(c->stream, f->xev, 0), "hipStreamWaitEvent");
+    c->fine_calls = f->calls;
+}
+
 int hpg_mg_restrict(hpg_ctx* c) {
     if (!c) return -2;
     if (c->coarse_level) {
         // tri_hp/movco.cpp:41-102: fine residual and state onto this coarse mesh
         HPG_TRY(c, {
             hpg_ctx* f = c->fine;
-            check(hipEventRecord(f->xev, f->stream), "hipEventRecord");
-            check(hipStreamWaitEvent(c->stream, f->xev, 0), "hipStreamWaitEvent");
+            wait_for_fine(c);
             c->isfrst = true;
             c->coarse_flag = true;
             if (c->nv == NVC) {
@@ -2129,6 +2144,8 @@ int hpg_mg_prolongate(hpg_ctx* c) {
         HPG_TRY(c, {
             hpg_ctx* f = c->fine;
             const long n = (long)c->npnt * c->nv;
+            // the fine state and residual are changed here: after what f's stream still holds
+            if (c->fine_calls != f->calls) wait_for_fine(c);
             hipLaunchKernelGGL(k_hcorr, dim3(nblk(n)), dim3(256), 0, c->stream, n, c->vug_frst, c->ugv);
             if (c->nv == NVC)
                 hipLaunchKernelGGL(k_hprolong<NVC>, dim3(nblk(f->npnt)), dim3(256), 0, c->stream, f->npnt, c->hp_cv,

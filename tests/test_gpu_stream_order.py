@@ -35,6 +35,35 @@ def test_upload_to_the_fine_mesh_between_restriction_and_prolongation(oracle_mod
     assert not np.array_equal(out[0][0], st[0])  # the correction is not zero
 
 
+@pytest.mark.parametrize("physics", ["ins", "cns"])
+def test_update_of_the_fine_mesh_between_restriction_and_prolongation(oracle_mod, physics):
+    """The correction is added to the fine state that the updates leave."""
+    _case(f"fine updates, mg_prolongate {physics} 32x32 -> 16x16 p=2")
+    _, (G, Gc), _ = _stacks(oracle_mod, physics, 32, 1, 2)
+    if physics == "cns":
+        # the explicit compressible relaxation stays admissible at CFL ~ (8 h)^2 / p^3 0.01
+        for x in (G, Gc):
+            x.set_cfl([0.01 / 16 / 8] * 4)
+    base = G.get_state()
+    out = []
+    for wait in (False, True):
+        G.set_state(*base)
+        assert G.setup_preconditioner() == 0
+        G.rsdl()
+        Gc.mg_restrict()
+        assert Gc.setup_preconditioner() == 0
+        Gc.update()
+        Gc.synchronize()
+        for _ in range(20):
+            G.update()
+        if wait:
+            G.synchronize()
+        Gc.mg_prolongate()
+        out.append([*G.get_state(), *G.get_residual()])
+    for a, b in zip(*out):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
 def test_upload_to_a_coarse_mesh_before_a_replayed_cycle(oracle_mod):
     """A replayed cycle runs on the fine stream and overwrites the coarse states: an upload to
     a coarse context just before it lands before it."""
